@@ -416,7 +416,8 @@ class Neighbours:
         return self.out
 
     def __del__(self):
-        self.L.pth_gtree_free(self.h)
+        if self.ctx.handle:  # (at interpreter exit the contexts are closed first)
+            self.L.pth_gtree_free(self.h)
 
 
 class Evaluation:
