@@ -1149,38 +1149,19 @@ int pth_resident_results(pth_resident *r, double *acc, double *pot, long long *n
     if (!r) return PTH_ERR_ARG;
     pth_ctx *c = r->ctx;
     if (!r->ran) return c->fail(PTH_ERR_STATE, "pth_resident_results: no evaluation run");
-    int rc = pth_resident_sync(r);
-    if (rc) return rc;
+    HIPCHK(c, hipSetDevice(c->device), "hipSetDevice");
     const long long n = r->plan.ni_tot;
-    std::vector<double4> a(std::max<long long>(n, 1));
-    std::vector<int> nb(std::max<long long>(n, 1));
-    if (n > 0) {
-        HIPCHK(c, hipMemcpy(a.data(), r->out_accp.p, sizeof(double4) * n, hipMemcpyDeviceToHost), "result download");
-        HIPCHK(c, hipMemcpy(nb.data(), r->out_nnb.p, sizeof(int) * n, hipMemcpyDeviceToHost), "result download");
-    }
-    if (r->co) {
-        const int nw = (int)r->plan.walks.size();
-        std::vector<int> err(std::max(nw, 1));
-        if (nw > 0)
-            HIPCHK(c, hipMemcpy(err.data(), r->work.walk_err.p, sizeof(int) * nw, hipMemcpyDeviceToHost),
-                   "result download");
-        for (int w = 0; w < nw; w++)
-            if (err[w])
-                return c->fail(PTH_ERR_ARG, "pth_resident_results: changeover mode: an i-particle of walk " +
-                                                std::to_string(w) + " has no EPJ with its id in the walk's list");
-        if (pot_tot && n > 0)
-            HIPCHK(c, hipMemcpy(pot_tot, r->out_pott.p, sizeof(double) * n, hipMemcpyDeviceToHost),
-                   "result download");
-    }
-    for (long long i = 0; i < n; i++) {
-        if (acc) {
-            acc[3 * i] = a[i].x;
-            acc[3 * i + 1] = a[i].y;
-            acc[3 * i + 2] = a[i].z;
-        }
-        if (pot) pot[i] = a[i].w;
-        if (nnb) nnb[i] = nb[i];
-    }
+    const int nw = r->co ? (int)r->plan.walks.size() : 0;
+    int bad = -1;
+    const hipError_t e =
+        results_to_host(c->stream, r->ring, r->out_accp.as<double4>(), r->out_nnb.as<int>(),
+                        r->co ? r->out_pott.as<double>() : nullptr, n, acc, pot, nnb, pot_tot,
+                        nw > 0 ? r->work.walk_err.as<int>() : nullptr, nw, &bad);
+    HIPCHK(c, e, "result download");
+    if (bad >= 0)
+        return c->fail(PTH_ERR_ARG, "pth_resident_results: changeover mode: an i-particle of walk " +
+                                        std::to_string(bad) + " has no EPJ with its id in the walk's list");
+    HIPCHK(c, hipGetLastError(), "kernel execution");
     return PTH_OK;
 }
 
@@ -1309,6 +1290,7 @@ void pth_resident_free(pth_resident *r)
     r->out_pott.release();
     r->plan_dev.release();
     r->work.release();
+    r->ring.release();
     for (int k = 0; k < 4; k++)
         if (r->ev[k]) (void)hipEventDestroy(r->ev[k]);
     for (hipEvent_t x : r->side_done)
@@ -1363,6 +1345,68 @@ long long pth_plan_debug(int n_walk, const int *n_epi, const int *n_epj, const i
 }  // extern "C"
 
 namespace pth {
+
+void unpack_results(const char *src, long long n, bool co, double *acc, double *pot, long long *nnb, double *pot_tot)
+{
+    const double *a = reinterpret_cast<const double *>(src), *p = a + 3 * n, *pt = p + n;
+    const int *nb = reinterpret_cast<const int *>(co ? pt + n : pt);
+    auto part = [&](long long b, long long e) {
+        if (acc) std::memcpy(acc + 3 * b, a + 3 * b, 24 * (size_t)(e - b));
+        if (pot) std::memcpy(pot + b, p + b, 8 * (size_t)(e - b));
+        if (co && pot_tot) std::memcpy(pot_tot + b, pt + b, 8 * (size_t)(e - b));
+        if (nnb)
+            for (long long i = b; i < e; i++) nnb[i] = nb[i];
+    };
+    // the caller's arrays are often fresh memory: the copy is mostly page
+    // faults, which threads take side by side
+    const int t = (int)std::min<long long>(omp_get_max_threads(), n / 4096);
+    if (t < 2) {
+        part(0, n);
+        return;
+    }
+#pragma omp parallel for num_threads(t) schedule(static, 1)
+    for (int k = 0; k < t; k++) part(n * k / t, n * (k + 1) / t);
+}
+
+hipError_t results_to_host(hipStream_t st, ResultRing &ring, const double4 *accp, const int *out_nnb,
+                           const double *pott, long long n, double *acc, double *pot, long long *nnb, double *pot_tot,
+                           const int *err, int n_err, int *bad)
+{
+    hipError_t e;
+    const bool co = pott != nullptr;
+    const long long n_chunk = (n + RESULT_CHUNK - 1) / RESULT_CHUNK;
+    const int nb = (int)std::min<long long>(n_chunk, RESULT_RING);
+    const size_t head = err ? align256(sizeof(int) * (size_t)n_err) : 0;  // in front of buffer 0's chunk
+    auto count = [&](long long k) { return (int)std::min<long long>(RESULT_CHUNK, n - k * RESULT_CHUNK); };
+    for (int k = 0; k < nb; k++) {
+        if ((e = ring.buf[k].ensure((k ? 0 : head) + results_bytes(count(0), co)))) return e;
+        if (!ring.ev[k] && (e = hipEventCreateWithFlags(&ring.ev[k], hipEventDisableTiming))) return e;
+    }
+    auto at = [&](long long k) { return ring.buf[k % RESULT_RING].as<char>() + (k % RESULT_RING ? 0 : head); };
+    auto pack = [&](long long k) -> hipError_t {
+        const hipError_t r = launch_results(accp, out_nnb, pott, k * RESULT_CHUNK, count(k),
+                                            reinterpret_cast<double *>(at(k)), st);
+        return r ? r : hipEventRecord(ring.ev[k % RESULT_RING], st);
+    };
+    if (n <= 0) return hipStreamSynchronize(st);
+    if (err && (e = hipMemcpyAsync(ring.buf[0].p, err, sizeof(int) * (size_t)n_err, hipMemcpyDeviceToHost, st))) return e;
+    for (long long k = 0; k < nb; k++)
+        if ((e = pack(k))) return e;
+    for (long long k = 0; k < n_chunk; k++) {
+        if ((e = hipEventSynchronize(ring.ev[k % RESULT_RING]))) return e;
+        if (k == 0 && err)
+            for (int w = 0; w < n_err; w++)
+                if (ring.buf[0].as<int>()[w]) {
+                    *bad = w;
+                    return hipStreamSynchronize(st);
+                }
+        const long long i0 = k * RESULT_CHUNK;
+        unpack_results(at(k), count(k), co, acc ? acc + 3 * i0 : nullptr, pot ? pot + i0 : nullptr,
+                       nnb ? nnb + i0 : nullptr, pot_tot ? pot_tot + i0 : nullptr);
+        if (k + RESULT_RING < n_chunk && (e = pack(k + RESULT_RING))) return e;
+    }
+    return hipSuccess;
+}
 
 int resident_setup(pth_resident *r, int n_walk, const int *n_epi, const int *n_epj, const int *n_spj,
                    long long n_ide, long long n_ids, int n_epj_tot, int n_spj_tot, const char *who, Plan *pre,

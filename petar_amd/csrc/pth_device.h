@@ -193,6 +193,12 @@ hipError_t launch_stage(const BatchDev &b, int k, hipStream_t st);
 // classes: bit c set launches the items of i-per-lane class c + 1
 hipError_t launch_force(const BatchDev &b, int k, hipStream_t st, unsigned classes = 0xFu);
 hipError_t launch_reduce(const BatchDev &b, int k, hipStream_t st);
+// Results of particles [i0, i0 + n) as packed arrays acc [n][3], pot [n],
+// pot_tot [n] (when pott is not null) and nnb [n] at dst (pinned host memory),
+// in that order; results_bytes(n, co) long.
+hipError_t launch_results(const double4 *accp, const int *nnb, const double *pott, long long i0, int n, double *dst,
+                          hipStream_t st);
+constexpr size_t results_bytes(long long n, bool co) { return (size_t)n * (co ? 44 : 36); }
 // All segments of a batch in order on one stream.
 hipError_t launch_all(const BatchDev &b, hipStream_t st);
 

@@ -1096,6 +1096,26 @@ __global__ __launch_bounds__(256) void k_reduce(const RItem *__restrict__ ritems
 }
 
 // ---------------------------------------------------------------------------
+// Results [i0, i0 + n) packed for the host: consecutive threads write
+// consecutive words, so that the stores to host memory leave as whole lines
+// (the {ax, ay, az, pot} records are read from L2 at a stride instead).
+__global__ __launch_bounds__(256) void k_results(const double4 *__restrict__ accp, const int *__restrict__ nnb,
+                                                 const double *__restrict__ pott, long long i0, int n,
+                                                 double *__restrict__ dst)
+{
+    const double *in = reinterpret_cast<const double *>(accp + i0);
+    double *pot = dst + 3 * (size_t)n, *pt = pot + n;
+    int *nb = reinterpret_cast<int *>(pott ? pt + n : pt);
+    const int step = (int)(gridDim.x * 256), t0 = (int)(blockIdx.x * 256 + threadIdx.x);
+    for (int k = t0; k < 3 * n; k += step) dst[k] = in[4 * (k / 3) + k % 3];
+    for (int k = t0; k < n; k += step) {
+        pot[k] = in[4 * (size_t)k + 3];
+        if (pott) pt[k] = pott[i0 + k];
+        nb[k] = nnb[i0 + k];
+    }
+}
+
+// ---------------------------------------------------------------------------
 // index lists sent as runs (pth_dispatch): workgroup g expands part
 // g / (2 n_walk) of n_part of the EPJ list (g % (2 n_walk) < n_walk) or the
 // SPJ list of one walk.  The part's first run is found by a binary search
@@ -1355,6 +1375,15 @@ hipError_t launch_reduce(const BatchDev &b, int k, hipStream_t st)
     else
         hipLaunchKernelGGL(k_reduce<false>, dim3((unsigned)g.n_ritems), dim3(256), 0, st, ri, b.part_accp,
                            b.part_nnb, b.part_pott, b.G, b.out_accp, b.out_nnb, b.out_pott);
+    return hipGetLastError();
+}
+
+hipError_t launch_results(const double4 *accp, const int *nnb, const double *pott, long long i0, int n, double *dst,
+                          hipStream_t st)
+{
+    if (n <= 0) return hipSuccess;
+    const unsigned nblk = (unsigned)std::min(512, (n + 255) / 256);
+    hipLaunchKernelGGL(k_results, dim3(nblk), dim3(256), 0, st, accp, nnb, pott, i0, n, dst);
     return hipGetLastError();
 }
 

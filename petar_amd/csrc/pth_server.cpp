@@ -189,6 +189,7 @@ struct pth_server {
     hipStream_t cap = nullptr;   // graph capture
     hipStream_t xfer = nullptr;  // result copies (evictions, pth_server_results)
     hipEvent_t ev_evicted = nullptr;  // the latest eviction copy
+    ResultRing ring;             // of pth_server_results
     long long n_evict_copies = 0;
     long long gen_clock = 0;     // placements of cluster ranges and scratch ranges
     std::mutex mu;
@@ -884,18 +885,14 @@ int pth_server_results(pth_server *s, int k, double *acc, double *pot, long long
     if (c.off >= 0) {
         // resident: its last request has completed; copy the outputs now
         // (the worker is held off by the lock meanwhile)
-        if (n > 0) {
-            const char *base = s->pool.as<char>() + c.off;
-            HIPCHK(s->ctx, hipMemcpyAsync(c.h_accp.p, base + c.L.out_accp, sizeof(double4) * n,
-                                          hipMemcpyDeviceToHost, s->xfer), "result download");
-            HIPCHK(s->ctx, hipMemcpyAsync(c.h_nnb.p, base + c.L.out_nnb, sizeof(int) * n, hipMemcpyDeviceToHost,
-                                          s->xfer), "result download");
-            HIPCHK(s->ctx, hipStreamSynchronize(s->xfer), "result download");
-        }
-    } else {
-        if (!c.saved_valid) return s->ctx->fail(PTH_ERR_STATE, "pth_server_results: results not kept");
-        HIPCHK(s->ctx, hipEventSynchronize(c.saved), "result download");
+        const char *base = s->pool.as<char>() + c.off;
+        HIPCHK(s->ctx, results_to_host(s->xfer, s->ring, reinterpret_cast<const double4 *>(base + c.L.out_accp),
+                                       reinterpret_cast<const int *>(base + c.L.out_nnb), nullptr, n, acc, pot, nnb,
+                                       nullptr), "result download");
+        return PTH_OK;
     }
+    if (!c.saved_valid) return s->ctx->fail(PTH_ERR_STATE, "pth_server_results: results not kept");
+    HIPCHK(s->ctx, hipEventSynchronize(c.saved), "result download");
     const double4 *a = c.h_accp.as<double4>();
     const int *nb = c.h_nnb.as<int>();
     for (long long i = 0; i < n; i++) {
@@ -966,6 +963,7 @@ void pth_server_free(pth_server *s)
     if (s->cap) (void)hipStreamDestroy(s->cap);
     if (s->xfer) (void)hipStreamDestroy(s->xfer);
     s->pool.release();
+    s->ring.release();
     if (s->pctx) pth_destroy(s->pctx);
     delete s;
 }

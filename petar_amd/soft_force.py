@@ -533,12 +533,12 @@ class Resident:
 
     def results(self):
         """acc [ni, 3], pot [ni], nnb [ni] (+ pot_tot [ni] in changeover mode)."""
-        acc = np.zeros((self.ni, 3))
-        pot = np.zeros(self.ni)
-        nnb = np.zeros(self.ni, np.int64)
-        pt = np.zeros(self.ni)
+        acc = np.empty((self.ni, 3))
+        pot = np.empty(self.ni)
+        nnb = np.empty(self.ni, np.int64)
+        pt = np.empty(self.ni if self.co else 0)
         self.ctx.check(lib().pth_resident_results(self._h, _ptr(acc, C.c_double), _ptr(pot, C.c_double),
-                                                  _ptr(nnb, C.c_longlong), _ptr(pt, C.c_double)),
+                                                  _ptr(nnb, C.c_longlong), _ptr(pt, C.c_double) if self.co else None),
                        "pth_resident_results")
         return (acc, pot, nnb, pt) if self.co else (acc, pot, nnb)
 
@@ -820,7 +820,7 @@ class Server:
 
     def results(self, cluster):
         n = self._ni[cluster]
-        acc, pot, nnb = np.zeros((n, 3)), np.zeros(n), np.zeros(n, np.int64)
+        acc, pot, nnb = np.empty((n, 3)), np.empty(n), np.empty(n, np.int64)
         self.ctx.check(lib().pth_server_results(self._h, cluster, _ptr(acc, C.c_double), _ptr(pot, C.c_double),
                                                 _ptr(nnb, C.c_longlong)), "pth_server_results")
         return acc, pot, nnb

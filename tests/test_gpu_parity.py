@@ -752,3 +752,46 @@ def test_two_tags_in_flight_are_bit_identical(c1):
     f = np.concatenate(out)
     got = (f["acc"], f["pot"], f["n_ngb"])
     assert all(np.array_equal(x, y) for x, y in zip(want, got))
+
+
+@pytest.mark.parametrize("n", [2, 255, 65535, 65536, 65537, 3 * 65536 + 1])
+@pytest.mark.parametrize("co", [0, 1])
+def test_results_over_chunk_edges(n, co):
+    """Results reach the caller's arrays in chunks of 65,536 particles through
+    three buffers: every array of every size equals what the hooks retrieve
+    (another route for the same walks), and a call that leaves arrays out
+    fills the others alike."""
+    r_out = 1e-3  # short lists: the routes are what is compared
+    m, x, _ = host.cluster(n, "plummer", seed=n)
+    L = host.build_lists(x, m, 1.5 * r_out, theta=0.9)
+    rin, rout = np.full(n, 0.1 * r_out), np.full(n, r_out)
+    ctx = sf.Context(0, eps2=0.0, rcut2=r_out ** 2, changeover=co)
+    r = sf.Resident.from_lists(ctx, L, rin, rout)
+    r.run()
+    got = r.results()
+    acc, nnb = np.full((n, 3), np.nan), np.full(n, -1, np.int64)
+    ctx.check(sf.lib().pth_resident_results(r._h, acc.ctypes.data_as(sf.C.POINTER(sf.C.c_double)), None,
+                                            nnb.ctypes.data_as(sf.C.POINTER(sf.C.c_longlong)), None), "results")
+    assert np.array_equal(acc, got[0]) and np.array_equal(nnb, got[2])
+    r.close()
+    ctx.close()
+    f = sf.CalcForceWithLinearCutoffMultiWalk(0, 0.0, r_out ** 2, 1.0, changeover=co)
+    epj, spj = np.zeros(n, sf.EPJ_SOFT), np.zeros(len(L.spj_mass), sf.SPJ_SOFT)
+    epj["id"], epj["pos"], epj["mass"], epj["r_search"] = np.arange(n), L.epj_pos, L.epj_mass, L.epj_rs
+    epj["r_in"], epj["r_out"] = rin, rout
+    spj["pos"], spj["mass"] = L.spj_pos, L.spj_mass
+    for k, q in enumerate(("xx", "yy", "zz", "xy", "xz", "yz")):
+        spj["quad"][q] = L.spj_quad[:, k]
+    epi = np.zeros(n, sf.EPI_SOFT)
+    epi["id"], epi["pos"], epi["r_search"] = np.arange(n), L.epj_pos, L.epj_rs
+    force = np.zeros(n, sf.FORCE_SOFT_CO if co else sf.FORCE_SOFT)
+    eo, so = L.walk_offsets()
+    f(0, 0, [], [], [], [], [], [], epj, n, spj, len(spj), True)
+    for b in range(0, L.n_walk, 200):
+        ws = range(b, min(b + 200, L.n_walk))
+        own = [slice(L.epi_begin[w], L.epi_begin[w] + L.n_epi[w]) for w in ws]
+        f(0, len(ws), [epi[s] for s in own], L.n_epi[b:b + 200], [L.id_epj[eo[w]:eo[w + 1]] for w in ws],
+          L.n_epj[b:b + 200], [L.id_spj[so[w]:so[w + 1]] for w in ws], L.n_spj[b:b + 200], None, 0, None, 0, False)
+        f.retrieve(0, len(ws), L.n_epi[b:b + 200], [force[s] for s in own])
+    for k, v in zip(("acc", "pot", "n_ngb", "pot_tot"), got):
+        assert np.array_equal(force[k], v), k
