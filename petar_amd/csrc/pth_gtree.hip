@@ -6,14 +6,18 @@
 // (src/petar.hpp:894-899):
 //   1. bounding cube (FP64 min/max), 63-bit Morton keys, stable radix sort of
 //      (key, index);
-//   2. nodes level by level: a node with more than n_leaf_limit particles is
-//      split into its non-empty octants (binary search of the key ranges);
-//      the nodes of a level follow their parents' order, octants in order;
+//   2. nodes of every level at once: a cell that starts at a particle is a
+//      node when its parent holds more than n_leaf_limit particles, which a
+//      few keys around the particle decide; per-block counts of every level,
+//      one scan and a writing pass number the nodes level by level, each
+//      level in Morton order (so children follow their parents' order), with
+//      one wait for the host (the counts) in the whole build;
 //   3. moments bottom-up (mass, centre of mass, raw second moment about it,
 //      particle box and box widened by r_search), each node by one thread in
 //      the host's summation order;
 //   4. i-groups: largest cells with at most n_group_limit particles (or
-//      leaves), in Morton order;
+//      leaves), in Morton order (decided and counted with the nodes, as are
+//      the neighbour search's tiles of at most 64);
 //   5. walk: one wave per group traverses the tree with a stack in LDS,
 //      popping up to 64 nodes at a time; a node is opened when it contains
 //      the group, when the group box is closer to its centre of mass than
@@ -106,205 +110,411 @@ __global__ __launch_bounds__(256) void k_bbox(const double *__restrict__ pos, co
     }
 }
 
-__global__ __launch_bounds__(256) void k_keys(const double *__restrict__ pos, long long n, double r0, double r1,
-                                              double r2, double scale, unsigned long long *__restrict__ key,
-                                              long long *__restrict__ idx)
+// What the host reads back from a build: the root cube and the sizes.
+struct TreeMeta {
+    double root[3], scale, len, rs_max, bad;
+    int level_start[GT_MAX_LEVEL + 2];  // first node of each level, then the node count
+    int n_group, n_tile;
+};
+
+// The root cube from the nb blocks' partial boxes (the host tree's
+// expressions).
+__global__ __launch_bounds__(64) void k_root(const double *__restrict__ part, int nb, TreeMeta *__restrict__ meta)
+{
+    double v[8];
+    for (int d = 0; d < 8; d++) {
+        v[d] = d < 3 ? 1e300 : d < 6 ? -1e300 : 0.0;
+        for (int b = threadIdx.x; b < nb; b += 64) v[d] = d < 3 ? fmin(v[d], part[8 * b + d]) : fmax(v[d], part[8 * b + d]);
+        for (int off = 32; off > 0; off >>= 1) {
+            const double o = __shfl_xor(v[d], off, 64);
+            v[d] = d < 3 ? fmin(v[d], o) : fmax(v[d], o);
+        }
+    }
+    if (threadIdx.x) return;
+    double len = 0;
+    for (int d = 0; d < 3; d++) len = fmax(len, v[3 + d] - v[d]);
+    len = (len > 0) ? len * (1.0 + 1e-9) : 1.0;
+    for (int d = 0; d < 3; d++) meta->root[d] = 0.5 * (v[d] + v[3 + d]) - 0.5 * len;
+    meta->scale = (double)(1u << GT_MAX_LEVEL) / len;
+    meta->len = len;
+    meta->rs_max = v[6];
+    meta->bad = v[7];
+}
+
+__global__ __launch_bounds__(256) void k_keys(const double *__restrict__ pos, long long n,
+                                              const TreeMeta *__restrict__ meta, unsigned long long *__restrict__ key,
+                                              int *__restrict__ idx)
 {
     const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
     if (i >= n) return;
-    const double r[3] = {r0, r1, r2};
+    const double scale = meta->scale;
     unsigned long long c[3];
     for (int d = 0; d < 3; d++) {
-        const double f = (pos[3 * i + d] - r[d]) * scale;
+        const double f = (pos[3 * i + d] - meta->root[d]) * scale;
         long long v = (long long)floor(f);
         v = min(max(v, 0LL), (long long)(1u << GT_MAX_LEVEL) - 1);
         c[d] = (unsigned long long)v;
     }
     key[i] = spread3(c[0]) << 2 | spread3(c[1]) << 1 | spread3(c[2]);
-    idx[i] = i;
+    idx[i] = (int)i;
 }
 
-__global__ __launch_bounds__(256) void k_gather(long long n, const long long *__restrict__ order,
-                                                const double *__restrict__ pos, const double *__restrict__ mass,
+__global__ __launch_bounds__(256) void k_gather(long long n, const int *__restrict__ sidx,
+                                                long long *__restrict__ order, const double *__restrict__ pos, const double *__restrict__ mass,
                                                 const double *__restrict__ rs, double *__restrict__ spos,
                                                 double *__restrict__ smass, double *__restrict__ srs)
 {
     const long long k = (long long)blockIdx.x * 256 + threadIdx.x;
     if (k >= n) return;
-    const long long i = order[k];
+    const long long i = sidx[k];
+    order[k] = i;
     for (int d = 0; d < 3; d++) spos[3 * k + d] = pos[3 * i + d];
     smass[k] = mass[i];
     srs[k] = rs ? rs[i] : 0.0;
 }
 
-// octant boundaries and non-empty child count of nodes [lb, lb + nl)
-__global__ __launch_bounds__(256) void k_split_count(const GNode *__restrict__ nodes, long long lb, long long nl,
-                                                     const unsigned long long *__restrict__ key, int n_leaf_limit,
-                                                     long long *__restrict__ bnd, int *__restrict__ cnt)
+// ---- nodes ------------------------------------------------------------------
+// A cell of level l is a maximal run of equal 3l-bit key prefixes; it is a
+// node when its parent holds more than n_leaf particles (level 0: always).
+// The cells that start at particle k are those of the levels from
+// d = 1 + (levels shared with particle k - 1) on, so the nodes starting at k
+// are consecutive levels d .. e: all down to the first with at most n_leaf
+// particles, which key k + n_leaf decides, and the one of level d only if
+// its parent (which starts before k) is large enough.  So all levels come
+// from one pass over the keys, where splitting level by level took three
+// launches and a wait for the host each (bound by those: 16,384 particles,
+// 9 levels, 550 us for the tree; 176 us now, 1,048,576 particles 1.21 ms and
+// 0.56 ms).
+
+// levels on which two keys agree (21: the same key)
+__device__ __forceinline__ int common_levels(unsigned long long a, unsigned long long b)
+{
+    const unsigned long long x = a ^ b;
+    return x ? GT_MAX_LEVEL - 1 - (63 - __clzll((long long)x)) / 3 : GT_MAX_LEVEL;
+}
+
+// whether particle k's cell of level l holds more than m particles
+__device__ bool cell_holds(const unsigned long long *__restrict__ key, long long n, long long k, int l, long long m)
+{
+    const unsigned long long kk = key[k];
+    // the largest r <= m with k + r (then k - r) still in the cell
+    long long right = 0, left = 0;
+    for (long long hi = min(m, n - 1 - k); right < hi;) {
+        const long long mid = (right + hi + 1) >> 1;
+        if (common_levels(kk, key[k + mid]) >= l) right = mid;
+        else hi = mid - 1;
+    }
+    if (right >= m) return true;
+    for (long long hi = min(m - right, k); left < hi;) {
+        const long long mid = (left + hi + 1) >> 1;
+        if (common_levels(kk, key[k - mid]) >= l) left = mid;
+        else hi = mid - 1;
+    }
+    return left + right + 1 > m;
+}
+
+// The nodes starting at one particle: levels d .. e (none when e < d), and
+// the level of the group and of the tile among them (-1: none).
+struct Starts {
+    int d, e, group, tile;
+};
+__device__ Starts starts_at(const unsigned long long *__restrict__ key, long long n, long long k, long long n_leaf,
+                            long long n_group, long long n_tile)
+{
+    const unsigned long long kk = key[k];
+    Starts s{k > 0 ? common_levels(key[k - 1], kk) + 1 : 0, -1, -1, -1};
+    if (s.d > GT_MAX_LEVEL) return s;
+    auto shared = [&](long long m) { return k + m < n ? common_levels(kk, key[k + m]) : -1; };
+    const int c = shared(n_leaf);
+    if (c >= s.d || k == 0) s.e = min(GT_MAX_LEVEL, c + 1);
+    else if (cell_holds(key, n, k, s.d - 1, n_leaf)) s.e = s.d;
+    else return s;
+    // the largest cell of at most m particles, or the leaf: the first such
+    // level on the way down, unless it is d and its parent is one already
+    auto largest = [&](long long m) {
+        const int q = min(max(s.d, shared(m) + 1), s.e);
+        return (q > s.d || q == 0 || cell_holds(key, n, k, s.d - 1, m)) ? q : -1;
+    };
+    s.group = largest(n_group);
+    s.tile = largest(n_tile);
+    return s;
+}
+
+// Rows of the per-block counts: nodes of each level, nodes, groups, tiles.
+constexpr int ROW_NODES = GT_MAX_LEVEL + 1, ROW_GROUPS = ROW_NODES + 1, ROW_TILES = ROW_NODES + 2,
+              N_ROWS = ROW_NODES + 3;
+
+// Counts per block of 256 particles (row-major, entry N_ROWS nblk zeroed so
+// that the scan ends with the total); st: the particles' starts, packed.
+__global__ __launch_bounds__(256) void k_starts(const unsigned long long *__restrict__ key, long long n, int n_leaf,
+                                                int n_group, int n_tile, int nblk, int *__restrict__ cnt,
+                                                unsigned *__restrict__ st)
+{
+    __shared__ int w[N_ROWS][4];
+    const long long k = (long long)blockIdx.x * 256 + threadIdx.x;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    Starts s{0, -1, -1, -1};
+    if (k < n) {
+        s = starts_at(key, n, k, n_leaf, n_group, n_tile);
+        st[k] = (unsigned)(s.d | (s.e + 1) << 8 | (s.group + 1) << 16 | (s.tile + 1) << 24);
+    }
+    const int n_lev = max(s.e - s.d + 1, 0);
+    int nodes = 0;
+    for (int l = 0; l <= GT_MAX_LEVEL; l++) {
+        const int c = __popcll(__ballot(n_lev > 0 && s.d <= l && l <= s.e));
+        nodes += c;
+        if (lane == 0) w[l][wave] = c;
+    }
+    const int g = __popcll(__ballot(s.group >= 0)), t = __popcll(__ballot(s.tile >= 0));
+    if (lane == 0) {
+        w[ROW_NODES][wave] = nodes;
+        w[ROW_GROUPS][wave] = g;
+        w[ROW_TILES][wave] = t;
+    }
+    __syncthreads();
+    const int r = threadIdx.x;
+    if (r < N_ROWS) cnt[(size_t)r * nblk + blockIdx.x] = w[r][0] + w[r][1] + w[r][2] + w[r][3];
+    if (blockIdx.x == 0 && r == 0) cnt[(size_t)N_ROWS * nblk] = 0;
+}
+
+// Level table and totals from the scanned counts.
+__global__ __launch_bounds__(64) void k_tree_sizes(const int *__restrict__ off, int nblk, TreeMeta *__restrict__ meta)
+{
+    const int r = threadIdx.x;
+    if (r <= ROW_NODES) meta->level_start[r] = off[(size_t)r * nblk];
+    if (r == 0) {
+        const int nn = off[(size_t)ROW_NODES * nblk], g0 = off[(size_t)ROW_GROUPS * nblk],
+                  t0 = off[(size_t)ROW_TILES * nblk];
+        meta->n_group = t0 - g0;
+        meta->n_tile = off[(size_t)N_ROWS * nblk] - t0;
+        (void)nn;
+    }
+}
+
+// Nodes (all but end and n_child), their preorder numbers (a depth-first
+// walk's order: by first particle, then level) and the inverse, the groups
+// and the tiles in Morton order.
+__global__ __launch_bounds__(256) void k_nodes(long long n, int nblk, const int *__restrict__ off,
+                                               const unsigned *__restrict__ st, GNode *__restrict__ nodes,
+                                               int *__restrict__ pre, int *__restrict__ node_at,
+                                               int *__restrict__ groups, int *__restrict__ tiles)
+{
+    __shared__ int w[N_ROWS][4];
+    const long long k = (long long)blockIdx.x * 256 + threadIdx.x;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const unsigned v = k < n ? st[k] : 0u;
+    const int d = (int)(v & 255u), e = (int)(v >> 8 & 255u) - 1, group = (int)(v >> 16 & 255u) - 1,
+              tile = (int)(v >> 24) - 1;
+    const unsigned long long below = lane ? ~0ull >> (64 - lane) : 0ull;
+    // counts of the waves before this one, and the lanes' ranks
+    int mine = 0, nodes_before = 0;  // nodes of the lanes before this one
+    for (int l = 0; l <= GT_MAX_LEVEL; l++) {
+        const unsigned long long b = __ballot(d <= l && l <= e);
+        if (lane == 0) w[l][wave] = __popcll(b);
+        mine += __popcll(b);
+        nodes_before += __popcll(b & below);
+    }
+    const unsigned long long bg = __ballot(group >= 0), bt = __ballot(tile >= 0);
+    if (lane == 0) {
+        w[ROW_NODES][wave] = mine;
+        w[ROW_GROUPS][wave] = __popcll(bg);
+        w[ROW_TILES][wave] = __popcll(bt);
+    }
+    __syncthreads();
+    auto base = [&](int r) {
+        int o = off[(size_t)r * nblk + blockIdx.x];
+        for (int q = 0; q < 3; q++)
+            if (q < wave) o += w[r][q];
+        return o;
+    };
+    const int p0 = base(ROW_NODES) - off[(size_t)ROW_NODES * nblk] + nodes_before;
+    int child = -1;
+    for (int l = GT_MAX_LEVEL; l >= 0; l--) {
+        const bool in = d <= l && l <= e;
+        const unsigned long long b = __ballot(in);
+        if (b == 0) continue;
+        const int at = base(l) + __popcll(b & below);
+        if (!in) continue;
+        nodes[at] = GNode{k, 0, l, 0, child};
+        const int p = p0 + (l - d);
+        pre[at] = p;
+        node_at[p] = at;
+        if (l == group) groups[base(ROW_GROUPS) - off[(size_t)ROW_GROUPS * nblk] + __popcll(bg & below)] = at;
+        if (l == tile) tiles[base(ROW_TILES) - off[(size_t)ROW_TILES * nblk] + __popcll(bt & below)] = at;
+        child = at;
+    }
+}
+
+// End and child count of every node: the end by a search of the keys
+// (doubling steps from the smallest possible size), the children being the
+// nodes of the next level that start before it.
+__global__ __launch_bounds__(256) void k_node_ends(GNode *__restrict__ nodes, long long nn, long long n, int n_leaf,
+                                                   const unsigned long long *__restrict__ key)
 {
     const long long k = (long long)blockIdx.x * 256 + threadIdx.x;
-    if (k == 0) cnt[nl] = 0;  // so that the scan's entry nl is the level's child count
-    if (k >= nl) return;
-    const GNode nd = nodes[lb + k];
-    long long *b = bnd + 9 * k;
-    const long long m = nd.end - nd.begin;
-    if (m <= n_leaf_limit || nd.level >= GT_MAX_LEVEL) {
-        cnt[k] = 0;
-        return;
-    }
-    const int shift = 3 * (GT_MAX_LEVEL - 1 - nd.level);
-    b[0] = nd.begin;
-    b[8] = nd.end;
-    for (int d = 1; d < 8; d++) {
-        // first position in [begin, end) whose octant digit is >= d
-        long long lo = nd.begin, hi = nd.end;
-        while (lo < hi) {
-            const long long mid = (lo + hi) >> 1;
-            if ((int)((key[mid] >> shift) & 7u) < d) lo = mid + 1;
-            else hi = mid;
+    if (k >= nn) return;
+    const long long b = nodes[k].begin, fc = nodes[k].first_child;
+    const int l = nodes[k].level;
+    const unsigned long long kk = key[b];
+    long long in = b, step = fc >= 0 ? (long long)n_leaf : 1;  // particle in is in the cell
+    long long out = n;                                         // particle out is not
+    while (in + step < n) {
+        if (common_levels(kk, key[in + step]) < l) {
+            out = in + step;
+            break;
         }
-        b[d] = lo;
+        in += step;
+        step *= 2;
     }
-    int c = 0;
-    for (int d = 0; d < 8; d++) c += (b[d + 1] > b[d]);
-    cnt[k] = c;
+    while (out - in > 1) {
+        const long long mid = (in + out) >> 1;
+        if (common_levels(kk, key[mid]) >= l) in = mid;
+        else out = mid;
+    }
+    nodes[k].end = out;
+    if (fc < 0) return;
+    int c = 1;
+    for (int j = 1; j < 8; j++)
+        if (fc + j < nn && nodes[fc + j].level == l + 1 && nodes[fc + j].begin < out) c = j + 1;
+    nodes[k].n_child = c;
 }
 
-__global__ __launch_bounds__(256) void k_split_write(GNode *__restrict__ nodes, long long lb, long long nl,
-                                                     long long le, const long long *__restrict__ bnd,
-                                                     const int *__restrict__ cnt, const int *__restrict__ off)
+// Boxes and reciprocal data of a node's moments, written to the node arrays.
+struct Moments {
+    double M, c[3], q[6], bi[6], bo[6];
+};
+struct MomentArrays {
+    double *mass, *com, *quad, *box_in, *box_out;
+};
+__device__ __forceinline__ void moments_init(Moments &v)
+{
+    v.M = 0;
+    for (int d = 0; d < 3; d++) {
+        v.c[d] = 0;
+        v.bi[d] = v.bo[d] = 1e300;
+        v.bi[3 + d] = v.bo[3 + d] = -1e300;
+    }
+    for (int d = 0; d < 6; d++) v.q[d] = 0;
+}
+__device__ __forceinline__ void moments_centre(Moments &v)
+{
+    if (v.M > 0) {
+        for (int d = 0; d < 3; d++) v.c[d] /= v.M;
+    } else {
+        for (int d = 0; d < 3; d++) v.c[d] = 0.5 * (v.bi[d] + v.bi[3 + d]);
+    }
+}
+__device__ __forceinline__ void moments_store(const Moments &v, const MomentArrays &o, long long k)
+{
+    o.mass[k] = v.M;
+    for (int d = 0; d < 3; d++) o.com[3 * k + d] = v.c[d];
+    for (int d = 0; d < 6; d++) {
+        o.quad[6 * k + d] = v.q[d];
+        o.box_in[6 * k + d] = v.bi[d];
+        o.box_out[6 * k + d] = v.bo[d];
+    }
+}
+
+// Moments of the leaves, one thread each, the host's sums in its order; the
+// particles are loaded four at a time, so that a leaf of 20 waits for memory
+// ten times and not forty.
+__global__ __launch_bounds__(256) void k_leaf_moments(const GNode *__restrict__ nodes, long long nn,
+                                                      const double *__restrict__ pos, const double *__restrict__ mass,
+                                                      const double *__restrict__ rs, const MomentArrays out)
 {
     const long long k = (long long)blockIdx.x * 256 + threadIdx.x;
-    if (k >= nl || cnt[k] == 0) return;
-    GNode &nd = nodes[lb + k];
-    nd.first_child = le + off[k];
-    nd.n_child = cnt[k];
-    const long long *b = bnd + 9 * k;
-    long long c = nd.first_child;
-    for (int d = 0; d < 8; d++)
-        if (b[d + 1] > b[d]) nodes[c++] = GNode{b[d], b[d + 1], nd.level + 1, 0, -1};
+    if (k >= nn) return;
+    const GNode nd = nodes[k];
+    if (nd.n_child != 0) return;
+    Moments v;
+    moments_init(v);
+    for (long long i0 = nd.begin; i0 < nd.end; i0 += 4) {
+        double x[4][3], m[4], r[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const long long i = min(i0 + u, nd.end - 1);
+            for (int d = 0; d < 3; d++) x[u][d] = pos[3 * i + d];
+            m[u] = mass[i];
+            r[u] = rs[i];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            if (i0 + u >= nd.end) break;
+            v.M += m[u];
+            for (int d = 0; d < 3; d++) {
+                v.c[d] += m[u] * x[u][d];
+                v.bi[d] = fmin(v.bi[d], x[u][d]);
+                v.bi[3 + d] = fmax(v.bi[3 + d], x[u][d]);
+                v.bo[d] = fmin(v.bo[d], x[u][d] - r[u]);
+                v.bo[3 + d] = fmax(v.bo[3 + d], x[u][d] + r[u]);
+            }
+        }
+    }
+    moments_centre(v);
+    for (long long i0 = nd.begin; i0 < nd.end; i0 += 4) {
+        double p[4][3], m4[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const long long i = min(i0 + u, nd.end - 1);
+            for (int d = 0; d < 3; d++) p[u][d] = pos[3 * i + d];
+            m4[u] = mass[i];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            if (i0 + u >= nd.end) break;
+            const double x = p[u][0] - v.c[0], y = p[u][1] - v.c[1], z = p[u][2] - v.c[2], m = m4[u];
+            v.q[0] += m * x * x;
+            v.q[1] += m * y * y;
+            v.q[2] += m * z * z;
+            v.q[3] += m * x * y;
+            v.q[4] += m * x * z;
+            v.q[5] += m * y * z;
+        }
+    }
+    moments_store(v, out, k);
 }
 
-// moments of nodes [a, b) (children are done): the host's sums in its order
-__global__ __launch_bounds__(256) void k_moments(const GNode *__restrict__ nodes, long long a, long long b,
-                                                 const double *__restrict__ pos, const double *__restrict__ mass,
-                                                 const double *__restrict__ rs, double *__restrict__ nmass,
-                                                 double *__restrict__ ncom, double *__restrict__ nquad,
-                                                 double *__restrict__ box_in, double *__restrict__ box_out)
+// Moments of the inner nodes of [a, b), one level (its children are done).
+__global__ __launch_bounds__(64) void k_inner_moments(const GNode *__restrict__ nodes, long long a, long long b,
+                                                      const MomentArrays o)
 {
-    const long long k = a + (long long)blockIdx.x * 256 + threadIdx.x;
+    const long long k = a + (long long)blockIdx.x * 64 + threadIdx.x;
     if (k >= b) return;
     const GNode nd = nodes[k];
-    double M = 0, c[3] = {0, 0, 0}, q[6] = {0, 0, 0, 0, 0, 0};
-    double bi[6] = {1e300, 1e300, 1e300, -1e300, -1e300, -1e300};
-    double bo[6] = {1e300, 1e300, 1e300, -1e300, -1e300, -1e300};
-    if (nd.n_child == 0) {
-        for (long long i = nd.begin; i < nd.end; i++) {
-            M += mass[i];
-            for (int d = 0; d < 3; d++) {
-                const double x = pos[3 * i + d];
-                c[d] += mass[i] * x;
-                bi[d] = fmin(bi[d], x);
-                bi[3 + d] = fmax(bi[3 + d], x);
-                bo[d] = fmin(bo[d], x - rs[i]);
-                bo[3 + d] = fmax(bo[3 + d], x + rs[i]);
-            }
-        }
-        if (M > 0) {
-            for (int d = 0; d < 3; d++) c[d] /= M;
-        } else {
-            for (int d = 0; d < 3; d++) c[d] = 0.5 * (bi[d] + bi[3 + d]);
-        }
-        for (long long i = nd.begin; i < nd.end; i++) {
-            const double x = pos[3 * i] - c[0], y = pos[3 * i + 1] - c[1], z = pos[3 * i + 2] - c[2], m = mass[i];
-            q[0] += m * x * x;
-            q[1] += m * y * y;
-            q[2] += m * z * z;
-            q[3] += m * x * y;
-            q[4] += m * x * z;
-            q[5] += m * y * z;
-        }
-    } else {
-        for (int ch = 0; ch < nd.n_child; ch++) {
-            const long long cc = nd.first_child + ch;
-            M += nmass[cc];
-            for (int d = 0; d < 3; d++) {
-                c[d] += nmass[cc] * ncom[3 * cc + d];
-                bi[d] = fmin(bi[d], box_in[6 * cc + d]);
-                bi[3 + d] = fmax(bi[3 + d], box_in[6 * cc + 3 + d]);
-                bo[d] = fmin(bo[d], box_out[6 * cc + d]);
-                bo[3 + d] = fmax(bo[3 + d], box_out[6 * cc + 3 + d]);
-            }
-        }
-        if (M > 0) {
-            for (int d = 0; d < 3; d++) c[d] /= M;
-        } else {
-            for (int d = 0; d < 3; d++) c[d] = 0.5 * (bi[d] + bi[3 + d]);
-        }
-        for (int ch = 0; ch < nd.n_child; ch++) {
-            const long long cc = nd.first_child + ch;
-            const double m = nmass[cc];
-            const double x = ncom[3 * cc] - c[0], y = ncom[3 * cc + 1] - c[1], z = ncom[3 * cc + 2] - c[2];
-            const double *qc = nquad + 6 * cc;
-            q[0] += qc[0] + m * x * x;
-            q[1] += qc[1] + m * y * y;
-            q[2] += qc[2] + m * z * z;
-            q[3] += qc[3] + m * x * y;
-            q[4] += qc[4] + m * x * z;
-            q[5] += qc[5] + m * y * z;
-        }
-    }
-    nmass[k] = M;
-    for (int d = 0; d < 3; d++) ncom[3 * k + d] = c[d];
-    for (int d = 0; d < 6; d++) {
-        nquad[6 * k + d] = q[d];
-        box_in[6 * k + d] = bi[d];
-        box_out[6 * k + d] = bo[d];
-    }
-}
-
-// group flags: the root when it qualifies (at most n_group_limit particles,
-// or a leaf); k_group_children adds the qualifying children of every
-// non-qualifying node, i.e. the largest qualifying cells
-__global__ __launch_bounds__(256) void k_group_flags(const GNode *__restrict__ nodes, long long nn, int n_group_limit,
-                                                     char *__restrict__ flag)
-{
-    const long long k = (long long)blockIdx.x * 256 + threadIdx.x;
-    if (k >= nn) return;
-    char f = 0;
-    if (k == 0) {
-        const GNode nd = nodes[0];
-        f = (char)((nd.end - nd.begin <= n_group_limit) || nd.n_child == 0);
-    }
-    flag[k] = f;
-}
-
-// marks the children of every non-qualifying internal node that qualify
-__global__ __launch_bounds__(256) void k_group_children(const GNode *__restrict__ nodes, long long nn,
-                                                        int n_group_limit, char *__restrict__ flag)
-{
-    const long long k = (long long)blockIdx.x * 256 + threadIdx.x;
-    if (k >= nn) return;
-    const GNode nd = nodes[k];
-    const bool q = (nd.end - nd.begin <= n_group_limit) || nd.n_child == 0;
-    if (q) return;
+    if (nd.n_child == 0) return;
+    Moments v;
+    moments_init(v);
     for (int ch = 0; ch < nd.n_child; ch++) {
-        const GNode c = nodes[nd.first_child + ch];
-        if ((c.end - c.begin <= n_group_limit) || c.n_child == 0) flag[nd.first_child + ch] = 1;
+        const long long cc = nd.first_child + ch;
+        const double m = o.mass[cc];
+        v.M += m;
+        for (int d = 0; d < 3; d++) {
+            v.c[d] += m * o.com[3 * cc + d];
+            v.bi[d] = fmin(v.bi[d], o.box_in[6 * cc + d]);
+            v.bi[3 + d] = fmax(v.bi[3 + d], o.box_in[6 * cc + 3 + d]);
+            v.bo[d] = fmin(v.bo[d], o.box_out[6 * cc + d]);
+            v.bo[3 + d] = fmax(v.bo[3 + d], o.box_out[6 * cc + 3 + d]);
+        }
     }
+    moments_centre(v);
+    for (int ch = 0; ch < nd.n_child; ch++) {
+        const long long cc = nd.first_child + ch;
+        const double m = o.mass[cc];
+        const double x = o.com[3 * cc] - v.c[0], y = o.com[3 * cc + 1] - v.c[1], z = o.com[3 * cc + 2] - v.c[2];
+        const double *qc = o.quad + 6 * cc;
+        v.q[0] += qc[0] + m * x * x;
+        v.q[1] += qc[1] + m * y * y;
+        v.q[2] += qc[2] + m * z * z;
+        v.q[3] += qc[3] + m * x * y;
+        v.q[4] += qc[4] + m * x * z;
+        v.q[5] += qc[5] + m * y * z;
+    }
+    moments_store(v, o, k);
 }
 
 __global__ __launch_bounds__(64) void k_fill_int(int *__restrict__ p, long long n, int v)
 {
     for (long long k = threadIdx.x; k < n; k += 64) p[k] = v;
-}
-
-__global__ __launch_bounds__(256) void k_group_keys(const GNode *__restrict__ nodes, const int *__restrict__ gnode,
-                                                    long long ng, long long *__restrict__ gbeg)
-{
-    const long long g = (long long)blockIdx.x * 256 + threadIdx.x;
-    if (g >= ng) return;
-    gbeg[g] = nodes[gnode[g]].begin;
 }
 
 // per group: first particle, size, list lengths (host copy for the planner)
@@ -771,11 +981,11 @@ __global__ __launch_bounds__(64) void k_ngb(const NgbArgs a)
 
 struct pth_gtree {
     pth_ctx *ctx = nullptr;
-    long long n = 0, n_node = 0, n_group = 0, n_le = 0, n_ls = 0;
-    DevBuf order, key, skey, sidx, spos, smass, srs, nodes, nmass, ncom, nquad, box_in, box_out, groups, off_e, off_s,
+    long long n = 0, n_node = 0, n_group = 0, n_tile = 0, n_le = 0, n_ls = 0;
+    DevBuf order, key, skey, sidx, sidx2, spos, smass, srs, nodes, nmass, ncom, nquad, box_in, box_out, groups, off_e, off_s,
         id_epj, id_spj, tmp;
     // build-time scratch, released when the build ends (or by pth_gtree_free)
-    DevBuf dpos, dmass, drs, part, bnd, cnt, off, flag, gsel, nsel, gkey, gkey2, ce, cs, alt, lkey, lkey2, info;
+    DevBuf dpos, dmass, drs, part, cnt, off, starts, ce, cs, alt, lkey, lkey2, info;
     // neighbour lists (pth_gtree_neighbors): count per input index, offsets,
     // entries; tile boxes, candidate counts / offsets / lists, tile records
     DevBuf ngb_cnt, ngb_off, ngb, tiles, tbox, tcnt, toff, tl, tl_alt, tinfo;
@@ -784,7 +994,10 @@ struct pth_gtree {
     DevBuf pad_off, pad_e, pad_s;
     std::vector<long long> pad_h;
     int walk_passes = 0;  // of the last build: 1 (one padded pass) or 2 (count, then write)
-    void *pinned = nullptr;  // pinned host block for small read-backs and uploads (PIN_* layout)
+    DevBuf meta;             // TreeMeta of the last build
+    DevBuf pre, node_at;     // preorder number of each node, and the inverse
+    void *pinned = nullptr;  // pinned host copy of meta
+    hipEvent_t ev_meta = nullptr;  // that copy
     // one-pass tile walks of the neighbour search: the last search's
     // candidate counts per tile (nt + 1 entries), padded offsets, lists
     std::vector<long long> tcnt_h, tpad_h;
@@ -801,11 +1014,9 @@ struct pth_gtree {
     float ms_ngb = 0.f;
     void release_scratch()
     {
-        DevBuf *s[] = {&dpos, &dmass, &drs, &part, &bnd, &cnt, &off, &flag, &gsel, &nsel, &gkey, &gkey2, &ce, &cs,
-                       &alt, &lkey, &lkey2, &info};
+        DevBuf *s[] = {&dpos, &dmass, &drs, &part, &cnt, &off, &starts, &ce, &cs, &alt, &lkey, &lkey2, &info};
         for (DevBuf *b : s) b->release();
     }
-    std::vector<long long> level_start;
     std::vector<int4> groups_h;  // per group: first particle, size, n_epj, n_spj
     // the plan of a resident evaluation of the last build's lists, made on
     // the host while the device writes and orders them, and the parameters
@@ -830,22 +1041,17 @@ namespace {
         if (e_ != hipSuccess) return t->ctx->hip_fail(e_, what); \
     } while (0)
 
-inline unsigned blocks(long long n) { return (unsigned)((n + 255) / 256); }
+constexpr int TILE_LIMIT = 64;  // particles of a neighbour-search tile
 
-// Pinned host block of a tree: small counts read back at byte 0, the root
-// node's upload at byte 64, the bounding-box partials (8 doubles for each of
-// at most 1024 blocks) from byte 128.
-constexpr size_t PIN_COUNT = 0, PIN_ROOT = 64, PIN_BBOX = 128, PIN_BYTES = PIN_BBOX + 8 * 8 * 1024;
+inline unsigned blocks(long long n) { return (unsigned)((n + 255) / 256); }
 
 hipError_t ensure_pinned(pth_gtree *t)
 {
     if (t->pinned) return hipSuccess;
-    const hipError_t e = hipHostMalloc(&t->pinned, PIN_BYTES, hipHostMallocDefault);
+    const hipError_t e = hipHostMalloc(&t->pinned, sizeof(TreeMeta), hipHostMallocDefault);
     if (e != hipSuccess) t->pinned = nullptr;
-    return e;
+    return e ? e : hipEventCreateWithFlags(&t->ev_meta, hipEventDisableTiming);
 }
-
-template <class T> T *pinned_at(pth_gtree *t, size_t off) { return reinterpret_cast<T *>(static_cast<char *>(t->pinned) + off); }
 
 // temp storage for a hipcub call, grown on demand
 hipError_t cub_temp(pth_gtree *t, size_t bytes) { return t->tmp.ensure(std::max<size_t>(bytes, 256)); }
@@ -853,49 +1059,6 @@ hipError_t cub_temp(pth_gtree *t, size_t bytes) { return t->tmp.ensure(std::max<
 }  // namespace
 
 namespace {
-
-// The largest cells with at most `limit` particles (or leaves), as node
-// indices in Morton order (by first particle): the i-groups for limit =
-// n_group_limit, the neighbour-search tiles for limit = 64.
-int select_cells(pth_gtree *t, int limit, DevBuf &out, long long &n_out)
-{
-    pth_ctx *ctx = t->ctx;
-    hipStream_t st = ctx->stream;
-    const long long nn = t->n_node;
-    size_t tb = 0;
-    hipError_t e;
-    DevBuf &flag = t->flag, &gsel = t->gsel, &nsel = t->nsel, &gkey = t->gkey, &gkey2 = t->gkey2;
-    if ((e = flag.ensure(nn)) || (e = gsel.ensure(sizeof(int) * nn)) || (e = nsel.ensure(sizeof(int))))
-        return ctx->hip_fail(e, "cell selection allocation");
-    hipLaunchKernelGGL(k_group_flags, dim3(blocks(nn)), dim3(256), 0, st, t->nodes.as<GNode>(), nn, limit,
-                       flag.as<char>());
-    hipLaunchKernelGGL(k_group_children, dim3(blocks(nn)), dim3(256), 0, st, t->nodes.as<GNode>(), nn, limit,
-                       flag.as<char>());
-    hipcub::CountingInputIterator<int> it(0);
-    if ((e = hipcub::DeviceSelect::Flagged(nullptr, tb, it, flag.as<char>(), gsel.as<int>(), nsel.as<int>(), (int)nn,
-                                           st)) ||
-        (e = cub_temp(t, tb)) ||
-        (e = hipcub::DeviceSelect::Flagged(t->tmp.p, tb, it, flag.as<char>(), gsel.as<int>(), nsel.as<int>(),
-                                           (int)nn, st)))
-        return ctx->hip_fail(e, "cell selection");
-    if ((e = ensure_pinned(t)) ||
-        (e = hipMemcpyAsync(pinned_at<int>(t, PIN_COUNT), nsel.p, sizeof(int), hipMemcpyDeviceToHost, st)) ||
-        (e = hipStreamSynchronize(st)))
-        return ctx->hip_fail(e, "cell count");
-    const long long ng = *static_cast<volatile int *>(pinned_at<int>(t, PIN_COUNT));
-    if ((e = gkey.ensure(8 * ng)) || (e = gkey2.ensure(8 * ng)) || (e = out.ensure(sizeof(int) * std::max(ng, 1LL))))
-        return ctx->hip_fail(e, "cell selection allocation");
-    hipLaunchKernelGGL(k_group_keys, dim3(blocks(ng)), dim3(256), 0, st, t->nodes.as<GNode>(), gsel.as<int>(), ng,
-                       gkey.as<long long>());
-    if ((e = hipcub::DeviceRadixSort::SortPairs(nullptr, tb, gkey.as<long long>(), gkey2.as<long long>(),
-                                                gsel.as<int>(), out.as<int>(), (int)ng, 0, 32, st)) ||
-        (e = cub_temp(t, tb)) ||
-        (e = hipcub::DeviceRadixSort::SortPairs(t->tmp.p, tb, gkey.as<long long>(), gkey2.as<long long>(),
-                                                gsel.as<int>(), out.as<int>(), (int)ng, 0, 32, st)))
-        return ctx->hip_fail(e, "cell sort");
-    n_out = ng;
-    return PTH_OK;
-}
 
 // Builds (or rebuilds, reusing t's device memory) the tree of n particles.
 // pos / mass / rs are host arrays, or device arrays when on_device.
@@ -933,127 +1096,86 @@ int gtree_run(pth_gtree *t, long long n, const double *pos, const double *mass, 
         dmass = t->dmass.as<double>();
         drs = r_search ? t->drs.as<double>() : nullptr;
     }
-    // 1. bounding cube (per-block partials reduced on the host)
+    // 1. bounding cube
     const int nb = (int)std::min<long long>(1024, (n + 255) / 256);
     DevBuf &part = t->part;
-    if ((e = ensure_pinned(t))) return ctx->hip_fail(e, "pinned buffer");
-    const double *hp = pinned_at<double>(t, PIN_BBOX);
-    if ((e = part.ensure(sizeof(double) * 8 * nb))) return ctx->hip_fail(e, "bbox");
-    hipLaunchKernelGGL(k_bbox, dim3(nb), dim3(256), 0, st, dpos, drs, n, part.as<double>());
-    if ((e = hipMemcpyAsync(pinned_at<double>(t, PIN_BBOX), part.p, sizeof(double) * 8 * nb, hipMemcpyDeviceToHost,
-                            st)) ||
-        (e = hipStreamSynchronize(st)))
+    if ((e = ensure_pinned(t)) || (e = part.ensure(sizeof(double) * 8 * nb)) || (e = t->meta.ensure(sizeof(TreeMeta))))
         return ctx->hip_fail(e, "bbox");
-    double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
-    t->rs_max = 0.0;
-    bool bad = false;
-    for (int b = 0; b < nb; b++) {
-        for (int d = 0; d < 3; d++) {
-            lo[d] = std::min(lo[d], hp[8 * b + d]);
-            hi[d] = std::max(hi[d], hp[8 * b + 3 + d]);
-        }
-        t->rs_max = std::max(t->rs_max, hp[8 * b + 6]);
-        bad = bad || hp[8 * b + 7] != 0.0;
-    }
-    if (bad) return ctx->fail(PTH_ERR_ARG, "pth_gtree: non-finite particle positions or r_search");
-    double len = 0;
-    for (int d = 0; d < 3; d++) len = std::max(len, hi[d] - lo[d]);
-    len = (len > 0) ? len * (1.0 + 1e-9) : 1.0;
-    double root[3];
-    for (int d = 0; d < 3; d++) root[d] = 0.5 * (lo[d] + hi[d]) - 0.5 * len;
-    const double scale = (double)(1u << GT_MAX_LEVEL) / len;
-    t->root_len = len;
+    TreeMeta *meta = t->meta.as<TreeMeta>();
+    hipLaunchKernelGGL(k_bbox, dim3(nb), dim3(256), 0, st, dpos, drs, n, part.as<double>());
+    hipLaunchKernelGGL(k_root, dim3(1), dim3(64), 0, st, part.as<double>(), nb, meta);
     // 2. keys, stable sort of (key, index), sorted particles
     if ((e = t->key.ensure(8 * (size_t)n)) || (e = t->skey.ensure(8 * (size_t)n)) ||
-        (e = t->sidx.ensure(8 * (size_t)n)) || (e = t->order.ensure(8 * (size_t)n)))
+        (e = t->sidx.ensure(4 * (size_t)n)) || (e = t->sidx2.ensure(4 * (size_t)n)) ||
+        (e = t->order.ensure(8 * (size_t)n)))
         return ctx->hip_fail(e, "key allocation");
-    hipLaunchKernelGGL(k_keys, dim3(blocks(n)), dim3(256), 0, st, dpos, n, root[0], root[1], root[2],
-                       scale, t->key.as<unsigned long long>(), t->sidx.as<long long>());
+    hipLaunchKernelGGL(k_keys, dim3(blocks(n)), dim3(256), 0, st, dpos, n, meta, t->key.as<unsigned long long>(),
+                       t->sidx.as<int>());
     size_t tb = 0;
     if ((e = hipcub::DeviceRadixSort::SortPairs(nullptr, tb, t->key.as<unsigned long long>(),
-                                                t->skey.as<unsigned long long>(), t->sidx.as<long long>(),
-                                                t->order.as<long long>(), n, 0, 3 * GT_MAX_LEVEL, st)) ||
+                                                t->skey.as<unsigned long long>(), t->sidx.as<int>(),
+                                                t->sidx2.as<int>(), n, 0, 3 * GT_MAX_LEVEL, st)) ||
         (e = cub_temp(t, tb)) ||
         (e = hipcub::DeviceRadixSort::SortPairs(t->tmp.p, tb, t->key.as<unsigned long long>(),
-                                                t->skey.as<unsigned long long>(), t->sidx.as<long long>(),
-                                                t->order.as<long long>(), n, 0, 3 * GT_MAX_LEVEL, st)))
+                                                t->skey.as<unsigned long long>(), t->sidx.as<int>(),
+                                                t->sidx2.as<int>(), n, 0, 3 * GT_MAX_LEVEL, st)))
         return ctx->hip_fail(e, "key sort");
     if ((e = t->spos.ensure(24 * (size_t)n)) || (e = t->smass.ensure(8 * (size_t)n)) ||
         (e = t->srs.ensure(8 * (size_t)n)))
         return ctx->hip_fail(e, "particle allocation");
-    hipLaunchKernelGGL(k_gather, dim3(blocks(n)), dim3(256), 0, st, n, t->order.as<long long>(), dpos,
-                       dmass, drs, t->spos.as<double>(),
-                       t->smass.as<double>(), t->srs.as<double>());
-    // 3. nodes level by level
-    if ((e = t->nodes.ensure(sizeof(GNode) * std::max<long long>(2 * n / std::max(n_leaf_limit, 1) + 64, 1024))))
+    // 3. nodes, groups and tiles: counts, one scan, one wait for the sizes
+    const int nblk = (int)blocks(n);
+    const unsigned long long *skey = t->skey.as<unsigned long long>();
+    const int n_cnt = N_ROWS * nblk + 1;
+    if ((e = t->cnt.ensure(sizeof(int) * (size_t)n_cnt)) || (e = t->off.ensure(sizeof(int) * (size_t)n_cnt)) ||
+        (e = t->starts.ensure(4 * (size_t)n)))
+        return ctx->hip_fail(e, "node counts");
+    hipLaunchKernelGGL(k_starts, dim3(nblk), dim3(256), 0, st, skey, n, n_leaf_limit, n_group_limit, TILE_LIMIT, nblk,
+                       t->cnt.as<int>(), t->starts.as<unsigned>());
+    if ((e = hipcub::DeviceScan::ExclusiveSum(nullptr, tb, t->cnt.as<int>(), t->off.as<int>(), n_cnt, st)) ||
+        (e = cub_temp(t, tb)) ||
+        (e = hipcub::DeviceScan::ExclusiveSum(t->tmp.p, tb, t->cnt.as<int>(), t->off.as<int>(), n_cnt, st)))
+        return ctx->hip_fail(e, "node scan");
+    hipLaunchKernelGGL(k_tree_sizes, dim3(1), dim3(64), 0, st, t->off.as<int>(), nblk, meta);
+    if ((e = hipMemcpyAsync(t->pinned, meta, sizeof(TreeMeta), hipMemcpyDeviceToHost, st)) ||
+        (e = hipEventRecord(t->ev_meta, st)))
+        return ctx->hip_fail(e, "tree sizes");
+    // (beside the wait)
+    hipLaunchKernelGGL(k_gather, dim3(blocks(n)), dim3(256), 0, st, n, t->sidx2.as<int>(), t->order.as<long long>(),
+                       dpos, dmass, drs, t->spos.as<double>(), t->smass.as<double>(), t->srs.as<double>());
+    if ((e = hipEventSynchronize(t->ev_meta))) return ctx->hip_fail(e, "tree sizes");
+    TreeMeta M;
+    std::memcpy(&M, t->pinned, sizeof M);
+    if (M.bad != 0.0) return ctx->fail(PTH_ERR_ARG, "pth_gtree: non-finite particle positions or r_search");
+    const double len = M.len;
+    t->rs_max = M.rs_max;
+    t->root_len = len;
+    const long long nn = M.level_start[GT_MAX_LEVEL + 1];
+    t->n_node = nn;
+    t->n_group = M.n_group;
+    t->n_tile = M.n_tile;
+    if ((e = t->nodes.ensure(sizeof(GNode) * nn)) || (e = t->pre.ensure(4 * nn)) || (e = t->node_at.ensure(4 * nn)) ||
+        (e = t->groups.ensure(4 * t->n_group)) || (e = t->tiles.ensure(4 * t->n_tile)))
         return ctx->hip_fail(e, "node allocation");
-    long long cap = (long long)(t->nodes.cap / sizeof(GNode));
-    // (from pinned memory: the copy is ordered before the level loop's
-    // launches and needs no wait)
-    *pinned_at<GNode>(t, PIN_ROOT) = GNode{0, n, 0, 0, -1};
-    if ((e = hipMemcpyAsync(t->nodes.p, pinned_at<GNode>(t, PIN_ROOT), sizeof(GNode), hipMemcpyHostToDevice, st)))
-        return ctx->hip_fail(e, "node upload");
-    t->level_start.assign(1, 0);
-    long long lb = 0, le = 1;
-    DevBuf &bnd = t->bnd, &cnt = t->cnt, &off = t->off;
-    for (;;) {
-        t->level_start.push_back(le);
-        const long long nl = le - lb;
-        if ((e = bnd.ensure(sizeof(long long) * 9 * nl)) || (e = cnt.ensure(sizeof(int) * (nl + 1))) ||
-            (e = off.ensure(sizeof(int) * (nl + 1))))
-            return ctx->hip_fail(e, "level buffers");
-        hipLaunchKernelGGL(k_split_count, dim3(blocks(nl)), dim3(256), 0, st, t->nodes.as<GNode>(), lb, nl,
-                           t->skey.as<unsigned long long>(), n_leaf_limit, bnd.as<long long>(), cnt.as<int>());
-        if ((e = hipcub::DeviceScan::ExclusiveSum(nullptr, tb, cnt.as<int>(), off.as<int>(), (int)nl + 1, st)) ||
-            (e = cub_temp(t, tb)) ||
-            (e = hipcub::DeviceScan::ExclusiveSum(t->tmp.p, tb, cnt.as<int>(), off.as<int>(), (int)nl + 1, st)))
-            return ctx->hip_fail(e, "level scan");
-        // one small copy into pinned memory per level
-        if ((e = hipMemcpyAsync(pinned_at<int>(t, PIN_COUNT), off.as<int>() + nl, sizeof(int), hipMemcpyDeviceToHost,
-                                st)) ||
-            (e = hipStreamSynchronize(st)))
-            return ctx->hip_fail(e, "level size");
-        const long long total = *static_cast<volatile int *>(pinned_at<int>(t, PIN_COUNT));
-        if (total == 0) break;
-        if (le + total > cap) {
-            // grow the node array, keeping its contents
-            const long long ncap = std::max(2 * cap, le + total);
-            DevBuf nb2;
-            if ((e = nb2.ensure(sizeof(GNode) * ncap)) ||
-                (e = hipMemcpyAsync(nb2.p, t->nodes.p, sizeof(GNode) * le, hipMemcpyDeviceToDevice, st)) ||
-                (e = hipStreamSynchronize(st)))
-                return ctx->hip_fail(e, "node growth");
-            t->nodes.release();
-            t->nodes = nb2;
-            cap = ncap;
-        }
-        hipLaunchKernelGGL(k_split_write, dim3(blocks(nl)), dim3(256), 0, st, t->nodes.as<GNode>(), lb, nl, le,
-                           bnd.as<long long>(), cnt.as<int>(), off.as<int>());
-        lb = le;
-        le += total;
-    }
-    t->n_node = le;
-    if (le > 0x7fffffffLL)  // the walks keep node indices as int32
-        return ctx->fail(PTH_ERR_CAPACITY, "pth_gtree: node count exceeds the int32 range");
-    const long long nn = le;
-    // 4. moments bottom-up
+    hipLaunchKernelGGL(k_nodes, dim3(nblk), dim3(256), 0, st, n, nblk, t->off.as<int>(), t->starts.as<unsigned>(),
+                       t->nodes.as<GNode>(), t->pre.as<int>(), t->node_at.as<int>(), t->groups.as<int>(),
+                       t->tiles.as<int>());
+    hipLaunchKernelGGL(k_node_ends, dim3(blocks(nn)), dim3(256), 0, st, t->nodes.as<GNode>(), nn, n, n_leaf_limit,
+                       skey);
+    // 4. moments: the leaves, then the inner nodes level by level
     if ((e = t->nmass.ensure(8 * nn)) || (e = t->ncom.ensure(24 * nn)) || (e = t->nquad.ensure(48 * nn)) ||
         (e = t->box_in.ensure(48 * nn)) || (e = t->box_out.ensure(48 * nn)))
         return ctx->hip_fail(e, "moment allocation");
-    for (int l = (int)t->level_start.size() - 2; l >= 0; l--) {
-        const long long a = t->level_start[l], b = t->level_start[l + 1];
-        if (b <= a) continue;
-        hipLaunchKernelGGL(k_moments, dim3(blocks(b - a)), dim3(256), 0, st, t->nodes.as<GNode>(), a, b,
-                           t->spos.as<double>(), t->smass.as<double>(), t->srs.as<double>(), t->nmass.as<double>(),
-                           t->ncom.as<double>(), t->nquad.as<double>(), t->box_in.as<double>(),
-                           t->box_out.as<double>());
-    }
-    // 5. groups in Morton order
-    {
-        long long ng_sel = 0;
-        const int rc = select_cells(t, n_group_limit, t->groups, ng_sel);
-        if (rc != PTH_OK) return rc;
-        t->n_group = ng_sel;
+    const MomentArrays mo{t->nmass.as<double>(), t->ncom.as<double>(), t->nquad.as<double>(), t->box_in.as<double>(),
+                          t->box_out.as<double>()};
+    hipLaunchKernelGGL(k_leaf_moments, dim3(blocks(nn)), dim3(256), 0, st, t->nodes.as<GNode>(), nn,
+                       t->spos.as<double>(), t->smass.as<double>(), t->srs.as<double>(), mo);
+    for (int l = GT_MAX_LEVEL; l >= 0; l--) {
+        // (the deepest level holds leaves only)
+        const long long a = M.level_start[l], b = M.level_start[l + 1];
+        if (b <= a || b == nn) continue;
+        hipLaunchKernelGGL(k_inner_moments, dim3((unsigned)((b - a + 63) / 64)), dim3(64), 0, st,
+                           t->nodes.as<GNode>(), a, b, mo);
     }
     const long long ng = t->n_group;
     if ((e = hipStreamSynchronize(st))) return ctx->hip_fail(e, "tree build");
@@ -1442,11 +1564,7 @@ int pth_gtree_neighbors(pth_gtree *t, long long *n_total)
     // 1. candidate lists: one overlap-only walk per tile (the largest cells
     //    with at most 64 particles; theta opening off: inv_theta2 = 0), the
     //    group walk's symmetric r_search tests on widened tile boxes
-    long long nt = 0;
-    {
-        const int rc = select_cells(t, 64, t->tiles, nt);
-        if (rc != PTH_OK) return rc;
-    }
+    const long long nt = t->n_tile;
     HIPCHK(c, t->tbox.ensure(sizeof(double) * 12 * nt), "neighbour buffers");
     HIPCHK(c, t->tcnt.ensure(sizeof(long long) * (nt + 1)), "neighbour buffers");
     HIPCHK(c, t->toff.ensure(sizeof(long long) * (nt + 1)), "neighbour buffers");
@@ -1649,14 +1767,16 @@ void pth_gtree_free(pth_gtree *t)
         (void)hipSetDevice(t->ctx->device);
         if (t->ctx->stream) (void)hipStreamSynchronize(t->ctx->stream);
     }
-    DevBuf *all[] = {&t->order, &t->key, &t->skey, &t->sidx, &t->spos, &t->smass, &t->srs, &t->nodes, &t->nmass,
+    DevBuf *all[] = {&t->order, &t->key, &t->skey, &t->sidx, &t->sidx2, &t->spos, &t->smass, &t->srs, &t->nodes, &t->nmass,
                      &t->ncom, &t->nquad, &t->box_in, &t->box_out, &t->groups, &t->off_e, &t->off_s, &t->id_epj,
                      &t->id_spj, &t->tmp, &t->ngb_cnt, &t->ngb_off, &t->ngb, &t->tiles, &t->tbox, &t->tcnt,
                      &t->toff, &t->tl, &t->tl_alt, &t->tinfo, &t->pad_off, &t->pad_e, &t->pad_s,
-                     &t->tpad_off, &t->tl_pad, &t->ngb_cap, &t->ngb_poff, &t->ngb_pad, &t->ngb_flag};
+                     &t->tpad_off, &t->tl_pad, &t->ngb_cap, &t->ngb_poff, &t->ngb_pad, &t->ngb_flag,
+                     &t->meta, &t->pre, &t->node_at};
     for (DevBuf *b : all) b->release();
     t->release_scratch();
     if (t->pinned) (void)hipHostFree(t->pinned);
+    if (t->ev_meta) (void)hipEventDestroy(t->ev_meta);
     delete t;
 }
 

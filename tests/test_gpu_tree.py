@@ -68,6 +68,21 @@ def test_device_tree_limits():
     _compare(20000, 5, 0.3, 0.4, leaf=1, group=1)
 
 
+@pytest.mark.parametrize("n", [20, 21, 255, 256, 257, 3001])
+@pytest.mark.parametrize("leaf,group", [(1, 64), (20, 512), (20, 7), (64, 64), (300, 20)])
+def test_device_tree_block_edges_and_coincident_particles(n, leaf, group):
+    """The nodes of every level are decided from a few keys around each
+    particle, in blocks of 256 particles: sizes around a block and a leaf,
+    cells that straddle blocks, runs of coincident particles longer and
+    shorter than the limits (leaves at the deepest level), group limits below
+    and above the leaf limit."""
+    rng = np.random.default_rng(n)
+    m, x, _ = host.cluster(n, "plummer", f_bin=0.5, seed=n)
+    x[n // 2:n // 2 + min(40, n // 4)] = x[0]  # coincident particles
+    x[-3:] = x[-1] + 1e-13 * rng.standard_normal((3, 3))
+    _compare(n, 0, 0.0, 0.5, leaf=leaf, group=group, mx=(m, x))
+
+
 def test_device_tree_batch_order():
     _compare(30000, 4, 0.3, 0.3, canonical=False)
 
