@@ -425,10 +425,10 @@ int pth_gtree_sizes(const pth_gtree *tree, long long *n_node, long long *n_group
 int pth_gtree_download(const pth_gtree *tree, long long *order, long long *node_begin, long long *node_end,
                        int *node_level, double *node_mass, double *node_com, double *node_quad,
                        long long *epi_begin, int *n_epi, int *n_epj, int *n_spj, int *id_epj, int *id_spj);
-/* Host wall time of the last build (ms): tree (upload, sort, nodes, moments,
- * groups), walk (first walk pass, scan, list sizes) and the rest (writing
- * pass or the move of the lists written by the first pass, canonical
- * ordering when asked for, and meanwhile on the host the plan of a resident
+/* Host wall time of the last build (ms): tree (upload, sort, nodes; the
+ * moments are enqueued), walk (moments, first walk pass, list sizes) and the
+ * rest (writing pass when one is due, the final lists, in canonical order
+ * when asked for, and meanwhile on the host the plan of a resident
  * evaluation under the context's parameters, which pth_resident_from_gtree /
  * pth_resident_refill then take over). */
 int pth_gtree_timing(const pth_gtree *tree, float *ms_build, float *ms_walk, float *ms_order);

@@ -22,10 +22,12 @@
 //      popping up to 64 nodes at a time; a node is opened when it contains
 //      the group, when the group box is closer to its centre of mass than
 //      L/theta, or when the boxes overlap with either side widened by
-//      r_search; opened leaves give their particles (EPJ), closed nodes give
-//      one SPJ.  A counting pass, a scan, then a writing pass.
-//   6. optionally (canonical order) a segmented sort of every list into the
-//      host walk's depth-first order: EPJ ascending, SPJ by first particle.
+//      r_search; opened leaves go to the group's leaf list, closed nodes to
+//      its node list, both in batch order, in regions of the last build's
+//      lengths (a first build counts before it writes);
+//   6. lists: one workgroup per group puts its nodes and leaves into the host
+//      walk's depth-first order (canonical order) and expands the leaves
+//      into their particles.
 // Every decision is the same FP64 expression as on the host (no FMA
 // contraction in this file), so the lists are the host's lists as sets, and
 // entry for entry after the canonical ordering.
@@ -119,18 +121,21 @@ struct TreeMeta {
 
 // The root cube from the nb blocks' partial boxes (the host tree's
 // expressions).
-__global__ __launch_bounds__(64) void k_root(const double *__restrict__ part, int nb, TreeMeta *__restrict__ meta)
+__global__ __launch_bounds__(1024) void k_root(const double *__restrict__ part, int nb, TreeMeta *__restrict__ meta)
 {
-    double v[8];
-    for (int d = 0; d < 8; d++) {
-        v[d] = d < 3 ? 1e300 : d < 6 ? -1e300 : 0.0;
-        for (int b = threadIdx.x; b < nb; b += 64) v[d] = d < 3 ? fmin(v[d], part[8 * b + d]) : fmax(v[d], part[8 * b + d]);
-        for (int off = 32; off > 0; off >>= 1) {
-            const double o = __shfl_xor(v[d], off, 64);
-            v[d] = d < 3 ? fmin(v[d], o) : fmax(v[d], o);
-        }
+    // thread t reduces component t % 8 over the blocks t / 8, t / 8 + 128, ..
+    __shared__ double red[128][8];
+    const int c = threadIdx.x & 7, row = threadIdx.x >> 3;
+    double q = c < 3 ? 1e300 : c < 6 ? -1e300 : 0.0;
+    for (int b = row; b < nb; b += 128) q = c < 3 ? fmin(q, part[8 * b + c]) : fmax(q, part[8 * b + c]);
+    red[row][c] = q;
+    __syncthreads();
+    for (int half = 64; half > 0; half >>= 1) {
+        if (row < half) red[row][c] = c < 3 ? fmin(red[row][c], red[row + half][c]) : fmax(red[row][c], red[row + half][c]);
+        __syncthreads();
     }
     if (threadIdx.x) return;
+    const double *v = red[0];
     double len = 0;
     for (int d = 0; d < 3; d++) len = fmax(len, v[3 + d] - v[d]);
     len = (len > 0) ? len * (1.0 + 1e-9) : 1.0;
@@ -349,7 +354,8 @@ __global__ __launch_bounds__(256) void k_nodes(long long n, int nblk, const int 
 // (doubling steps from the smallest possible size), the children being the
 // nodes of the next level that start before it.
 __global__ __launch_bounds__(256) void k_node_ends(GNode *__restrict__ nodes, long long nn, long long n, int n_leaf,
-                                                   const unsigned long long *__restrict__ key)
+                                                   const unsigned long long *__restrict__ key,
+                                                   const int *__restrict__ pre, int2 *__restrict__ range)
 {
     const long long k = (long long)blockIdx.x * 256 + threadIdx.x;
     if (k >= nn) return;
@@ -372,6 +378,7 @@ __global__ __launch_bounds__(256) void k_node_ends(GNode *__restrict__ nodes, lo
         else out = mid;
     }
     nodes[k].end = out;
+    range[pre[k]] = make_int2((int)b, (int)(out - b));
     if (fc < 0) return;
     int c = 1;
     for (int j = 1; j < 8; j++)
@@ -379,12 +386,9 @@ __global__ __launch_bounds__(256) void k_node_ends(GNode *__restrict__ nodes, lo
     nodes[k].n_child = c;
 }
 
-// Boxes and reciprocal data of a node's moments, written to the node arrays.
+// A node's moments and boxes.
 struct Moments {
     double M, c[3], q[6], bi[6], bo[6];
-};
-struct MomentArrays {
-    double *mass, *com, *quad, *box_in, *box_out;
 };
 __device__ __forceinline__ void moments_init(Moments &v)
 {
@@ -404,7 +408,56 @@ __device__ __forceinline__ void moments_centre(Moments &v)
         for (int d = 0; d < 3; d++) v.c[d] = 0.5 * (v.bi[d] + v.bi[3 + d]);
     }
 }
-__device__ __forceinline__ void moments_store(const Moments &v, const MomentArrays &o, long long k)
+// What the walks read of a node, in FP32 relative to the root cube's centre:
+// the centre of mass and the two boxes, the boxes' bounds pushed outwards by
+// walk_margin (more than every rounding involved), the particle range, level,
+// child count, first child and preorder number.  52 B per visited node in
+// the group walk (A, B, C, F), in loads of 16 B that neighbouring lanes'
+// sibling nodes share lines of, against 152 B of FP64 moments: the walk is
+// bound by these gathers (1,048,576 particles, 67M visits: 1.32 ms on the
+// FP64 moments, 0.37 ms on these; 4,194,304: 4.6 and 1.27 ms).
+struct WalkRec {
+    float4 *A;  // centre of mass, first particle (int bits)
+    float4 *B;  // low corner of the box widened by r_search (joined with the
+                // particle box, should an r_search be negative), last particle + 1
+    float4 *C;  // its high corner, level << 8 | child count
+    float4 *D, *E;  // particle box (tile walks)
+    int2 *F;    // first child, preorder number
+};
+// Above every error of an FP32 coordinate difference inside the root cube
+// widened by r_search: each coordinate and difference is off by at most
+// 2^-24 (len + 2 rs_max), and at most four of them meet.
+__host__ __device__ inline float walk_margin(double len, double rs_max) { return (float)((len + 2.0 * rs_max) * 0x1p-21); }
+
+struct MomentArrays {
+    double *mass, *com, *quad, *box_in, *box_out;
+    WalkRec rec;
+    const TreeMeta *meta;
+    const int *pre;
+};
+
+__device__ void walk_rec_store(const WalkRec &w, const TreeMeta *__restrict__ meta, const GNode &nd,
+                               const Moments &v, int pre, long long k)
+{
+    float p[3], ol[3], oh[3], il[3], ih[3];
+    const float m = walk_margin(meta->len, meta->rs_max);
+    for (int d = 0; d < 3; d++) {
+        const double c = meta->root[d] + 0.5 * meta->len;
+        p[d] = (float)(v.c[d] - c);
+        ol[d] = (float)(fmin(v.bo[d], v.bi[d]) - c) - m;
+        oh[d] = (float)(fmax(v.bo[3 + d], v.bi[3 + d]) - c) + m;
+        il[d] = (float)(v.bi[d] - c) - m;
+        ih[d] = (float)(v.bi[3 + d] - c) + m;
+    }
+    w.A[k] = make_float4(p[0], p[1], p[2], __int_as_float((int)nd.begin));
+    w.B[k] = make_float4(ol[0], ol[1], ol[2], __int_as_float((int)nd.end));
+    w.C[k] = make_float4(oh[0], oh[1], oh[2], __int_as_float(nd.level << 8 | nd.n_child));
+    w.D[k] = make_float4(il[0], il[1], il[2], 0.f);
+    w.E[k] = make_float4(ih[0], ih[1], ih[2], 0.f);
+    w.F[k] = make_int2((int)nd.first_child, pre);
+}
+
+__device__ __forceinline__ void moments_store(const Moments &v, const MomentArrays &o, const GNode &nd, long long k)
 {
     o.mass[k] = v.M;
     for (int d = 0; d < 3; d++) o.com[3 * k + d] = v.c[d];
@@ -413,6 +466,7 @@ __device__ __forceinline__ void moments_store(const Moments &v, const MomentArra
         o.box_in[6 * k + d] = v.bi[d];
         o.box_out[6 * k + d] = v.bo[d];
     }
+    walk_rec_store(o.rec, o.meta, nd, v, o.pre[k], k);
 }
 
 // Moments of the leaves, one thread each, the host's sums in its order; the
@@ -471,7 +525,7 @@ __global__ __launch_bounds__(256) void k_leaf_moments(const GNode *__restrict__ 
             v.q[5] += m * y * z;
         }
     }
-    moments_store(v, out, k);
+    moments_store(v, out, nd, k);
 }
 
 // Moments of the inner nodes of [a, b), one level (its children are done).
@@ -509,7 +563,7 @@ __global__ __launch_bounds__(64) void k_inner_moments(const GNode *__restrict__ 
         v.q[4] += qc[4] + m * x * z;
         v.q[5] += qc[5] + m * y * z;
     }
-    moments_store(v, o, k);
+    moments_store(v, o, nd, k);
 }
 
 __global__ __launch_bounds__(64) void k_fill_int(int *__restrict__ p, long long n, int v)
@@ -517,25 +571,70 @@ __global__ __launch_bounds__(64) void k_fill_int(int *__restrict__ p, long long 
     for (long long k = threadIdx.x; k < n; k += 64) p[k] = v;
 }
 
-// per group: first particle, size, list lengths (host copy for the planner)
-__global__ __launch_bounds__(256) void k_group_info(const GNode *__restrict__ nodes, const int *__restrict__ groups,
-                                                    long long ng, const long long *__restrict__ off_e,
-                                                    const long long *__restrict__ off_s, int4 *__restrict__ info)
+// Exclusive sums of up to three count arrays (block b takes in[b]), n + 1
+// entries each; with pad > 0 every count counts as c + c/4 + pad (a region
+// for the next build's list).
+struct Sums {
+    const int *in[3];
+    long long *out[3];
+};
+__global__ __launch_bounds__(1024) void k_sums(long long n, const Sums s, int pad)
 {
-    const long long g = (long long)blockIdx.x * 256 + threadIdx.x;
-    if (g >= ng) return;
-    const GNode G = nodes[groups[g]];
-    info[g] = make_int4((int)G.begin, (int)(G.end - G.begin), (int)(off_e[g + 1] - off_e[g]),
-                        (int)(off_s[g + 1] - off_s[g]));
+    constexpr int U = 4;
+    __shared__ long long ws[16];
+    const int *__restrict__ in = s.in[blockIdx.x];
+    long long *__restrict__ out = s.out[blockIdx.x];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    long long carry = 0;
+    for (long long k0 = 0; k0 < n; k0 += 1024 * U) {
+        const long long k = k0 + U * (long long)threadIdx.x;
+        long long v[U], sum = 0;
+        for (int u = 0; u < U; u++) {
+            const int c = k + u < n ? in[k + u] : 0;
+            v[u] = (pad > 0 && k + u < n) ? (long long)c + c / 4 + pad : c;
+            sum += v[u];
+        }
+        long long inc = sum;
+        for (int off = 1; off < 64; off <<= 1) {
+            const long long t = __shfl_up(inc, off, 64);
+            if (lane >= off) inc += t;
+        }
+        if (lane == 63) ws[wave] = inc;
+        __syncthreads();
+        long long before = carry, total = 0;
+        for (int w = 0; w < 16; w++) {
+            if (w < wave) before += ws[w];
+            total += ws[w];
+        }
+        before += inc - sum;
+        for (int u = 0; u < U; u++) {
+            if (k + u < n) out[k + u] = before;
+            before += v[u];
+        }
+        carry += total;
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) out[n] = carry;
 }
 
-// sort key of an SPJ entry: the node's first particle
-__global__ __launch_bounds__(256) void k_spj_keys(const GNode *__restrict__ nodes, const int *__restrict__ id_spj,
-                                                  long long n, int *__restrict__ key)
+// What the host reads back from a walk, and (behind it) the groups' records
+// {first particle, size, EPJ entries, SPJ entries} for the planner.
+struct WalkTotals {
+    long long e, s, l;
+    int over, pad;
+};
+__global__ __launch_bounds__(256) void k_group_info(const GNode *__restrict__ nodes, const int *__restrict__ groups,
+                                                    long long ng, const int *__restrict__ cnt_e,
+                                                    const int *__restrict__ cnt_s, const long long *__restrict__ off_e,
+                                                    const long long *__restrict__ off_s,
+                                                    const long long *__restrict__ off_l, const int *__restrict__ over,
+                                                    WalkTotals *__restrict__ tot, int4 *__restrict__ info)
 {
-    const long long k = (long long)blockIdx.x * 256 + threadIdx.x;
-    if (k >= n) return;
-    key[k] = (int)nodes[id_spj[k]].begin;
+    const long long g = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (g == 0) *tot = WalkTotals{off_e[ng], off_s ? off_s[ng] : 0, off_l[ng], *over, 0};
+    if (g >= ng) return;
+    const GNode G = nodes[groups[g]];
+    info[g] = make_int4((int)G.begin, (int)(G.end - G.begin), cnt_e[g], cnt_s ? cnt_s[g] : 0);
 }
 
 // resident records from the tree (the conversions of pth_resident_create)
@@ -564,9 +663,10 @@ __global__ __launch_bounds__(256) void k_res_particles(long long n, const double
     epj[k] = j;
 }
 
-__global__ __launch_bounds__(256) void k_res_nodes(long long nn, const double *__restrict__ nmass,
-                                                   const double *__restrict__ ncom, const double *__restrict__ nquad,
-                                                   pth::SpjDev *__restrict__ spj)
+// (the SPJ lists name nodes by preorder number)
+__global__ __launch_bounds__(256) void k_res_nodes(long long nn, const int *__restrict__ pre,
+                                                   const double *__restrict__ nmass, const double *__restrict__ ncom,
+                                                   const double *__restrict__ nquad, pth::SpjDev *__restrict__ spj)
 {
     const long long k = (long long)blockIdx.x * 256 + threadIdx.x;
     if (k >= nn) return;
@@ -583,11 +683,12 @@ __global__ __launch_bounds__(256) void k_res_nodes(long long nn, const double *_
     r.qxz = (float)q[4];
     r.qyz = (float)q[5];
     r.pad[0] = r.pad[1] = r.pad[2] = 0.f;
-    spj[k] = r;
+    spj[pre[k]] = r;
 }
 
 // monopole superparticles: the node's mass at its centre of mass
-__global__ __launch_bounds__(256) void k_res_nodes_mono(long long nn, const double *__restrict__ nmass,
+__global__ __launch_bounds__(256) void k_res_nodes_mono(long long nn, const int *__restrict__ pre,
+                                                        const double *__restrict__ nmass,
                                                         const double *__restrict__ ncom,
                                                         pth::EpjDev *__restrict__ spj)
 {
@@ -599,26 +700,26 @@ __global__ __launch_bounds__(256) void k_res_nodes_mono(long long nn, const doub
     r.z = ncom[3 * k + 2];
     r.m = (float)nmass[k];
     r.rs = 0.f;
-    spj[k] = r;
+    spj[pre[k]] = r;
 }
 
 struct WalkArgs {
-    const GNode *nodes;
+    WalkRec rec;
     const double *ncom, *box_in, *box_out;
+    const TreeMeta *meta;
     const int *groups;
     long long n_group;
-    // tile walks (tbox != null): group g is node groups[g] with the boxes
-    // tbox[12 g ..] (particle box, box widened by r_search) instead of the
-    // node's own
+    // tile walks: group g is node groups[g] with the boxes tbox[12 g ..]
+    // (particle box, box widened by r_search) instead of the node's own
     const double *tbox;
-    double root_len, inv_theta2;
+    double inv_theta2;
     int theta_pos;
-    long long *cnt_e, *cnt_s;                // counting pass (and a padded writing pass)
-    const long long *off_e, *off_s;          // writing pass
-    int *id_epj, *id_spj;
-    // padded writing pass: group g writes into [off[g], off[g + 1]) at most,
-    // skipping what does not fit, and stores its exact counts
-    int padded;
+    int *cnt_e, *cnt_s, *cnt_l;             // EPJ entries, closed nodes, opened leaves
+    // writing pass: group g's region of each raw list; what does not fit is
+    // counted, not written, and sets *over
+    const long long *off_l, *off_s;
+    int *raw_l, *raw_s;  // preorder numbers
+    int *over;
 };
 
 __device__ __forceinline__ bool overlap6(const double *a, const double *b)
@@ -628,42 +729,58 @@ __device__ __forceinline__ bool overlap6(const double *a, const double *b)
     return true;
 }
 
-// inclusive wave scan of v
-__device__ __forceinline__ long long wave_scan(long long v, int lane)
+// false only if boxes (lo, hi) and (l, h) do not meet; NaN bounds meet
+__device__ __forceinline__ bool meet(const float (&lo)[3], const float (&hi)[3], const float4 &l, const float4 &h)
 {
-    for (int off = 1; off < 64; off <<= 1) {
-        const long long t = __shfl_up(v, off, 64);
-        if (lane >= off) v += t;
-    }
-    return v;
+    return !(lo[0] > h.x || l.x > hi[0] || lo[1] > h.y || l.y > hi[1] || lo[2] > h.z || l.z > hi[2]);
 }
 
-// One 64-thread workgroup (one wave) per group at a time.
-template <bool WRITE>
+// One 64-thread workgroup (one wave) per group at a time.  The opening test
+// is decided in FP32 where its bounds, widened by the margin, leave no doubt,
+// and otherwise (a node at the edge of the theta sphere, or whose widened box
+// meets the group's) by the host's FP64 expressions; a tile walk takes every
+// node whose FP32 boxes meet (a superset: its lists are filtered exactly).
+template <bool WRITE, bool TILE>
 __global__ __launch_bounds__(64) void k_walk(const WalkArgs a)
 {
     __shared__ int stk[WALK_STACK];
+    __shared__ float lim[GT_MAX_LEVEL + 1];  // (L / theta)^2 of each level
     const int lane = threadIdx.x;
+    const double len = a.meta->len;
+    const float mg = walk_margin(len, a.meta->rs_max);
+    if (lane <= GT_MAX_LEVEL) {
+        const double L = len / (double)(1LL << lane);
+        lim[lane] = (float)(L * L * a.inv_theta2);
+    }
+    const unsigned long long below = lane ? ~0ull >> (64 - lane) : 0ull;
     for (long long g = blockIdx.x; g < a.n_group; g += gridDim.x) {
-        const int gn = a.groups[g];
-        const GNode G = a.nodes[gn];
-        const long long gb = G.begin, ge = G.end;
-        double bin[6], bout[6];
-        for (int d = 0; d < 6; d++) {
-            bin[d] = a.tbox ? a.tbox[12 * g + d] : a.box_in[6 * (long long)gn + d];
-            bout[d] = a.tbox ? a.tbox[12 * g + 6 + d] : a.box_out[6 * (long long)gn + d];
+        const long long gn = a.groups[g];
+        const int gb = __float_as_int(a.rec.A[gn].w), ge = __float_as_int(a.rec.B[gn].w);
+        const double *bin = TILE ? a.tbox + 12 * g : a.box_in + 6 * gn;
+        const double *bout = TILE ? a.tbox + 12 * g + 6 : a.box_out + 6 * gn;
+        // the group's boxes: the particle box as it rounds, both pushed out
+        float bl[3], bh[3], il[3], ih[3], ol[3], oh[3];
+        for (int d = 0; d < 3; d++) {
+            const double c = a.meta->root[d] + 0.5 * len;
+            bl[d] = (float)(bin[d] - c);
+            bh[d] = (float)(bin[3 + d] - c);
+            il[d] = bl[d] - mg;
+            ih[d] = bh[d] + mg;
+            ol[d] = (float)(fmin(bout[d], bin[d]) - c) - mg;
+            oh[d] = (float)(fmax(bout[3 + d], bin[3 + d]) - c) + mg;
         }
-        long long ne = 0, ns = 0;
-        int *oe = nullptr, *os = nullptr;
-        long long cap_e = LLONG_MAX, cap_s = LLONG_MAX;
+        int my_e = 0, nl = 0, ns = 0;
+        int *ol_raw = nullptr, *os_raw = nullptr;
+        long long cap_l = 0, cap_s = 0;
         if (WRITE) {
-            oe = a.id_epj + a.off_e[g];
-            if (a.id_spj) os = a.id_spj + a.off_s[g];
-            if (a.padded) {
-                cap_e = a.off_e[g + 1] - a.off_e[g];
-                if (a.id_spj) cap_s = a.off_s[g + 1] - a.off_s[g];
+            ol_raw = a.raw_l + a.off_l[g];
+            cap_l = a.off_l[g + 1] - a.off_l[g];
+            if (!TILE) {
+                os_raw = a.raw_s + a.off_s[g];
+                cap_s = a.off_s[g + 1] - a.off_s[g];
             }
         }
+        __syncthreads();
         if (lane == 0) stk[0] = 0;
         int size = 1;
         __syncthreads();
@@ -678,74 +795,315 @@ __global__ __launch_bounds__(64) void k_walk(const WalkArgs a)
             int c = 0;
             if (act) c = stk[size - 1 - lane];
             __syncthreads();
-            long long me = 0, mc = 0, ms = 0;
-            GNode nd{0, 0, 0, 0, 0};
+            bool open = false;
+            int begin = 0, end = 0, kids = 0;
+            int2 F = make_int2(-1, 0);
             if (act) {
-                nd = a.nodes[c];
-                bool open;
-                if (nd.begin <= gb && ge <= nd.end) open = true;
-                else if (!a.theta_pos) open = true;
-                else {
-                    const double L = a.root_len / (double)(1LL << nd.level);
-                    double s = 0;
-                    for (int d = 0; d < 3; d++) {
-                        const double p = a.ncom[3 * (long long)c + d];
-                        double e = 0;
-                        if (p < bin[d]) e = bin[d] - p;
-                        else if (p > bin[3 + d]) e = p - bin[3 + d];
-                        s += e * e;
-                    }
-                    open = s < L * L * a.inv_theta2 || overlap6(bout, a.box_in + 6 * (long long)c) ||
-                           overlap6(bin, a.box_out + 6 * (long long)c);
-                }
-                if (open) {
-                    if (nd.n_child == 0) me = nd.end - nd.begin;
-                    else mc = nd.n_child;
+                const float4 A = a.rec.A[c], B = a.rec.B[c], C = a.rec.C[c];
+                F = a.rec.F[c];
+                begin = __float_as_int(A.w);
+                end = __float_as_int(B.w);
+                const int lv = __float_as_int(C.w);
+                kids = lv & 255;
+                if ((begin <= gb && ge <= end) || !a.theta_pos) open = true;
+                else if (TILE) {
+                    const float4 D = a.rec.D[c], E = a.rec.E[c];
+                    open = meet(ol, oh, D, E) || meet(il, ih, B, C);
                 } else {
-                    ms = 1;
+                    const float p[3] = {A.x, A.y, A.z};
+                    float far = 0.f, near = 0.f;  // bounds of the squared distance
+                    for (int d = 0; d < 3; d++) {
+                        const float e = fmaxf(fmaxf(bl[d] - p[d], p[d] - bh[d]), 0.f);
+                        const float ep = e + mg, em = fmaxf(e - mg, 0.f);
+                        far = __builtin_fmaf(ep, ep, far);
+                        near = __builtin_fmaf(em, em, near);
+                    }
+                    const float T = lim[lv >> 8];
+                    if (far * 1.00001f < T * 0.99999f) open = true;
+                    else if (!(near * 0.99999f > T * 1.00001f) || meet(ol, oh, B, C)) {
+                        const double L = len / (double)(1LL << (lv >> 8));
+                        double s = 0;
+                        for (int d = 0; d < 3; d++) {
+                            const double q = a.ncom[3 * (long long)c + d];
+                            double e = 0;
+                            if (q < bin[d]) e = bin[d] - q;
+                            else if (q > bin[3 + d]) e = q - bin[3 + d];
+                            s += e * e;
+                        }
+                        open = s < L * L * a.inv_theta2 || overlap6(bout, a.box_in + 6 * (long long)c) ||
+                               overlap6(bin, a.box_out + 6 * (long long)c);
+                    }
                 }
             }
-            // the three counts scanned as one word: EPJ entries in bits 0-31
-            // (a step's popped leaves are distinct, so their total is at most
-            // n < 2^31), children in 32-47 (at most 8 per lane), SPJ entries
-            // in 48-63 (at most 1 per lane)
-            const long long pk = wave_scan(me | (mc << 32) | (ms << 48), lane);
-            const long long tk = __shfl(pk, 63, 64);
-            const long long pe = pk & 0xffffffffLL, pc = (pk >> 32) & 0xffff, ps = (pk >> 48) & 0xffff;
-            const long long te = tk & 0xffffffffLL, tc = (tk >> 32) & 0xffff, ts = (tk >> 48) & 0xffff;
+            const bool leaf = open && kids == 0, closed = act && !open;
+            const int mc = (open && !leaf) ? kids : 0;
+            const unsigned long long ml = __ballot(leaf), ms = TILE ? 0ull : __ballot(closed);
+            // exclusive sum of the child counts (0 .. 8) from their bits
+            int pc = 0, tc = 0;
+#pragma unroll
+            for (int b = 0; b < 4; b++) {
+                const unsigned long long m = __ballot((mc >> b) & 1);
+                pc += __popcll(m & below) << b;
+                tc += __popcll(m) << b;
+            }
+            if (leaf) my_e += end - begin;
             if (WRITE) {
-                for (long long t = 0; t < me; t++) {
-                    const long long k = ne + pe - me + t;
-                    if (k < cap_e) oe[k] = (int)(nd.begin + t);
-                }
-                if (ms && os && ns + ps - 1 < cap_s) os[ns + ps - 1] = c;
+                const int pl = nl + __popcll(ml & below), ps = ns + __popcll(ms & below);
+                if (leaf && pl < cap_l) ol_raw[pl] = F.y;
+                if (!TILE && closed && ps < cap_s) os_raw[ps] = F.y;
             }
-            ne += te;
-            ns += ts;
+            nl += __popcll(ml);
+            ns += __popcll(ms);
             size -= k;
-            for (long long t = 0; t < mc; t++) stk[size + (pc - mc) + t] = (int)(nd.first_child + (mc - 1 - t));
-            size += (int)tc;
+            for (int t = 0; t < mc; t++) stk[size + pc + t] = F.x + (mc - 1 - t);
+            size += tc;
             __syncthreads();
         }
-        if ((!WRITE || a.padded) && lane == 0) {
-            a.cnt_e[g] = ne;
-            if (a.cnt_s) a.cnt_s[g] = ns;
+        for (int off = 32; off > 0; off >>= 1) my_e += __shfl_xor(my_e, off, 64);
+        if (lane == 0) {
+            a.cnt_e[g] = my_e;
+            a.cnt_l[g] = nl;
+            if (!TILE) a.cnt_s[g] = ns;
+            if (WRITE && (nl > cap_l || ns > cap_s)) atomicOr(a.over, 1);
         }
+    }
+}
+
+// The final lists from the raw ones, one workgroup per group or tile.  The raw
+// entries are preorder numbers, and a depth-first walk's order is their
+// ascending order, so a list is put in order without moving it: each entry
+// sets a bit of a map of the tree's nodes in LDS (a window of it at a time,
+// for trees of more nodes), and the set bits are read off in order.  A
+// segmented radix sort moved every particle and node entry through memory
+// three times (1,048,576 particles, 34M + 53M entries: 1.9 ms with its keys,
+// and 0.17 ms to move the lists to their places; 0.21 ms here.  4,194,304
+// particles: 7.9 and 2.0 ms).
+struct OrderArgs {
+    const int2 *range;  // first particle and size of each node, in preorder
+    int n_words;        // of the node map
+    int window;         // words of it held in LDS
+    long long n_group;
+    const int *cnt_l;
+    const long long *roff_l, *roff_s, *off_e, *off_s;
+    const int *raw_l, *raw_s;
+    int *sort_l;  // room for long ordered leaf lists, in raw_l's layout
+    int *id_epj, *id_spj;
+};
+
+// Inclusive wave sum in the vector ALU's own lane shifts (DPP): six
+// dependent adds, where six LDS permutes would each wait for LDS.
+__device__ __forceinline__ int wave_inclusive(int v)
+{
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr:1
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);  // row_shr:2
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);  // row_shr:4
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);  // row_shr:8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1, 3
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2, 3
+    return v;
+}
+
+// Sets the bits of the m entries of raw that fall into words [w0, w0 + nw) of
+// the map and returns whether this thread set any.  Neighbouring entries are siblings, i.e.
+// bits of one word: a thread takes a run of entries (in aligned quads, which
+// may hold up to three words before and after the region's entries) and
+// joins the bits of a word before its LDS atomic, and the threads of a wave
+// are on different words (lane-strided entries met on a few words and waited
+// for each other).
+template <int WG>
+__device__ __forceinline__ int set_bits(const int *__restrict__ raw, int m, int w0, int nw, unsigned *map)
+{
+    const int lead = (int)((reinterpret_cast<size_t>(raw) >> 2) & 3);
+    const int4 *quads = reinterpret_cast<const int4 *>(raw - lead);
+    const int nq = (m + lead + 3) >> 2;
+    const int q0 = (int)((long long)nq * threadIdx.x / WG), q1 = (int)((long long)nq * (threadIdx.x + 1) / WG);
+    int word = -1, any = 0;
+    unsigned bits = 0;
+    auto flush = [&]() {
+        if (word < 0 || word >= nw) return;
+        atomicOr(&map[word], bits);
+        any = 1;
+    };
+    for (int q = q0; q < q1; q++) {
+        const int4 v4 = quads[q];
+        const int v[4] = {v4.x, v4.y, v4.z, v4.w};
+        const int k = 4 * q - lead;  // entry of v[0]
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            if (k + u < 0 || k + u >= m) continue;
+            const int w = (v[u] >> 5) - w0;
+            if (w != word) {
+                flush();
+                word = w;
+                bits = 0;
+            }
+            bits |= 1u << (v[u] & 31);
+        }
+    }
+    flush();
+    return any;
+}
+
+// The m entries of raw to out in ascending order: an entry's place is the
+// number of bits set below its own, i.e. the sum of its chunk of 64 words
+// (sums), of its word in the chunk (below) and the bits below in the word.
+// So every entry is placed by itself; reading the bits off word by word left
+// most lanes idle, the near cells' bits being packed into a few words.  All
+// threads of the block call it; map, below and sums hold `window` words.
+template <int WG>
+__device__ void order_by_map(const int *__restrict__ raw, int m, int n_words, int window, unsigned *map, int *wtot,
+                             int *out)
+{
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    constexpr int NW = WG / 64, U = 4;
+    int *sums = reinterpret_cast<int *>(map + window);
+    unsigned short *below = reinterpret_cast<unsigned short *>(sums + (window + 63) / 64);
+    int done = 0;
+    for (int w0 = 0; w0 < n_words; w0 += window) {
+        const int nw = min(window, n_words - w0), nc = (nw + 63) >> 6;
+        for (int k = tid; k < nw; k += WG) map[k] = 0u;
+        __syncthreads();
+        // (a leaf list often leaves a window empty)
+        if (!__syncthreads_or(set_bits<WG>(raw, m, w0, nw, map))) continue;
+        for (int c = wave; c < nc; c += NW) {
+            const int k = c * 64 + lane;
+            const int own = k < nw ? __popc(map[k]) : 0, inc = wave_inclusive(own);
+            if (k < nw) below[k] = (unsigned short)(inc - own);
+            if (lane == 63) sums[c] = inc;
+        }
+        __syncthreads();
+        if (wave == 0) {
+            int carry = 0;
+            for (int c0 = 0; c0 < nc; c0 += 64) {
+                const int own = c0 + lane < nc ? sums[c0 + lane] : 0, inc = wave_inclusive(own);
+                if (c0 + lane < nc) sums[c0 + lane] = carry + inc - own;
+                carry += __builtin_amdgcn_readlane(inc, 63);
+            }
+            if (lane == 0) *wtot = carry;
+        }
+        __syncthreads();
+        for (int k0 = tid; k0 < m; k0 += WG * U) {
+            int v[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) v[u] = k0 + u * WG < m ? raw[k0 + u * WG] : -1;
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int q = (v[u] >> 5) - w0;
+                if (v[u] < 0 || q < 0 || q >= nw) continue;
+                out[done + sums[q >> 6] + below[q] + __popc(map[q] & ((1u << (v[u] & 31)) - 1u))] = v[u];
+            }
+        }
+        done += *wtot;
+        __syncthreads();
+    }
+}
+// LDS bytes of a map of `window` words (even) with its sums.
+constexpr size_t map_bytes(int window) { return 6 * (size_t)window + 4 * (size_t)((window + 63) / 64); }
+
+// Writes the particles of m leaves (preorder numbers, in order) to out.  All
+// threads of the block call it; eight lanes write a leaf.
+template <int WG, int RMAX>
+__device__ void expand_leaves(const int *leaves, int m, const int2 *__restrict__ range, int *l_begin, int *l_off,
+                              int *wsum, int *__restrict__ out)
+{
+    static_assert(RMAX % WG == 0, "leaves per pass");
+    constexpr int PER = RMAX / WG, NW = WG / 64;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    int done = 0;  // entries written
+    for (int l0 = 0; l0 < m; l0 += RMAX) {
+        const int nl = min(RMAX, m - l0);
+        int v[PER], sum = 0;
+        for (int u = 0; u < PER; u++) {
+            const int k = tid * PER + u;
+            v[u] = 0;
+            if (k < nl) {
+                const int2 q = range[leaves[l0 + k]];
+                l_begin[k] = q.x;
+                v[u] = q.y;
+            }
+            sum += v[u];
+        }
+        const int inc = wave_inclusive(sum);
+        if (lane == 63) wsum[wave] = inc;
+        __syncthreads();
+        int before = inc - sum, total = 0;
+        for (int w = 0; w < NW; w++) {
+            if (w < wave) before += wsum[w];
+            total += wsum[w];
+        }
+        for (int u = 0; u < PER; u++) {
+            l_off[tid * PER + u] = before;
+            before += v[u];
+        }
+        if (tid == WG - 1) l_off[RMAX] = before;
+        __syncthreads();
+        for (int k = tid >> 3; k < nl; k += WG / 8) {
+            const int o = l_off[k], n = l_off[k + 1] - o, p = l_begin[k];
+            for (int j = tid & 7; j < n; j += 8) out[done + o + j] = p + j;
+        }
+        done += total;
         __syncthreads();
     }
 }
 
-// Group g's list, written by a padded walk at poff[g], moved to off[g]
-// (off[g + 1] - off[g] entries, checked on the host to fit the region).
-__global__ __launch_bounds__(256) void k_compact(long long ng, const long long *__restrict__ poff,
-                                                 const long long *__restrict__ off, const int *__restrict__ src,
-                                                 int *__restrict__ dst)
+// Groups: SORT for canonical order, else batch order.
+template <int WG, int RMAX, bool SORT> __global__ __launch_bounds__(WG) void k_order(const OrderArgs a)
 {
-    for (long long g = blockIdx.x; g < ng; g += gridDim.x) {
-        const long long n = off[g + 1] - off[g];
-        const int *s = src + poff[g];
-        int *d = dst + off[g];
-        for (long long k = threadIdx.x; k < n; k += 256) d[k] = s[k];
+    extern __shared__ unsigned map[];
+    __shared__ int l_pre[SORT ? RMAX : 1], l_begin[RMAX], l_off[RMAX + 1], wsum[WG / 64];
+    for (long long g = blockIdx.x; g < a.n_group; g += gridDim.x) {
+        const int ms = (int)(a.off_s[g + 1] - a.off_s[g]), ml = a.cnt_l[g];
+        const int *raw_s = a.raw_s + a.roff_s[g], *leaves = a.raw_l + a.roff_l[g];
+        int *out_s = a.id_spj + a.off_s[g];
+        if constexpr (SORT) {
+            // ordered leaves: in LDS when they fit
+            int *sorted = ml <= RMAX ? l_pre : a.sort_l + a.roff_l[g];
+            order_by_map<WG>(raw_s, ms, a.n_words, a.window, map, wsum, out_s);
+            order_by_map<WG>(leaves, ml, a.n_words, a.window, map, wsum, sorted);
+            leaves = sorted;
+            __threadfence_block();
+            __syncthreads();
+        } else {
+            for (int k = threadIdx.x; k < ms; k += WG) out_s[k] = raw_s[k];
+        }
+        expand_leaves<WG, RMAX>(leaves, ml, a.range, l_begin, l_off, wsum, a.id_epj + a.off_e[g]);
+    }
+}
+
+// Neighbour-search tiles (leaf lists only, a dozen entries each), one wave
+// per tile: an entry's rank is the number of smaller ones; lists of more than
+// RMAX entries (degenerate trees) go through the map.
+template <int RMAX> __global__ __launch_bounds__(64) void k_order_tiles(const OrderArgs a)
+{
+    extern __shared__ unsigned map[];
+    __shared__ __attribute__((aligned(16))) int l_raw[RMAX];
+    __shared__ int l_pre[RMAX], l_begin[RMAX], l_off[RMAX + 1], wsum[1];
+    static_assert(RMAX % 64 == 0, "leaves per pass");
+    const int lane = threadIdx.x;
+    for (long long g = blockIdx.x; g < a.n_group; g += gridDim.x) {
+        const int m = a.cnt_l[g];
+        const int *raw = a.raw_l + a.roff_l[g];
+        int *sorted = l_pre;
+        if (m <= RMAX) {
+            const int m4 = (m + 3) & ~3;
+            for (int k = lane; k < m4; k += 64) l_raw[k] = k < m ? raw[k] : INT_MAX;
+            __syncthreads();
+            for (int k = lane; k < m; k += 64) {
+                const int v = l_raw[k];
+                int r = 0;
+                for (int j = 0; j < m4; j += 4) {
+                    const int4 q = *reinterpret_cast<const int4 *>(l_raw + j);
+                    r += (q.x < v) + (q.y < v) + (q.z < v) + (q.w < v);
+                }
+                l_pre[r] = v;
+            }
+        } else {
+            sorted = a.sort_l + a.roff_l[g];
+            order_by_map<64>(raw, m, a.n_words, a.window, map, wsum, sorted);
+            __threadfence_block();
+        }
+        __syncthreads();
+        expand_leaves<64, RMAX>(sorted, m, a.range, l_begin, l_off, wsum, a.id_epj + a.off_e[g]);
     }
 }
 
@@ -799,17 +1157,6 @@ __global__ __launch_bounds__(256) void k_tile_boxes(const int *__restrict__ tile
         tbox[12 * t + 6 + d] = lo2 - (fabs(lo2) + rs_max) * m;
         tbox[12 * t + 9 + d] = hi2 + (fabs(hi2) + rs_max) * m;
     }
-}
-
-// per tile: first particle, size, candidate count (k_ngb's group record)
-__global__ __launch_bounds__(256) void k_tile_info(const GNode *__restrict__ nodes, const int *__restrict__ tiles,
-                                                   long long nt, const long long *__restrict__ off,
-                                                   int4 *__restrict__ info)
-{
-    const long long t = (long long)blockIdx.x * 256 + threadIdx.x;
-    if (t >= nt) return;
-    const GNode c = nodes[tiles[t]];
-    info[t] = make_int4((int)c.begin, (int)(c.end - c.begin), (int)(off[t + 1] - off[t]), 0);
 }
 
 // Neighbour search (src/soft_force.hpp:11-34, SearchNeighborEpEpNoSimd) on
@@ -979,29 +1326,45 @@ __global__ __launch_bounds__(64) void k_ngb(const NgbArgs a)
 // ---------------------------------------------------------------------------
 // host side
 
+// The lists of a walk: counts per group (EPJ entries, closed nodes, opened
+// leaves), offsets, the raw lists and their regions, the read-back.  Kept
+// from walk to walk: the counts size the next one's regions.
+struct WalkLists {
+    DevBuf cnt, off, reg, raw_l, raw_s, sort_l, back;
+    PinBuf host;  // WalkTotals, then one int4 per group
+    long long n = -1, tot_l = 0, tot_s = 0;
+    int passes = 0;
+    const int4 *info() const { return reinterpret_cast<const int4 *>(host.as<WalkTotals>() + 1); }
+    void release()
+    {
+        for (DevBuf *b : {&cnt, &off, &reg, &raw_l, &raw_s, &sort_l, &back}) b->release();
+        host.release();
+    }
+};
+
 struct pth_gtree {
     pth_ctx *ctx = nullptr;
     long long n = 0, n_node = 0, n_group = 0, n_tile = 0, n_le = 0, n_ls = 0;
-    DevBuf order, key, skey, sidx, sidx2, spos, smass, srs, nodes, nmass, ncom, nquad, box_in, box_out, groups, off_e, off_s,
+    DevBuf order, key, skey, sidx, sidx2, spos, smass, srs, nodes, nmass, ncom, nquad, box_in, box_out, rec, groups,
         id_epj, id_spj, tmp;
+    WalkLists walk, tile_walk;  // the group walk, the neighbour search's
+    WalkRec walk_rec() const
+    {
+        float4 *p = rec.as<float4>();
+        return WalkRec{p, p + n_node, p + 2 * n_node, p + 3 * n_node, p + 4 * n_node,
+                       reinterpret_cast<int2 *>(p + 5 * n_node)};
+    }
     // build-time scratch, released when the build ends (or by pth_gtree_free)
-    DevBuf dpos, dmass, drs, part, cnt, off, starts, ce, cs, alt, lkey, lkey2, info;
+    DevBuf dpos, dmass, drs, part, cnt, off, starts;
     // neighbour lists (pth_gtree_neighbors): count per input index, offsets,
-    // entries; tile boxes, candidate counts / offsets / lists, tile records
-    DevBuf ngb_cnt, ngb_off, ngb, tiles, tbox, tcnt, toff, tl, tl_alt, tinfo;
-    // one-pass walks: list regions sized from the previous build's lengths
-    // (padded offsets, EPJ then SPJ), the lists written there
-    DevBuf pad_off, pad_e, pad_s;
-    std::vector<long long> pad_h;
+    // entries; tiles, tile boxes, candidate lists
+    DevBuf ngb_cnt, ngb_off, ngb, tiles, tbox, tl;
     int walk_passes = 0;  // of the last build: 1 (one padded pass) or 2 (count, then write)
     DevBuf meta;             // TreeMeta of the last build
     DevBuf pre, node_at;     // preorder number of each node, and the inverse
+    DevBuf range;            // the nodes' particle ranges, in preorder
     void *pinned = nullptr;  // pinned host copy of meta
     hipEvent_t ev_meta = nullptr;  // that copy
-    // one-pass tile walks of the neighbour search: the last search's
-    // candidate counts per tile (nt + 1 entries), padded offsets, lists
-    std::vector<long long> tcnt_h, tpad_h;
-    DevBuf tpad_off, tl_pad;
     int tile_passes = 0;  // of the last search's tile walk
     // one-pass neighbour filters: regions from the last completed search's
     // per-particle counts (ngb_cnt), valid while ngb_prev_ok
@@ -1014,7 +1377,7 @@ struct pth_gtree {
     float ms_ngb = 0.f;
     void release_scratch()
     {
-        DevBuf *s[] = {&dpos, &dmass, &drs, &part, &cnt, &off, &starts, &ce, &cs, &alt, &lkey, &lkey2, &info};
+        DevBuf *s[] = {&dpos, &dmass, &drs, &part, &cnt, &off, &starts};
         for (DevBuf *b : s) b->release();
     }
     std::vector<int4> groups_h;  // per group: first particle, size, n_epj, n_spj
@@ -1060,6 +1423,128 @@ hipError_t cub_temp(pth_gtree *t, size_t bytes) { return t->tmp.ensure(std::max<
 
 namespace {
 
+// The tree's part of a walk's arguments.
+WalkArgs walk_args(pth_gtree *t)
+{
+    WalkArgs wa{};
+    wa.rec = t->walk_rec();
+    wa.ncom = t->ncom.as<double>();
+    wa.box_in = t->box_in.as<double>();
+    wa.box_out = t->box_out.as<double>();
+    wa.meta = t->meta.as<TreeMeta>();
+    return wa;
+}
+
+// Walks the groups of wa into W's raw lists and reads the counts back: one
+// writing pass into regions of the last walk's lengths when that was a walk
+// of as many groups (and again_ok says its counts still stand), else a
+// counting pass; the writing pass that either may still need is walk_finish's.
+template <bool TILE> int walk_run(pth_gtree *t, WalkArgs &wa, WalkLists &W, bool again_ok, long long ng)
+{
+    pth_ctx *ctx = t->ctx;
+    hipStream_t st = ctx->stream;
+    hipError_t e;
+    const bool again = ng > 0 && again_ok && W.n == ng;
+    W.n = -1;  // the counts are about to be rewritten
+    W.passes = 0;
+    const size_t nc = (size_t)ng + 1, bytes = sizeof(WalkTotals) + sizeof(int4) * (size_t)ng;
+    if ((e = W.cnt.ensure(sizeof(int) * (3 * nc + 1))) || (e = W.off.ensure(8 * 3 * nc)) ||
+        (e = W.reg.ensure(8 * 2 * nc)) || (e = W.back.ensure(bytes)) || (e = W.host.ensure(bytes)))
+        return ctx->hip_fail(e, "walk allocation");
+    wa.cnt_e = W.cnt.as<int>();
+    wa.cnt_s = wa.cnt_e + nc;
+    wa.cnt_l = wa.cnt_s + nc;
+    wa.over = wa.cnt_l + nc;
+    long long *off_e = W.off.as<long long>(), *off_s = off_e + nc, *off_l = off_s + nc;
+    long long *reg_l = W.reg.as<long long>(), *reg_s = reg_l + nc;
+    const unsigned wg = (unsigned)std::min<long long>(ng, 65536);
+    hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, st, wa.over, 1, 0);
+    if (again) {
+        // (a tile has a dozen leaves: 64 spare ones each would be mostly holes)
+        const int pad = TILE ? 8 : 64;
+        // (the regions' sum: each at most its length + 1/4 + pad)
+        auto room = [&](long long n) { return 4 * (size_t)(n + n / 4 + pad * ng + 64); };
+        if ((e = W.raw_l.ensure(room(W.tot_l))) || (!TILE && (e = W.raw_s.ensure(room(W.tot_s)))))
+            return ctx->hip_fail(e, "raw list allocation");
+        const Sums s{{wa.cnt_l, wa.cnt_s, nullptr}, {reg_l, reg_s, nullptr}};
+        hipLaunchKernelGGL(k_sums, dim3(TILE ? 1 : 2), dim3(1024), 0, st, ng, s, pad);
+        wa.off_l = reg_l;
+        wa.off_s = reg_s;
+        wa.raw_l = W.raw_l.as<int>();
+        wa.raw_s = W.raw_s.as<int>();
+        hipLaunchKernelGGL((k_walk<true, TILE>), dim3(wg), dim3(64), 0, st, wa);
+    } else if (ng > 0) {
+        hipLaunchKernelGGL((k_walk<false, TILE>), dim3(wg), dim3(64), 0, st, wa);
+    }
+    const Sums s{{wa.cnt_e, wa.cnt_l, wa.cnt_s}, {off_e, off_l, off_s}};
+    hipLaunchKernelGGL(k_sums, dim3(TILE ? 2 : 3), dim3(1024), 0, st, ng, s, 0);
+    hipLaunchKernelGGL(k_group_info, dim3(std::max(1u, blocks(ng))), dim3(256), 0, st, t->nodes.as<GNode>(), wa.groups,
+                       ng, wa.cnt_e, TILE ? nullptr : wa.cnt_s, off_e, TILE ? nullptr : off_s, off_l, wa.over,
+                       W.back.as<WalkTotals>(), reinterpret_cast<int4 *>(W.back.as<WalkTotals>() + 1));
+    // (a tile walk's records stay on the device)
+    if ((e = hipGetLastError()) ||
+        (e = hipMemcpyAsync(W.host.p, W.back.p, TILE ? sizeof(WalkTotals) : bytes, hipMemcpyDeviceToHost, st)) ||
+        (e = hipStreamSynchronize(st)))
+        return ctx->hip_fail(e, "tree walk");
+    const WalkTotals &tot = *W.host.as<WalkTotals>();
+    W.tot_l = tot.l;
+    W.tot_s = tot.s;
+    W.n = ng;
+    W.passes = again && !tot.over ? 1 : 2;
+    return PTH_OK;
+}
+
+// The writing pass, if one is due, and the final lists.
+template <bool TILE> int walk_finish(pth_gtree *t, WalkArgs &wa, WalkLists &W, bool canonical, int *id_epj, int *id_spj)
+{
+    pth_ctx *ctx = t->ctx;
+    hipStream_t st = ctx->stream;
+    hipError_t e;
+    const long long ng = wa.n_group;
+    if (ng <= 0) return PTH_OK;
+    const size_t nc = (size_t)ng + 1;
+    long long *off_e = W.off.as<long long>(), *off_s = off_e + nc, *off_l = off_s + nc;
+    if (W.passes == 2) {
+        if ((e = W.raw_l.ensure(4 * (size_t)(W.tot_l + 8))) ||
+            (!TILE && (e = W.raw_s.ensure(4 * (size_t)(W.tot_s + 8)))))
+            return ctx->hip_fail(e, "raw list allocation");
+        wa.off_l = off_l;
+        wa.off_s = off_s;
+        wa.raw_l = W.raw_l.as<int>();
+        wa.raw_s = W.raw_s.as<int>();
+        hipLaunchKernelGGL((k_walk<true, TILE>), dim3((unsigned)std::min<long long>(ng, 65536)), dim3(64), 0, st, wa);
+    }
+    if ((e = W.sort_l.ensure(W.raw_l.cap))) return ctx->hip_fail(e, "leaf list allocation");
+    OrderArgs o{};
+    o.range = t->range.as<int2>();
+    o.n_words = (int)((t->n_node + 31) / 32);
+    o.n_group = ng;
+    o.cnt_l = wa.cnt_l;
+    o.roff_l = wa.off_l;
+    o.roff_s = wa.off_s;
+    o.off_e = off_e;
+    o.off_s = off_s;
+    o.raw_l = wa.raw_l;
+    o.raw_s = wa.raw_s;
+    o.sort_l = W.sort_l.as<int>();
+    o.id_epj = id_epj;
+    o.id_spj = id_spj;
+    const dim3 grid((unsigned)std::min<long long>(ng, 65536));
+    // map windows: 36 KB for a group (three workgroups of 512 per CU; trees of
+    // up to 196,608 nodes in one window), 3 KB for a tile
+    if constexpr (TILE) {
+        o.window = std::min(o.n_words, 512);
+        hipLaunchKernelGGL(k_order_tiles<256>, grid, dim3(64), map_bytes(o.window), st, o);
+    } else {
+        o.window = std::min(o.n_words, 6144);
+        if (canonical)
+            hipLaunchKernelGGL((k_order<512, 1024, true>), grid, dim3(512), map_bytes(o.window), st, o);
+        else hipLaunchKernelGGL((k_order<512, 1024, false>), grid, dim3(512), 0, st, o);
+    }
+    if ((e = hipGetLastError())) return ctx->hip_fail(e, "list kernels");
+    return PTH_OK;
+}
+
 // Builds (or rebuilds, reusing t's device memory) the tree of n particles.
 // pos / mass / rs are host arrays, or device arrays when on_device.
 int gtree_run(pth_gtree *t, long long n, const double *pos, const double *mass, const double *r_search,
@@ -1103,7 +1588,7 @@ int gtree_run(pth_gtree *t, long long n, const double *pos, const double *mass, 
         return ctx->hip_fail(e, "bbox");
     TreeMeta *meta = t->meta.as<TreeMeta>();
     hipLaunchKernelGGL(k_bbox, dim3(nb), dim3(256), 0, st, dpos, drs, n, part.as<double>());
-    hipLaunchKernelGGL(k_root, dim3(1), dim3(64), 0, st, part.as<double>(), nb, meta);
+    hipLaunchKernelGGL(k_root, dim3(1), dim3(1024), 0, st, part.as<double>(), nb, meta);
     // 2. keys, stable sort of (key, index), sorted particles
     if ((e = t->key.ensure(8 * (size_t)n)) || (e = t->skey.ensure(8 * (size_t)n)) ||
         (e = t->sidx.ensure(4 * (size_t)n)) || (e = t->sidx2.ensure(4 * (size_t)n)) ||
@@ -1155,19 +1640,21 @@ int gtree_run(pth_gtree *t, long long n, const double *pos, const double *mass, 
     t->n_group = M.n_group;
     t->n_tile = M.n_tile;
     if ((e = t->nodes.ensure(sizeof(GNode) * nn)) || (e = t->pre.ensure(4 * nn)) || (e = t->node_at.ensure(4 * nn)) ||
+        (e = t->range.ensure(8 * nn)) ||
         (e = t->groups.ensure(4 * t->n_group)) || (e = t->tiles.ensure(4 * t->n_tile)))
         return ctx->hip_fail(e, "node allocation");
     hipLaunchKernelGGL(k_nodes, dim3(nblk), dim3(256), 0, st, n, nblk, t->off.as<int>(), t->starts.as<unsigned>(),
                        t->nodes.as<GNode>(), t->pre.as<int>(), t->node_at.as<int>(), t->groups.as<int>(),
                        t->tiles.as<int>());
     hipLaunchKernelGGL(k_node_ends, dim3(blocks(nn)), dim3(256), 0, st, t->nodes.as<GNode>(), nn, n, n_leaf_limit,
-                       skey);
+                       skey, t->pre.as<int>(), t->range.as<int2>());
     // 4. moments: the leaves, then the inner nodes level by level
     if ((e = t->nmass.ensure(8 * nn)) || (e = t->ncom.ensure(24 * nn)) || (e = t->nquad.ensure(48 * nn)) ||
         (e = t->box_in.ensure(48 * nn)) || (e = t->box_out.ensure(48 * nn)))
         return ctx->hip_fail(e, "moment allocation");
+    if ((e = t->rec.ensure((5 * sizeof(float4) + sizeof(int2)) * (size_t)nn))) return ctx->hip_fail(e, "node records");
     const MomentArrays mo{t->nmass.as<double>(), t->ncom.as<double>(), t->nquad.as<double>(), t->box_in.as<double>(),
-                          t->box_out.as<double>()};
+                          t->box_out.as<double>(), t->walk_rec(), meta, t->pre.as<int>()};
     hipLaunchKernelGGL(k_leaf_moments, dim3(blocks(nn)), dim3(256), 0, st, t->nodes.as<GNode>(), nn,
                        t->spos.as<double>(), t->smass.as<double>(), t->srs.as<double>(), mo);
     for (int l = GT_MAX_LEVEL; l >= 0; l--) {
@@ -1178,159 +1665,36 @@ int gtree_run(pth_gtree *t, long long n, const double *pos, const double *mass, 
                            t->nodes.as<GNode>(), a, b, mo);
     }
     const long long ng = t->n_group;
-    if ((e = hipStreamSynchronize(st))) return ctx->hip_fail(e, "tree build");
     const auto t1 = std::chrono::steady_clock::now();
     t->ms_build = std::chrono::duration<float, std::milli>(t1 - t0).count();
-    // 6. walk. With the previous build's list lengths per group at hand (same
+    // 5. walk.  With the previous build's list lengths per group at hand (same
     //    number of groups: a rebuild of slowly moving particles), one writing
     //    pass into regions of those lengths + 1/4 + 64 that also counts;
-    //    otherwise a counting pass first.  Either way the exact counts give
-    //    the list offsets; a region that turned out too small (checked on the
-    //    host) means a second, exact writing pass.
-    WalkArgs wa{};
-    wa.nodes = t->nodes.as<GNode>();
-    wa.ncom = t->ncom.as<double>();
-    wa.box_in = t->box_in.as<double>();
-    wa.box_out = t->box_out.as<double>();
+    //    otherwise a counting pass first.  A list that outgrew its region
+    //    means a second, exact writing pass.
+    WalkArgs wa = walk_args(t);
     wa.groups = t->groups.as<int>();
     wa.n_group = ng;
-    wa.root_len = len;
     wa.inv_theta2 = (theta > 0) ? 1.0 / (theta * theta) : 0.0;
     wa.theta_pos = theta > 0;
-    DevBuf &ce = t->ce, &cs = t->cs;
-    if ((e = ce.ensure(8 * (ng + 1))) || (e = cs.ensure(8 * (ng + 1))) || (e = t->off_e.ensure(8 * (ng + 1))) ||
-        (e = t->off_s.ensure(8 * (ng + 1))))
-        return ctx->hip_fail(e, "walk allocation");
-    wa.cnt_e = ce.as<long long>();
-    wa.cnt_s = cs.as<long long>();
-    const unsigned wg = (unsigned)std::min<long long>(ng, 65536);
-    const bool one_pass = ng > 0 && was_built && (long long)t->groups_h.size() == ng;
-    if (one_pass) {
-        std::vector<long long> &ph = t->pad_h;  // padded offsets: EPJ [0, ng], SPJ [ng + 1, 2 ng + 1]
-        ph.assign(2 * (ng + 1), 0);
-        long long pe = 0, ps = 0;
-        for (long long g = 0; g < ng; g++) {
-            const long long le = std::max(t->groups_h[g].z, 0), ls = std::max(t->groups_h[g].w, 0);
-            ph[g] = pe;
-            ph[ng + 1 + g] = ps;
-            pe += le + le / 4 + 64;
-            ps += ls + ls / 4 + 64;
-        }
-        ph[ng] = pe;
-        ph[2 * ng + 1] = ps;
-        if ((e = t->pad_off.ensure(8 * ph.size())) || (e = t->pad_e.ensure(4 * (size_t)pe)) ||
-            (e = t->pad_s.ensure(4 * (size_t)ps)) ||
-            (e = hipMemcpyAsync(t->pad_off.p, ph.data(), 8 * ph.size(), hipMemcpyHostToDevice, st)))
-            return ctx->hip_fail(e, "padded list allocation");
-        wa.off_e = t->pad_off.as<long long>();
-        wa.off_s = t->pad_off.as<long long>() + ng + 1;
-        wa.id_epj = t->pad_e.as<int>();
-        wa.id_spj = t->pad_s.as<int>();
-        wa.padded = 1;
-        hipLaunchKernelGGL(k_walk<true>, dim3(wg), dim3(64), 0, st, wa);
-    } else if (ng > 0) {
-        hipLaunchKernelGGL(k_walk<false>, dim3(wg), dim3(64), 0, st, wa);
-    }
-    long long zero = 0;
-    if ((e = hipMemcpyAsync(ce.as<long long>() + ng, &zero, 8, hipMemcpyHostToDevice, st)) ||
-        (e = hipMemcpyAsync(cs.as<long long>() + ng, &zero, 8, hipMemcpyHostToDevice, st)))
-        return ctx->hip_fail(e, "walk counts");
-    if ((e = hipcub::DeviceScan::ExclusiveSum(nullptr, tb, ce.as<long long>(), t->off_e.as<long long>(), (int)ng + 1,
-                                              st)) ||
-        (e = cub_temp(t, tb)) ||
-        (e = hipcub::DeviceScan::ExclusiveSum(t->tmp.p, tb, ce.as<long long>(), t->off_e.as<long long>(), (int)ng + 1,
-                                              st)) ||
-        (e = hipcub::DeviceScan::ExclusiveSum(t->tmp.p, tb, cs.as<long long>(), t->off_s.as<long long>(), (int)ng + 1,
-                                              st)))
-        return ctx->hip_fail(e, "walk scan");
-    // per-group sizes (first particle, size, list lengths) and the totals
-    t->groups_h.assign(ng, make_int4(0, 0, 0, 0));
-    if ((e = t->info.ensure(sizeof(int4) * std::max<long long>(ng, 1)))) return ctx->hip_fail(e, "group sizes");
-    if (ng > 0)
-        hipLaunchKernelGGL(k_group_info, dim3(blocks(ng)), dim3(256), 0, st, t->nodes.as<GNode>(), t->groups.as<int>(),
-                           ng, t->off_e.as<long long>(), t->off_s.as<long long>(), t->info.as<int4>());
-    long long tot[2] = {0, 0};
-    if ((ng > 0 &&
-         (e = hipMemcpyAsync(t->groups_h.data(), t->info.p, sizeof(int4) * ng, hipMemcpyDeviceToHost, st))) ||
-        (e = hipMemcpyAsync(&tot[0], t->off_e.as<long long>() + ng, 8, hipMemcpyDeviceToHost, st)) ||
-        (e = hipMemcpyAsync(&tot[1], t->off_s.as<long long>() + ng, 8, hipMemcpyDeviceToHost, st)) ||
-        (e = hipStreamSynchronize(st)))
-        return ctx->hip_fail(e, "walk totals");
-    if (tot[0] > 0x7fffffffLL || tot[1] > 0x7fffffffLL)
+    WalkLists &W = t->walk;
+    int rc = walk_run<false>(t, wa, W, was_built, ng);
+    if (rc != PTH_OK) return rc;
+    const WalkTotals tot = *W.host.as<WalkTotals>();
+    t->groups_h.assign(W.info(), W.info() + ng);
+    if (tot.e > 0x7fffffffLL || tot.s > 0x7fffffffLL)
         return ctx->fail(PTH_ERR_CAPACITY, "pth_gtree_build: lists exceed the int32 range");
-    t->n_le = tot[0];
-    t->n_ls = tot[1];
-    // did every group's lists fit the padded regions?
-    bool rewalk = !one_pass;
-    for (long long g = 0; g < ng && !rewalk; g++)
-        rewalk = t->groups_h[g].z > t->pad_h[g + 1] - t->pad_h[g] ||
-                 t->groups_h[g].w > t->pad_h[ng + 2 + g] - t->pad_h[ng + 1 + g];
-    t->walk_passes = ng > 0 ? (one_pass && !rewalk ? 1 : 2) : 0;
-    // every buffer of the write pass and the ordering sorts, before anything
-    // is enqueued (a growing buffer's free would wait for the device)
-    const bool order = t->canonical && ng > 0;
-    int bits = 1;
-    while (bits < 31 && (1LL << bits) < n) bits++;  // keys are particle positions < n
-    const long long *ob = t->off_e.as<long long>(), *osp = t->off_s.as<long long>();
-    size_t tb_e = 0, tb_s = 0;
-    // the ordering swaps id_epj / id_spj with alt, so each of the three may
-    // hold either list next: all three are sized for the longer one
-    const size_t lbytes = 4 * (size_t)std::max<long long>(std::max(tot[0], tot[1]), 1);
-    if ((e = t->id_epj.ensure(lbytes)) || (e = t->id_spj.ensure(lbytes)))
-        return ctx->hip_fail(e, "list allocation");
-    if (order) {
-        if ((e = t->alt.ensure(lbytes)) || (e = t->lkey.ensure(4 * std::max<long long>(tot[1], 1))) ||
-            (e = t->lkey2.ensure(4 * std::max<long long>(tot[1], 1))) ||
-            (e = hipcub::DeviceSegmentedRadixSort::SortKeys(nullptr, tb_e, t->id_epj.as<int>(), t->alt.as<int>(),
-                                                            (int)tot[0], (int)ng, ob, ob + 1, 0, bits, st)) ||
-            (e = hipcub::DeviceSegmentedRadixSort::SortPairs(nullptr, tb_s, t->lkey.as<int>(), t->lkey2.as<int>(),
-                                                             t->id_spj.as<int>(), t->alt.as<int>(), (int)tot[1],
-                                                             (int)ng, osp, osp + 1, 0, bits, st)) ||
-            (e = cub_temp(t, std::max(tb_e, tb_s))))
-            return ctx->hip_fail(e, "list ordering allocation");
-    }
-    // write pass (or the move of the padded lists), then the ordering, all
-    // enqueued without waits
-    wa.off_e = t->off_e.as<long long>();
-    wa.off_s = t->off_s.as<long long>();
-    wa.id_epj = t->id_epj.as<int>();
-    wa.id_spj = t->id_spj.as<int>();
-    wa.padded = 0;
+    t->n_le = tot.e;
+    t->n_ls = tot.s;
+    t->walk_passes = ng > 0 ? W.passes : 0;
     const auto t2 = std::chrono::steady_clock::now();
     t->ms_walk = std::chrono::duration<float, std::milli>(t2 - t1).count();
-    if (t->id_epj.cap < 4 * (size_t)tot[0] || t->id_spj.cap < 4 * (size_t)tot[1])
-        return ctx->fail(PTH_ERR_STATE, "pth_gtree: list buffers smaller than the lists");
-    if (ng > 0 && rewalk) {
-        hipLaunchKernelGGL(k_walk<true>, dim3(wg), dim3(64), 0, st, wa);
-    } else if (ng > 0) {
-        // every group fits its region (checked above): n <= region size
-        hipLaunchKernelGGL(k_compact, dim3(wg), dim3(256), 0, st, ng, t->pad_off.as<long long>(),
-                           t->off_e.as<long long>(), t->pad_e.as<int>(), t->id_epj.as<int>());
-        hipLaunchKernelGGL(k_compact, dim3(wg), dim3(256), 0, st, ng, t->pad_off.as<long long>() + ng + 1,
-                           t->off_s.as<long long>(), t->pad_s.as<int>(), t->id_spj.as<int>());
-    }
-    // 7. canonical order: segmented sorts of the lists (one segment per group)
-    if (order) {
-        if (t->alt.cap < lbytes || t->id_epj.cap < lbytes || t->id_spj.cap < lbytes ||
-            t->lkey.cap < 4 * (size_t)tot[1] || t->lkey2.cap < 4 * (size_t)tot[1] ||
-            t->tmp.cap < std::max(tb_e, tb_s))
-            return ctx->fail(PTH_ERR_STATE, "pth_gtree: ordering buffers smaller than the lists");
-        if (tot[0] > 0) {
-            if ((e = hipcub::DeviceSegmentedRadixSort::SortKeys(t->tmp.p, tb_e, t->id_epj.as<int>(), t->alt.as<int>(),
-                                                                (int)tot[0], (int)ng, ob, ob + 1, 0, bits, st)))
-                return ctx->hip_fail(e, "EPJ list ordering");
-            std::swap(t->id_epj, t->alt);
-        }
-        if (tot[1] > 0) {
-            hipLaunchKernelGGL(k_spj_keys, dim3(blocks(tot[1])), dim3(256), 0, st, t->nodes.as<GNode>(),
-                               t->id_spj.as<int>(), tot[1], t->lkey.as<int>());
-            if ((e = hipcub::DeviceSegmentedRadixSort::SortPairs(t->tmp.p, tb_s, t->lkey.as<int>(), t->lkey2.as<int>(),
-                                                                 t->id_spj.as<int>(), t->alt.as<int>(), (int)tot[1],
-                                                                 (int)ng, osp, osp + 1, 0, bits, st)))
-                return ctx->hip_fail(e, "SPJ list ordering");
-            std::swap(t->id_spj, t->alt);
-        }
-    }
+    // 6. the lists, enqueued without waits
+    if ((e = t->id_epj.ensure(4 * (size_t)std::max<long long>(tot.e, 1))) ||
+        (e = t->id_spj.ensure(4 * (size_t)std::max<long long>(tot.s, 1))))
+        return ctx->hip_fail(e, "list allocation");
+    rc = walk_finish<false>(t, wa, W, t->canonical, t->id_epj.as<int>(), t->id_spj.as<int>());
+    if (rc != PTH_OK) return rc;
     // meanwhile, the plan of a resident evaluation of these lists under the
     // context's parameters (pth_resident_from_gtree / _refill take it over)
     {
@@ -1411,10 +1775,10 @@ int resident_fill_gtree(pth_resident *r, const pth_gtree *t, const char *who)
                        r->epj.as<EpjDev>());
     if (P.mono)
         hipLaunchKernelGGL(k_res_nodes_mono, dim3(blocks(t->n_node)), dim3(256), 0, st, t->n_node,
-                           t->nmass.as<double>(), t->ncom.as<double>(), r->spj.as<EpjDev>());
+                           t->pre.as<int>(), t->nmass.as<double>(), t->ncom.as<double>(), r->spj.as<EpjDev>());
     else
-        hipLaunchKernelGGL(k_res_nodes, dim3(blocks(t->n_node)), dim3(256), 0, st, t->n_node, t->nmass.as<double>(),
-                           t->ncom.as<double>(), t->nquad.as<double>(), r->spj.as<SpjDev>());
+        hipLaunchKernelGGL(k_res_nodes, dim3(blocks(t->n_node)), dim3(256), 0, st, t->n_node, t->pre.as<int>(),
+                           t->nmass.as<double>(), t->ncom.as<double>(), t->nquad.as<double>(), r->spj.as<SpjDev>());
     if ((e = hipGetLastError()) || (e = hipStreamSynchronize(st))) return bail(e, "resident records");
     if ((e = resident_finish(r))) return bail(e, "resident SPJ table");
     return PTH_OK;
@@ -1491,6 +1855,12 @@ int pth_gtree_download(const pth_gtree *t, long long *order, long long *node_beg
     HIPCHK(c, d2h(node_quad, t->nquad, 48 * nn), "download");
     HIPCHK(c, d2h(id_epj, t->id_epj, 4 * t->n_le), "download");
     HIPCHK(c, d2h(id_spj, t->id_spj, 4 * t->n_ls), "download");
+    if (id_spj && t->n_ls > 0) {
+        // (the lists name nodes by preorder number on the device)
+        std::vector<int> at(nn);
+        HIPCHK(c, d2h(at.data(), t->node_at, 4 * nn), "download");
+        for (long long k = 0; k < t->n_ls; k++) id_spj[k] = at[id_spj[k]];
+    }
     std::vector<GNode> nodes(nn);
     HIPCHK(c, d2h(nodes.data(), t->nodes, sizeof(GNode) * nn), "download");
     for (long long k = 0; k < nn; k++) {
@@ -1566,100 +1936,28 @@ int pth_gtree_neighbors(pth_gtree *t, long long *n_total)
     //    group walk's symmetric r_search tests on widened tile boxes
     const long long nt = t->n_tile;
     HIPCHK(c, t->tbox.ensure(sizeof(double) * 12 * nt), "neighbour buffers");
-    HIPCHK(c, t->tcnt.ensure(sizeof(long long) * (nt + 1)), "neighbour buffers");
-    HIPCHK(c, t->toff.ensure(sizeof(long long) * (nt + 1)), "neighbour buffers");
-    HIPCHK(c, t->tinfo.ensure(sizeof(int4) * nt), "neighbour buffers");
     hipLaunchKernelGGL(k_tile_boxes, dim3(blocks(nt)), dim3(256), 0, st, t->tiles.as<int>(), nt,
                        t->box_in.as<double>(), t->box_out.as<double>(), t->rs_max, t->tbox.as<double>());
-    WalkArgs wa{};
-    wa.nodes = t->nodes.as<GNode>();
-    wa.ncom = t->ncom.as<double>();
-    wa.box_in = t->box_in.as<double>();
-    wa.box_out = t->box_out.as<double>();
+    WalkArgs wa = walk_args(t);
     wa.groups = t->tiles.as<int>();
     wa.n_group = nt;
     wa.tbox = t->tbox.as<double>();
-    wa.root_len = t->root_len;
-    wa.inv_theta2 = 0.0;
     wa.theta_pos = 1;
-    wa.cnt_e = t->tcnt.as<long long>();
     const unsigned wgt = (unsigned)std::min<long long>(nt, 65536);
-    // as many tiles as the last search (the same tree, or one rebuilt from
-    // particles that moved a little): one writing pass into regions of the
-    // last search's candidate counts + 1/4 + 64 that also counts; otherwise
-    // a counting pass first (a region that turns out too small means an
-    // exact writing pass, as for the group walk)
-    const bool one_pass = nt > 0 && (long long)t->tcnt_h.size() == nt + 1;
-    if (one_pass) {
-        std::vector<long long> &ph = t->tpad_h;
-        ph.assign(nt + 1, 0);
-        long long pe = 0;
-        for (long long g = 0; g < nt; g++) {
-            const long long k = std::max(t->tcnt_h[g], 0LL);
-            ph[g] = pe;
-            pe += k + k / 4 + 64;
-        }
-        ph[nt] = pe;
-        HIPCHK(c, t->tpad_off.ensure(8 * (size_t)(nt + 1)), "neighbour buffers");
-        HIPCHK(c, t->tl_pad.ensure(4 * (size_t)pe), "neighbour buffers");
-        HIPCHK(c, hipMemcpyAsync(t->tpad_off.p, ph.data(), 8 * (size_t)(nt + 1), hipMemcpyHostToDevice, st),
-               "neighbour regions");
-        wa.off_e = t->tpad_off.as<long long>();
-        wa.id_epj = t->tl_pad.as<int>();
-        wa.padded = 1;
-        hipLaunchKernelGGL(k_walk<true>, dim3(wgt), dim3(64), 0, st, wa);
-    } else if (nt > 0) {
-        hipLaunchKernelGGL(k_walk<false>, dim3(wgt), dim3(64), 0, st, wa);
-    }
-    const long long zero = 0;
-    HIPCHK(c, hipMemcpyAsync(t->tcnt.as<long long>() + nt, &zero, 8, hipMemcpyHostToDevice, st), "neighbour counts");
-    if ((e = hipcub::DeviceScan::ExclusiveSum(nullptr, tb, t->tcnt.as<long long>(), t->toff.as<long long>(),
-                                              (int)(nt + 1), st)) ||
-        (e = cub_temp(t, tb)) ||
-        (e = hipcub::DeviceScan::ExclusiveSum(t->tmp.p, tb, t->tcnt.as<long long>(), t->toff.as<long long>(),
-                                              (int)(nt + 1), st)))
-        return c->hip_fail(e, "candidate scan");
-    long long ncand = 0;
-    t->tcnt_h.resize(nt + 1);
-    HIPCHK(c, hipMemcpyAsync(&ncand, t->toff.as<long long>() + nt, 8, hipMemcpyDeviceToHost, st), "candidates");
-    HIPCHK(c, hipMemcpyAsync(t->tcnt_h.data(), t->tcnt.p, 8 * (size_t)(nt + 1), hipMemcpyDeviceToHost, st),
-           "candidates");
-    HIPCHK(c, hipStreamSynchronize(st), "candidates");
+    // (regions of the last search's lengths when it had as many tiles)
+    WalkLists &W = t->tile_walk;
+    int rc = walk_run<true>(t, wa, W, true, nt);
+    if (rc != PTH_OK) return rc;
+    const long long ncand = W.host.as<WalkTotals>()->e;
     if (ncand > 0x7fffffffLL) {
-        t->tcnt_h.clear();
+        W.n = -1;
         return c->fail(PTH_ERR_CAPACITY, "pth_gtree_neighbors: candidates exceed the int32 range");
     }
-    // did every tile's candidates fit its region?
-    bool rewalk = !one_pass;
-    for (long long g = 0; g < nt && !rewalk; g++) rewalk = t->tcnt_h[g] > t->tpad_h[g + 1] - t->tpad_h[g];
-    t->tile_passes = nt > 0 ? (rewalk ? 2 : 1) : 0;
+    t->tile_passes = nt > 0 ? W.passes : 0;
     HIPCHK(c, t->tl.ensure(sizeof(int) * std::max<long long>(ncand, 1)), "neighbour buffers");
-    HIPCHK(c, t->tl_alt.ensure(sizeof(int) * std::max<long long>(ncand, 1)), "neighbour buffers");
-    wa.off_e = t->toff.as<long long>();
-    wa.id_epj = t->tl.as<int>();
-    wa.padded = 0;
-    if (nt > 0 && rewalk) {
-        hipLaunchKernelGGL(k_walk<true>, dim3(wgt), dim3(64), 0, st, wa);
-    } else if (nt > 0) {
-        // every tile fits its region (checked above)
-        hipLaunchKernelGGL(k_compact, dim3(wgt), dim3(256), 0, st, nt, t->tpad_off.as<long long>(),
-                           t->toff.as<long long>(), t->tl_pad.as<int>(), t->tl.as<int>());
-    }
     // candidates ascending in tree order, so rows come out in that order
-    if (ncand > 0) {
-        int bits = 1;
-        while (bits < 31 && (1LL << bits) < n) bits++;
-        const long long *ob = t->toff.as<long long>();
-        if ((e = hipcub::DeviceSegmentedRadixSort::SortKeys(nullptr, tb, t->tl.as<int>(), t->tl_alt.as<int>(),
-                                                            (int)ncand, (int)nt, ob, ob + 1, 0, bits, st)) ||
-            (e = cub_temp(t, tb)) ||
-            (e = hipcub::DeviceSegmentedRadixSort::SortKeys(t->tmp.p, tb, t->tl.as<int>(), t->tl_alt.as<int>(),
-                                                            (int)ncand, (int)nt, ob, ob + 1, 0, bits, st)))
-            return c->hip_fail(e, "candidate ordering");
-        std::swap(t->tl, t->tl_alt);
-    }
-    hipLaunchKernelGGL(k_tile_info, dim3(blocks(nt)), dim3(256), 0, st, t->nodes.as<GNode>(), t->tiles.as<int>(), nt,
-                       t->toff.as<long long>(), t->tinfo.as<int4>());
+    rc = walk_finish<true>(t, wa, W, true, t->tl.as<int>(), nullptr);
+    if (rc != PTH_OK) return rc;
     // 2. exact FP64 filter of the candidates.  After a completed search of
     //    as many particles: one writing pass into regions of that search's
     //    counts + 1/4 + 4 that also counts (their total is at most 1.25 times
@@ -1677,8 +1975,8 @@ int pth_gtree_neighbors(pth_gtree *t, long long *n_total)
     na.spos = t->spos.as<double>();
     na.srs = t->srs.as<double>();
     na.order = t->order.as<long long>();
-    na.info = t->tinfo.as<int4>();
-    na.off_e = t->toff.as<long long>();
+    na.info = reinterpret_cast<const int4 *>(W.back.as<WalkTotals>() + 1);
+    na.off_e = W.off.as<long long>();
     na.id_epj = t->tl.as<int>();
     na.n_group = nt;
     na.cnt = t->ngb_cnt.as<int>();
@@ -1767,12 +2065,12 @@ void pth_gtree_free(pth_gtree *t)
         (void)hipSetDevice(t->ctx->device);
         if (t->ctx->stream) (void)hipStreamSynchronize(t->ctx->stream);
     }
-    DevBuf *all[] = {&t->order, &t->key, &t->skey, &t->sidx, &t->sidx2, &t->spos, &t->smass, &t->srs, &t->nodes, &t->nmass,
-                     &t->ncom, &t->nquad, &t->box_in, &t->box_out, &t->groups, &t->off_e, &t->off_s, &t->id_epj,
-                     &t->id_spj, &t->tmp, &t->ngb_cnt, &t->ngb_off, &t->ngb, &t->tiles, &t->tbox, &t->tcnt,
-                     &t->toff, &t->tl, &t->tl_alt, &t->tinfo, &t->pad_off, &t->pad_e, &t->pad_s,
-                     &t->tpad_off, &t->tl_pad, &t->ngb_cap, &t->ngb_poff, &t->ngb_pad, &t->ngb_flag,
-                     &t->meta, &t->pre, &t->node_at};
+    DevBuf *all[] = {&t->order, &t->key, &t->skey, &t->sidx, &t->sidx2, &t->spos, &t->smass, &t->srs, &t->nodes,
+                     &t->nmass, &t->ncom, &t->nquad, &t->box_in, &t->box_out, &t->rec, &t->groups, &t->id_epj,
+                     &t->id_spj, &t->tmp, &t->ngb_cnt, &t->ngb_off, &t->ngb, &t->tiles, &t->tbox, &t->tl,
+                     &t->ngb_cap, &t->ngb_poff, &t->ngb_pad, &t->ngb_flag, &t->meta, &t->pre, &t->node_at, &t->range};
+    t->walk.release();
+    t->tile_walk.release();
     for (DevBuf *b : all) b->release();
     t->release_scratch();
     if (t->pinned) (void)hipHostFree(t->pinned);

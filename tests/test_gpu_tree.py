@@ -83,6 +83,28 @@ def test_device_tree_block_edges_and_coincident_particles(n, leaf, group):
     _compare(n, 0, 0.0, 0.5, leaf=leaf, group=group, mx=(m, x))
 
 
+@pytest.mark.parametrize("n,theta,leaf,group,canonical", [
+    (40000, 0.05, 2, 512, True), (40000, 0.05, 2, 512, False),  # leaf lists over 1,024 entries
+    (40000, 1.5, 8, 2048, True),                                # few entries per list
+    (230000, 0.7, 1, 2048, True),                               # node map in several windows
+    (5000, 0.0, 1, 5000, True)])                                # one group that opens every leaf
+def test_device_tree_list_ordering(n, theta, leaf, group, canonical):
+    """Lists put in order through the map of the tree's nodes: leaf lists
+    longer and shorter than one expansion pass, maps of one and of several
+    windows, a list of every leaf."""
+    _compare(n, 17, 0.5, theta, leaf=leaf, group=group, canonical=canonical)
+
+
+@pytest.mark.parametrize("scale,shift", [(1e-12, 0.0), (1e9, 0.0), (1.0, 1e6), (1e-25, 0.0)])
+def test_device_tree_opening_test_precision(scale, shift):
+    """The opening test is decided in FP32 relative to the root cube only
+    where that leaves no doubt: lists stay the FP64 ones for clusters far
+    smaller or larger than 1 (squares that leave the FP32 range) and for one
+    whose offset takes most of the FP64 digits."""
+    m, x, _ = host.cluster(6000, "plummer", f_bin=0.3, seed=23)
+    _compare(6000, 0, 0.0, 0.5, r_search=0.015 * scale, mx=(m, x * scale + shift))
+
+
 def test_device_tree_batch_order():
     _compare(30000, 4, 0.3, 0.3, canonical=False)
 
