@@ -190,6 +190,9 @@ hipError_t launch_expand_runs(const WalkDev *walks, int w_begin, int n_walk, con
 
 // Launches of segment k of a batch (k < b.n_seg).
 hipError_t launch_stage(const BatchDev &b, int k, hipStream_t st);
+// Whether segment k's items run a quarter per wave, classes 1 and 2 together
+// (launch_force then launches them with bit 1 of classes).
+bool split_launch(const BatchDev &b, int k);
 // classes: bit c set launches the items of i-per-lane class c + 1
 hipError_t launch_force(const BatchDev &b, int k, hipStream_t st, unsigned classes = 0xFu);
 hipError_t launch_reduce(const BatchDev &b, int k, hipStream_t st);

@@ -39,6 +39,7 @@
 // G multiplies the FP64 sums once at the end.
 #include <hip/hip_runtime.h>
 
+#include <climits>
 #include <mutex>
 #include <unordered_map>
 
@@ -457,8 +458,9 @@ struct Consts {
 // walk-relative coordinates, (x_j - x_i) + (xlo_j - xlo_i): the FP32 high
 // parts of two close particles differ exactly, so the separation keeps FP32
 // relative precision however far the pair lies from the walk centre.
-template <int IPL, int NNB_LE, bool NEAR, bool VC, bool DF = false>
-__device__ __forceinline__ void epj_blocks(cfp se, int b_begin, int b_end, const float (&xi)[IPL],
+// end(b) is called after the sums up to block b are in A.
+template <int IPL, int NNB_LE, bool NEAR, bool VC, bool DF = false, class F>
+__device__ __forceinline__ void epj_blocks(F &end, cfp se, int b_begin, int b_end, const float (&xi)[IPL],
                                            const float (&yi)[IPL], const float (&zi)[IPL],
                                            const float (&rsi2)[IPL], const Consts &K, double (&A)[IPL][4],
                                            int (&nnb)[IPL], cfp sel = nullptr, const float *xil = nullptr,
@@ -527,6 +529,7 @@ __device__ __forceinline__ void epj_blocks(cfp se, int b_begin, int b_end, const
             A[q][3] += (double)p[q];
             nnb[q] += nb[q];
         }
+        end(b1);
     }
 }
 
@@ -574,8 +577,9 @@ __device__ __forceinline__ void co_pair(float r2, float mj, float mp, float rin_
 // only add zeros there.
 // The self pair's -m_i/r_out is removed by the caller (src/hard.hpp:1669-1673
 // adds the same term back on the CPU).
-template <int IPL, int NNB_LE>
-__device__ __forceinline__ void epj_near_co(cfp se, cfp sec, int b_begin, int b_end, const float (&xi)[IPL],
+// end as in epj_blocks.
+template <int IPL, int NNB_LE, class F>
+__device__ __forceinline__ void epj_near_co(F &end, cfp se, cfp sec, int b_begin, int b_end, const float (&xi)[IPL],
                                             const float (&yi)[IPL], const float (&zi)[IPL],
                                             const float (&xil)[IPL], const float (&yil)[IPL],
                                             const float (&zil)[IPL], const float (&rsi2)[IPL],
@@ -670,6 +674,7 @@ __device__ __forceinline__ void epj_near_co(cfp se, cfp sec, int b_begin, int b_
             PT[q] += (double)pt[q];
             nnb[q] += nb[q];
         }
+        end(b1);
     }
 }
 
@@ -748,9 +753,9 @@ __device__ __forceinline__ void spj_flush(const float (&ax)[IPL], const float (&
 // position after it are loaded before the current record is used (scalar
 // loads in flight during the pair arithmetic instead of a wait at the top of
 // every record; the table index comes from the position loaded one record
-// earlier).
-template <int IPL, bool VC>
-__device__ __forceinline__ void spj_records(cfp ss, cfp tab, int s_begin, int s_end, const float (&xi)[IPL],
+// earlier).  end(s) is called after the sums up to record s are in A.
+template <int IPL, bool VC, class F>
+__device__ __forceinline__ void spj_records(F &end, cfp ss, cfp tab, int s_begin, int s_end, const float (&xi)[IPL],
                                             const float (&yi)[IPL], const float (&zi)[IPL], const Consts &K,
                                             double (&A)[IPL][4])
 {
@@ -772,6 +777,7 @@ __device__ __forceinline__ void spj_records(cfp ss, cfp tab, int s_begin, int s_
             pn = pnn;
         }
         spj_flush<IPL>(ax, ay, az, p, A);
+        end(s1);
     }
 }
 
@@ -779,6 +785,7 @@ __device__ __forceinline__ void spj_records(cfp ss, cfp tab, int s_begin, int s_
 struct ForceArgs {
     const Item *items;
     int n_items;
+    const Item *items1;  // split launches: the items of 1 i per lane
     // persistent launches: the class's 8 item counters (one per XCD) and the
     // slots of each XCD's run of items
     int *counter;
@@ -801,94 +808,9 @@ struct ForceArgs {
     double *part_pott;  // changeover mode
 };
 
-template <int IPL, int NNB_LE, bool VC, bool CO, bool DF>
-__device__ __forceinline__ void run_tile(const ForceArgs &a, const Item &it, int near_end, int lane,
-                                         const Consts &K)
+__device__ __forceinline__ Item load_item(const Item *items, int idx)
 {
-    const int n_i = item_n_i(it.n_i_ipl);
-    float xi[IPL], yi[IPL], zi[IPL], rsi2[IPL];
-    double A[IPL][4], PT[IPL];
-    int nnb[IPL];
-    int self[IPL];
-    float rin_i[IPL], rout_i[IPL], m_i[IPL], xil[IPL], yil[IPL], zil[IPL];
-#pragma unroll
-    for (int q = 0; q < IPL; q++) {
-        const bool in = lane + 64 * q < n_i;
-        float4 v = make_float4(0.f, 0.f, 0.f, -1.f);
-        if (in) v = a.staged_i[it.i_begin + lane + 64 * q];
-        xi[q] = v.x;
-        yi[q] = v.y;
-        zi[q] = v.z;
-        rsi2[q] = v.w;
-        A[q][0] = A[q][1] = A[q][2] = A[q][3] = 0.0;
-        PT[q] = 0.0;
-        nnb[q] = 0;
-        if constexpr (DF) {
-            float4 l = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (in) l = a.staged_il[it.i_begin + lane + 64 * q];
-            xil[q] = l.x;
-            yil[q] = l.y;
-            zil[q] = l.z;
-        }
-        if constexpr (CO) {
-            float4 c = make_float4(__int_as_float(-2), 0.f, 0.f, 0.f);
-            if (in) c = a.staged_ic[it.i_begin + lane + 64 * q];
-            self[q] = __float_as_int(c.x);
-            rin_i[q] = c.y;
-            rout_i[q] = c.z;
-            m_i[q] = c.w;
-            float4 l = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (in) l = a.staged_il[it.i_begin + lane + 64 * q];
-            xil[q] = l.x;
-            yil[q] = l.y;
-            zil[q] = l.z;
-        }
-    }
-    const cfp se = as_const(a.staged_e);
-    const int e_mid = min(max(near_end, it.e_blk_begin), it.e_blk_end);
-    if constexpr (CO) {
-        epj_near_co<IPL, NNB_LE>(se, as_const(a.staged_ec), it.e_blk_begin, e_mid, xi, yi, zi, xil, yil, zil, rsi2,
-                                 self, rin_i, rout_i, K, a.ngb2, A, PT, nnb);
-        // remove the self pair's linear-cutoff potential -m_i / max(eps, r_out)
-        // (added above with these same FP32 operations) in the item whose
-        // j-range holds the i's own entry
-#pragma unroll
-        for (int q = 0; q < IPL; q++) {
-            const int sb = self[q] >> 3;
-            if (self[q] >= 0 && sb >= it.e_blk_begin && sb < e_mid)
-                A[q][3] += (double)(m_i[q] * __builtin_amdgcn_rsqf(__builtin_fmaxf(K.eps2, K.rout2)));
-        }
-    } else if constexpr (DF) {
-        epj_blocks<IPL, NNB_LE, true, VC, true>(se, it.e_blk_begin, e_mid, xi, yi, zi, rsi2, K, A, nnb,
-                                                as_const(a.staged_el), xil, yil, zil);
-    } else
-        epj_blocks<IPL, NNB_LE, true, VC>(se, it.e_blk_begin, e_mid, xi, yi, zi, rsi2, K, A, nnb);
-    epj_blocks<IPL, NNB_LE, false, VC>(se, e_mid, it.e_blk_end, xi, yi, zi, rsi2, K, A, nnb);
-    spj_records<IPL, VC>(as_const(a.staged_s), as_const(reinterpret_cast<const float *>(a.spj_tab)), it.s_begin,
-                         it.s_end, xi, yi, zi, K, A);
-    const double G = a.G;
-#pragma unroll
-    for (int q = 0; q < IPL; q++) {
-        const int i = lane + 64 * q;
-        if (i >= n_i) continue;
-        if (it.part < 0) {
-            a.out_accp[it.i_begin + i] = make_double4(G * A[q][0], G * A[q][1], G * A[q][2], G * A[q][3]);
-            a.out_nnb[it.i_begin + i] = nnb[q];
-            if constexpr (CO) a.out_pott[it.i_begin + i] = G * (A[q][3] + PT[q]);
-        } else {
-            const size_t slot = (size_t)(it.part + q) * 64 + lane;
-            a.part_accp[slot] = make_double4(A[q][0], A[q][1], A[q][2], A[q][3]);
-            a.part_nnb[slot] = nnb[q];
-            if constexpr (CO) a.part_pott[slot] = A[q][3] + PT[q];
-        }
-    }
-}
-
-// Work item idx of this class's launch (empty slots have walk < 0).
-template <int NNB_LE, int IPL, bool VC, bool CO, bool DF>
-__device__ __forceinline__ void force_item(const ForceArgs &a, int idx)
-{
-    const cip ci = (cip)(a.items) + (size_t)idx * 8;
+    const cip ci = (cip)(items) + (size_t)idx * 8;
     Item it;
     it.walk = ci[0];
     it.i_begin = ci[1];
@@ -898,10 +820,311 @@ __device__ __forceinline__ void force_item(const ForceArgs &a, int idx)
     it.s_begin = ci[5];
     it.s_end = ci[6];
     it.part = ci[7];
-    if (it.walk < 0) return;
+    return it;
+}
+
+// A work item's j-range falls into four quarters of about equal cost, cut
+// where the FP32 partial sums are flushed: each quarter is summed in FP64 by
+// itself, and the quarters' sums are added in order.  So one wave that takes
+// the quarters in turn and four waves that take one each give the same bits,
+// and a launch is free to do either.
+struct Cut {
+    bool in_e;  // among the EPJ blocks (at most their end), or the SPJ records
+    int e, s;   // blocks before e and records before s come before the cut
+};
+__device__ __forceinline__ Cut cut_at(const Item &it, int near_end, int k)
+{
+    const int nb = it.e_blk_end - it.e_blk_begin, ns = it.s_end - it.s_begin;
+    const int m = min(max(near_end, it.e_blk_begin), it.e_blk_end);
+    const long long ue = 8ll * nb, u = (ue + 2ll * ns) * k / 4;
+    Cut c{k < 4 && u <= ue, it.e_blk_end, it.s_begin};
+    // whole flush groups: 8 blocks from the range's begin, or from where its
+    // far part begins; 32 records
+    if (c.in_e) {
+        const int x = min(nb, ((int)(u >> 3) + PTH_FLUSH_BLOCKS / 2) & ~(PTH_FLUSH_BLOCKS - 1));
+        c.e = it.e_blk_begin + x;
+        if (c.e > m && x < nb)
+            c.e = min(m + ((c.e - m + PTH_FLUSH_BLOCKS - 1) & ~(PTH_FLUSH_BLOCKS - 1)), it.e_blk_end);
+    } else if (k < 4) {
+        c.s += min(ns, ((int)((u - ue) >> 1) + PTH_FLUSH_SPJ / 2) & ~(PTH_FLUSH_SPJ - 1));
+    } else {
+        c.s = it.s_end;
+    }
+    return c;
+}
+
+// The i of a tile held by one lane (i = i_begin + lane + 64 k).
+template <int IPL> struct Tile {
+    float x[IPL], y[IPL], z[IPL], rs2[IPL];
+    float xl[IPL], yl[IPL], zl[IPL];               // low parts (DF, CO)
+    float rin[IPL], rout[IPL], m[IPL];             // CO
+    int self[IPL];                                 // CO
+};
+template <int IPL, bool CO, bool DF>
+__device__ __forceinline__ void load_tile(const ForceArgs &a, const Item &it, int lane, Tile<IPL> &t)
+{
+    const int n_i = item_n_i(it.n_i_ipl);
+#pragma unroll
+    for (int q = 0; q < IPL; q++) {
+        const bool in = lane + 64 * q < n_i;
+        float4 v = make_float4(0.f, 0.f, 0.f, -1.f);
+        if (in) v = a.staged_i[it.i_begin + lane + 64 * q];
+        t.x[q] = v.x;
+        t.y[q] = v.y;
+        t.z[q] = v.z;
+        t.rs2[q] = v.w;
+        if constexpr (DF || CO) {
+            float4 l = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (in) l = a.staged_il[it.i_begin + lane + 64 * q];
+            t.xl[q] = l.x;
+            t.yl[q] = l.y;
+            t.zl[q] = l.z;
+        }
+        if constexpr (CO) {
+            float4 c = make_float4(__int_as_float(-2), 0.f, 0.f, 0.f);
+            if (in) c = a.staged_ic[it.i_begin + lane + 64 * q];
+            t.self[q] = __float_as_int(c.x);
+            t.rin[q] = c.y;
+            t.rout[q] = c.z;
+            t.m[q] = c.w;
+        }
+    }
+}
+
+// Components of an i's FP64 sums: acc, pot and, in changeover mode, the
+// potential still missing from the total.
+template <bool CO> constexpr int n_sum = CO ? 5 : 4;
+
+// Adds the tile's sums over EPJ blocks [e0, e_mid) near and [e_mid, e1) far
+// and SPJ records [s0, s1) to A, PT and nnb; between the blocks and the
+// records, and wherever sums are flushed, end is told how far they go.
+template <int IPL, int NNB_LE, bool VC, bool CO, bool DF, class F>
+__device__ __forceinline__ void sum_range(F &end, const ForceArgs &a, const Tile<IPL> &t, int e0, int e_mid, int e1,
+                                          int s0, int s1, const Consts &K, double (&A)[IPL][4], double (&PT)[IPL],
+                                          int (&nnb)[IPL])
+{
+    const cfp se = as_const(a.staged_e);
+    if constexpr (CO) {
+        epj_near_co<IPL, NNB_LE>(end, se, as_const(a.staged_ec), e0, e_mid, t.x, t.y, t.z, t.xl, t.yl, t.zl, t.rs2,
+                                 t.self, t.rin, t.rout, K, a.ngb2, A, PT, nnb);
+    } else if constexpr (DF) {
+        epj_blocks<IPL, NNB_LE, true, VC, true>(end, se, e0, e_mid, t.x, t.y, t.z, t.rs2, K, A, nnb,
+                                                as_const(a.staged_el), t.xl, t.yl, t.zl);
+    } else
+        epj_blocks<IPL, NNB_LE, true, VC>(end, se, e0, e_mid, t.x, t.y, t.z, t.rs2, K, A, nnb);
+    epj_blocks<IPL, NNB_LE, false, VC>(end, se, e_mid, e1, t.x, t.y, t.z, t.rs2, K, A, nnb);
+    end.records(s0);
+    spj_records<IPL, VC>(end, as_const(a.staged_s), as_const(reinterpret_cast<const float *>(a.spj_tab)), s0, s1, t.x,
+                         t.y, t.z, K, A);
+}
+
+// Changeover mode: the self pairs' linear-cutoff potentials -m_i / max(eps,
+// r_out) (added in the near loop with these same FP32 operations) are removed
+// in the item whose j-range [e0, e_mid) holds the i's own entry, once all its
+// sums are made.
+template <int IPL>
+__device__ __forceinline__ void drop_self(const Tile<IPL> &t, int e0, int e_mid, const Consts &K, double (&A)[IPL][4])
+{
+#pragma unroll
+    for (int q = 0; q < IPL; q++) {
+        const int sb = t.self[q] >> 3;
+        if (t.self[q] >= 0 && sb >= e0 && sb < e_mid)
+            A[q][3] += (double)(t.m[q] * __builtin_amdgcn_rsqf(__builtin_fmaxf(K.eps2, K.rout2)));
+    }
+}
+
+// Sums of slot q of a tile to the outputs, or to the item's partial slot.
+template <bool CO>
+__device__ __forceinline__ void store_sums(const ForceArgs &a, const Item &it, int lane, int q, const double (&A)[4],
+                                           double PT, int nnb)
+{
+    const int i = lane + 64 * q;
+    if (i >= item_n_i(it.n_i_ipl)) return;
+    const double G = a.G;
+    if (it.part < 0) {
+        a.out_accp[it.i_begin + i] = make_double4(G * A[0], G * A[1], G * A[2], G * A[3]);
+        a.out_nnb[it.i_begin + i] = nnb;
+        if constexpr (CO) a.out_pott[it.i_begin + i] = G * (A[3] + PT);
+    } else {
+        const size_t slot = (size_t)(it.part + q) * 64 + lane;
+        a.part_accp[slot] = make_double4(A[0], A[1], A[2], A[3]);
+        a.part_nnb[slot] = nnb;
+        if constexpr (CO) a.part_pott[slot] = A[3] + PT;
+    }
+}
+
+// Ends the quarters of an item that one wave takes: the sums up to each cut
+// go to LDS (T, this wave's n_sum IPL rows of 64; in registers they would
+// cost the 2-i kernel a wave per SIMD).  `at` is the next cut among the
+// blocks (records, after records()).
+template <int IPL, bool CO> struct Quarters {
+    static constexpr int NC = n_sum<CO>;
+    const ForceArgs &a;
+    int idx, k, at;
+    bool first;
+    double *T;
+    double (&A)[IPL][4], (&PT)[IPL];
+    // the next cut after position pos (of the blocks or, with rec, records)
+    __device__ __forceinline__ void next(int pos, bool rec)
+    {
+        // (the item is read again: its words would take scalar registers all
+        // through the j loops, which need every one)
+        asm volatile("" : "+s"(idx));
+        const Item it = load_item(a.items, idx);
+        const int near_end = ((cip)(a.near_blk))[it.walk];
+        at = INT_MAX;
+        for (; k < 4; k++) {
+            const Cut c = cut_at(it, near_end, k);
+            if (c.in_e == rec) {
+                if (!rec) break;  // the cuts left are among the records
+                continue;
+            }
+            if ((rec ? c.s : c.e) > pos) {
+                at = rec ? c.s : c.e;
+                break;
+            }
+        }
+    }
+    __device__ __forceinline__ void close()
+    {
+        const int lane = threadIdx.x & 63;
+#pragma unroll
+        for (int q = 0; q < IPL; q++) {
+            double *Tq = T + (size_t)(q * NC) * 64 + lane;
+#pragma unroll
+            for (int c = 0; c < NC; c++) {
+                double &v = c < 4 ? A[q][c] : PT[q];
+                Tq[c * 64] = first ? v : Tq[c * 64] + v;
+                v = 0.0;
+            }
+        }
+        first = false;
+    }
+    __device__ __forceinline__ void operator()(int pos)
+    {
+        if (pos < at) return;
+        close();
+        next(pos, rec_);
+    }
+    bool rec_ = false;
+    // between the blocks and the records: a cut may lie just there
+    __device__ __forceinline__ void records(int s0)
+    {
+        rec_ = true;
+        const int k0 = k;
+        next(s0, true);
+        if (k > k0) close();
+    }
+    // the item's sums
+    __device__ __forceinline__ void finish()
+    {
+        if (first) return;
+        const int lane = threadIdx.x & 63;
+#pragma unroll
+        for (int q = 0; q < IPL; q++) {
+            const double *Tq = T + (size_t)(q * NC) * 64 + lane;
+#pragma unroll
+            for (int c = 0; c < 4; c++) A[q][c] = Tq[c * 64] + A[q][c];
+            if constexpr (CO) PT[q] = Tq[4 * 64] + PT[q];
+        }
+    }
+};
+struct NoQuarters {
+    __device__ __forceinline__ void operator()(int) const {}
+    __device__ __forceinline__ void records(int) const {}
+};
+
+// One item by one wave.
+template <int IPL, int NNB_LE, bool VC, bool CO, bool DF>
+__device__ __forceinline__ void run_tile(const ForceArgs &a, int idx, int lane, const Consts &K, double *T)
+{
+    Tile<IPL> t;
+    double A[IPL][4], PT[IPL];
+    int nnb[IPL];
+#pragma unroll
+    for (int q = 0; q < IPL; q++) {
+        nnb[q] = 0;
+        A[q][0] = A[q][1] = A[q][2] = A[q][3] = PT[q] = 0.0;
+    }
+    const Item it = load_item(a.items, idx);
+    if (it.walk < 0) return;  // an empty slot
+    load_tile<IPL, CO, DF>(a, it, lane, t);
+    const int e_mid = min(max(((cip)(a.near_blk))[it.walk], it.e_blk_begin), it.e_blk_end);
+    Quarters<IPL, CO> end{a, idx, 1, 0, true, T, A, PT};
+    end.next(it.e_blk_begin, false);
+    sum_range<IPL, NNB_LE, VC, CO, DF>(end, a, t, it.e_blk_begin, e_mid, it.e_blk_end, it.s_begin, it.s_end, K, A, PT,
+                                       nnb);
+    end.finish();
+    if constexpr (CO) drop_self<IPL>(t, it.e_blk_begin, e_mid, K, A);
+#pragma unroll
+    for (int q = 0; q < IPL; q++) store_sums<CO>(a, it, lane, q, A[q], PT[q], nnb[q]);
+}
+
+// One item by the four waves of a workgroup, a quarter each; wave q then adds
+// up the sums of slot q.  All waves of the workgroup call it with the same
+// item.
+template <int IPL, int NNB_LE, bool CO, bool DF>
+__device__ __forceinline__ void run_tile_split(const ForceArgs &a, const Item *items, int idx, int wave, int lane,
+                                               const Consts &K, double *T, int *N)
+{
+    constexpr int NC = n_sum<CO>;
+    Tile<IPL> t;
+    double A[IPL][4], PT[IPL];
+    int nnb[IPL];
+#pragma unroll
+    for (int q = 0; q < IPL; q++) {
+        nnb[q] = 0;
+        A[q][0] = A[q][1] = A[q][2] = A[q][3] = PT[q] = 0.0;
+    }
+    const Item it = load_item(items, idx);
+    if (it.walk < 0) return;  // an empty slot
+    load_tile<IPL, CO, DF>(a, it, lane, t);
     const int near_end = ((cip)(a.near_blk))[it.walk];
+    const int e_mid = min(max(near_end, it.e_blk_begin), it.e_blk_end);
+    const Cut c0 = cut_at(it, near_end, wave), c1 = cut_at(it, near_end, wave + 1);
+    const int e0 = wave ? c0.e : it.e_blk_begin, s0 = wave ? c0.s : it.s_begin;
+    NoQuarters end;
+    sum_range<IPL, NNB_LE, false, CO, DF>(end, a, t, e0, min(max(e_mid, e0), c1.e), c1.e, s0, c1.s, K, A, PT, nnb);
+#pragma unroll
+    for (int q = 0; q < IPL; q++) {
+        double *Tq = T + (size_t)((wave * IPL + q) * NC) * 64 + lane;
+#pragma unroll
+        for (int c = 0; c < 4; c++) Tq[c * 64] = A[q][c];
+        if constexpr (CO) Tq[4 * 64] = PT[q];
+        N[(wave * IPL + q) * 64 + lane] = nnb[q];
+    }
+    __syncthreads();
+    if (wave >= IPL) return;
+    nnb[0] = 0;
+#pragma unroll
+    for (int w = 0; w < 4; w++) {
+        const double *Tq = T + (size_t)((w * IPL + wave) * NC) * 64 + lane;
+#pragma unroll
+        for (int c = 0; c < 4; c++) A[0][c] = w ? A[0][c] + Tq[c * 64] : Tq[c * 64];
+        if constexpr (CO) PT[0] = w ? PT[0] + Tq[4 * 64] : Tq[4 * 64];
+        nnb[0] += N[(w * IPL + wave) * 64 + lane];
+    }
+    if constexpr (CO) {
+        // (each lane's i of slot `wave`)
+#pragma unroll
+        for (int q = 1; q < IPL; q++)
+            if (wave == q) {
+                t.self[0] = t.self[q];
+                t.m[0] = t.m[q];
+            }
+        const int sb = t.self[0] >> 3;
+        if (t.self[0] >= 0 && sb >= it.e_blk_begin && sb < e_mid)
+            A[0][3] += (double)(t.m[0] * __builtin_amdgcn_rsqf(__builtin_fmaxf(K.eps2, K.rout2)));
+    }
+    store_sums<CO>(a, it, lane, wave, A[0], PT[0], nnb[0]);
+}
+
+// Work item idx of this class's launch (empty slots have walk < 0).
+template <int NNB_LE, int IPL, bool VC, bool CO, bool DF>
+__device__ __forceinline__ void force_item(const ForceArgs &a, int idx, double *T)
+{
     const Consts K{jv<VC>(a.eps2), jv<VC>(a.rout2), jv<VC>(0.5f), jv<VC>(2.5f)};
-    run_tile<IPL, NNB_LE, VC, CO, DF>(a, it, near_end, threadIdx.x & 63, K);
+    run_tile<IPL, NNB_LE, VC, CO, DF>(a, idx, threadIdx.x & 63, K, T);
 }
 
 // One launch per i-per-lane class: items [0, n_items) of this class, one
@@ -912,6 +1135,8 @@ __device__ __forceinline__ void force_item(const ForceArgs &a, int idx)
 template <int NNB_LE, int IPL, bool VC, bool CO, bool DF, bool P>
 __device__ __forceinline__ void force_items(const ForceArgs &a)
 {
+    __shared__ double sums[4 * IPL * n_sum<CO> * 64];
+    double *T = sums + (size_t)uniform((int)threadIdx.x >> 6) * (IPL * n_sum<CO> * 64);
     if constexpr (P) {
         const int x = (int)blockIdx.x & 7;
         int *cnt = a.counter + x;
@@ -920,12 +1145,12 @@ __device__ __forceinline__ void force_items(const ForceArgs &a)
             if ((threadIdx.x & 63) == 0) k = atomicAdd(cnt, 1);
             k = uniform(k);
             if (k >= a.n_run) break;
-            force_item<NNB_LE, IPL, VC, CO, DF>(a, ((k >> 2) * 8 + x) * 4 + (k & 3));
+            force_item<NNB_LE, IPL, VC, CO, DF>(a, ((k >> 2) * 8 + x) * 4 + (k & 3), T);
         }
     } else {
         const int idx = uniform((int)blockIdx.x * 4 + ((int)threadIdx.x >> 6));
         if (idx >= a.n_items) return;
-        force_item<NNB_LE, IPL, VC, CO, DF>(a, idx);
+        force_item<NNB_LE, IPL, VC, CO, DF>(a, idx, T);
     }
 }
 
@@ -943,6 +1168,35 @@ template <int NNB_LE, int IPL, bool VC, bool P = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(IPL <= 2 ? 7 : 1))) void k_force_co(const ForceArgs a)
 {
     force_items<NNB_LE, IPL, VC, true, false, P>(a);
+}
+
+// Small launches: one item per workgroup, a quarter per wave, and the items
+// of 2 and of 1 i per lane in one launch (a.items and its n_items slots, then
+// the rest of the grid's slots at a.items1).  With few items a wave per item
+// leaves the SIMDs with one or two waves that wait for their scalar loads,
+// and the launch lasts as long as its longest item: 1,702 items (16,384
+// particles) 140 us, 70 us in quarters.  Workgroup b, on XCD b % 8, takes the
+// items of that XCD's runs.
+template <int NNB_LE, bool CO, bool DF> __device__ __forceinline__ void force_split(const ForceArgs &a)
+{
+    __shared__ double sums[4 * 2 * n_sum<CO> * 64];
+    __shared__ int ngb[4 * 2 * 64];
+    const int wave = uniform((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const bool two = (int)blockIdx.x < a.n_items;
+    const int b = two ? (int)blockIdx.x : (int)blockIdx.x - a.n_items;
+    const int idx = ((b >> 5) * 8 + (b & 7)) * 4 + ((b >> 3) & 3);
+    const Consts K{a.eps2, a.rout2, 0.5f, 2.5f};
+    if (two) run_tile_split<2, NNB_LE, CO, DF>(a, a.items, idx, wave, lane, K, sums, ngb);
+    else run_tile_split<1, NNB_LE, CO, DF>(a, a.items1, idx, wave, lane, K, sums, ngb);
+}
+template <int NNB_LE, bool DF> __global__ __launch_bounds__(256) void k_force_split(const ForceArgs a)
+{
+    force_split<NNB_LE, false, DF>(a);
+}
+template <int NNB_LE>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) void k_force_split_co(const ForceArgs a)
+{
+    force_split<NNB_LE, true, false>(a);
 }
 
 // ---------------------------------------------------------------------------
@@ -1264,6 +1518,23 @@ static unsigned fit_blocks(const void *f)
     return (unsigned)(it->second * cus[dev]);
 }
 
+// Whether segment k's force launch takes an item per workgroup (and both
+// i-per-lane classes at once).  A launch ends with its longest items, and one
+// of a few rounds of waves (8,192 slots) is much of it tail: quarters of items
+// shorten that.  Against that stand the four loads of a tile's i and a
+// barrier.  us per evaluation, a wave against a workgroup per item, by items
+// of a launch: 1,702 (16,384 particles) 259 and 204; 20,000 (262,144) 2,795
+// and 2,540; 37,000 (524,288) 5,700 and 5,030; 29,000 (1,048,576) 10,550 and
+// 10,220; 57,000 (2M) 20,700 and 20,370; 124,000 (4,194,304) 43,050 and
+// 43,830.  The kernel holds 1 and 2 i per lane.
+constexpr int SPLIT_MAX_ITEMS = 65536;
+bool split_launch(const BatchDev &b, int k)
+{
+    const SegDev &g = b.seg[k];
+    return !b.plain && !b.persistent && !b.j_vgpr && g.seg_count[2] + g.seg_count[3] == 0 &&
+           g.seg_count[0] + g.seg_count[1] <= SPLIT_MAX_ITEMS;
+}
+
 // nblk blocks of one item per wave; persistent (P): as many blocks as the
 // device holds, at most nblk, a multiple of 8 so that every XCD's run of
 // items has blocks that drain it
@@ -1311,7 +1582,7 @@ hipError_t launch_force(const BatchDev &b, int k, hipStream_t st, unsigned class
         return hipGetLastError();
     }
     static const int ipls[PLAN_CLASSES] = {1, 2, 3, 4};
-    ForceArgs a;
+    ForceArgs a{};
     a.near_blk = b.near_blk;
     a.staged_i = b.staged_i;
     a.staged_e = b.staged_e;
@@ -1331,6 +1602,25 @@ hipError_t launch_force(const BatchDev &b, int k, hipStream_t st, unsigned class
     a.part_accp = b.part_accp;
     a.part_nnb = b.part_nnb;
     a.part_pott = b.part_pott;
+    if (split_launch(b, k)) {
+        if (!(classes & 2u)) return hipSuccess;  // both classes go with the 2-i launch
+        a.items = b.items + g.seg_begin[1];
+        a.n_items = g.seg_count[1];
+        a.items1 = b.items + g.seg_begin[0];
+        const dim3 grid((unsigned)(g.seg_count[0] + g.seg_count[1]));
+        if (grid.x == 0) return hipSuccess;
+        if (b.co) {
+            if (b.nnb_le) hipLaunchKernelGGL(k_force_split_co<1>, grid, dim3(256), 0, st, a);
+            else hipLaunchKernelGGL(k_force_split_co<0>, grid, dim3(256), 0, st, a);
+        } else if (b.df) {
+            if (b.nnb_le) hipLaunchKernelGGL((k_force_split<1, true>), grid, dim3(256), 0, st, a);
+            else hipLaunchKernelGGL((k_force_split<0, true>), grid, dim3(256), 0, st, a);
+        } else {
+            if (b.nnb_le) hipLaunchKernelGGL((k_force_split<1, false>), grid, dim3(256), 0, st, a);
+            else hipLaunchKernelGGL((k_force_split<0, false>), grid, dim3(256), 0, st, a);
+        }
+        return hipGetLastError();
+    }
     // the longer classes first: the 1-i launch is about one round of waves,
     // and its run-down tail then overlaps the other force stream's work
     // instead of holding back a longer launch behind it on this stream

@@ -795,3 +795,50 @@ def test_results_over_chunk_edges(n, co):
         f.retrieve(0, len(ws), L.n_epi[b:b + 200], [force[s] for s in own])
     for k, v in zip(("acc", "pot", "n_ngb", "pot_tot"), got):
         assert np.array_equal(force[k], v), k
+
+
+@pytest.mark.parametrize("co", [0, 1])
+@pytest.mark.parametrize("nj,ns", [(0, 70), (5, 0), (64, 0), (65, 1), (500, 3), (513, 255), (900, 2000), (4000, 31),
+                                   (4000, 33)])
+def test_quarters_of_items_are_bit_identical(nj, ns, co):
+    """An item's j-range is summed in four quarters, cut where the FP32 sums
+    are flushed (64 EPJ from the range's and from the far part's begin, 32
+    SPJ): four waves that take one each (default launches) give the bits of
+    one wave that takes them in turn (persistent launches), for ranges of
+    EPJ only, SPJ only, less than a flush, with the near part's end anywhere
+    in them, and agree with the FP64 oracle."""
+    rng = np.random.default_rng(nj + ns)
+    n_epi = np.array([100, 1, 64, 37], np.int32)
+    ni = int(n_epi.sum())
+    ni_w = [n_epi[:w].sum() for w in range(5)]
+    n = nj + 2 * ni + 200
+    pos = rng.normal(0, 0.02, (n, 3))  # half of the j within the cutoff region of the i
+    pos[ni:] += rng.choice([0.0, 0.3], (n - ni, 1))
+    mass, rs = rng.uniform(0.5, 1.5, n) / n, np.full(n, 0.03)
+    spos, smass = rng.normal(0, 0.1, (max(ns, 1), 3)) + 2.0, np.full(max(ns, 1), 0.1)
+    quad = np.zeros((max(ns, 1), 6))
+    quad[:, :3] = rng.uniform(0.01, 0.02, (max(ns, 1), 3))
+    nje = max(nj, int(n_epi.max())) if co else nj  # (changeover: each i's own EPJ is on its list)
+    ide = [np.concatenate([np.arange(ni_w[w], ni_w[w + 1]),
+                           rng.permutation(np.arange(ni, n))])[:nje] if co else rng.integers(0, n, nje) for w in range(4)]
+    a = dict(n_epi=n_epi, n_epj=np.full(4, nje, np.int32), n_spj=np.full(4, ns, np.int32), epi_pos=pos[:ni],
+             epi_rs=rs[:ni], id_epj=np.concatenate(ide).astype(np.int32),
+             id_spj=np.tile(np.arange(ns, dtype=np.int32), 4), epj_pos=pos, epj_mass=mass, epj_rs=rs, spj_pos=spos,
+             spj_mass=smass, spj_quad=quad)
+    out = []
+    for persistent in (0, 1):
+        for chunk in (0, 1 << 20):
+            ctx = sf.Context(0, eps2=1e-6, rcut2=4e-4, changeover=co, persistent=persistent, chunk_j=chunk)
+            r = sf.Resident(ctx, **a)
+            if co:
+                r.changeover(np.arange(ni), np.arange(n), np.full(n, 0.002), np.full(n, 0.02))
+            r.run()
+            out.append(r.results())
+            r.close()
+            ctx.close()
+    for k in (0, 1):
+        assert all(np.array_equal(x, y) for x, y in zip(out[k], out[k + 2]))
+    if not co:
+        racc, rpot, _ = O.soft_force_walks(**a, eps2=1e-6, rout2=4e-4)
+        for acc, pot, _ in out:
+            assert np.median(rel_err(acc, racc)) <= MED and np.median(rel_err(pot, rpot)) <= MED
