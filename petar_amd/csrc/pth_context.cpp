@@ -501,7 +501,7 @@ int pth_dispatch(pth_ctx *c, int tag, int n_walk, const void *const *epi, const 
     {
 #pragma omp single nowait
         plan_ok = make_plan(n_walk, n_epi, n_epj, n_spj, c->par.exec_mode, c->par.chunk_j, c->par.max_ipl, P, 1,
-                            c->mono_sent);
+                            c->mono_sent, 0, true);
 #pragma omp for schedule(dynamic) nowait
         for (int w = 0; w < n_walk; w++) {
             const int ne = n_epj[w], ns = n_spj[w];
@@ -554,7 +554,7 @@ int pth_dispatch(pth_ctx *c, int tag, int n_walk, const void *const *epi, const 
     Arena A;
     if (runs) A.layout(P, n_ide, n_ids, co, n_re, n_rs);
     else A.layout(P, n_ide, n_ids, co);
-    HIPCHK(c, c->h_arena.ensure_keep(A.total, A.walks), "pinned arena allocation");
+    HIPCHK(c, c->h_arena.ensure_keep(A.upload, A.walks), "pinned arena allocation");
     const bool grow = A.total > c->d_arena.cap;
     if (grow) HIPCHK(c, hipStreamSynchronize(c->stream), "hipStreamSynchronize");
     HIPCHK(c, c->d_arena.ensure(A.total), "device arena allocation");
@@ -653,10 +653,11 @@ int pth_dispatch(pth_ctx *c, int tag, int n_walk, const void *const *epi, const 
     c->prof.n_call += 1;
     T.timed = c->prof_on;
     if (T.timed) HIPCHK(c, hipEventRecord(T.prof[0], c->stream), "hipEventRecord");
-    HIPCHK(c, hipMemcpyAsync(c->d_arena.p, h, A.total, hipMemcpyHostToDevice, c->stream), "batch upload");
+    HIPCHK(c, hipMemcpyAsync(c->d_arena.p, h, A.upload, hipMemcpyHostToDevice, c->stream), "batch upload");
     HIPCHK(c, hipEventRecord(c->ev_upload, c->stream), "hipEventRecord");
     if (T.timed) HIPCHK(c, hipEventRecord(T.prof[1], c->stream), "hipEventRecord");
     if (c->par.exec_mode == PTH_EXEC_PLAIN) HIPCHK(c, hipStreamSynchronize(c->stream), "upload sync");
+    HIPCHK(c, plan_items(P, A, c->d_arena.as<char>(), c->stream), "planning kernel");
     BatchDev b;
     // the SPJ table of the sent superparticles (quadrupole form), for this
     // batch's eps2
@@ -925,7 +926,7 @@ int pth_resident_create(pth_ctx *c, pth_resident **out, int n_walk, const int *n
     };
     hipError_t e;
     // host mirrors (pageable is fine: uploaded once)
-    std::vector<char> h(r->A.total);
+    std::vector<char> h(r->A.upload);
     EpiDev *he = reinterpret_cast<EpiDev *>(h.data() + r->A.epi);
     for (long long i = 0; i < P.ni_tot; i++) {
         he[i].x = epi_pos[3 * i];
@@ -968,7 +969,7 @@ int pth_resident_create(pth_ctx *c, pth_resident **out, int n_walk, const int *n
         sj[i].qyz = (float)q[5];
         sj[i].pad[0] = sj[i].pad[1] = sj[i].pad[2] = 0.f;
     }
-    if ((e = hipMemcpy(r->arena.p, h.data(), r->A.total, hipMemcpyHostToDevice))) return bail(e, "resident upload");
+    if ((e = hipMemcpy(r->arena.p, h.data(), r->A.upload, hipMemcpyHostToDevice))) return bail(e, "resident upload");
     if (n_epj_tot && (e = hipMemcpy(r->epj.p, ej.data(), sizeof(EpjDev) * n_epj_tot, hipMemcpyHostToDevice)))
         return bail(e, "resident upload");
     if (n_spj_tot && (e = P.mono ? hipMemcpy(r->spj.p, sm.data(), sizeof(EpjDev) * n_spj_tot, hipMemcpyHostToDevice)
@@ -1423,7 +1424,7 @@ int resident_setup(pth_resident *r, int n_walk, const int *n_epi, const int *n_e
         if (!pre_ok) return c->fail(PTH_ERR_CAPACITY, std::string(who) + ": sizes exceed the int32 index range");
         std::swap(r->plan, *pre);
     } else if (!make_plan(n_walk, n_epi, n_epj, n_spj, c->par.exec_mode, c->par.chunk_j, c->par.max_ipl, r->plan,
-                          r->n_seg, c->par.spj_monopole != 0, seg_pairs(c->par)))
+                          r->n_seg, c->par.spj_monopole != 0, seg_pairs(c->par), true))
         return c->fail(PTH_ERR_CAPACITY, std::string(who) + ": sizes exceed the int32 index range");
     const Plan &P = r->plan;
     r->co = c->par.changeover != 0;
@@ -1491,6 +1492,7 @@ hipError_t resident_finish(pth_resident *r)
 {
     const Plan &P = r->plan;
     pth_ctx *c = r->ctx;
+    if (const hipError_t e = plan_items(P, r->A, r->arena.as<char>(), c->stream)) return e;
     if (!P.mono) {
         const hipError_t e = launch_spj_table(r->spj.as<SpjDev>(), r->n_spj_tot, (float)c->par.eps2,
                                               r->spj_tab.as<SpjTab>(), c->stream);

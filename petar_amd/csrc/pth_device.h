@@ -112,6 +112,34 @@ struct RItem {
     int out, n_i, part_first, n_part, ipl, pad[3];
 };
 
+// What the device needs to write a walk's items (k_plan): where the walk's
+// items of 1 and of 2 i per lane, its reduction items and its partial slots
+// begin (items counted over all walks, class by class), its tiles of 128 i,
+// its chunks and its segment.
+struct WalkPlan {
+    int item[2];
+    int ritem, part;
+    int n2, nch, seg, pad;
+};
+// A segment's items of 1 and of 2 i per lane: first slot, slots, first item,
+// and where each XCD's run of items begins (in items from the first; entry 8:
+// their number).
+struct SegPlan {
+    int begin[2], slots[2], first[2];
+    int run[2][9];
+};
+
+// Chunk k of nch of a walk's list of nb staged EPJ blocks and ns staged SPJ
+// records: list units [k units / nch, (k + 1) units / nch) (an EPJ slot
+// counts 1, an SPJ record 2), EPJ bounds rounded up to whole blocks.
+__host__ __device__ inline void chunk_cut(long long nb, long long ns, long long nch, long long k, int &e, int &s)
+{
+    const long long ue = nb * 8, units = ue + 2 * ns, u = k * units / nch;
+    const long long eb = ((u < ue ? u : ue) + 7) / 8, sb = ((u > ue ? u - ue : 0) + 1) / 2;
+    e = (int)(k == nch || eb > nb ? nb : eb);
+    s = (int)(k == nch || sb > ns ? ns : sb);
+}
+
 // One segment of a batch: its walks, its items per ipl class and its
 // reduction items (the launches of one segment run in order on one stream).
 struct SegDev {
@@ -187,6 +215,11 @@ hipError_t launch_spj_table(const SpjDev *spj, long long n, float eps2, SpjTab *
 hipError_t launch_expand_runs(const WalkDev *walks, int w_begin, int n_walk, const int *rid_e, const int *rpos_e,
                               const int *run_eo, const int *rid_s, const int *rpos_s, const int *run_so, int *out_e,
                               int *out_s, hipStream_t st);
+
+// Writes the items and reduction items of a plan made on the device (tiles of
+// at most 128 i).
+hipError_t launch_plan(const WalkDev *walks, const WalkPlan *wplan, int n_walk, const SegPlan *splan, int n_seg,
+                       const long long *es_off, const long long *ss_off, Item *items, RItem *ritems, hipStream_t st);
 
 // Launches of segment k of a batch (k < b.n_seg).
 hipError_t launch_stage(const BatchDev &b, int k, hipStream_t st);

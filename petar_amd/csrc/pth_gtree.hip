@@ -1710,7 +1710,7 @@ int gtree_run(pth_gtree *t, long long n, const double *pos, const double *mass, 
                              seg_pairs(par)};
         t->pre_ok = make_plan((int)ng, ni.data(), nje.data(), njs.data(), t->pre_key.exec_mode, t->pre_key.chunk_j,
                               t->pre_key.max_ipl, t->pre_plan, t->pre_key.n_seg, t->pre_key.mono != 0,
-                              t->pre_key.min_seg_pairs);
+                              t->pre_key.min_seg_pairs, true);
         t->pre_valid = true;
     }
     if ((e = hipGetLastError()) || (e = hipStreamSynchronize(st))) return ctx->hip_fail(e, "tree walk");
@@ -1764,6 +1764,8 @@ int resident_fill_gtree(pth_resident *r, const pth_gtree *t, const char *who)
     if ((e = h2d(A.walks, P.walks.data(), sizeof(WalkDev) * P.walks.size())) ||
         (e = h2d(A.es, P.es_off.data(), sizeof(long long) * P.es_off.size())) ||
         (e = h2d(A.ss, P.ss_off.data(), sizeof(long long) * P.ss_off.size())) ||
+        (e = h2d(A.wplan, P.wplan.data(), sizeof(WalkPlan) * P.wplan.size())) ||
+        (e = h2d(A.splan, P.splan.data(), sizeof(SegPlan) * P.splan.size())) ||
         (e = h2d(A.items, P.items.data(), sizeof(Item) * P.items.size())) ||
         (e = h2d(A.ritems, P.ritems.data(), sizeof(RItem) * P.ritems.size())))
         return bail(e, "resident upload");

@@ -119,7 +119,8 @@ inline size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 // int32 per run), run_eo / run_so the walks'
 // run offsets (n_walk + 1 each), and the lists are expanded on the device.
 struct Arena {
-    size_t epi, epi_id, walks, es, ss, ide, ids, items, ritems, run_e, run_s, run_eo, run_so, total;
+    size_t epi, epi_id, walks, es, ss, wplan, splan, ide, ids, items, ritems, run_e, run_s, run_eo, run_so, total;
+    size_t upload;  // what the host fills: all, or all but the items, which then come last
     bool runs = false;
     // the i records (and ids) lead: [0, i_part(ni_tot, co)), i ids at
     // i_id_offset(ni_tot)
@@ -138,15 +139,19 @@ struct Arena {
         walks = o; o = align256(o + sizeof(WalkDev) * P.walks.size());
         es = o; o = align256(o + sizeof(long long) * P.es_off.size());
         ss = o; o = align256(o + sizeof(long long) * P.ss_off.size());
+        wplan = o; o = align256(o + sizeof(WalkPlan) * P.wplan.size());
+        splan = o; o = align256(o + sizeof(SegPlan) * P.splan.size());
         ide = o; o = align256(o + (runs ? 0 : sizeof(int) * (size_t)n_ide));
         ids = o; o = align256(o + (runs ? 0 : sizeof(int) * (size_t)n_ids));
-        items = o; o = align256(o + sizeof(Item) * P.items.size());
-        ritems = o; o = align256(o + sizeof(RItem) * P.ritems.size());
         run_e = o; o = align256(o + (runs ? 2 * sizeof(int) * (size_t)n_run_e : 0));
         run_s = o; o = align256(o + (runs ? 2 * sizeof(int) * (size_t)n_run_s : 0));
         run_eo = o; o = align256(o + (runs ? sizeof(int) * (P.walks.size() + 1) : 0));
         run_so = o; o = align256(o + (runs ? sizeof(int) * (P.walks.size() + 1) : 0));
+        upload = o;
+        items = o; o = align256(o + sizeof(Item) * (size_t)P.n_slots);
+        ritems = o; o = align256(o + sizeof(RItem) * (size_t)P.n_ritems);
         total = o;
+        if (!P.on_device) upload = o;
     }
 };
 
@@ -288,8 +293,8 @@ inline void fill_batch(BatchDev &b, const Plan &P, const pth_params &par, const 
     b.ni_tot = P.ni_tot;
     b.n_e_slots = P.n_e_slots;
     b.n_s_rec = P.n_s_rec;
-    b.n_items = (int)P.items.size();
-    b.n_ritems = (int)P.ritems.size();
+    b.n_items = P.n_slots;
+    b.n_ritems = P.n_ritems;
     set_segments(b, P);
     b.j_vgpr = par.j_vgpr ? 1 : 0;
     b.plain = (par.exec_mode == PTH_EXEC_PLAIN);
@@ -376,11 +381,26 @@ inline const char *co_plan_error(const Plan &P)
     return nullptr;
 }
 
+// Enqueues the making of the items of a plan that left them to the device, in
+// the arena at base (its upload enqueued before).
+inline hipError_t plan_items(const Plan &P, const Arena &A, char *base, hipStream_t st)
+{
+    if (!P.on_device) return hipSuccess;
+    return launch_plan(reinterpret_cast<const WalkDev *>(base + A.walks),
+                       reinterpret_cast<const WalkPlan *>(base + A.wplan), (int)P.walks.size(),
+                       reinterpret_cast<const SegPlan *>(base + A.splan), (int)P.splan.size(),
+                       reinterpret_cast<const long long *>(base + A.es),
+                       reinterpret_cast<const long long *>(base + A.ss), reinterpret_cast<Item *>(base + A.items),
+                       reinterpret_cast<RItem *>(base + A.ritems), st);
+}
+
 inline void copy_plan_to_arena(char *h, const Plan &P, const Arena &A)
 {
     std::memcpy(h + A.walks, P.walks.data(), sizeof(WalkDev) * P.walks.size());
     std::memcpy(h + A.es, P.es_off.data(), sizeof(long long) * P.es_off.size());
     std::memcpy(h + A.ss, P.ss_off.data(), sizeof(long long) * P.ss_off.size());
+    if (!P.wplan.empty()) std::memcpy(h + A.wplan, P.wplan.data(), sizeof(WalkPlan) * P.wplan.size());
+    if (!P.splan.empty()) std::memcpy(h + A.splan, P.splan.data(), sizeof(SegPlan) * P.splan.size());
     if (!P.items.empty()) std::memcpy(h + A.items, P.items.data(), sizeof(Item) * P.items.size());
     if (!P.ritems.empty()) std::memcpy(h + A.ritems, P.ritems.data(), sizeof(RItem) * P.ritems.size());
 }

@@ -1434,7 +1434,70 @@ __global__ __launch_bounds__(256) void k_expand_runs(const WalkDev *__restrict__
 }
 
 // ---------------------------------------------------------------------------
+// The work items of a plan whose sizes the host made (make_plan with
+// on_device): block b < n_walk writes walk b's items and reduction items,
+// block n_walk + g the empty slots behind the runs of segment g.  A run's
+// items are in walk order (the host's planner puts the most expensive first;
+// their costs differ by at most a factor of two, chunks being of equal size).
+__global__ __launch_bounds__(64) void k_plan(const WalkDev *__restrict__ walks, const WalkPlan *__restrict__ wplan,
+                                             int n_walk, const SegPlan *__restrict__ splan,
+                                             const long long *__restrict__ es_off,
+                                             const long long *__restrict__ ss_off, Item *__restrict__ items,
+                                             RItem *__restrict__ ritems)
+{
+    // slot of item k of run x of a class that begins at slot `begin`
+    auto slot = [](int begin, int x, int k) { return begin + ((k >> 2) * 8 + x) * 4 + (k & 3); };
+    const int lane = threadIdx.x;
+    if ((int)blockIdx.x >= n_walk) {
+        const SegPlan &sp = splan[(int)blockIdx.x - n_walk];
+        const int x = lane & 7;
+        for (int c = 0; c < 2; c++)
+            for (int k = sp.run[c][x + 1] - sp.run[c][x] + (lane >> 3); k < sp.slots[c] / 8; k += 8)
+                items[slot(sp.begin[c], x, k)] = Item{-1, 0, 0, 0, 0, 0, 0, -1};
+        return;
+    }
+    const int w = (int)blockIdx.x;
+    const WalkDev W = walks[w];
+    const WalkPlan wp = wplan[w];
+    const SegPlan &sp = splan[wp.seg];
+    const long long es = es_off[w] >> 3, ss = ss_off[w], nb = (es_off[w + 1] >> 3) - es, ns = ss_off[w + 1] - ss;
+    const int n1 = max(0, (W.n_i - 128 * wp.n2 + 63) >> 6), nt = wp.n2 + n1;
+    for (int j = lane; j < nt * wp.nch; j += 64) {
+        const int t = j / wp.nch, k = j - t * wp.nch;
+        const bool two = t < wp.n2;
+        const int c = two ? 1 : 0, u = two ? t : t - wp.n2;
+        const int begin = two ? 128 * t : 128 * wp.n2 + 64 * u, n = min(two ? 128 : 64, W.n_i - begin);
+        Item it;
+        it.walk = w;
+        it.i_begin = W.i_off + begin;
+        it.n_i_ipl = item_pack(n, c + 1);
+        int e0, e1, s0, s1;
+        chunk_cut(nb, ns, wp.nch, k, e0, s0);
+        chunk_cut(nb, ns, wp.nch, k + 1, e1, s1);
+        it.e_blk_begin = (int)es + e0;
+        it.e_blk_end = (int)es + e1;
+        it.s_begin = (int)ss + s0;
+        it.s_end = (int)ss + s1;
+        const int part_first = wp.part + (two ? 2 * t : 2 * wp.n2 + u) * wp.nch;
+        it.part = wp.nch > 1 ? part_first + k * (c + 1) : -1;
+        const int idx = wp.item[c] + u * wp.nch + k - sp.first[c];
+        int x = 0;
+        for (int q = 1; q < 8; q++) x += idx >= sp.run[c][q];
+        items[slot(sp.begin[c], x, idx - sp.run[c][x])] = it;
+        if (k == 0 && wp.nch > 1) ritems[wp.ritem + t] = RItem{it.i_begin, n, part_first, wp.nch, c + 1, {0, 0, 0}};
+    }
+}
+
+// ---------------------------------------------------------------------------
 // launchers (host)
+
+hipError_t launch_plan(const WalkDev *walks, const WalkPlan *wplan, int n_walk, const SegPlan *splan, int n_seg,
+                       const long long *es_off, const long long *ss_off, Item *items, RItem *ritems, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_plan, dim3((unsigned)(n_walk + n_seg)), dim3(64), 0, st, walks, wplan, n_walk, splan, es_off,
+                       ss_off, items, ritems);
+    return hipGetLastError();
+}
 
 hipError_t launch_spj_table(const SpjDev *spj, long long n, float eps2, SpjTab *tab, hipStream_t st)
 {

@@ -185,7 +185,7 @@ extern "C" int pth_resident_eval_noalloc(pth_ctx *c, int n_walk, const int *n_ep
     // the plan: one segment on the context's stream (a walk's items and
     // results do not depend on the segmentation)
     Plan &P = c->na_plan;
-    if (!make_plan(n_walk, n_epi, n_epj, n_spj, PTH_EXEC_FUSED, c->par.chunk_j, c->par.max_ipl, P, 1, mono))
+    if (!make_plan(n_walk, n_epi, n_epj, n_spj, PTH_EXEC_FUSED, c->par.chunk_j, c->par.max_ipl, P, 1, mono, 0, true))
         return c->fail(PTH_ERR_CAPACITY, W + ": sizes exceed the int32 index range");
     Arena A{};
     A.layout(P, n_ide, n_ids, false);
@@ -239,6 +239,8 @@ extern "C" int pth_resident_eval_noalloc(pth_ctx *c, int n_walk, const int *n_ep
     if ((e = up(o_arena + A.walks, P.walks.data(), sizeof(WalkDev) * P.walks.size())) ||
         (e = up(o_arena + A.es, P.es_off.data(), sizeof(long long) * P.es_off.size())) ||
         (e = up(o_arena + A.ss, P.ss_off.data(), sizeof(long long) * P.ss_off.size())) ||
+        (e = up(o_arena + A.wplan, P.wplan.data(), sizeof(WalkPlan) * P.wplan.size())) ||
+        (e = up(o_arena + A.splan, P.splan.data(), sizeof(SegPlan) * P.splan.size())) ||
         (e = up(o_arena + A.items, P.items.data(), sizeof(Item) * P.items.size())) ||
         (e = up(o_arena + A.ritems, P.ritems.data(), sizeof(RItem) * P.ritems.size())) ||
         (e = up(o_arena + A.ide, id_epj, sizeof(int) * (size_t)n_ide)) ||
@@ -266,6 +268,7 @@ extern "C" int pth_resident_eval_noalloc(pth_ctx *c, int n_walk, const int *n_ep
                                (const double *)(base + o_sq), (SpjDev *)(base + o_spj));
     }
     HIPCHK(c, hipGetLastError(), "packing kernels");
+    HIPCHK(c, plan_items(P, A, base + o_arena, st), "planning kernel");
     if (!mono) HIPCHK(c, launch_spj_table((const SpjDev *)(base + o_spj), n_spj_tot, (float)c->par.eps2,
                                           (SpjTab *)(base + o_tab), st), "SPJ table kernel");
 

@@ -20,7 +20,9 @@
 #include <algorithm>
 #include <omp.h>
 #include <array>
+#include <atomic>
 #include <climits>
+#include <cmath>
 #include <cstdint>
 #include <cstring>
 
@@ -77,13 +79,13 @@ template <class F> void parallel_for(int n, int grain, F f)
 constexpr int PLAN_WALKS_PER_THREAD = 512;
 constexpr int PLAN_ITEMS_PER_THREAD = 32768;
 
-// Least-cost cover of n i-particles by tiles of 256 (ipl 4), 192 (ipl 3),
-// 128 (ipl 2) and 64 (ipl 1) lanes x i, for a walk with n_e EPJ and n_s
-// SPJ; ties go to the cover with fewer 1-i tiles (the least efficient
-// class: most idle lanes, least work per scalar load).
-void tile_walk(int n, long long n_e, long long n_s, int max_ipl, std::vector<Tile> &out)
+// Least-cost cover of n i-particles by n_tile[k] tiles of 64 (k + 1) i (k + 1
+// per lane), for a walk with n_e EPJ and n_s SPJ; ties go to the cover with
+// fewer 1-i tiles (the least efficient class: most idle lanes, least work per
+// scalar load).
+void cover(int n, long long n_e, long long n_s, int max_ipl, int (&n_tile)[PLAN_CLASSES])
 {
-    out.clear();
+    for (int &t : n_tile) t = 0;
     if (n <= 0) return;
     auto cost = [&](int ipl) { return 64.0 * ipl * (epj_unit_cost(ipl) * n_e + spj_unit_cost(ipl) * n_s); };
     // the largest allowed class any number of times, each smaller one (but
@@ -92,21 +94,28 @@ void tile_walk(int n, long long n_e, long long n_s, int max_ipl, std::vector<Til
     const int dmax = (max_ipl >= 4) ? 3 : (max_ipl == 3) ? (n + 191) / 192 : 0;
     const int bmax = (max_ipl >= 3) ? 3 : (max_ipl == 2) ? (n + 127) / 128 : 0;
     double best = -1;
-    int ba = 0, bd = 0, bb = 0, bc = 0;
     for (int a = 0; a <= amax; a++)
         for (int d = 0; d <= dmax; d++)
             for (int b = 0; b <= bmax; b++) {
                 const long long covered = 256LL * a + 192LL * d + 128LL * b;
                 const int c = covered >= n ? 0 : (int)((n - covered + 63) / 64);
                 const double t = a * cost(4) + d * cost(3) + b * cost(2) + c * cost(1);
-                if (best < 0 || t < best - 1e-9 || (t < best + 1e-9 && c < bc)) {
+                if (best < 0 || t < best - 1e-9 || (t < best + 1e-9 && c < n_tile[0])) {
                     best = t;
-                    ba = a;
-                    bd = d;
-                    bb = b;
-                    bc = c;
+                    n_tile[3] = a;
+                    n_tile[2] = d;
+                    n_tile[1] = b;
+                    n_tile[0] = c;
                 }
             }
+}
+
+void tile_walk(int n, long long n_e, long long n_s, int max_ipl, std::vector<Tile> &out)
+{
+    out.clear();
+    if (n <= 0) return;
+    int n_tile[PLAN_CLASSES];
+    cover(n, n_e, n_s, max_ipl, n_tile);
     int pos = 0;
     auto emit = [&](int count, int ipl) {
         for (int k = 0; k < count && pos < n; k++) {
@@ -115,16 +124,151 @@ void tile_walk(int n, long long n_e, long long n_s, int max_ipl, std::vector<Til
             pos += m;
         }
     };
-    emit(ba, 4);
-    emit(bd, 3);
-    emit(bb, 2);
-    emit(bc, 1);
+    for (int ipl = PLAN_CLASSES; ipl > 0; ipl--) emit(n_tile[ipl - 1], ipl);
+}
+
+// Cost of the nch items of one tile of a walk.
+double tile_cost(int ipl, long long nb, long long ns, long long nch)
+{
+    return 64.0 * ipl * (epj_unit_cost(ipl) * 8.0 * nb + spj_unit_cost(ipl) * ns + 50.0 * nch);
+}
+
+// Segments: contiguous walk ranges of about equal item cost (wcost: its
+// prefix sums over the walks).  The first one gets half the cost of the
+// others: its staging is the one part of a pipelined evaluation that nothing
+// overlaps.  A pipeline pays for its launches and cross-stream events, so each
+// segment gets at least min_seg_pairs interactions.
+std::vector<int> segment_cuts(const Plan &P, const std::vector<double> &wcost, int n_seg, long long min_seg_pairs)
+{
+    const int n_walk = (int)P.walks.size();
+    n_seg = std::min(std::max(n_seg, 1), MAX_SEGMENTS);
+    if (n_seg > n_walk) n_seg = std::max(n_walk, 1);
+    if (min_seg_pairs > 0)
+        n_seg = (int)std::min<long long>(n_seg, std::max<long long>(1, (P.n_epep + P.n_epsp) / min_seg_pairs));
+    std::vector<int> cut(n_seg + 1, 0);
+    cut[n_seg] = n_walk;
+    for (int g = 1; g < n_seg; g++) {
+        const double target = wcost[n_walk] * (g - 0.5) / (n_seg - 0.5);
+        cut[g] = (int)(std::lower_bound(wcost.begin(), wcost.end(), target) - wcost.begin());
+        cut[g] = std::min(std::max(cut[g], cut[g - 1]), n_walk);
+    }
+    return cut;
+}
+
+// The sizes of a plan whose items the device makes (walks, staged offsets and
+// interaction counts of P are there).
+bool size_plan(Plan &P, long long cj, int max_ipl, int n_seg, long long min_seg_pairs, std::vector<double> &wcost)
+{
+    const int n_walk = (int)P.walks.size();
+    P.on_device = true;
+    P.wplan.resize(n_walk);
+    wcost.assign(n_walk + 1, 0.0);
+    auto blocks = [&](int w) { return (P.es_off[w + 1] - P.es_off[w]) / 8; };
+    auto recs = [&](int w) { return P.ss_off[w + 1] - P.ss_off[w]; };
+    auto tiles1 = [&](int w) { return std::max(0, (P.walks[w].n_i - 128 * P.wplan[w].n2 + 63) / 64); };
+    std::atomic<bool> fits(true);
+    parallel_for(n_walk, PLAN_WALKS_PER_THREAD, [&](int wb, int we) {
+        for (int w = wb; w < we; w++) {
+            const WalkDev &W = P.walks[w];
+            WalkPlan &p = P.wplan[w];
+            p = WalkPlan{};
+            if (W.n_i <= 0) continue;
+            const long long nb = blocks(w), ns = recs(w);
+            const long long nch = std::max(1LL, (8 * nb + 2 * ns + cj - 1) / cj);
+            int n_tile[PLAN_CLASSES];
+            cover(W.n_i, P.mono ? (long long)W.n_e + W.n_s : W.n_e, P.mono ? 0 : W.n_s, max_ipl, n_tile);
+            if (nch * (n_tile[0] + 2LL * n_tile[1]) > INT_MAX) fits = false;
+            p.n2 = n_tile[1];
+            p.nch = (int)nch;
+            wcost[w + 1] = n_tile[1] * tile_cost(2, nb, ns, nch) + n_tile[0] * tile_cost(1, nb, ns, nch);
+        }
+    });
+    if (!fits) return false;
+    long long item[2] = {0, 0}, ritem = 0, part = 0;
+    for (int w = 0; w < n_walk; w++) {
+        WalkPlan &p = P.wplan[w];
+        const long long n1 = tiles1(w), n2 = p.n2;
+        p.item[0] = (int)item[0];
+        p.item[1] = (int)item[1];
+        p.ritem = (int)ritem;
+        p.part = (int)part;
+        item[0] += n1 * p.nch;
+        item[1] += n2 * p.nch;
+        if (p.nch > 1) {
+            ritem += n1 + n2;
+            part += (n1 + 2 * n2) * p.nch;
+        }
+        if (item[0] > INT_MAX || item[1] > INT_MAX || part > INT_MAX) return false;
+        wcost[w + 1] += wcost[w];
+    }
+    P.n_real_items = (int)(item[0] + item[1]);
+    P.n_ritems = (int)ritem;
+    P.n_part = (int)part;
+    const std::vector<int> cut = segment_cuts(P, wcost, n_seg, min_seg_pairs);
+    n_seg = (int)cut.size() - 1;
+    P.segs.resize(n_seg);
+    P.splan.resize(n_seg);
+    auto first_item = [&](int w, int c) { return w < n_walk ? (long long)P.wplan[w].item[c] : item[c]; };
+    parallel_for(n_seg, 1, [&](int gb, int ge) {
+        for (int g = gb; g < ge; g++) {
+            SegPlan &sp = P.splan[g];
+            sp = SegPlan{};
+            for (int w = cut[g]; w < cut[g + 1]; w++) P.wplan[w].seg = g;
+            for (int c = 0; c < 2; c++) {
+                auto cost = [&](int w) {
+                    return (c ? P.wplan[w].n2 : tiles1(w)) * tile_cost(c + 1, blocks(w), recs(w), P.wplan[w].nch);
+                };
+                // eight runs of equal cost, cut at items: a walk's items of
+                // a class have about equal costs
+                double total = 0, acc = 0;
+                for (int w = cut[g]; w < cut[g + 1]; w++) total += cost(w);
+                const long long i0 = first_item(cut[g], c), i1 = first_item(cut[g + 1], c);
+                sp.first[c] = (int)i0;
+                int x = 1;
+                for (int w = cut[g]; w < cut[g + 1] && x < XCDS; w++) {
+                    const double cw = cost(w);
+                    const long long k0 = first_item(w, c), n = first_item(w + 1, c) - k0;
+                    for (; x < XCDS && n > 0 && acc + cw > total * x / XCDS; x++) {
+                        const long long m = (long long)std::ceil((total * x / XCDS - acc) * (double)n / cw);
+                        sp.run[c][x] = (int)(k0 - i0 + std::min(std::max(m, 0LL), n));
+                    }
+                    acc += cw;
+                }
+                for (; x <= XCDS; x++) sp.run[c][x] = (int)(i1 - i0);
+                int longest = 0;
+                for (int q = 0; q < XCDS; q++) longest = std::max(longest, sp.run[c][q + 1] - sp.run[c][q]);
+                sp.slots[c] = (longest + ITEMS_PER_BLOCK - 1) / ITEMS_PER_BLOCK * ITEMS_PER_BLOCK * XCDS;
+            }
+        }
+    });
+    long long cursor = 0;
+    for (int g = 0; g < n_seg; g++) {
+        PlanSeg &sg = P.segs[g];
+        sg = PlanSeg();
+        sg.walk_begin = cut[g];
+        sg.walk_end = cut[g + 1];
+        sg.ritem_begin = cut[g] < n_walk ? P.wplan[cut[g]].ritem : P.n_ritems;
+        sg.ritem_count = (cut[g + 1] < n_walk ? P.wplan[cut[g + 1]].ritem : P.n_ritems) - sg.ritem_begin;
+        for (int c = 0; c < 2; c++) {
+            P.splan[g].begin[c] = sg.seg_begin[c] = (int)cursor;
+            sg.seg_count[c] = P.splan[g].slots[c];
+            cursor += P.splan[g].slots[c];
+            if (cursor > INT_MAX) return false;
+        }
+        sg.seg_begin[2] = sg.seg_begin[3] = (int)cursor;
+    }
+    P.n_slots = (int)cursor;
+    for (int c = 0; c < PLAN_CLASSES; c++) {
+        P.seg_begin[c] = P.segs[0].seg_begin[c];
+        P.seg_count[c] = P.segs[0].seg_count[c];
+    }
+    return true;
 }
 
 }  // namespace
 
 bool make_plan(int n_walk, const int *n_epi, const int *n_epj, const int *n_spj, int exec_mode,
-               int chunk_j, int max_ipl, Plan &P, int n_seg, bool mono, long long min_seg_pairs)
+               int chunk_j, int max_ipl, Plan &P, int n_seg, bool mono, long long min_seg_pairs, bool on_device)
 {
     // the item array keeps its size from the previous plan (every slot is
     // written below, so growing it is the only initialisation it needs)
@@ -169,6 +313,7 @@ bool make_plan(int n_walk, const int *n_epi, const int *n_epj, const int *n_spj,
 
     const long long cj = (chunk_j > 0) ? chunk_j : DEFAULT_CHUNK_J;
     static thread_local Scratch S;
+    if (on_device && max_ipl <= 2) return size_plan(P, cj, max_ipl, n_seg, min_seg_pairs, S.wcost);
     // chunking of walk w: nch chunks, EPJ block / SPJ record bounds
     auto chunks = [&](int w, std::vector<long long> &eb, std::vector<long long> &sb) -> long long {
         const long long nb = (P.es_off[w + 1] - P.es_off[w]) / 8;
@@ -176,17 +321,14 @@ bool make_plan(int n_walk, const int *n_epi, const int *n_epj, const int *n_spj,
         const long long units = nb * 8 + 2LL * n_s;
         long long nch = (units + cj - 1) / cj;
         if (nch < 1) nch = 1;
-        // chunk k covers list units [k*units/nch, (k+1)*units/nch); EPJ
-        // boundaries are rounded to whole blocks of 8
         eb.resize(nch + 1);
         sb.resize(nch + 1);
         for (long long k = 0; k <= nch; k++) {
-            const long long u = (k == nch) ? units : (k * units) / nch;
-            eb[k] = std::min((std::min(u, nb * 8) + 7) / 8, nb);
-            sb[k] = std::min((std::max(0LL, u - nb * 8) + 1) / 2, n_s);
+            int e, r;
+            chunk_cut(nb, n_s, nch, k, e, r);
+            eb[k] = e;
+            sb[k] = r;
         }
-        eb[nch] = nb;
-        sb[nch] = n_s;
         return nch;
     };
     // 1. per walk: items (tiles x chunks), reduction items and partial slots
@@ -273,25 +415,10 @@ bool make_plan(int n_walk, const int *n_epi, const int *n_epj, const int *n_spj,
         }
     });
     P.n_real_items = (int)seq.size();
-    // 2. segments: contiguous walk ranges of about equal item cost (the
-    //    first one half of it)
-    if (n_seg < 1) n_seg = 1;
-    if (n_seg > MAX_SEGMENTS) n_seg = MAX_SEGMENTS;
-    if (n_seg > n_walk) n_seg = std::max(n_walk, 1);
-    // a pipeline pays for its launches and cross-stream events, so each
-    // segment gets at least min_seg_pairs interactions
-    if (min_seg_pairs > 0)
-        n_seg = (int)std::min<long long>(n_seg, std::max<long long>(1, (P.n_epep + P.n_epsp) / min_seg_pairs));
+    // 2. segments
     for (int w = 0; w < n_walk; w++) wcost[w + 1] += wcost[w];
-    // the first segment gets half the cost of the others: its staging is the
-    // one part of a pipelined evaluation that nothing overlaps
-    std::vector<int> cut(n_seg + 1, 0);
-    cut[n_seg] = n_walk;
-    for (int g = 1; g < n_seg; g++) {
-        const double target = wcost[n_walk] * (g - 0.5) / (n_seg - 0.5);
-        cut[g] = (int)(std::lower_bound(wcost.begin(), wcost.end(), target) - wcost.begin());
-        cut[g] = std::min(std::max(cut[g], cut[g - 1]), n_walk);
-    }
+    const std::vector<int> cut = segment_cuts(P, wcost, n_seg, min_seg_pairs);
+    n_seg = (int)cut.size() - 1;
     // 3. cost buckets for the most-expensive-first order inside a run: a
     //    counting sort on the cost's binary exponent and top 4 mantissa bits
     //    (16 steps per octave), stable inside a bucket
@@ -389,6 +516,8 @@ bool make_plan(int n_walk, const int *n_epi, const int *n_epj, const int *n_spj,
                 }
             }
     });
+    P.n_slots = (int)P.items.size();
+    P.n_ritems = (int)P.ritems.size();
     for (int cls = 0; cls < PLAN_CLASSES; cls++) {  // whole-plan view (one segment)
         P.seg_begin[cls] = P.segs[0].seg_begin[cls];
         P.seg_count[cls] = P.segs[0].seg_count[cls];

@@ -248,8 +248,8 @@ void bind(SCluster &c, BatchDev &b, char *base, char *sc, const pth_params &par)
     b.ni_tot = P.ni_tot;
     b.n_e_slots = P.n_e_slots;
     b.n_s_rec = P.n_s_rec;
-    b.n_items = (int)P.items.size();
-    b.n_ritems = (int)P.ritems.size();
+    b.n_items = P.n_slots;
+    b.n_ritems = P.n_ritems;
     set_segments(b, P);
     b.j_vgpr = par.j_vgpr ? 1 : 0;
     b.nnb_le = (par.nnb_mode == 1);

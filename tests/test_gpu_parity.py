@@ -842,3 +842,39 @@ def test_quarters_of_items_are_bit_identical(nj, ns, co):
         racc, rpot, _ = O.soft_force_walks(**a, eps2=1e-6, rout2=4e-4)
         for acc, pot, _ in out:
             assert np.median(rel_err(acc, racc)) <= MED and np.median(rel_err(pot, rpot)) <= MED
+
+
+@pytest.mark.parametrize("max_ipl,segments", [(1, 1), (2, 1), (2, 5)])
+def test_device_plan_equals_host_plan(max_ipl, segments):
+    """A resident evaluation's items are written by the device (max_ipl 1 or
+    2); after a re-plan with the same tiles and chunks they come from the host's
+    planner.  The results are the same bit for bit, for walks with no i, no
+    lists, one chunk and many, tiles of every remainder."""
+    rng = np.random.default_rng(7)
+    nw = 150
+    n_epi = rng.integers(0, 300, nw)
+    n_epi[:8] = (0, 1, 63, 64, 65, 127, 128, 129)
+    n_epj, n_spj = (10 ** rng.uniform(0, 4, nw)).astype(int), (10 ** rng.uniform(0, 3.5, nw)).astype(int)
+    n_epj[10:14], n_spj[12:16] = 0, 0
+    ni, n = int(n_epi.sum()), 20000
+    pos, spos = rng.normal(0, 0.3, (n, 3)), rng.normal(0, 0.3, (4000, 3)) + 3.0
+    a = dict(n_epi=n_epi, n_epj=n_epj, n_spj=n_spj, epi_pos=rng.normal(0, 0.3, (ni, 3)), epi_rs=np.full(ni, 0.01),
+             id_epj=rng.integers(0, n, int(n_epj.sum())), id_spj=rng.integers(0, 4000, int(n_spj.sum())),
+             epj_pos=pos, epj_mass=rng.uniform(1, 2, n) / n, epj_rs=np.full(n, 0.01), spj_pos=spos,
+             spj_mass=np.full(4000, 0.01), spj_quad=rng.uniform(0, 1e-4, (4000, 6)))
+    for persistent in (0, 1):
+        ctx = sf.Context(0, eps2=1e-8, rcut2=1e-4, max_ipl=max_ipl, segments=segments, min_seg_pairs=1.0,
+                         persistent=persistent)
+        r = sf.Resident(ctx, **a)
+        r.run()
+        dev, n_items = r.results(), r.stats()["n_items"]
+        r.replan(max_ipl, 0)
+        r.run()
+        host_ = r.results()
+        assert r.stats()["n_items"] == n_items
+        assert all(np.array_equal(x, y) for x, y in zip(dev, host_))
+        r.close()
+        ctx.close()
+    racc, rpot, rnnb = O.soft_force_walks(**a, eps2=1e-8, rout2=1e-4)
+    assert np.median(rel_err(dev[0], racc)[np.abs(racc).sum(1) > 0]) <= MED
+    assert np.mean(dev[2] != rnnb) <= 1e-3
