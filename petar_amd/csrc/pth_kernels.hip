@@ -41,6 +41,7 @@
 
 #include <climits>
 #include <mutex>
+#include <type_traits>
 #include <unordered_map>
 
 #include "pth_device.h"
@@ -151,10 +152,31 @@ struct StageArgs {
     int *counters;
 };
 
+// The reduction of a wave's values by op (idempotent: min or max), in lane 63:
+// the vector ALU's lane shifts (DPP) instead of 84 LDS permutes (staging of
+// the 16,384-particle cluster 47 to 43 us, of 4,096 particles 21 to 17).
+template <class F> __device__ __forceinline__ double wave_last(double v, F op)
+{
+    auto step = [&](auto ctrl, auto rows) {
+        const int lo = __double2loint(v), hi = __double2hiint(v);
+        v = op(v, __hiloint2double(
+                      __builtin_amdgcn_update_dpp(hi, hi, decltype(ctrl)::value, decltype(rows)::value, 0xf, false),
+                      __builtin_amdgcn_update_dpp(lo, lo, decltype(ctrl)::value, decltype(rows)::value, 0xf, false)));
+    };
+    using std::integral_constant;
+    step(integral_constant<int, 0x111>(), integral_constant<int, 0xf>());  // row_shr:1
+    step(integral_constant<int, 0x112>(), integral_constant<int, 0xf>());  // row_shr:2
+    step(integral_constant<int, 0x114>(), integral_constant<int, 0xf>());  // row_shr:4
+    step(integral_constant<int, 0x118>(), integral_constant<int, 0xf>());  // row_shr:8
+    step(integral_constant<int, 0x142>(), integral_constant<int, 0xa>());  // row_bcast:15 into rows 1, 3
+    step(integral_constant<int, 0x143>(), integral_constant<int, 0xc>());  // row_bcast:31 into rows 2, 3
+    return v;
+}
+
 // SPJ list entries [k_begin, k_end) of walk w: positions relative to the
 // centre and table indices, U per thread and pass so that U gathers are in
 // flight
-template <int U>
+template <int U, int WG>
 __device__ __forceinline__ void stage_spj(const StageArgs &a, int w, const WalkDev &wk, const double (&c)[3],
                                           int k_begin, int k_end)
 {
@@ -162,11 +184,11 @@ __device__ __forceinline__ void stage_spj(const StageArgs &a, int w, const WalkD
     const int *ids = a.id_spj + wk.s_off;
     const SpjDev *__restrict__ spj = a.spj;
     const int tid = (int)threadIdx.x;
-    for (int k0 = k_begin; k0 < k_end; k0 += 256 * U) {
+    for (int k0 = k_begin; k0 < k_end; k0 += WG * U) {
         int id[U];
 #pragma unroll
         for (int u = 0; u < U; u++) {
-            const int k = k0 + 256 * u + tid;
+            const int k = k0 + WG * u + tid;
             id[u] = k < k_end ? ids[k] : -1;
         }
         double px[U], py[U], pz[U];
@@ -179,7 +201,7 @@ __device__ __forceinline__ void stage_spj(const StageArgs &a, int w, const WalkD
             }
 #pragma unroll
         for (int u = 0; u < U; u++)
-            if (id[u] >= 0) put_spj(out_s + (k0 + 256 * u + tid), px[u], py[u], pz[u], c, id[u]);
+            if (id[u] >= 0) put_spj(out_s + (k0 + WG * u + tid), px[u], py[u], pz[u], c, id[u]);
     }
 }
 
@@ -194,12 +216,14 @@ __device__ __forceinline__ void stage_spj(const StageArgs &a, int w, const WalkD
 // staged_ic (the force kernel drops the self pair by slot and takes the i's
 // changeover radii from there).  walk_err counts i with no such entry.
 // EU: EPJ entries per thread and pass of the near/far split, all gathers in
-// flight at once: 4 where the launch has few walks (its latency is exposed),
-// 2 where it has many (fewer registers, so that staging waves fit beside the
-// force kernels of other segments) and in changeover mode
-template <bool CO, int EU>
-__global__ __launch_bounds__(256) void k_stage_walk(const StageArgs a)
+// flight at once, of WG threads per walk.  A pass is a chain of two gathers
+// and two barriers (3.5 us): 4 entries where the launch has few walks (its
+// latency is exposed), 2 where it has many (fewer registers, so that staging
+// waves fit beside the force kernels of other segments)
+template <bool CO, int EU, int WG>
+__global__ __launch_bounds__(WG) void k_stage_walk(const StageArgs a)
 {
+    constexpr int NW = WG / 64;
     // the SPJ blocks need only the walk's centre: they run beside the EPJ
     // split, which is sequential within a walk
     const int nw = a.n_walk;
@@ -215,17 +239,17 @@ __global__ __launch_bounds__(256) void k_stage_walk(const StageArgs a)
     float4 *__restrict__ staged_i = a.staged_i;
     float *__restrict__ staged_e = a.staged_e;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    __shared__ double red[4][7];
-    __shared__ int cnt[2 * EU][4];
+    __shared__ double red[NW][7];
+    __shared__ int cnt[2 * EU][NW];
     __shared__ int co_idx[CO ? PTH_CO_HASH : 1];
     __shared__ int co_self[CO ? PTH_CO_MAX_NI : 1];
     __shared__ float co_rin[CO ? PTH_CO_MAX_NI : 1], co_rout[CO ? PTH_CO_MAX_NI : 1], co_m[CO ? PTH_CO_MAX_NI : 1];
     const int n_co = (CO && !spj_wg) ? min(wk.n_i, PTH_CO_MAX_NI) : 0;
     if constexpr (CO) {
         if (!spj_wg) {
-            for (int k = tid; k < PTH_CO_HASH; k += 256) co_idx[k] = -1;
+            for (int k = tid; k < PTH_CO_HASH; k += WG) co_idx[k] = -1;
             __syncthreads();
-            for (int k = tid; k < n_co; k += 256) {
+            for (int k = tid; k < n_co; k += WG) {
                 const long long id = a.epi_id[wk.i_off + k];
                 unsigned h = co_hash(id);
                 // at most PTH_CO_MAX_NI keys in PTH_CO_HASH buckets: a free one exists
@@ -240,33 +264,35 @@ __global__ __launch_bounds__(256) void k_stage_walk(const StageArgs a)
     }
     // -- bounding box and largest r_search of the walk's i
     double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300}, rsm = 0.0;
-    for (int k = tid; k < wk.n_i; k += 256) {
+    for (int k = tid; k < wk.n_i; k += WG) {
         const EpiDev e = epi[wk.i_off + k];
         lo[0] = fmin(lo[0], e.x); hi[0] = fmax(hi[0], e.x);
         lo[1] = fmin(lo[1], e.y); hi[1] = fmax(hi[1], e.y);
         lo[2] = fmin(lo[2], e.z); hi[2] = fmax(hi[2], e.z);
         rsm = fmax(rsm, (double)e.rs);
     }
-    for (int off = 32; off > 0; off >>= 1) {
-        for (int d = 0; d < 3; d++) {
-            lo[d] = fmin(lo[d], __shfl_xor(lo[d], off, 64));
-            hi[d] = fmax(hi[d], __shfl_xor(hi[d], off, 64));
-        }
-        rsm = fmax(rsm, __shfl_xor(rsm, off, 64));
+    for (int d = 0; d < 3; d++) {
+        lo[d] = wave_last(lo[d], [](double x, double y) { return fmin(x, y); });
+        hi[d] = wave_last(hi[d], [](double x, double y) { return fmax(x, y); });
     }
-    if (lane == 0) {
+    rsm = wave_last(rsm, [](double x, double y) { return fmax(x, y); });
+    if (lane == 63) {
         for (int d = 0; d < 3; d++) { red[wave][d] = lo[d]; red[wave][3 + d] = hi[d]; }
         red[wave][6] = rsm;
     }
     __syncthreads();
     double c[3], h[3];
     for (int d = 0; d < 3; d++) {
-        const double l = fmin(fmin(red[0][d], red[1][d]), fmin(red[2][d], red[3][d]));
-        const double u = fmax(fmax(red[0][3 + d], red[1][3 + d]), fmax(red[2][3 + d], red[3][3 + d]));
+        double l = red[0][d], u = red[0][3 + d];
+        for (int v = 1; v < NW; v++) {
+            l = fmin(l, red[v][d]);
+            u = fmax(u, red[v][3 + d]);
+        }
         c[d] = (wk.n_i > 0) ? 0.5 * (l + u) : 0.0;
         h[d] = (wk.n_i > 0) ? 0.5 * (u - l) : 0.0;
     }
-    rsm = fmax(fmax(red[0][6], red[1][6]), fmax(red[2][6], red[3][6]));
+    rsm = red[0][6];
+    for (int v = 1; v < NW; v++) rsm = fmax(rsm, red[v][6]);
     if (spj_wg) {
         const int part = ((int)blockIdx.x - nw) / nw;
         const int k_begin = (int)((long long)wk.n_s * part / a.spj_parts);
@@ -274,11 +300,11 @@ __global__ __launch_bounds__(256) void k_stage_walk(const StageArgs a)
         // (two in changeover mode: fewer registers, so the staging of the
         // next segment fits beside the changeover force kernels, which are
         // held to 7 waves per SIMD)
-        stage_spj<CO ? 2 : 4>(a, w, wk, c, k_begin, k_end);
+        stage_spj<CO ? 2 : 4, WG>(a, w, wk, c, k_begin, k_end);
         return;
     }
     if (tid == 0) a.centre[w] = make_double4(c[0], c[1], c[2], 0.0);
-    for (int k = tid; k < wk.n_i; k += 256) {
+    for (int k = tid; k < wk.n_i; k += WG) {
         const EpiDev e = epi[wk.i_off + k];
         const double rs = (double)e.rs;
         const double dx = e.x - c[0], dy = e.y - c[1], dz = e.z - c[2];
@@ -366,10 +392,10 @@ __global__ __launch_bounds__(256) void k_stage_walk(const StageArgs a)
         }
     };
     const unsigned long long below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-    for (int t0 = 0; t0 < wk.n_e; t0 += 256 * EU) {
+    for (int t0 = 0; t0 < wk.n_e; t0 += WG * EU) {
         Ent q[EU];
 #pragma unroll
-        for (int u = 0; u < EU; u++) q[u] = load(t0 + 256 * u + tid);
+        for (int u = 0; u < EU; u++) q[u] = load(t0 + WG * u + tid);
 #pragma unroll
         for (int u = 0; u < EU; u++) classify(q[u]);
         unsigned long long bn[EU], bf[EU];
@@ -390,7 +416,7 @@ __global__ __launch_bounds__(256) void k_stage_walk(const StageArgs a)
 #pragma unroll
         for (int u = 0; u < EU; u++) {
             int pn = 0, pf = 0, tn = 0, tf = 0;
-            for (int v = 0; v < 4; v++) {
+            for (int v = 0; v < NW; v++) {
                 const int cn = cnt[2 * u][v], cf = cnt[2 * u + 1][v];
                 if (v < wave) {
                     pn += cn;
@@ -412,7 +438,7 @@ __global__ __launch_bounds__(256) void k_stage_walk(const StageArgs a)
     // order from the back
     if (a.mono) {
         const int *__restrict__ mid = a.id_spj + wk.s_off;
-        for (int k = tid; k < wk.n_s; k += 256) {
+        for (int k = tid; k < wk.n_s; k += WG) {
             const EpjDev e = a.spj_mono[mid[k]];
             put_epj(staged_e, base + cap - 1 - (n_far + k), (float)(e.x - c[0]), (float)(e.y - c[1]),
                     (float)(e.z - c[2]), e.m, 0.f);
@@ -421,7 +447,7 @@ __global__ __launch_bounds__(256) void k_stage_walk(const StageArgs a)
     }
     // pad the gap between the two regions (far, massless); the padding of the
     // last near block is read by the double-float near loop: zero low parts
-    for (long long s = base + n_near + tid; s < base + cap - n_far; s += 256) {
+    for (long long s = base + n_near + tid; s < base + cap - n_far; s += WG) {
         put_epj(staged_e, s, 1e18f, 1e18f, 1e18f, 0.f, 0.f);
         if (!CO && a.df) {
             float *blk = a.staged_el + (s >> 3) * PTH_DF_EXTRA;
@@ -433,7 +459,7 @@ __global__ __launch_bounds__(256) void k_stage_walk(const StageArgs a)
     if constexpr (CO) {
         // (the loop above ended with a barrier: co_self is complete)
         int miss = 0;
-        for (int k = tid; k < wk.n_i; k += 256) {
+        for (int k = tid; k < wk.n_i; k += WG) {
             const bool in = k < n_co;
             const int s = in ? co_self[k] : -1;
             a.staged_ic[wk.i_off + k] =
@@ -1555,9 +1581,15 @@ hipError_t launch_stage(const BatchDev &b, int k, hipStream_t st)
     a.n_walk = g.n_walk;
     a.spj_parts = b.mono ? 0 : std::max(1, std::min(8, 2048 / g.n_walk));
     const unsigned nblk = (unsigned)g.n_walk * (1u + (unsigned)a.spj_parts);
-    if (b.co) hipLaunchKernelGGL((k_stage_walk<true, 2>), dim3(nblk), dim3(256), 0, st, a);
-    else if (g.n_walk <= 2048) hipLaunchKernelGGL((k_stage_walk<false, 4>), dim3(nblk), dim3(256), 0, st, a);
-    else hipLaunchKernelGGL((k_stage_walk<false, 2>), dim3(nblk), dim3(256), 0, st, a);
+    // in changeover mode an entry also costs a hash search: 512 threads of 4
+    // entries per walk where a launch has few walks (the 131,071-particle hooks
+    // 2,566 to 2,466 us); without it a walk's gathers keep its CU busy, and
+    // they gain nothing (16,384 particles 43 to 37 us, 40,000 43 to 53)
+    if (b.co && g.n_walk <= 512)
+        hipLaunchKernelGGL((k_stage_walk<true, 4, 512>), dim3(nblk), dim3(512), 0, st, a);
+    else if (b.co) hipLaunchKernelGGL((k_stage_walk<true, 2, 256>), dim3(nblk), dim3(256), 0, st, a);
+    else if (g.n_walk <= 2048) hipLaunchKernelGGL((k_stage_walk<false, 4, 256>), dim3(nblk), dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((k_stage_walk<false, 2, 256>), dim3(nblk), dim3(256), 0, st, a);
     return hipGetLastError();
 }
 
