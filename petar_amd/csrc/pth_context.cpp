@@ -210,6 +210,8 @@ void pth_destroy(pth_ctx *c)
     for (hipEvent_t &x : c->prof_send)
         if (x) (void)hipEventDestroy(x);
     c->d_ids.release();
+    c->h_rid.release();
+    c->h_rpos.release();
     c->d_spj_tab.release();
     if (c->ev_send) (void)hipEventDestroy(c->ev_send);
     if (c->ev_upload) (void)hipEventDestroy(c->ev_upload);
@@ -474,20 +476,22 @@ int pth_dispatch(pth_ctx *c, int tag, int n_walk, const void *const *epi, const 
     if ((c->par.spj_monopole != 0) != c->mono_sent)
         return c->fail(PTH_ERR_STATE, "pth_dispatch: spj_monopole differs from the last pth_send_j");
     HIPCHK(c, hipSetDevice(c->device), "hipSetDevice");
-    // the pinned arena may still feed the previous batch's copy
+    // the pinned arena and runs may still feed the previous batch
     HIPCHK(c, hipEventSynchronize(c->ev_upload), "hipEventSynchronize");
     // the i records lead the arena: packed before its full size is known
     HIPCHK(c, c->h_arena.ensure(Arena::i_part(ni_tot, co)), "pinned arena allocation");
     double t_pack = wall_s();
     const bool encode = c->list_runs != 0;
     const int nj_lim = c->n_epj, ns_lim = c->n_spj;
-    if (encode && (long long)c->h_rid.size() < n_ide + n_ids) {
-        c->h_rid.resize((size_t)(n_ide + n_ids));
-        c->h_rpos.resize((size_t)(n_ide + n_ids));
+    if (encode) {
+        // (16 more: the encoder stores whole vectors)
+        const size_t bytes = sizeof(int) * (size_t)(n_ide + n_ids + 16);
+        HIPCHK(c, c->h_rid.ensure(bytes), "pinned list allocation");
+        HIPCHK(c, c->h_rpos.ensure(bytes), "pinned list allocation");
     }
     c->run_ne.assign(n_walk + 1, 0);
     c->run_ns.assign(n_walk + 1, 0);
-    int *hrid = c->h_rid.data(), *hrpos = c->h_rpos.data();
+    int *hrid = c->h_rid.as<int>(), *hrpos = c->h_rpos.as<int>();
     EpiDev *he = c->h_arena.as<EpiDev>();
     long long *hid = reinterpret_cast<long long *>(c->h_arena.as<char>() + Arena::i_id_offset(ni_tot));
     Plan &P = c->d_plan;
@@ -552,8 +556,7 @@ int pth_dispatch(pth_ctx *c, int tag, int n_walk, const void *const *epi, const 
                       (c->list_runs < 0 && 8 * (n_re + n_rs + n_walk + 1) <= 2 * (n_ide + n_ids));
     c->prof.copy_s += wall_s() - t_pack;
     Arena A;
-    if (runs) A.layout(P, n_ide, n_ids, co, n_re, n_rs);
-    else A.layout(P, n_ide, n_ids, co);
+    A.layout(P, n_ide, n_ids, co, runs);
     HIPCHK(c, c->h_arena.ensure_keep(A.upload, A.walks), "pinned arena allocation");
     const bool grow = A.total > c->d_arena.cap;
     if (grow) HIPCHK(c, hipStreamSynchronize(c->stream), "hipStreamSynchronize");
@@ -606,40 +609,13 @@ int pth_dispatch(pth_ctx *c, int tag, int n_walk, const void *const *epi, const 
     char *h = c->h_arena.as<char>();
     int *hide = reinterpret_cast<int *>(h + A.ide);
     int *hids = reinterpret_cast<int *>(h + A.ids);
-    // runs: first indices of all of the batch's runs, then their positions
-    int *hre = reinterpret_cast<int *>(h + A.run_e);
-    int *hrs = reinterpret_cast<int *>(h + A.run_s);
-    int *hreo = reinterpret_cast<int *>(h + A.run_eo);
-    int *hrso = reinterpret_cast<int *>(h + A.run_so);
     if (runs) {
-        // run offsets: walk w's runs start at the count of the walks before it
-        int oe = 0, os = 0;
-        for (int w = 0; w < n_walk; w++) {
-            const int ne = c->run_ne[w], ns = c->run_ns[w];
-            c->run_ne[w] = oe;
-            c->run_ns[w] = os;
-            oe += ne;
-            os += ns;
-        }
-        c->run_ne[n_walk] = oe;
-        c->run_ns[n_walk] = os;
-        std::memcpy(hreo, c->run_ne.data(), sizeof(int) * (n_walk + 1));
-        std::memcpy(hrso, c->run_ns.data(), sizeof(int) * (n_walk + 1));
-    }
+        std::memcpy(h + A.n_re, c->run_ne.data(), sizeof(int) * (size_t)n_walk);
+        std::memcpy(h + A.n_rs, c->run_ns.data(), sizeof(int) * (size_t)n_walk);
+    } else {
 #pragma omp parallel for schedule(dynamic)
-    for (int w = 0; w < n_walk; w++) {
-        const WalkDev &W = P.walks[w];
-        if (runs) {
-            const int ne = c->run_ne[w + 1] - c->run_ne[w], ns = c->run_ns[w + 1] - c->run_ns[w];
-            if (ne) {
-                std::memcpy(hre + c->run_ne[w], hrid + W.e_off, sizeof(int) * ne);
-                std::memcpy(hre + n_re + c->run_ne[w], hrpos + W.e_off, sizeof(int) * ne);
-            }
-            if (ns) {
-                std::memcpy(hrs + c->run_ns[w], hrid + n_ide + W.s_off, sizeof(int) * ns);
-                std::memcpy(hrs + n_rs + c->run_ns[w], hrpos + n_ide + W.s_off, sizeof(int) * ns);
-            }
-        } else {
+        for (int w = 0; w < n_walk; w++) {
+            const WalkDev &W = P.walks[w];
             if (W.n_e) std::memcpy(hide + W.e_off, id_epj[w], sizeof(int) * W.n_e);
             if (W.n_s) std::memcpy(hids + W.s_off, id_spj[w], sizeof(int) * W.n_s);
         }
@@ -654,7 +630,7 @@ int pth_dispatch(pth_ctx *c, int tag, int n_walk, const void *const *epi, const 
     T.timed = c->prof_on;
     if (T.timed) HIPCHK(c, hipEventRecord(T.prof[0], c->stream), "hipEventRecord");
     HIPCHK(c, hipMemcpyAsync(c->d_arena.p, h, A.upload, hipMemcpyHostToDevice, c->stream), "batch upload");
-    HIPCHK(c, hipEventRecord(c->ev_upload, c->stream), "hipEventRecord");
+    if (!runs) HIPCHK(c, hipEventRecord(c->ev_upload, c->stream), "hipEventRecord");
     if (T.timed) HIPCHK(c, hipEventRecord(T.prof[1], c->stream), "hipEventRecord");
     if (c->par.exec_mode == PTH_EXEC_PLAIN) HIPCHK(c, hipStreamSynchronize(c->stream), "upload sync");
     HIPCHK(c, plan_items(P, A, c->d_arena.as<char>(), c->stream), "planning kernel");
@@ -677,12 +653,11 @@ int pth_dispatch(pth_ctx *c, int tag, int n_walk, const void *const *epi, const 
     if (runs) {
         char *d = c->d_arena.as<char>();
         int *ide_dev = c->d_ids.as<int>();
-        const int *re = reinterpret_cast<const int *>(d + A.run_e);
-        const int *rs = reinterpret_cast<const int *>(d + A.run_s);
-        HIPCHK(c, launch_expand_runs(b.walks, 0, n_walk, re, re + n_re, reinterpret_cast<const int *>(d + A.run_eo),
-                                     rs, rs + n_rs, reinterpret_cast<const int *>(d + A.run_so), ide_dev,
+        HIPCHK(c, launch_expand_runs(b.walks, n_walk, hrid, hrpos, reinterpret_cast<const int *>(d + A.n_re),
+                                     hrid + n_ide, hrpos + n_ide, reinterpret_cast<const int *>(d + A.n_rs), ide_dev,
                                      ide_dev + n_ide, c->stream),
                "list expansion kernel");
+        HIPCHK(c, hipEventRecord(c->ev_upload, c->stream), "hipEventRecord");
         b.id_epj = ide_dev;
         b.id_spj = ide_dev + n_ide;
     }

@@ -207,14 +207,13 @@ hipError_t launch_spj_table(const SpjDev *spj, long long n, float eps2, SpjTab *
 // Floats per staged SPJ record.
 #define PTH_SPJ_STAGED 4
 
-// Expands index lists sent as runs of consecutive indices for walks
-// [w_begin, w_begin + n_walk): for walk w, runs roff[w] .. roff[w + 1] - 1
-// start at position rpos[k] of the walk's list with index rid[k]; the list
-// of walk w (n entries from walks[w].e_off for EPJ, or walks[w].s_off for
-// SPJ) goes to out_e / out_s.
-hipError_t launch_expand_runs(const WalkDev *walks, int w_begin, int n_walk, const int *rid_e, const int *rpos_e,
-                              const int *run_eo, const int *rid_s, const int *rpos_s, const int *run_so, int *out_e,
-                              int *out_s, hipStream_t st);
+// Expands index lists given as runs of consecutive indices: walk w's EPJ list
+// (n_e entries at e_off of out_e) is its n_re[w] runs from rid_e, rpos_e +
+// e_off on, run k starting at position rpos with index rid; its SPJ list
+// likewise.  The runs may lie in pinned host memory.
+hipError_t launch_expand_runs(const WalkDev *walks, int n_walk, const int *rid_e, const int *rpos_e, const int *n_re,
+                              const int *rid_s, const int *rpos_s, const int *n_rs, int *out_e, int *out_s,
+                              hipStream_t st);
 
 // Writes the items and reduction items of a plan made on the device (tiles of
 // at most 128 i).

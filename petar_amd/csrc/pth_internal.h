@@ -113,13 +113,11 @@ struct PinBuf {
 inline size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 
 // Layout of one upload arena (pinned host mirror and device copy).  The
-// index lists travel either as they are (ide, ids) or, with n_run >= 0, as
-// runs of consecutive indices (pth_dispatch): run_e / run_s hold the first
-// index of every run, then every run's position in its walk's list (two
-// int32 per run), run_eo / run_so the walks'
-// run offsets (n_walk + 1 each), and the lists are expanded on the device.
+// index lists travel either as they are (ide, ids) or, with runs
+// (pth_dispatch), as runs of consecutive indices that the device reads where
+// they were encoded: n_re / n_rs then hold the walks' run counts.
 struct Arena {
-    size_t epi, epi_id, walks, es, ss, wplan, splan, ide, ids, items, ritems, run_e, run_s, run_eo, run_so, total;
+    size_t epi, epi_id, walks, es, ss, wplan, splan, ide, ids, items, ritems, n_re, n_rs, total;
     size_t upload;  // what the host fills: all, or all but the items, which then come last
     bool runs = false;
     // the i records (and ids) lead: [0, i_part(ni_tot, co)), i ids at
@@ -129,10 +127,9 @@ struct Arena {
     {
         return align256(i_id_offset(ni_tot) + (co ? sizeof(long long) * (size_t)ni_tot : 0));
     }
-    void layout(const Plan &P, long long n_ide, long long n_ids, bool co, long long n_run_e = -1,
-                long long n_run_s = -1)
+    void layout(const Plan &P, long long n_ide, long long n_ids, bool co, bool as_runs = false)
     {
-        runs = n_run_e >= 0 && n_run_s >= 0;
+        runs = as_runs;
         epi = 0;
         epi_id = i_id_offset(P.ni_tot);
         size_t o = i_part(P.ni_tot, co);
@@ -143,10 +140,8 @@ struct Arena {
         splan = o; o = align256(o + sizeof(SegPlan) * P.splan.size());
         ide = o; o = align256(o + (runs ? 0 : sizeof(int) * (size_t)n_ide));
         ids = o; o = align256(o + (runs ? 0 : sizeof(int) * (size_t)n_ids));
-        run_e = o; o = align256(o + (runs ? 2 * sizeof(int) * (size_t)n_run_e : 0));
-        run_s = o; o = align256(o + (runs ? 2 * sizeof(int) * (size_t)n_run_s : 0));
-        run_eo = o; o = align256(o + (runs ? sizeof(int) * (P.walks.size() + 1) : 0));
-        run_so = o; o = align256(o + (runs ? sizeof(int) * (P.walks.size() + 1) : 0));
+        n_re = o; o = align256(o + (runs ? sizeof(int) * P.walks.size() : 0));
+        n_rs = o; o = align256(o + (runs ? sizeof(int) * P.walks.size() : 0));
         upload = o;
         items = o; o = align256(o + sizeof(Item) * (size_t)P.n_slots);
         ritems = o; o = align256(o + sizeof(RItem) * (size_t)P.n_ritems);
@@ -439,10 +434,10 @@ struct pth_ctx {
     // batch upload
     PinBuf h_arena;
     DevBuf d_arena;
-    // index lists as runs: host encoding space (reused), the walks' run
-    // counts, and the device lists they expand into (shared by all tags, as
-    // the work buffers)
-    std::vector<int> h_rid, h_rpos;
+    // index lists as runs: encoding space (reused; pinned, the device reads the
+    // runs there), the walks' run counts, and the device lists they expand
+    // into (shared by all tags, as the work buffers)
+    PinBuf h_rid, h_rpos;
     std::vector<int> run_ne, run_ns;
     std::vector<long long> w_off;  // pth_dispatch: prefix sums of the walks' i, EPJ, SPJ counts
     std::vector<int> ident;  // 0, 1, 2, ...: the lists of pth_dispatch_copies
@@ -461,7 +456,7 @@ struct pth_ctx {
     bool zero_copy = true;
     hipStream_t side = nullptr;
     hipEvent_t ev_fork = nullptr, ev_join = nullptr;
-    hipEvent_t ev_upload = nullptr;
+    hipEvent_t ev_upload = nullptr;  // the last batch's inputs have been read
     Work work;
     TagState tag[MAX_TAG];
     // profile of the hooks (pth_profile_*)

@@ -1396,56 +1396,45 @@ __global__ __launch_bounds__(256) void k_results(const double4 *__restrict__ acc
 }
 
 // ---------------------------------------------------------------------------
-// index lists sent as runs (pth_dispatch): workgroup g expands part
-// g / (2 n_walk) of n_part of the EPJ list (g % (2 n_walk) < n_walk) or the
-// SPJ list of one walk.  The part's first run is found by a binary search
-// over the walk's run positions; the runs are then taken EXPAND_RUNS at a
-// time into LDS (first index, position); each entry of the part that those
-// runs cover finds its run by a binary search in LDS and is written
-// coalesced.  The first run of a non-empty list has position 0 and
-// positions ascend.
+// Index lists given as runs of consecutive indices (pth_dispatch), read where
+// the host encoded them (pinned memory): workgroup g expands part g / (2
+// n_walk) of n_part of the runs of the EPJ list (g % (2 n_walk) < n_walk) or
+// of the SPJ list of one walk.  A part is a range of runs, so that it reads
+// nothing else over the link; the runs are taken EXPAND_RUNS at a time into
+// LDS (first index, position), each entry they cover finds its run by a binary
+// search in LDS and is written coalesced.  Bound by the link (1.6 MB of runs
+// per 200-walk batch of the 1,048,576-particle cluster; against copying the
+// runs together and uploading them first, that cluster's hooks 20.2 to 19.3
+// ms).
 #define EXPAND_RUNS 1024
-__global__ __launch_bounds__(256) void k_expand_runs(const WalkDev *__restrict__ walks, int w_begin, int n_walk,
-                                                     int n_part, const int *__restrict__ rid_e,
-                                                     const int *__restrict__ rpos_e, const int *__restrict__ run_eo,
-                                                     const int *__restrict__ rid_s, const int *__restrict__ rpos_s,
-                                                     const int *__restrict__ run_so, int *__restrict__ out_e,
-                                                     int *__restrict__ out_s)
+__global__ __launch_bounds__(256) void k_expand_runs(const WalkDev *__restrict__ walks, int n_walk, int n_part,
+                                                     const int *__restrict__ rid_e, const int *__restrict__ rpos_e,
+                                                     const int *__restrict__ n_re, const int *__restrict__ rid_s,
+                                                     const int *__restrict__ rpos_s, const int *__restrict__ n_rs,
+                                                     int *__restrict__ out_e, int *__restrict__ out_s)
 {
-    __shared__ int l_id[EXPAND_RUNS], l_pos[EXPAND_RUNS];
+    __shared__ int l_id[EXPAND_RUNS], l_pos[EXPAND_RUNS + 1];
     const int part = (int)blockIdx.x / (2 * n_walk), g = (int)blockIdx.x % (2 * n_walk);
     const bool sp = g >= n_walk;
-    const int w = w_begin + (sp ? g - n_walk : g);
+    const int w = sp ? g - n_walk : g;
     const WalkDev wk = walks[w];
-    const int n = sp ? wk.n_s : wk.n_e;
-    const int *__restrict__ rid = sp ? rid_s : rid_e;
-    const int *__restrict__ rpos = sp ? rpos_s : rpos_e;
-    const int *__restrict__ ro = sp ? run_so : run_eo;
-    const int r0 = ro[w], r1 = ro[w + 1];
-    // this part's entries [q0, q1)
-    const int q0 = (int)((long long)n * part / n_part), q1 = (int)((long long)n * (part + 1) / n_part);
-    if (q0 >= q1) return;
-    // its first run: the last one whose position is <= q0 (the first run of a
-    // non-empty list has position 0)
-    int f = r0;
-    for (int hi = r1 - 1; f < hi;) {
-        const int mid = (f + hi + 1) >> 1;
-        if (rpos[mid] <= q0) f = mid;
-        else hi = mid - 1;
-    }
-    int *__restrict__ out = sp ? out_s + wk.s_off : out_e + wk.e_off;
+    const int n = sp ? wk.n_s : wk.n_e, off = sp ? wk.s_off : wk.e_off, nr = sp ? n_rs[w] : n_re[w];
+    // a walk's runs lie where its list would
+    const int *__restrict__ rid = (sp ? rid_s : rid_e) + off;
+    const int *__restrict__ rpos = (sp ? rpos_s : rpos_e) + off;
+    int *__restrict__ out = (sp ? out_s : out_e) + off;
+    const int r0 = (int)((long long)nr * part / n_part), r1 = (int)((long long)nr * (part + 1) / n_part);
     const int tid = (int)threadIdx.x;
-    for (int c0 = f; c0 < r1; c0 += EXPAND_RUNS) {
+    for (int c0 = r0; c0 < r1; c0 += EXPAND_RUNS) {
         const int nc = min(EXPAND_RUNS, r1 - c0);
-        for (int k = tid; k < nc; k += 256) {
-            l_id[k] = rid[c0 + k];
-            l_pos[k] = rpos[c0 + k];
+        for (int k = tid; k <= nc; k += 256) {
+            // (entry nc: where the next run begins)
+            if (k < nc) l_id[k] = rid[c0 + k];
+            l_pos[k] = c0 + k < nr ? rpos[c0 + k] : n;
         }
         __syncthreads();
-        // the part's entries these runs cover: up to the next chunk's first run
-        const int next = (c0 + nc < r1) ? rpos[c0 + nc] : n;
-        const int p0 = max(l_pos[0], q0), p1 = min(next, q1);
-        for (int k = p0 + tid; k < p1; k += 256) {
+        const int p1 = l_pos[nc];
+        for (int k = l_pos[0] + tid; k < p1; k += 256) {
             int lo = 0, hi = nc - 1;
             while (lo < hi) {
                 const int mid = (lo + hi + 1) >> 1;
@@ -1455,7 +1444,6 @@ __global__ __launch_bounds__(256) void k_expand_runs(const WalkDev *__restrict__
             out[k] = l_id[lo] + (k - l_pos[lo]);
         }
         __syncthreads();
-        if (next >= q1) break;
     }
 }
 
@@ -1532,15 +1520,15 @@ hipError_t launch_spj_table(const SpjDev *spj, long long n, float eps2, SpjTab *
     return hipGetLastError();
 }
 
-hipError_t launch_expand_runs(const WalkDev *walks, int w_begin, int n_walk, const int *rid_e, const int *rpos_e,
-                              const int *run_eo, const int *rid_s, const int *rpos_s, const int *run_so, int *out_e,
-                              int *out_s, hipStream_t st)
+hipError_t launch_expand_runs(const WalkDev *walks, int n_walk, const int *rid_e, const int *rpos_e, const int *n_re,
+                              const int *rid_s, const int *rpos_s, const int *n_rs, int *out_e, int *out_s,
+                              hipStream_t st)
 {
     if (n_walk <= 0) return hipSuccess;
     // parts per list: a few blocks per CU for a batch of a few hundred walks
     const int n_part = std::max(1, std::min(8, 4096 / (2 * n_walk)));
-    hipLaunchKernelGGL(k_expand_runs, dim3(2u * (unsigned)n_walk * (unsigned)n_part), dim3(256), 0, st, walks,
-                       w_begin, n_walk, n_part, rid_e, rpos_e, run_eo, rid_s, rpos_s, run_so, out_e, out_s);
+    hipLaunchKernelGGL(k_expand_runs, dim3(2u * (unsigned)n_walk * (unsigned)n_part), dim3(256), 0, st, walks, n_walk,
+                       n_part, rid_e, rpos_e, n_re, rid_s, rpos_s, n_rs, out_e, out_s);
     return hipGetLastError();
 }
 
