@@ -1346,10 +1346,60 @@ void unpack_results(const char *src, long long n, bool co, double *acc, double *
     for (int k = 0; k < t; k++) part(n * k / t, n * (k + 1) / t);
 }
 
+// Has the pages of [p, p + bytes) mapped, without changing a byte: the caller's
+// arrays are often fresh memory, whose faults would otherwise come chunk by
+// chunk, several threads waiting for one (2 MB) page at a time.
+static void map_pages(void *p, size_t bytes)
+{
+    if (!p || bytes < (size_t)4 << 20) return;
+    char *b = static_cast<char *>(p);
+    const int t = omp_get_max_threads();
+#pragma omp parallel for num_threads(t) schedule(static, 1)
+    for (int k = 0; k < t; k++)
+        for (size_t q = bytes * k / t; q < bytes * (k + 1) / t; q += 4096)
+            asm volatile("lock orb $0, %0" : "+m"(b[q]));
+}
+
+hipError_t copy_to_host(hipStream_t st, ResultRing &ring, const std::vector<HostCopy> &pieces)
+{
+    constexpr size_t CHUNK = results_bytes(RESULT_CHUNK, false);
+    std::lock_guard<std::mutex> lk(ring.m);
+    std::vector<HostCopy> part;
+    for (const HostCopy &c : pieces)
+        for (size_t o = 0; c.dst && o < c.bytes; o += CHUNK)
+            part.push_back(HostCopy{(char *)c.dst + o, (const char *)c.src + o, std::min(CHUNK, c.bytes - o)});
+    hipError_t e;
+    auto start = [&](size_t k) -> hipError_t {
+        PinBuf &b = ring.buf[k % RESULT_RING];
+        hipEvent_t &x = ring.ev[k % RESULT_RING];
+        hipError_t r;
+        if ((r = b.ensure(part.size() > 1 ? CHUNK : part[k].bytes))) return r;
+        if (!x && (r = hipEventCreateWithFlags(&x, hipEventDisableTiming))) return r;
+        if ((r = hipMemcpyAsync(b.p, part[k].src, part[k].bytes, hipMemcpyDeviceToHost, st))) return r;
+        return hipEventRecord(x, st);
+    };
+    for (size_t k = 0; k < part.size() && k < RESULT_RING; k++)
+        if ((e = start(k))) return e;
+    for (const HostCopy &c : pieces)
+        if (c.dst) map_pages(c.dst, c.bytes);
+    for (size_t k = 0; k < part.size(); k++) {
+        if ((e = hipEventSynchronize(ring.ev[k % RESULT_RING]))) return e;
+        const char *src = ring.buf[k % RESULT_RING].as<char>();
+        const size_t n = part[k].bytes;
+        const int t = (int)std::max<size_t>(1, std::min<size_t>(omp_get_max_threads(), n >> 17));
+#pragma omp parallel for num_threads(t) schedule(static, 1) if (t > 1)
+        for (int q = 0; q < t; q++)
+            std::memcpy((char *)part[k].dst + n * q / t, src + n * q / t, n * (q + 1) / t - n * q / t);
+        if (k + RESULT_RING < part.size() && (e = start(k + RESULT_RING))) return e;
+    }
+    return hipStreamSynchronize(st);
+}
+
 hipError_t results_to_host(hipStream_t st, ResultRing &ring, const double4 *accp, const int *out_nnb,
                            const double *pott, long long n, double *acc, double *pot, long long *nnb, double *pot_tot,
                            const int *err, int n_err, int *bad)
 {
+    std::lock_guard<std::mutex> lk(ring.m);
     hipError_t e;
     const bool co = pott != nullptr;
     const long long n_chunk = (n + RESULT_CHUNK - 1) / RESULT_CHUNK;
@@ -1370,6 +1420,11 @@ hipError_t results_to_host(hipStream_t st, ResultRing &ring, const double4 *accp
     if (err && (e = hipMemcpyAsync(ring.buf[0].p, err, sizeof(int) * (size_t)n_err, hipMemcpyDeviceToHost, st))) return e;
     for (long long k = 0; k < nb; k++)
         if ((e = pack(k))) return e;
+    // (while the evaluation is still running)
+    map_pages(acc, 24 * (size_t)n);
+    map_pages(pot, 8 * (size_t)n);
+    map_pages(nnb, 8 * (size_t)n);
+    if (co) map_pages(pot_tot, 8 * (size_t)n);
     for (long long k = 0; k < n_chunk; k++) {
         if ((e = hipEventSynchronize(ring.ev[k % RESULT_RING]))) return e;
         if (k == 0 && err)

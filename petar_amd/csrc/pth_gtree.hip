@@ -1365,6 +1365,7 @@ struct pth_gtree {
     DevBuf range;            // the nodes' particle ranges, in preorder
     void *pinned = nullptr;  // pinned host copy of meta
     hipEvent_t ev_meta = nullptr;  // that copy
+    mutable ResultRing ring;       // of downloads
     int tile_passes = 0;  // of the last search's tile walk
     // one-pass neighbour filters: regions from the last completed search's
     // per-particle counts (ngb_cnt), valid while ngb_prev_ok
@@ -2051,11 +2052,9 @@ int pth_gtree_neighbors_download(const pth_gtree *t, int *count, long long *offs
     if (!t->built || t->n_ngb < 0)
         return c->fail(PTH_ERR_STATE, "pth_gtree_neighbors_download: no neighbour search since the last build");
     HIPCHK(c, hipSetDevice(c->device), "hipSetDevice");
-    if (count) HIPCHK(c, hipMemcpy(count, t->ngb_cnt.p, sizeof(int) * t->n, hipMemcpyDeviceToHost), "download");
-    if (offset)
-        HIPCHK(c, hipMemcpy(offset, t->ngb_off.p, sizeof(long long) * (t->n + 1), hipMemcpyDeviceToHost), "download");
-    if (ngb && t->n_ngb > 0)
-        HIPCHK(c, hipMemcpy(ngb, t->ngb.p, sizeof(int) * t->n_ngb, hipMemcpyDeviceToHost), "download");
+    HIPCHK(c, copy_to_host(c->stream, t->ring, {{count, t->ngb_cnt.p, sizeof(int) * (size_t)t->n},
+                                                {offset, t->ngb_off.p, sizeof(long long) * (size_t)(t->n + 1)},
+                                                {ngb, t->ngb.p, sizeof(int) * (size_t)t->n_ngb}}), "download");
     if (ms) *ms = t->ms_ngb;
     return PTH_OK;
 }
@@ -2077,6 +2076,7 @@ void pth_gtree_free(pth_gtree *t)
     t->release_scratch();
     if (t->pinned) (void)hipHostFree(t->pinned);
     if (t->ev_meta) (void)hipEventDestroy(t->ev_meta);
+    t->ring.release();
     delete t;
 }
 

@@ -8,6 +8,7 @@
 #include <algorithm>
 #include <cstdlib>
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -203,6 +204,7 @@ struct Work {
 // about 1 ms, 4,194,304 47 to 6 ms, 16,384 80 to 45 us.
 constexpr int RESULT_CHUNK = 65536, RESULT_RING = 3;
 struct ResultRing {
+    std::mutex m;  // one transfer at a time
     PinBuf buf[RESULT_RING];
     hipEvent_t ev[RESULT_RING] = {};
     void release()
@@ -222,6 +224,14 @@ struct ResultRing {
 hipError_t results_to_host(hipStream_t st, ResultRing &ring, const double4 *accp, const int *out_nnb,
                            const double *pott, long long n, double *acc, double *pot, long long *nnb, double *pot_tot,
                            const int *err = nullptr, int n_err = 0, int *bad = nullptr);
+// Copies device arrays to (pageable) host arrays through the ring, after the
+// work on stream st; pieces without bytes or destination are left out.
+struct HostCopy {
+    void *dst;
+    const void *src;
+    size_t bytes;
+};
+hipError_t copy_to_host(hipStream_t st, ResultRing &ring, const std::vector<HostCopy> &pieces);
 // The host side of one chunk of n results packed at src (launch_results).
 void unpack_results(const char *src, long long n, bool co, double *acc, double *pot, long long *nnb, double *pot_tot);
 
