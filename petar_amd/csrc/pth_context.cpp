@@ -1269,6 +1269,7 @@ void pth_resident_free(pth_resident *r)
     r->plan_dev.release();
     r->work.release();
     r->ring.release();
+    r->h_plan.release();
     for (int k = 0; k < 4; k++)
         if (r->ev[k]) (void)hipEventDestroy(r->ev[k]);
     for (hipEvent_t x : r->side_done)

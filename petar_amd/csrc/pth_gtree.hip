@@ -45,6 +45,7 @@
 namespace {
 
 constexpr int GT_MAX_LEVEL = 21;
+constexpr long long WALK_WIDE = 1024;
 constexpr int WALK_STACK = 2048;  // LDS node stack of one walking wave (8 KB: 20 waves per CU;
                                   // 4096 ran the precision workload's walk in 4.1 ms, 2048 and 2560
                                   // in 3.2 ms, 1536 in 4.7 ms, 1024 in 10.3 ms)
@@ -198,24 +199,40 @@ __device__ __forceinline__ int common_levels(unsigned long long a, unsigned long
     return x ? GT_MAX_LEVEL - 1 - (63 - __clzll((long long)x)) / 3 : GT_MAX_LEVEL;
 }
 
-// whether particle k's cell of level l holds more than m particles
-__device__ bool cell_holds(const unsigned long long *__restrict__ key, long long n, long long k, int l, long long m)
+// The sorted keys around a block of 256 particles: those up to KEY_HALO away
+// in LDS, the others in memory.  The decisions below are chains of some 30
+// dependent reads (binary searches), which from memory took 15 us at 16,384
+// particles and 43 us at 1,048,576 (10 and 36 so).
+constexpr int KEY_HALO = 512;
+struct KeyWindow {
+    const unsigned long long *__restrict__ key;
+    const unsigned long long *lds;  // keys [k0, k0 + n_lds)
+    long long k0;
+    int n_lds;
+    __device__ __forceinline__ unsigned long long operator[](long long k) const
+    {
+        const long long j = k - k0;
+        return j >= 0 && j < n_lds ? lds[j] : key[k];
+    }
+};
+
+// How many particles of k's cell of level l lie after k and before k (at most
+// m of each are looked at).
+__device__ void cell_reach(const KeyWindow &key, long long n, long long k, int l, long long m, long long &left,
+                           long long &right)
 {
     const unsigned long long kk = key[k];
-    // the largest r <= m with k + r (then k - r) still in the cell
-    long long right = 0, left = 0;
+    left = right = 0;
     for (long long hi = min(m, n - 1 - k); right < hi;) {
         const long long mid = (right + hi + 1) >> 1;
         if (common_levels(kk, key[k + mid]) >= l) right = mid;
         else hi = mid - 1;
     }
-    if (right >= m) return true;
-    for (long long hi = min(m - right, k); left < hi;) {
+    for (long long hi = min(m, k); left < hi;) {
         const long long mid = (left + hi + 1) >> 1;
         if (common_levels(kk, key[k - mid]) >= l) left = mid;
         else hi = mid - 1;
     }
-    return left + right + 1 > m;
 }
 
 // The nodes starting at one particle: levels d .. e (none when e < d), and
@@ -223,25 +240,37 @@ __device__ bool cell_holds(const unsigned long long *__restrict__ key, long long
 struct Starts {
     int d, e, group, tile;
 };
-__device__ Starts starts_at(const unsigned long long *__restrict__ key, long long n, long long k, long long n_leaf,
-                            long long n_group, long long n_tile)
+__device__ Starts starts_at(const KeyWindow &key, long long n, long long k, long long n_leaf, long long n_group,
+                            long long n_tile)
 {
     const unsigned long long kk = key[k];
     Starts s{k > 0 ? common_levels(key[k - 1], kk) + 1 : 0, -1, -1, -1};
     if (s.d > GT_MAX_LEVEL) return s;
     auto shared = [&](long long m) { return k + m < n ? common_levels(kk, key[k + m]) : -1; };
     const int c = shared(n_leaf);
+    long long left, right;
     if (c >= s.d || k == 0) s.e = min(GT_MAX_LEVEL, c + 1);
-    else if (cell_holds(key, n, k, s.d - 1, n_leaf)) s.e = s.d;
-    else return s;
+    else {
+        // (c == d - 1: the parent reaches n_leaf particles past k)
+        bool big = c == s.d - 1;
+        if (!big) {
+            cell_reach(key, n, k, s.d - 1, n_leaf, left, right);
+            big = left + right + 1 > n_leaf;
+        }
+        if (!big) return s;
+        s.e = s.d;
+    }
     // the largest cell of at most m particles, or the leaf: the first such
     // level on the way down, unless it is d and its parent is one already
-    auto largest = [&](long long m) {
-        const int q = min(max(s.d, shared(m) + 1), s.e);
-        return (q > s.d || q == 0 || cell_holds(key, n, k, s.d - 1, m)) ? q : -1;
-    };
-    s.group = largest(n_group);
-    s.tile = largest(n_tile);
+    auto level = [&](long long m) { return min(max(s.d, shared(m) + 1), s.e); };
+    s.group = level(n_group);
+    s.tile = level(n_tile);
+    const bool ask_g = s.group == s.d && s.d > 0, ask_t = s.tile == s.d && s.d > 0;
+    if (ask_g || ask_t) {
+        cell_reach(key, n, k, s.d - 1, max(ask_g ? n_group : 0, ask_t ? n_tile : 0), left, right);
+        if (ask_g && left + right + 1 <= n_group) s.group = -1;
+        if (ask_t && left + right + 1 <= n_tile) s.tile = -1;
+    }
     return s;
 }
 
@@ -256,11 +285,15 @@ __global__ __launch_bounds__(256) void k_starts(const unsigned long long *__rest
                                                 unsigned *__restrict__ st)
 {
     __shared__ int w[N_ROWS][4];
-    const long long k = (long long)blockIdx.x * 256 + threadIdx.x;
+    __shared__ unsigned long long near[256 + 2 * KEY_HALO];
+    const long long b0 = (long long)blockIdx.x * 256, k = b0 + threadIdx.x;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const long long w0 = max(b0 - KEY_HALO, 0LL), w1 = min(b0 + 256 + KEY_HALO, n);
+    for (int j = threadIdx.x; j < (int)(w1 - w0); j += 256) near[j] = key[w0 + j];
+    __syncthreads();
     Starts s{0, -1, -1, -1};
     if (k < n) {
-        s = starts_at(key, n, k, n_leaf, n_group, n_tile);
+        s = starts_at(KeyWindow{key, near, w0, (int)(w1 - w0)}, n, k, n_leaf, n_group, n_tile);
         st[k] = (unsigned)(s.d | (s.e + 1) << 8 | (s.group + 1) << 16 | (s.tile + 1) << 24);
     }
     const int n_lev = max(s.e - s.d + 1, 0);
@@ -388,7 +421,7 @@ __global__ __launch_bounds__(256) void k_node_ends(GNode *__restrict__ nodes, lo
 
 // A node's moments and boxes.
 struct Moments {
-    double M, c[3], q[6], bi[6], bo[6];
+    double M, c[3], bi[6], bo[6];
 };
 __device__ __forceinline__ void moments_init(Moments &v)
 {
@@ -398,7 +431,6 @@ __device__ __forceinline__ void moments_init(Moments &v)
         v.bi[d] = v.bo[d] = 1e300;
         v.bi[3 + d] = v.bo[3 + d] = -1e300;
     }
-    for (int d = 0; d < 6; d++) v.q[d] = 0;
 }
 __device__ __forceinline__ void moments_centre(Moments &v)
 {
@@ -436,134 +468,236 @@ struct MomentArrays {
     const int *pre;
 };
 
-__device__ void walk_rec_store(const WalkRec &w, const TreeMeta *__restrict__ meta, const GNode &nd,
-                               const Moments &v, int pre, long long k)
+// Moments are made by eight lanes per node, which load its children (or eight
+// of its particles at a time) side by side, pass them through LDS and each add
+// up one component: the host's sums in its order.  A level waits for the one
+// below it, so the chain of loads inside a node is what counts: with a thread
+// per node, going through its children or particles one after the other, the
+// leaves took 17 us and the inner levels 73 at 16,384 particles, 7 and 28 us so
+// (1,048,576: the inner levels 100 us, 48 so).
+constexpr int KID = 11;  // doubles per lane in LDS (odd, so that lanes' rows start on different banks)
+
+__device__ __forceinline__ void wave_sync()
 {
-    float p[3], ol[3], oh[3], il[3], ih[3];
-    const float m = walk_margin(meta->len, meta->rs_max);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+template <int CTRL> __device__ __forceinline__ double lane_swap(double v)
+{
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, false);
+    return __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double min8(double v)
+{
+    v = fmin(v, lane_swap<0xB1>(v));  // quad_perm [1,0,3,2]
+    v = fmin(v, lane_swap<0x4E>(v));  // quad_perm [2,3,0,1]
+    return fmin(v, lane_swap<0x141>(v));  // row_half_mirror
+}
+__device__ __forceinline__ double max8(double v)
+{
+    v = fmax(v, lane_swap<0xB1>(v));
+    v = fmax(v, lane_swap<0x4E>(v));
+    return fmax(v, lane_swap<0x141>(v));
+}
+// (by value: a choice among array elements would put the array into scratch)
+__device__ __forceinline__ double pick(int j, double a, double b, double c, double d = 0, double e = 0, double f = 0)
+{
+    const double lo = j == 0 ? a : j == 1 ? b : c, hi = j == 3 ? d : j == 4 ? e : f;
+    return j < 3 ? lo : hi;
+}
+
+// The eight lanes' boxes and sums (lane d < 3: m x_d, lane 3: m) joined: every
+// lane gets the mass, the boxes and the centre of mass.
+__device__ __forceinline__ void moments_join(Moments &v, double s, double *rows, int j)
+{
+#pragma unroll
     for (int d = 0; d < 3; d++) {
-        const double c = meta->root[d] + 0.5 * meta->len;
+        v.bi[d] = min8(v.bi[d]);
+        v.bi[3 + d] = max8(v.bi[3 + d]);
+        v.bo[d] = min8(v.bo[d]);
+        v.bo[3 + d] = max8(v.bo[3 + d]);
+    }
+    rows[j * KID + 5] = s;
+    wave_sync();
+    for (int d = 0; d < 3; d++) v.c[d] = rows[d * KID + 5];
+    v.M = rows[3 * KID + 5];
+    moments_centre(v);
+    wave_sync();
+}
+
+// Stores of node k's moments, lane j < 6 holding component j of the
+// quadrupole in q, and its walk record, a part per lane.
+__device__ __forceinline__ void moments_store(const Moments &v, double q, const MomentArrays &o, const GNode &nd,
+                                              long long k, int j)
+{
+    if (j == 7) o.mass[k] = v.M;
+    if (j < 3) o.com[3 * k + j] = pick(j, v.c[0], v.c[1], v.c[2]);
+    if (j < 6) {
+        o.quad[6 * k + j] = q;
+        o.box_in[6 * k + j] = pick(j, v.bi[0], v.bi[1], v.bi[2], v.bi[3], v.bi[4], v.bi[5]);
+        o.box_out[6 * k + j] = pick(j, v.bo[0], v.bo[1], v.bo[2], v.bo[3], v.bo[4], v.bo[5]);
+    }
+    const double len = o.meta->len;
+    const float m = walk_margin(len, o.meta->rs_max);
+    float p[3], ol[3], oh[3], il[3], ih[3];
+    for (int d = 0; d < 3; d++) {
+        const double c = o.meta->root[d] + 0.5 * len;
         p[d] = (float)(v.c[d] - c);
         ol[d] = (float)(fmin(v.bo[d], v.bi[d]) - c) - m;
         oh[d] = (float)(fmax(v.bo[3 + d], v.bi[3 + d]) - c) + m;
         il[d] = (float)(v.bi[d] - c) - m;
         ih[d] = (float)(v.bi[3 + d] - c) + m;
     }
-    w.A[k] = make_float4(p[0], p[1], p[2], __int_as_float((int)nd.begin));
-    w.B[k] = make_float4(ol[0], ol[1], ol[2], __int_as_float((int)nd.end));
-    w.C[k] = make_float4(oh[0], oh[1], oh[2], __int_as_float(nd.level << 8 | nd.n_child));
-    w.D[k] = make_float4(il[0], il[1], il[2], 0.f);
-    w.E[k] = make_float4(ih[0], ih[1], ih[2], 0.f);
-    w.F[k] = make_int2((int)nd.first_child, pre);
+    const WalkRec &w = o.rec;
+    if (j == 0) w.A[k] = make_float4(p[0], p[1], p[2], __int_as_float((int)nd.begin));
+    if (j == 1) w.B[k] = make_float4(ol[0], ol[1], ol[2], __int_as_float((int)nd.end));
+    if (j == 2) w.C[k] = make_float4(oh[0], oh[1], oh[2], __int_as_float(nd.level << 8 | nd.n_child));
+    if (j == 3) w.D[k] = make_float4(il[0], il[1], il[2], 0.f);
+    if (j == 4) w.E[k] = make_float4(ih[0], ih[1], ih[2], 0.f);
+    if (j == 5) w.F[k] = make_int2((int)nd.first_child, o.pre[k]);
 }
 
-__device__ __forceinline__ void moments_store(const Moments &v, const MomentArrays &o, const GNode &nd, long long k)
-{
-    o.mass[k] = v.M;
-    for (int d = 0; d < 3; d++) o.com[3 * k + d] = v.c[d];
-    for (int d = 0; d < 6; d++) {
-        o.quad[6 * k + d] = v.q[d];
-        o.box_in[6 * k + d] = v.bi[d];
-        o.box_out[6 * k + d] = v.bo[d];
-    }
-    walk_rec_store(o.rec, o.meta, nd, v, o.pre[k], k);
-}
-
-// Moments of the leaves, one thread each, the host's sums in its order; the
-// particles are loaded four at a time, so that a leaf of 20 waits for memory
-// ten times and not forty.
+// Moments of the leaves.  A lane holds four particles, so that a leaf of at
+// most 32 is read once.
 __global__ __launch_bounds__(256) void k_leaf_moments(const GNode *__restrict__ nodes, long long nn,
                                                       const double *__restrict__ pos, const double *__restrict__ mass,
                                                       const double *__restrict__ rs, const MomentArrays out)
 {
-    const long long k = (long long)blockIdx.x * 256 + threadIdx.x;
+    constexpr int U = 4;
+    __shared__ double lds[256 * KID];
+    const long long k = (long long)blockIdx.x * 32 + (threadIdx.x >> 3);
+    const int j = threadIdx.x & 7;
     if (k >= nn) return;
     const GNode nd = nodes[k];
     if (nd.n_child != 0) return;
+    double *rows = lds + (threadIdx.x & ~7) * KID, *row = rows + j * KID;
     Moments v;
     moments_init(v);
-    for (long long i0 = nd.begin; i0 < nd.end; i0 += 4) {
-        double x[4][3], m[4], r[4];
+    double x[U][3], m[U], s = 0, q = 0;
+    const int col = min(j, 3);
+    const bool once = nd.end - nd.begin <= 8 * U;
+    for (long long i0 = nd.begin; i0 < nd.end; i0 += 8 * U) {
+        double r[U];
 #pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const long long i = min(i0 + u, nd.end - 1);
+        for (int u = 0; u < U; u++) {
+            const long long i = min(i0 + 8 * u + j, nd.end - 1);
             for (int d = 0; d < 3; d++) x[u][d] = pos[3 * i + d];
             m[u] = mass[i];
             r[u] = rs[i];
         }
 #pragma unroll
-        for (int u = 0; u < 4; u++) {
-            if (i0 + u >= nd.end) break;
-            v.M += m[u];
-            for (int d = 0; d < 3; d++) {
-                v.c[d] += m[u] * x[u][d];
+        for (int u = 0; u < U; u++) {
+            const int n = (int)min(nd.end - i0 - 8 * u, 8LL);
+            if (n <= 0) break;
+            for (int d = 0; d < 3; d++) {  // (a lane past the end holds the last particle once more)
                 v.bi[d] = fmin(v.bi[d], x[u][d]);
                 v.bi[3 + d] = fmax(v.bi[3 + d], x[u][d]);
                 v.bo[d] = fmin(v.bo[d], x[u][d] - r[u]);
                 v.bo[3 + d] = fmax(v.bo[3 + d], x[u][d] + r[u]);
+                row[d] = x[u][d];
+            }
+            row[3] = 1.0;
+            row[4] = m[u];
+            wave_sync();
+            for (int t = 0; t < n; t++) s += rows[t * KID + 4] * rows[t * KID + col];
+            wave_sync();
+        }
+    }
+    moments_join(v, s, rows, j);
+    // components xx, yy, zz, xy, xz, yz
+    const int a = (0x100210 >> (4 * j)) & 3, b = (0x221210 >> (4 * j)) & 3;
+    for (long long i0 = nd.begin; i0 < nd.end; i0 += 8 * U) {
+        if (!once) {
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const long long i = min(i0 + 8 * u + j, nd.end - 1);
+                for (int d = 0; d < 3; d++) x[u][d] = pos[3 * i + d];
+                m[u] = mass[i];
             }
         }
-    }
-    moments_centre(v);
-    for (long long i0 = nd.begin; i0 < nd.end; i0 += 4) {
-        double p[4][3], m4[4];
 #pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const long long i = min(i0 + u, nd.end - 1);
-            for (int d = 0; d < 3; d++) p[u][d] = pos[3 * i + d];
-            m4[u] = mass[i];
-        }
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-            if (i0 + u >= nd.end) break;
-            const double x = p[u][0] - v.c[0], y = p[u][1] - v.c[1], z = p[u][2] - v.c[2], m = m4[u];
-            v.q[0] += m * x * x;
-            v.q[1] += m * y * y;
-            v.q[2] += m * z * z;
-            v.q[3] += m * x * y;
-            v.q[4] += m * x * z;
-            v.q[5] += m * y * z;
+        for (int u = 0; u < U; u++) {
+            const int n = (int)min(nd.end - i0 - 8 * u, 8LL);
+            if (n <= 0) break;
+            for (int d = 0; d < 3; d++) row[d] = x[u][d] - v.c[d];
+            row[4] = m[u];
+            wave_sync();
+            for (int t = 0; t < n; t++) q += rows[t * KID + 4] * rows[t * KID + a] * rows[t * KID + b];
+            wave_sync();
         }
     }
-    moments_store(v, out, nd, k);
+    moments_store(v, q, out, nd, k, j);
 }
 
-// Moments of the inner nodes of [a, b), one level (its children are done).
-__global__ __launch_bounds__(64) void k_inner_moments(const GNode *__restrict__ nodes, long long a, long long b,
-                                                      const MomentArrays o)
+// Moments of one inner node (its children are done), eight lanes.
+__device__ __forceinline__ void inner_moments(const GNode &nd, long long k, const MomentArrays &o, double *rows, int j)
 {
-    const long long k = a + (long long)blockIdx.x * 64 + threadIdx.x;
+    double *row = rows + j * KID;
+    const long long c = nd.first_child + min(j, nd.n_child - 1);
+    Moments v;
+    double m = o.mass[c], x[3], qc[6], s = 0, q = 0;
+    for (int d = 0; d < 3; d++) x[d] = o.com[3 * c + d];
+    for (int d = 0; d < 6; d++) {
+        v.bi[d] = o.box_in[6 * c + d];
+        v.bo[d] = o.box_out[6 * c + d];
+        qc[d] = o.quad[6 * c + d];
+    }
+    for (int d = 0; d < 3; d++) {
+        v.bi[d] = fmin(1e300, v.bi[d]);
+        v.bo[d] = fmin(1e300, v.bo[d]);
+        v.bi[3 + d] = fmax(-1e300, v.bi[3 + d]);
+        v.bo[3 + d] = fmax(-1e300, v.bo[3 + d]);
+        row[d] = x[d];
+    }
+    row[3] = 1.0;
+    row[4] = m;
+    wave_sync();
+    const int col = min(j, 3);
+    for (int t = 0; t < nd.n_child; t++) s += rows[t * KID + 4] * rows[t * KID + col];
+    wave_sync();
+    moments_join(v, s, rows, j);
+    for (int d = 0; d < 3; d++) x[d] -= v.c[d];
+    row[5] = qc[0] + m * x[0] * x[0];
+    row[6] = qc[1] + m * x[1] * x[1];
+    row[7] = qc[2] + m * x[2] * x[2];
+    row[8] = qc[3] + m * x[0] * x[1];
+    row[9] = qc[4] + m * x[0] * x[2];
+    row[10] = qc[5] + m * x[1] * x[2];
+    wave_sync();
+    for (int t = 0; t < nd.n_child; t++) q += rows[t * KID + 5 + min(j, 5)];
+    wave_sync();
+    moments_store(v, q, o, nd, k, j);
+}
+
+// The inner nodes of one level, [a, b).
+__global__ __launch_bounds__(256) void k_inner_moments(const GNode *__restrict__ nodes, long long a, long long b,
+                                                       const MomentArrays o)
+{
+    __shared__ double lds[256 * KID];
+    const long long k = a + (long long)blockIdx.x * 32 + (threadIdx.x >> 3);
     if (k >= b) return;
     const GNode nd = nodes[k];
-    if (nd.n_child == 0) return;
-    Moments v;
-    moments_init(v);
-    for (int ch = 0; ch < nd.n_child; ch++) {
-        const long long cc = nd.first_child + ch;
-        const double m = o.mass[cc];
-        v.M += m;
-        for (int d = 0; d < 3; d++) {
-            v.c[d] += m * o.com[3 * cc + d];
-            v.bi[d] = fmin(v.bi[d], o.box_in[6 * cc + d]);
-            v.bi[3 + d] = fmax(v.bi[3 + d], o.box_in[6 * cc + 3 + d]);
-            v.bo[d] = fmin(v.bo[d], o.box_out[6 * cc + d]);
-            v.bo[3 + d] = fmax(v.bo[3 + d], o.box_out[6 * cc + 3 + d]);
+    if (nd.n_child > 0) inner_moments(nd, k, o, lds + (threadIdx.x & ~7) * KID, threadIdx.x & 7);
+}
+
+// The inner nodes of the levels top .. 0, a level after the other, by one
+// workgroup: its waves share a CU, so that a barrier lets them see the level
+// before.
+constexpr int TOP_THREADS = 1024;
+constexpr int TOP_NODES = 256;  // per level, at most
+__global__ __launch_bounds__(TOP_THREADS) void k_top_moments(const GNode *__restrict__ nodes, int top, const MomentArrays o)
+{
+    __shared__ double lds[TOP_THREADS * KID];
+    for (int l = top; l >= 0; l--) {
+        const int a = o.meta->level_start[l], b = o.meta->level_start[l + 1];
+        for (int k = a + (int)(threadIdx.x >> 3); k < b; k += TOP_THREADS / 8) {
+            const GNode nd = nodes[k];
+            if (nd.n_child > 0) inner_moments(nd, k, o, lds + (threadIdx.x & ~7) * KID, threadIdx.x & 7);
         }
+        __threadfence_block();
+        __syncthreads();
     }
-    moments_centre(v);
-    for (int ch = 0; ch < nd.n_child; ch++) {
-        const long long cc = nd.first_child + ch;
-        const double m = o.mass[cc];
-        const double x = o.com[3 * cc] - v.c[0], y = o.com[3 * cc + 1] - v.c[1], z = o.com[3 * cc + 2] - v.c[2];
-        const double *qc = o.quad + 6 * cc;
-        v.q[0] += qc[0] + m * x * x;
-        v.q[1] += qc[1] + m * y * y;
-        v.q[2] += qc[2] + m * z * z;
-        v.q[3] += qc[3] + m * x * y;
-        v.q[4] += qc[4] + m * x * z;
-        v.q[5] += qc[5] + m * y * z;
-    }
-    moments_store(v, o, nd, k);
 }
 
 __global__ __launch_bounds__(64) void k_fill_int(int *__restrict__ p, long long n, int v)
@@ -573,13 +707,14 @@ __global__ __launch_bounds__(64) void k_fill_int(int *__restrict__ p, long long 
 
 // Exclusive sums of up to three count arrays (block b takes in[b]), n + 1
 // entries each; with pad > 0 every count counts as c + c/4 + pad (a region
-// for the next build's list).
+// for the next build's list).  *zero, if given, is set to 0.
 struct Sums {
     const int *in[3];
     long long *out[3];
 };
-__global__ __launch_bounds__(1024) void k_sums(long long n, const Sums s, int pad)
+__global__ __launch_bounds__(1024) void k_sums(long long n, const Sums s, int pad, int *__restrict__ zero)
 {
+    if (zero && blockIdx.x == 0 && threadIdx.x == 0) *zero = 0;
     constexpr int U = 4;
     __shared__ long long ws[16];
     const int *__restrict__ in = s.in[blockIdx.x];
@@ -735,22 +870,24 @@ __device__ __forceinline__ bool meet(const float (&lo)[3], const float (&hi)[3],
     return !(lo[0] > h.x || l.x > hi[0] || lo[1] > h.y || l.y > hi[1] || lo[2] > h.z || l.z > hi[2]);
 }
 
-// One 64-thread workgroup (one wave) per group at a time.  The opening test
+// One workgroup of NW waves per group at a time.  The opening test
 // is decided in FP32 where its bounds, widened by the margin, leave no doubt,
 // and otherwise (a node at the edge of the theta sphere, or whose widened box
 // meets the group's) by the host's FP64 expressions; a tile walk takes every
 // node whose FP32 boxes meet (a superset: its lists are filtered exactly).
-template <bool WRITE, bool TILE>
-__global__ __launch_bounds__(64) void k_walk(const WalkArgs a)
+template <bool WRITE, bool TILE, int NW>
+__global__ __launch_bounds__(64 * NW) void k_walk(const WalkArgs a)
 {
     __shared__ int stk[WALK_STACK];
     __shared__ float lim[GT_MAX_LEVEL + 1];  // (L / theta)^2 of each level
-    const int lane = threadIdx.x;
+    __shared__ int3 wave_n[NW];              // children, leaves and closed nodes of each wave
+    __shared__ int wave_e[NW];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, thread = threadIdx.x;
     const double len = a.meta->len;
     const float mg = walk_margin(len, a.meta->rs_max);
-    if (lane <= GT_MAX_LEVEL) {
-        const double L = len / (double)(1LL << lane);
-        lim[lane] = (float)(L * L * a.inv_theta2);
+    if (thread <= GT_MAX_LEVEL) {
+        const double L = len / (double)(1LL << thread);
+        lim[thread] = (float)(L * L * a.inv_theta2);
     }
     const unsigned long long below = lane ? ~0ull >> (64 - lane) : 0ull;
     for (long long g = blockIdx.x; g < a.n_group; g += gridDim.x) {
@@ -781,7 +918,7 @@ __global__ __launch_bounds__(64) void k_walk(const WalkArgs a)
             }
         }
         __syncthreads();
-        if (lane == 0) stk[0] = 0;
+        if (thread == 0) stk[0] = 0;
         int size = 1;
         __syncthreads();
         while (size > 0) {
@@ -790,11 +927,11 @@ __global__ __launch_bounds__(64) void k_walk(const WalkArgs a)
             // a time and a descent adds at most 7 entries per level (21
             // levels, 147 < 160), so the stack never overflows
             int k = (WALK_STACK - 160 - size) / 8;
-            k = max(1, min(64, min(k, size)));
-            const bool act = lane < k;
+            k = max(1, min(64 * NW, min(k, size)));
+            const bool act = thread < k;
             int c = 0;
-            if (act) c = stk[size - 1 - lane];
-            __syncthreads();
+            if (act) c = stk[size - 1 - thread];
+            if (NW == 1) __syncthreads();
             bool open = false;
             int begin = 0, end = 0, kids = 0;
             int2 F = make_int2(-1, 0);
@@ -847,20 +984,38 @@ __global__ __launch_bounds__(64) void k_walk(const WalkArgs a)
                 tc += __popcll(m) << b;
             }
             if (leaf) my_e += end - begin;
+            int3 tot = make_int3(tc, __popcll(ml), __popcll(ms)), off = make_int3(0, 0, 0);
+            if (NW > 1) {
+                if (lane == 0) wave_n[wave] = tot;
+                __syncthreads();
+                tot = make_int3(0, 0, 0);
+#pragma unroll
+                for (int w = 0; w < NW; w++) {
+                    const int3 n = wave_n[w];
+                    if (w == wave) off = tot;
+                    tot = make_int3(tot.x + n.x, tot.y + n.y, tot.z + n.z);
+                }
+            }
             if (WRITE) {
-                const int pl = nl + __popcll(ml & below), ps = ns + __popcll(ms & below);
+                const int pl = nl + off.y + __popcll(ml & below), ps = ns + off.z + __popcll(ms & below);
                 if (leaf && pl < cap_l) ol_raw[pl] = F.y;
                 if (!TILE && closed && ps < cap_s) os_raw[ps] = F.y;
             }
-            nl += __popcll(ml);
-            ns += __popcll(ms);
+            nl += tot.y;
+            ns += tot.z;
             size -= k;
-            for (int t = 0; t < mc; t++) stk[size + pc + t] = F.x + (mc - 1 - t);
-            size += tc;
+            for (int t = 0; t < mc; t++) stk[size + off.x + pc + t] = F.x + (mc - 1 - t);
+            size += tot.x;
             __syncthreads();
         }
         for (int off = 32; off > 0; off >>= 1) my_e += __shfl_xor(my_e, off, 64);
-        if (lane == 0) {
+        if (NW > 1) {
+            if (lane == 0) wave_e[wave] = my_e;
+            __syncthreads();
+            my_e = 0;
+            for (int w = 0; w < NW; w++) my_e += wave_e[w];
+        }
+        if (thread == 0) {
             a.cnt_e[g] = my_e;
             a.cnt_l[g] = nl;
             if (!TILE) a.cnt_s[g] = ns;
@@ -1436,6 +1591,17 @@ WalkArgs walk_args(pth_gtree *t)
     return wa;
 }
 
+// The walk of wa's groups: while there are few of them, four waves each (16,384
+// particles, 219 groups: 45 us with one wave, whose serial chain of pops
+// leaves the chip idle, 29 with four, 29 with eight).
+template <bool WRITE, bool TILE> void launch_walk(const WalkArgs &wa, hipStream_t st)
+{
+    const unsigned wg = (unsigned)std::min<long long>(wa.n_group, 65536);
+    if (wa.n_group <= WALK_WIDE)
+        hipLaunchKernelGGL((k_walk<WRITE, TILE, 4>), dim3(wg), dim3(256), 0, st, wa);
+    else hipLaunchKernelGGL((k_walk<WRITE, TILE, 1>), dim3(wg), dim3(64), 0, st, wa);
+}
+
 // Walks the groups of wa into W's raw lists and reads the counts back: one
 // writing pass into regions of the last walk's lengths when that was a walk
 // of as many groups (and again_ok says its counts still stand), else a
@@ -1458,8 +1624,6 @@ template <bool TILE> int walk_run(pth_gtree *t, WalkArgs &wa, WalkLists &W, bool
     wa.over = wa.cnt_l + nc;
     long long *off_e = W.off.as<long long>(), *off_s = off_e + nc, *off_l = off_s + nc;
     long long *reg_l = W.reg.as<long long>(), *reg_s = reg_l + nc;
-    const unsigned wg = (unsigned)std::min<long long>(ng, 65536);
-    hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, st, wa.over, 1, 0);
     if (again) {
         // (a tile has a dozen leaves: 64 spare ones each would be mostly holes)
         const int pad = TILE ? 8 : 64;
@@ -1468,17 +1632,17 @@ template <bool TILE> int walk_run(pth_gtree *t, WalkArgs &wa, WalkLists &W, bool
         if ((e = W.raw_l.ensure(room(W.tot_l))) || (!TILE && (e = W.raw_s.ensure(room(W.tot_s)))))
             return ctx->hip_fail(e, "raw list allocation");
         const Sums s{{wa.cnt_l, wa.cnt_s, nullptr}, {reg_l, reg_s, nullptr}};
-        hipLaunchKernelGGL(k_sums, dim3(TILE ? 1 : 2), dim3(1024), 0, st, ng, s, pad);
+        hipLaunchKernelGGL(k_sums, dim3(TILE ? 1 : 2), dim3(1024), 0, st, ng, s, pad, wa.over);
         wa.off_l = reg_l;
         wa.off_s = reg_s;
         wa.raw_l = W.raw_l.as<int>();
         wa.raw_s = W.raw_s.as<int>();
-        hipLaunchKernelGGL((k_walk<true, TILE>), dim3(wg), dim3(64), 0, st, wa);
+        launch_walk<true, TILE>(wa, st);
     } else if (ng > 0) {
-        hipLaunchKernelGGL((k_walk<false, TILE>), dim3(wg), dim3(64), 0, st, wa);
+        launch_walk<false, TILE>(wa, st);
     }
     const Sums s{{wa.cnt_e, wa.cnt_l, wa.cnt_s}, {off_e, off_l, off_s}};
-    hipLaunchKernelGGL(k_sums, dim3(TILE ? 2 : 3), dim3(1024), 0, st, ng, s, 0);
+    hipLaunchKernelGGL(k_sums, dim3(TILE ? 2 : 3), dim3(1024), 0, st, ng, s, 0, again ? nullptr : wa.over);
     hipLaunchKernelGGL(k_group_info, dim3(std::max(1u, blocks(ng))), dim3(256), 0, st, t->nodes.as<GNode>(), wa.groups,
                        ng, wa.cnt_e, TILE ? nullptr : wa.cnt_s, off_e, TILE ? nullptr : off_s, off_l, wa.over,
                        W.back.as<WalkTotals>(), reinterpret_cast<int4 *>(W.back.as<WalkTotals>() + 1));
@@ -1513,7 +1677,7 @@ template <bool TILE> int walk_finish(pth_gtree *t, WalkArgs &wa, WalkLists &W, b
         wa.off_s = off_s;
         wa.raw_l = W.raw_l.as<int>();
         wa.raw_s = W.raw_s.as<int>();
-        hipLaunchKernelGGL((k_walk<true, TILE>), dim3((unsigned)std::min<long long>(ng, 65536)), dim3(64), 0, st, wa);
+        launch_walk<true, TILE>(wa, st);
     }
     if ((e = W.sort_l.ensure(W.raw_l.cap))) return ctx->hip_fail(e, "leaf list allocation");
     OrderArgs o{};
@@ -1656,13 +1820,20 @@ int gtree_run(pth_gtree *t, long long n, const double *pos, const double *mass, 
     if ((e = t->rec.ensure((5 * sizeof(float4) + sizeof(int2)) * (size_t)nn))) return ctx->hip_fail(e, "node records");
     const MomentArrays mo{t->nmass.as<double>(), t->ncom.as<double>(), t->nquad.as<double>(), t->box_in.as<double>(),
                           t->box_out.as<double>(), t->walk_rec(), meta, t->pre.as<int>()};
-    hipLaunchKernelGGL(k_leaf_moments, dim3(blocks(nn)), dim3(256), 0, st, t->nodes.as<GNode>(), nn,
+    hipLaunchKernelGGL(k_leaf_moments, dim3((unsigned)((nn + 31) / 32)), dim3(256), 0, st, t->nodes.as<GNode>(), nn,
                        t->spos.as<double>(), t->smass.as<double>(), t->srs.as<double>(), mo);
     for (int l = GT_MAX_LEVEL; l >= 0; l--) {
         // (the deepest level holds leaves only)
         const long long a = M.level_start[l], b = M.level_start[l + 1];
         if (b <= a || b == nn) continue;
-        hipLaunchKernelGGL(k_inner_moments, dim3((unsigned)((b - a + 63) / 64)), dim3(64), 0, st,
+        // small levels, from here to the root, go together
+        bool small = true;
+        for (int q = 0; q <= l; q++) small = small && M.level_start[q + 1] - M.level_start[q] <= TOP_NODES;
+        if (small) {
+            hipLaunchKernelGGL(k_top_moments, dim3(1), dim3(TOP_THREADS), 0, st, t->nodes.as<GNode>(), l, mo);
+            break;
+        }
+        hipLaunchKernelGGL(k_inner_moments, dim3((unsigned)((b - a + 31) / 32)), dim3(256), 0, st,
                            t->nodes.as<GNode>(), a, b, mo);
     }
     const long long ng = t->n_group;
@@ -1758,17 +1929,17 @@ int resident_fill_gtree(pth_resident *r, const pth_gtree *t, const char *who)
     hipStream_t st = c->stream;
     hipError_t e;
     char *d = r->arena.as<char>();
-    // plan tables from the host, lists and records on the device
-    auto h2d = [&](size_t off, const void *h, size_t bytes) -> hipError_t {
-        return bytes ? hipMemcpyAsync(d + off, h, bytes, hipMemcpyHostToDevice, st) : hipSuccess;
-    };
-    if ((e = h2d(A.walks, P.walks.data(), sizeof(WalkDev) * P.walks.size())) ||
-        (e = h2d(A.es, P.es_off.data(), sizeof(long long) * P.es_off.size())) ||
-        (e = h2d(A.ss, P.ss_off.data(), sizeof(long long) * P.ss_off.size())) ||
-        (e = h2d(A.wplan, P.wplan.data(), sizeof(WalkPlan) * P.wplan.size())) ||
-        (e = h2d(A.splan, P.splan.data(), sizeof(SegPlan) * P.splan.size())) ||
-        (e = h2d(A.items, P.items.data(), sizeof(Item) * P.items.size())) ||
-        (e = h2d(A.ritems, P.ritems.data(), sizeof(RItem) * P.ritems.size())))
+    // plan tables from the host (one copy, from pinned memory: nothing waits
+    // for it; the caller has waited for the last refill's), lists and records
+    // on the device
+    const size_t tables = A.ide - A.walks;
+    if ((e = r->h_plan.ensure(tables))) return bail(e, "pinned plan");
+    copy_tables_to_arena(r->h_plan.as<char>() - A.walks, P, A);
+    if ((e = hipMemcpyAsync(d + A.walks, r->h_plan.p, tables, hipMemcpyHostToDevice, st)) ||
+        (!P.items.empty() && (e = hipMemcpyAsync(d + A.items, P.items.data(), sizeof(Item) * P.items.size(),
+                                                 hipMemcpyHostToDevice, st))) ||
+        (!P.ritems.empty() && (e = hipMemcpyAsync(d + A.ritems, P.ritems.data(), sizeof(RItem) * P.ritems.size(),
+                                                  hipMemcpyHostToDevice, st))))
         return bail(e, "resident upload");
     if ((t->n_le && (e = hipMemcpyAsync(d + A.ide, t->id_epj.p, 4 * (size_t)t->n_le, hipMemcpyDeviceToDevice, st))) ||
         (t->n_ls && (e = hipMemcpyAsync(d + A.ids, t->id_spj.p, 4 * (size_t)t->n_ls, hipMemcpyDeviceToDevice, st))))
@@ -1782,8 +1953,11 @@ int resident_fill_gtree(pth_resident *r, const pth_gtree *t, const char *who)
     else
         hipLaunchKernelGGL(k_res_nodes, dim3(blocks(t->n_node)), dim3(256), 0, st, t->n_node, t->pre.as<int>(),
                            t->nmass.as<double>(), t->ncom.as<double>(), t->nquad.as<double>(), r->spj.as<SpjDev>());
-    if ((e = hipGetLastError()) || (e = hipStreamSynchronize(st))) return bail(e, "resident records");
+    if ((e = hipGetLastError())) return bail(e, "resident records");
     if ((e = resident_finish(r))) return bail(e, "resident SPJ table");
+    // the tree's next build waits for its own context's stream: another one's
+    // copies are done before this returns (and those from the plan's own items)
+    if ((t->ctx != c || !P.on_device) && (e = hipStreamSynchronize(st))) return bail(e, "resident records");
     return PTH_OK;
 }
 

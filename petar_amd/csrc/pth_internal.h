@@ -399,13 +399,17 @@ inline hipError_t plan_items(const Plan &P, const Arena &A, char *base, hipStrea
                        reinterpret_cast<RItem *>(base + A.ritems), st);
 }
 
-inline void copy_plan_to_arena(char *h, const Plan &P, const Arena &A)
+inline void copy_tables_to_arena(char *h, const Plan &P, const Arena &A)
 {
     std::memcpy(h + A.walks, P.walks.data(), sizeof(WalkDev) * P.walks.size());
     std::memcpy(h + A.es, P.es_off.data(), sizeof(long long) * P.es_off.size());
     std::memcpy(h + A.ss, P.ss_off.data(), sizeof(long long) * P.ss_off.size());
     if (!P.wplan.empty()) std::memcpy(h + A.wplan, P.wplan.data(), sizeof(WalkPlan) * P.wplan.size());
     if (!P.splan.empty()) std::memcpy(h + A.splan, P.splan.data(), sizeof(SegPlan) * P.splan.size());
+}
+inline void copy_plan_to_arena(char *h, const Plan &P, const Arena &A)
+{
+    copy_tables_to_arena(h, P, A);
     if (!P.items.empty()) std::memcpy(h + A.items, P.items.data(), sizeof(Item) * P.items.size());
     if (!P.ritems.empty()) std::memcpy(h + A.ritems, P.ritems.data(), sizeof(RItem) * P.ritems.size());
 }
@@ -523,6 +527,7 @@ struct pth_resident {
     hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
     bool ran = false;
     ResultRing ring;
+    PinBuf h_plan;                       // plan tables on their way to the arena (refills from a tree)
     long long staged_bytes = 0;
 };
 

@@ -95,6 +95,13 @@ def test_device_tree_list_ordering(n, theta, leaf, group, canonical):
     _compare(n, 17, 0.5, theta, leaf=leaf, group=group, canonical=canonical)
 
 
+@pytest.mark.parametrize("leaf,group,theta", [(1, 512, 0.0), (1, 4, 0.05), (20, 8, 0.5), (20, 16, 0.5)])
+def test_device_tree_walk_widths(leaf, group, theta):
+    """Walks of few groups (four waves each) and of many (one wave each):
+    fronts that fill the node stack, and both sides of the limit between."""
+    _compare(12000, 29, 0.5, theta, leaf=leaf, group=group)
+
+
 @pytest.mark.parametrize("scale,shift", [(1e-12, 0.0), (1e9, 0.0), (1.0, 1e6), (1e-25, 0.0)])
 def test_device_tree_opening_test_precision(scale, shift):
     """The opening test is decided in FP32 relative to the root cube only
@@ -208,6 +215,33 @@ def _to_device(hip, a):
     assert hip.hipMalloc(C.byref(p), a.nbytes) == 0
     assert hip.hipMemcpy(p, a.ctypes.data, a.nbytes, 1) == 0  # host to device
     return p.value
+
+
+@pytest.mark.parametrize("max_ipl,own", [(2, True), (2, False), (4, True)])
+def test_device_tree_refills_in_a_row(max_ipl, own):
+    """A refill does not wait for the device: the next build and refill follow
+    at once, with the tree on the evaluation's context or on another, and with
+    plans made on the device (two i per lane at most) and on the host."""
+    par = dict(eps2=0.0, rcut2=R_OUT ** 2, G=1.0)
+    ctx = sf.Context(0, max_ipl=max_ipl, **par)
+    tctx = ctx if own else sf.Context(0, **par)
+    sets = [host.cluster(n, "plummer", f_bin=0.3, seed=n)[:2] for n in (9000, 15000, 4000)]
+    rs = [np.full(len(m), 1.5 * R_OUT) for m, _ in sets]
+    g = sf.GpuTree(tctx, sets[0][1], sets[0][0], rs[0])
+    r = sf.Resident.from_gtree(ctx, g)
+    for k in (1, 2, 0, 1):
+        g.update(sets[k][1], sets[k][0], rs[k])
+        r.refill(g)
+    g.update(sets[2][1], sets[2][0], rs[2])  # while the refill's copies may be on their way
+    r.run()
+    out = r.results()
+    f = sf.GpuTree(ctx, sets[1][1], sets[1][0], rs[1])
+    rf = sf.Resident.from_gtree(ctx, f)
+    rf.run()
+    for a, b in zip(out, rf.results()):
+        assert np.array_equal(a, b)
+    for o in (rf, f, r, g):
+        o.close()
 
 
 def test_device_tree_update_and_refill():
