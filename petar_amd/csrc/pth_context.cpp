@@ -213,6 +213,7 @@ void pth_destroy(pth_ctx *c)
     c->h_rid.release();
     c->h_rpos.release();
     c->d_spj_tab.release();
+    c->rings.release();
     if (c->ev_send) (void)hipEventDestroy(c->ev_send);
     if (c->ev_upload) (void)hipEventDestroy(c->ev_upload);
     if (c->ev_fork) (void)hipEventDestroy(c->ev_fork);
@@ -1010,6 +1011,7 @@ static int resident_enqueue(pth_resident *r, hipStream_t st, hipEvent_t fork_ev,
         if (timed) HIPCHK(c, hipEventRecord(r->ev[2], st), "hipEventRecord");
         for (int k = 0; k < r->b.n_seg; k++) HIPCHK(c, launch_reduce(r->b, k, st), "reduce kernel");
         r->pipelined = false;
+        r->ready.clear();
         return PTH_OK;
     }
     // a pipeline: the first side stream stages the segments one after
@@ -1017,6 +1019,7 @@ static int resident_enqueue(pth_resident *r, hipStream_t st, hipEvent_t fork_ev,
     // 1 + k mod (n - 1) once its staging is done, so the staging of the
     // segments after k overlaps k's force kernels
     const int ns = (int)r->side.size();
+    r->ready.clear();
     if (!timed) HIPCHK(c, hipEventRecord(fork_ev, st), "hipEventRecord");
     for (int s = 0; s < ns; s++) HIPCHK(c, hipStreamWaitEvent(r->side[s], fork_ev, 0), "hipStreamWaitEvent");
     for (int k = 0; k < r->b.n_seg; k++) {
@@ -1041,6 +1044,12 @@ static int resident_enqueue(pth_resident *r, hipStream_t st, hipEvent_t fork_ev,
             HIPCHK(c, launch_force(r->b, k, fs), "force kernel");
         }
         HIPCHK(c, launch_reduce(r->b, k, fs), "reduce kernel");
+        if (timed) {
+            const int we = r->plan.segs[k].walk_end;
+            const long long end = we < (int)r->plan.walks.size() ? r->plan.walks[we].i_off : r->plan.ni_tot;
+            HIPCHK(c, hipEventRecord(r->reduced[k], fs), "hipEventRecord");
+            r->ready.push_back(ResultsReady{end, r->reduced[k]});
+        }
     }
     for (int s = 0; s < ns; s++) {
         HIPCHK(c, hipEventRecord(r->side_done[s], r->side[s]), "hipEventRecord");
@@ -1094,6 +1103,7 @@ int pth_resident_run(pth_resident *r)
         return c->fail(PTH_ERR_STATE, "pth_resident_run: changeover mode needs pth_resident_changeover first");
     HIPCHK(c, hipSetDevice(c->device), "hipSetDevice");
     if (c->par.graph) {
+        r->ready.clear();
         const int rc = resident_capture(r);
         if (rc != PTH_OK) return rc;
         HIPCHK(c, hipEventRecord(r->ev[0], c->stream), "hipEventRecord");
@@ -1131,11 +1141,19 @@ int pth_resident_results(pth_resident *r, double *acc, double *pot, long long *n
     const long long n = r->plan.ni_tot;
     const int nw = r->co ? (int)r->plan.walks.size() : 0;
     int bad = -1;
+    // a pipelined evaluation: the first side stream, idle once it has staged
+    // the last segment, packs each chunk of results as soon as its segments
+    // are reduced, beside the force kernels of the segments after them (40 B
+    // per particle are 0.8 ms of 12.5 per step of 1,048,576, all after the
+    // evaluation before)
+    const bool early = !r->ready.empty();
     const hipError_t e =
-        results_to_host(c->stream, r->ring, r->out_accp.as<double4>(), r->out_nnb.as<int>(),
+        results_to_host(early ? r->side[0] : c->stream, c->rings, r->out_accp.as<double4>(), r->out_nnb.as<int>(),
                         r->co ? r->out_pott.as<double>() : nullptr, n, acc, pot, nnb, pot_tot,
-                        nw > 0 ? r->work.walk_err.as<int>() : nullptr, nw, &bad);
+                        nw > 0 ? r->work.walk_err.as<int>() : nullptr, nw, &bad, r->ready.data(),
+                        (int)r->ready.size());
     HIPCHK(c, e, "result download");
+    if (early) HIPCHK(c, hipStreamSynchronize(c->stream), "hipStreamSynchronize");
     if (bad >= 0)
         return c->fail(PTH_ERR_ARG, "pth_resident_results: changeover mode: an i-particle of walk " +
                                         std::to_string(bad) + " has no EPJ with its id in the walk's list");
@@ -1268,13 +1286,14 @@ void pth_resident_free(pth_resident *r)
     r->out_pott.release();
     r->plan_dev.release();
     r->work.release();
-    r->ring.release();
     r->h_plan.release();
     for (int k = 0; k < 4; k++)
         if (r->ev[k]) (void)hipEventDestroy(r->ev[k]);
     for (hipEvent_t x : r->side_done)
         if (x) (void)hipEventDestroy(x);
     for (hipEvent_t x : r->staged)
+        if (x) (void)hipEventDestroy(x);
+    for (hipEvent_t x : r->reduced)
         if (x) (void)hipEventDestroy(x);
     for (hipStream_t x : r->side)
         if (x) (void)hipStreamDestroy(x);
@@ -1361,10 +1380,28 @@ static void map_pages(void *p, size_t bytes)
             asm volatile("lock orb $0, %0" : "+m"(b[q]));
 }
 
-hipError_t copy_to_host(hipStream_t st, ResultRing &ring, const std::vector<HostCopy> &pieces)
+// A ring taken from the context's for one transfer; when that failed, the
+// ring goes back only after what was enqueued into it has ended.
+struct RingUse {
+    ResultRings &rings;
+    ResultRing *ring;
+    hipStream_t st;
+    bool done = false;
+    RingUse(ResultRings &r, hipStream_t s) : rings(r), ring(r.take()), st(s) {}
+    ~RingUse()
+    {
+        if (!ring) return;
+        if (!done) (void)hipStreamSynchronize(st);
+        rings.give(ring);
+    }
+};
+
+hipError_t copy_to_host(hipStream_t st, ResultRings &rings, const std::vector<HostCopy> &pieces)
 {
     constexpr size_t CHUNK = results_bytes(RESULT_CHUNK, false);
-    std::lock_guard<std::mutex> lk(ring.m);
+    RingUse use(rings, st);
+    if (!use.ring) return hipErrorOutOfMemory;
+    ResultRing &ring = *use.ring;
     std::vector<HostCopy> part;
     for (const HostCopy &c : pieces)
         for (size_t o = 0; c.dst && o < c.bytes; o += CHUNK)
@@ -1393,14 +1430,18 @@ hipError_t copy_to_host(hipStream_t st, ResultRing &ring, const std::vector<Host
             std::memcpy((char *)part[k].dst + n * q / t, src + n * q / t, n * (q + 1) / t - n * q / t);
         if (k + RESULT_RING < part.size() && (e = start(k + RESULT_RING))) return e;
     }
+    use.done = true;
     return hipStreamSynchronize(st);
 }
 
-hipError_t results_to_host(hipStream_t st, ResultRing &ring, const double4 *accp, const int *out_nnb,
+hipError_t results_to_host(hipStream_t st, ResultRings &rings, const double4 *accp, const int *out_nnb,
                            const double *pott, long long n, double *acc, double *pot, long long *nnb, double *pot_tot,
-                           const int *err, int n_err, int *bad)
+                           const int *err, int n_err, int *bad, const ResultsReady *ready, int n_ready)
 {
-    std::lock_guard<std::mutex> lk(ring.m);
+    if (n <= 0) return hipStreamSynchronize(st);
+    RingUse use(rings, st);
+    if (!use.ring) return hipErrorOutOfMemory;
+    ResultRing &ring = *use.ring;
     hipError_t e;
     const bool co = pott != nullptr;
     const long long n_chunk = (n + RESULT_CHUNK - 1) / RESULT_CHUNK;
@@ -1412,12 +1453,16 @@ hipError_t results_to_host(hipStream_t st, ResultRing &ring, const double4 *accp
         if (!ring.ev[k] && (e = hipEventCreateWithFlags(&ring.ev[k], hipEventDisableTiming))) return e;
     }
     auto at = [&](long long k) { return ring.buf[k % RESULT_RING].as<char>() + (k % RESULT_RING ? 0 : head); };
+    int waited = 0;
     auto pack = [&](long long k) -> hipError_t {
-        const hipError_t r = launch_results(accp, out_nnb, pott, k * RESULT_CHUNK, count(k),
+        hipError_t r;
+        const long long end = k * RESULT_CHUNK + count(k);
+        for (; waited < n_ready && (waited == 0 || ready[waited - 1].end < end); waited++)
+            if ((r = hipStreamWaitEvent(st, ready[waited].done, 0))) return r;
+        r = launch_results(accp, out_nnb, pott, k * RESULT_CHUNK, count(k),
                                             reinterpret_cast<double *>(at(k)), st);
         return r ? r : hipEventRecord(ring.ev[k % RESULT_RING], st);
     };
-    if (n <= 0) return hipStreamSynchronize(st);
     if (err && (e = hipMemcpyAsync(ring.buf[0].p, err, sizeof(int) * (size_t)n_err, hipMemcpyDeviceToHost, st))) return e;
     for (long long k = 0; k < nb; k++)
         if ((e = pack(k))) return e;
@@ -1439,6 +1484,7 @@ hipError_t results_to_host(hipStream_t st, ResultRing &ring, const double4 *accp
                        nnb ? nnb + i0 : nullptr, pot_tot ? pot_tot + i0 : nullptr);
         if (k + RESULT_RING < n_chunk && (e = pack(k + RESULT_RING))) return e;
     }
+    use.done = true;
     return hipSuccess;
 }
 
@@ -1450,6 +1496,7 @@ int resident_setup(pth_resident *r, int n_walk, const int *n_epi, const int *n_e
     r->ran = false;
     r->co_ready = false;
     r->pipelined = false;
+    r->ready.clear();
     r->n_seg = (c->par.exec_mode == PTH_EXEC_FUSED) ? c->par.segments : 1;
     if (pre) {
         if (!pre_ok) return c->fail(PTH_ERR_CAPACITY, std::string(who) + ": sizes exceed the int32 index range");
@@ -1494,6 +1541,10 @@ int resident_setup(pth_resident *r, int n_walk, const int *n_epi, const int *n_e
         while (r->staged.size() < P.segs.size()) {
             r->staged.push_back(nullptr);
             if ((e = hipEventCreateWithFlags(&r->staged.back(), hipEventDisableTiming))) return bail(e, "hipEventCreate");
+        }
+        while (r->reduced.size() < P.segs.size()) {
+            r->reduced.push_back(nullptr);
+            if ((e = hipEventCreateWithFlags(&r->reduced.back(), hipEventDisableTiming))) return bail(e, "hipEventCreate");
         }
     }
     r->n_epj_tot = n_epj_tot;

@@ -1520,7 +1520,6 @@ struct pth_gtree {
     DevBuf range;            // the nodes' particle ranges, in preorder
     void *pinned = nullptr;  // pinned host copy of meta
     hipEvent_t ev_meta = nullptr;  // that copy
-    mutable ResultRing ring;       // of downloads
     int tile_passes = 0;  // of the last search's tile walk
     // one-pass neighbour filters: regions from the last completed search's
     // per-particle counts (ngb_cnt), valid while ngb_prev_ok
@@ -2226,7 +2225,7 @@ int pth_gtree_neighbors_download(const pth_gtree *t, int *count, long long *offs
     if (!t->built || t->n_ngb < 0)
         return c->fail(PTH_ERR_STATE, "pth_gtree_neighbors_download: no neighbour search since the last build");
     HIPCHK(c, hipSetDevice(c->device), "hipSetDevice");
-    HIPCHK(c, copy_to_host(c->stream, t->ring, {{count, t->ngb_cnt.p, sizeof(int) * (size_t)t->n},
+    HIPCHK(c, copy_to_host(c->stream, c->rings, {{count, t->ngb_cnt.p, sizeof(int) * (size_t)t->n},
                                                 {offset, t->ngb_off.p, sizeof(long long) * (size_t)(t->n + 1)},
                                                 {ngb, t->ngb.p, sizeof(int) * (size_t)t->n_ngb}}), "download");
     if (ms) *ms = t->ms_ngb;
@@ -2250,7 +2249,6 @@ void pth_gtree_free(pth_gtree *t)
     t->release_scratch();
     if (t->pinned) (void)hipHostFree(t->pinned);
     if (t->ev_meta) (void)hipEventDestroy(t->ev_meta);
-    t->ring.release();
     delete t;
 }
 

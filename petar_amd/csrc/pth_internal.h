@@ -9,6 +9,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
+#include <new>
 #include <string>
 #include <vector>
 
@@ -195,16 +196,13 @@ struct Work {
 
 // Pinned buffers that results pass through on their way to the caller's
 // arrays: a chunk is packed into one by the device while the host copies the
-// chunks before it out of the others.  One per object that hands out results
-// (a resident evaluation, a server), so calls on different objects share
-// nothing.  RESULT_CHUNK particles (2.4 MB) keep a chunk's transfer (42 us at
+// chunks before it out of the others.  RESULT_CHUNK particles (2.4 MB) keep a chunk's transfer (42 us at
 // the link's 57 GB/s) well above the cost of its launch, event and parallel
 // loop.  Against two pageable copies and one host loop over all results
 // (bound by 18 GB/s, page faults and one core): 1,048,576 particles 10.9 to
 // about 1 ms, 4,194,304 47 to 6 ms, 16,384 80 to 45 us.
 constexpr int RESULT_CHUNK = 65536, RESULT_RING = 3;
 struct ResultRing {
-    std::mutex m;  // one transfer at a time
     PinBuf buf[RESULT_RING];
     hipEvent_t ev[RESULT_RING] = {};
     void release()
@@ -216,22 +214,67 @@ struct ResultRing {
         }
     }
 };
-// Copies n results, complete on stream st when the work enqueued there is, to
-// acc [n][3], pot [n], nnb [n] and pot_tot [n] (each may be null; pott null:
-// no total potential) and returns when they are there.  With n_err > 0 the
-// n_err words at err are looked at first: if one is not zero, nothing is
-// copied and bad receives its index.
-hipError_t results_to_host(hipStream_t st, ResultRing &ring, const double4 *accp, const int *out_nnb,
+// The rings of a context: a transfer takes one for its own use and gives it
+// back, so transfers of different objects and threads share none.  At most
+// MAX_FREE are kept (8 to 10 MB each) until the context is destroyed.  Rings
+// of the objects themselves cost every new one their pinning: a service's
+// first pass over 24 clusters 8.6 ms, with the context's 5.2; a changeover
+// evaluation's of 1,048,576 particles 20.4 and 12.8.
+struct ResultRings {
+    static constexpr int MAX_FREE = 4;
+    std::mutex m;
+    ResultRing *free[MAX_FREE] = {};
+    int n = 0;
+    ResultRing *take()
+    {
+        std::lock_guard<std::mutex> lk(m);
+        return n > 0 ? free[--n] : new (std::nothrow) ResultRing;
+    }
+    void give(ResultRing *r)
+    {
+        {
+            std::lock_guard<std::mutex> lk(m);
+            if (n < MAX_FREE) {
+                free[n++] = r;
+                return;
+            }
+        }
+        r->release();
+        delete r;
+    }
+    void release()
+    {
+        while (n > 0) {
+            free[--n]->release();
+            delete free[n];
+        }
+    }
+};
+// The results of particles [0, end) are complete when done (recorded on
+// another stream) and those of the ends before it are.
+struct ResultsReady {
+    long long end;
+    hipEvent_t done;
+};
+// Copies n results to acc [n][3], pot [n], nnb [n] and pot_tot [n] (each may
+// be null; pott null: no total potential) and returns when they are there.
+// They are complete when the work enqueued on stream st is and, with n_ready
+// > 0, the events of ready say so (ends ascending, the last one n): a chunk
+// then leaves while later ones are computed.  With n_err > 0 the
+// n_err words at err (complete on st) are looked at first: if one is not
+// zero, nothing is copied and bad receives its index.
+hipError_t results_to_host(hipStream_t st, ResultRings &rings, const double4 *accp, const int *out_nnb,
                            const double *pott, long long n, double *acc, double *pot, long long *nnb, double *pot_tot,
-                           const int *err = nullptr, int n_err = 0, int *bad = nullptr);
-// Copies device arrays to (pageable) host arrays through the ring, after the
+                           const int *err = nullptr, int n_err = 0, int *bad = nullptr,
+                           const ResultsReady *ready = nullptr, int n_ready = 0);
+// Copies device arrays to (pageable) host arrays through a ring, after the
 // work on stream st; pieces without bytes or destination are left out.
 struct HostCopy {
     void *dst;
     const void *src;
     size_t bytes;
 };
-hipError_t copy_to_host(hipStream_t st, ResultRing &ring, const std::vector<HostCopy> &pieces);
+hipError_t copy_to_host(hipStream_t st, ResultRings &rings, const std::vector<HostCopy> &pieces);
 // The host side of one chunk of n results packed at src (launch_results).
 void unpack_results(const char *src, long long n, bool co, double *acc, double *pot, long long *nnb, double *pot_tot);
 
@@ -471,6 +514,7 @@ struct pth_ctx {
     hipStream_t side = nullptr;
     hipEvent_t ev_fork = nullptr, ev_join = nullptr;
     hipEvent_t ev_upload = nullptr;  // the last batch's inputs have been read
+    ResultRings rings;
     Work work;
     TagState tag[MAX_TAG];
     // profile of the hooks (pth_profile_*)
@@ -514,6 +558,8 @@ struct pth_resident {
     std::vector<hipEvent_t> side_done;   // one per side stream
     std::vector<hipEvent_t> staged;      // one per segment: its staging is done
     bool pipelined = false;              // the last run used the side streams
+    std::vector<hipEvent_t> reduced;     // one per segment: its results are complete
+    std::vector<pth::ResultsReady> ready;  // of the last run, if pipelined (not replayed from the graph)
     // graph mode: the evaluation captured on its own stream (fork and join
     // events over the side streams) and replayed; b_gen counts rebuilds of
     // the launch descriptor, g_gen the one the graph holds
@@ -526,7 +572,6 @@ struct pth_resident {
     BatchDev b;
     hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
     bool ran = false;
-    ResultRing ring;
     PinBuf h_plan;                       // plan tables on their way to the arena (refills from a tree)
     long long staged_bytes = 0;
 };

@@ -189,7 +189,6 @@ struct pth_server {
     hipStream_t cap = nullptr;   // graph capture
     hipStream_t xfer = nullptr;  // result copies (evictions, pth_server_results)
     hipEvent_t ev_evicted = nullptr;  // the latest eviction copy
-    ResultRing ring;             // of pth_server_results
     long long n_evict_copies = 0;
     long long gen_clock = 0;     // placements of cluster ranges and scratch ranges
     std::mutex mu;
@@ -886,7 +885,7 @@ int pth_server_results(pth_server *s, int k, double *acc, double *pot, long long
         // resident: its last request has completed; copy the outputs now
         // (the worker is held off by the lock meanwhile)
         const char *base = s->pool.as<char>() + c.off;
-        HIPCHK(s->ctx, results_to_host(s->xfer, s->ring, reinterpret_cast<const double4 *>(base + c.L.out_accp),
+        HIPCHK(s->ctx, results_to_host(s->xfer, s->ctx->rings, reinterpret_cast<const double4 *>(base + c.L.out_accp),
                                        reinterpret_cast<const int *>(base + c.L.out_nnb), nullptr, n, acc, pot, nnb,
                                        nullptr), "result download");
         return PTH_OK;
@@ -963,7 +962,6 @@ void pth_server_free(pth_server *s)
     if (s->cap) (void)hipStreamDestroy(s->cap);
     if (s->xfer) (void)hipStreamDestroy(s->xfer);
     s->pool.release();
-    s->ring.release();
     if (s->pctx) pth_destroy(s->pctx);
     delete s;
 }
