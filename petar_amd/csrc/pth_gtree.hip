@@ -1316,20 +1316,23 @@ __global__ __launch_bounds__(256) void k_tile_boxes(const int *__restrict__ tile
 
 // Neighbour search (src/soft_force.hpp:11-34, SearchNeighborEpEpNoSimd) on
 // candidate lists that hold every symmetric-search neighbour (the tile walks
-// of pth_gtree_neighbors, or a group's EPJ list): for every i of a tile the
+// of pth_gtree_neighbors): for every i of a tile the
 // list entries j with |x_i - x_j|^2 < max(rs_i, rs_j)^2 in FP64, self
-// included.  One wave per tile at a time, up to NGB_T sub-tiles of 64 i per
-// pass (lane l holds i = l + 64 t), j staged
-// 64 at a time in LDS (read as broadcasts).  A (tile, chunk) pair is
-// skipped when the boxes of the tile's and the chunk's positions are at
-// least R = max(rs) apart: the gap g (per axis, >= 0) bounds every pair's
-// |dx| from below, and since each rounded operation is monotone,
-// gx*gx + gy*gy + gz*gz >= R*R implies dx*dx + dy*dy + dz*dz >= rs*rs in
-// the same FP64 arithmetic, so the skip never drops a neighbour.
+// included.  One wave per tile at a time, lane l holds i = l (a tile of more
+// than 64 particles is a leaf of as many, taken 64 at a time); 64 candidates
+// at a time are loaded, one per lane, and those that come within R =
+// max(rs of the tile, rs_j) of the tile's box go to LDS, in list order, to be
+// read as broadcasts by all lanes.  The gap g between box and j (per axis,
+// >= 0) bounds every pair's |dx| from below; g2 = gx^2 + gy^2 + gz^2 and the
+// pair's r2 are each within 3 ulp of their exact values however they are
+// contracted, so g2 > R^2 (1 + 2^-48) implies r2 >= rs^2 as computed below
+// and the skip never drops a neighbour.
+// What bounds it: the latency of the candidates' gathers and the pair loop.
+// A wave that held eight sub-tiles of 64 i (nearly all tiles have one), took
+// the boxes of all eight and of every 64 candidates and then tested all of
+// the 64 was 655 us at 1,048,576 particles; this 215.
 // Counting pass: cnt[input index of i]; writing pass: input indices of the
 // neighbours at ngb[off[input index of i]..], in list order.
-constexpr int NGB_T = 8;
-
 struct NgbArgs {
     const double *spos, *srs;
     const long long *order;
@@ -1362,115 +1365,75 @@ __device__ __forceinline__ double wave_max(double v)
     return v;
 }
 
-struct Box {
-    double lo[3], hi[3], rs;
-};
-
-// box of the lane values (inactive lanes pass act = false)
-__device__ __forceinline__ Box wave_box(bool act, double x, double y, double z, double rs)
-{
-    Box b;
-    b.lo[0] = wave_min(act ? x : 1e300);
-    b.lo[1] = wave_min(act ? y : 1e300);
-    b.lo[2] = wave_min(act ? z : 1e300);
-    b.hi[0] = wave_max(act ? x : -1e300);
-    b.hi[1] = wave_max(act ? y : -1e300);
-    b.hi[2] = wave_max(act ? z : -1e300);
-    b.rs = wave_max(act ? rs : 0.0);
-    return b;
-}
-
-// true when no pair between the two boxes can be neighbours
-__device__ __forceinline__ bool boxes_apart(const Box &a, const Box &b)
-{
-    const double gx = fmax(0.0, fmax(b.lo[0] - a.hi[0], a.lo[0] - b.hi[0]));
-    const double gy = fmax(0.0, fmax(b.lo[1] - a.hi[1], a.lo[1] - b.hi[1]));
-    const double gz = fmax(0.0, fmax(b.lo[2] - a.hi[2], a.lo[2] - b.hi[2]));
-    const double r = fmax(a.rs, b.rs);
-    return gx * gx + gy * gy + gz * gz >= r * r;
-}
-
 template <bool WRITE>
 __global__ __launch_bounds__(64) void k_ngb(const NgbArgs a)
 {
     __shared__ NgbJ sj[64];
     __shared__ int sid[64];
-    __shared__ Box tb[NGB_T];  // boxes of the tiles (wave-uniform)
     const int lane = threadIdx.x;
     for (long long g = blockIdx.x; g < a.n_group; g += gridDim.x) {
         const int4 G = a.info[g];
         const long long eb = a.off_e[g], ee = a.off_e[g + 1];
-        for (int s0 = 0; s0 < G.y; s0 += 64 * NGB_T) {
-            const int nt = min(NGB_T, (G.y - s0 + 63) / 64);
-            double xi[NGB_T], yi[NGB_T], zi[NGB_T], ri[NGB_T];
-            long long w[NGB_T];
-            int c[NGB_T], cap[NGB_T];
-            bool act[NGB_T];
-#pragma unroll
-            for (int t = 0; t < NGB_T; t++) {
-                c[t] = 0;
-                cap[t] = INT_MAX;
-                act[t] = false;
-                xi[t] = yi[t] = zi[t] = ri[t] = 0.0;
-                w[t] = 0;
-                if (t < nt) {
-                    act[t] = s0 + 64 * t + lane < G.y;
-                    if (act[t]) {
-                        const long long i = (long long)G.x + s0 + 64 * t + lane;
-                        xi[t] = a.spos[3 * i];
-                        yi[t] = a.spos[3 * i + 1];
-                        zi[t] = a.spos[3 * i + 2];
-                        ri[t] = a.srs[i];
-                        if (WRITE) {
-                            const long long oi = a.order[i];
-                            w[t] = a.off[oi];
-                            if (a.padded) cap[t] = (int)(a.off[oi + 1] - w[t]);
-                        }
-                    }
-                    const Box b = wave_box(act[t], xi[t], yi[t], zi[t], ri[t]);
-                    if (lane == 0) tb[t] = b;
+        for (int s0 = 0; s0 < G.y; s0 += 64) {
+            const bool act = s0 + lane < G.y;
+            double xi = 0, yi = 0, zi = 0, ri = 0;
+            long long oi = 0, w = 0;
+            int c = 0, cap = INT_MAX;
+            if (act) {
+                const long long i = (long long)G.x + s0 + lane;
+                xi = a.spos[3 * i];
+                yi = a.spos[3 * i + 1];
+                zi = a.spos[3 * i + 2];
+                ri = a.srs[i];
+                oi = a.order[i];
+                if (WRITE) {
+                    w = a.off[oi];
+                    if (a.padded) cap = (int)(a.off[oi + 1] - w);
                 }
             }
+            const double lx = wave_min(act ? xi : 1e300), hx = wave_max(act ? xi : -1e300);
+            const double ly = wave_min(act ? yi : 1e300), hy = wave_max(act ? yi : -1e300);
+            const double lz = wave_min(act ? zi : 1e300), hz = wave_max(act ? zi : -1e300);
+            const double rt = wave_max(act ? ri : 0.0);
             for (long long k0 = eb; k0 < ee; k0 += 64) {
                 const long long k = k0 + lane;
-                const bool jact = k < ee;
                 NgbJ J{0, 0, 0, 0};
-                if (jact) {
-                    const int j = a.id_epj[k];
+                bool near = false;
+                int j = 0;
+                if (k < ee) {
+                    j = a.id_epj[k];
                     J = NgbJ{a.spos[3 * (long long)j], a.spos[3 * (long long)j + 1], a.spos[3 * (long long)j + 2],
                              a.srs[j]};
-                    sj[lane] = J;
-                    if (WRITE) sid[lane] = (int)a.order[j];
+                    const double gx = fmax(0.0, fmax(lx - J.x, J.x - hx));
+                    const double gy = fmax(0.0, fmax(ly - J.y, J.y - hy));
+                    const double gz = fmax(0.0, fmax(lz - J.z, J.z - hz));
+                    const double R = fmax(rt, J.rs);
+                    near = !(gx * gx + gy * gy + gz * gz > R * R * (1 + 0x1p-48));
                 }
-                const Box cb = wave_box(jact, J.x, J.y, J.z, J.rs);
+                const unsigned long long found = __ballot(near);
+                if (near) {
+                    const int p = __popcll(found & ((1ull << lane) - 1));
+                    sj[p] = J;
+                    if (WRITE) sid[p] = (int)a.order[j];
+                }
                 __syncthreads();
-                const int m = (int)min((long long)64, ee - k0);
-#pragma unroll
-                for (int t = 0; t < NGB_T; t++) {
-                    if (t >= nt || boxes_apart(tb[t], cb)) continue;  // wave-uniform (LDS broadcast)
-                    if (act[t])
-                        for (int q = 0; q < m; q++) {
-                            const NgbJ Q = sj[q];
-                            const double dx = xi[t] - Q.x, dy = yi[t] - Q.y, dz = zi[t] - Q.z;
-                            const double r2 = dx * dx + dy * dy + dz * dz;
-                            const double rs = (ri[t] < Q.rs) ? Q.rs : ri[t];
-                            if (r2 < rs * rs) {
-                                if (WRITE && c[t] < cap[t]) a.ngb[w[t] + c[t]] = sid[q];
-                                c[t]++;
-                            }
+                const int m = __popcll(found);
+                if (act)
+                    for (int q = 0; q < m; q++) {
+                        const NgbJ Q = sj[q];
+                        const double dx = xi - Q.x, dy = yi - Q.y, dz = zi - Q.z;
+                        const double r2 = dx * dx + dy * dy + dz * dz;
+                        const double rs = (ri < Q.rs) ? Q.rs : ri;
+                        if (r2 < rs * rs) {
+                            if (WRITE && c < cap) a.ngb[w + c] = sid[q];
+                            c++;
                         }
-                }
+                    }
                 __syncthreads();
             }
             if (!WRITE || a.padded) {
-                bool over = false;
-#pragma unroll
-                for (int t = 0; t < NGB_T; t++)
-                    if (t < nt && act[t]) {
-                        a.cnt[a.order[(long long)G.x + s0 + 64 * t + lane]] = c[t];
-                        over = over || c[t] > cap[t];
-                    }
-                if (WRITE && over) atomicOr(a.flag, 1);
+                if (act) a.cnt[oi] = c;
+                if (WRITE && c > cap) atomicOr(a.flag, 1);
             }
         }
     }
