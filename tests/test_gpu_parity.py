@@ -441,6 +441,39 @@ def test_segments_are_bit_identical(c1, segments, streams):
     _check(out[1], ref, amb, f"segments={segments} streams={streams}")
 
 
+@pytest.mark.parametrize("segments,streams,n", [(8, 3, 300000), (5, 2, 70001), (16, 5, 9000)])
+def test_results_of_evaluations_in_turn(segments, streams, n):
+    """Two evaluations of one context share its streams and transfer buffers:
+    run one after the other and read in either order, also with graph replays
+    set on and off in between, their results (several chunks of 65,536, some
+    ending inside a segment) equal those of one stream bit for bit."""
+    m, x, _ = host.cluster(n, "plummer", kroupa=True, seed=5)
+    L = [host.build_lists(x[:k], m[:k], 1.5 * R_OUT, theta=0.6) for k in (n, n // 2)]
+    par = dict(eps2=0.0, rcut2=R_OUT ** 2, G=1.0, min_seg_pairs=1)
+    ctx = sf.Context(0, segments=1, streams=1, **par)
+    want = []
+    for l in L:
+        r = sf.Resident.from_lists(ctx, l)
+        r.run()
+        want.append(r.results())
+        r.close()
+    ctx.close()
+    ctx = sf.Context(0, segments=segments, streams=streams, **par)
+    rs = [sf.Resident.from_lists(ctx, l) for l in L]
+    for graph, order in ((0, (0, 1)), (0, (1, 0)), (1, (0, 1)), (0, (0, 1)), (1, (1, 0))):
+        p = ctx.get_params()
+        p.graph = graph
+        ctx.set_params(p)
+        for r in rs:
+            r.run()
+        for k in order:
+            got = rs[k].results()
+            assert all(np.array_equal(a, b) for a, b in zip(got, want[k])), (graph, order, k)
+    for r in rs:
+        r.close()
+    ctx.close()
+
+
 @pytest.mark.parametrize("exec_mode", [sf.EXEC_FUSED, sf.EXEC_PLAIN])
 def test_monopole_superparticles(c1, exec_mode):
     """spj_monopole = 1 (a PeTar build without USE_QUAD): the superparticles'

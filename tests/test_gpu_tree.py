@@ -383,6 +383,24 @@ def test_device_neighbors_equal_oracle(n, f_bin, theta, shift):
     assert np.array_equal(cnt, ecnt) and np.array_equal(off, eoff) and np.array_equal(ngb, engb)
 
 
+@pytest.mark.parametrize("leaf,same", [(1, 0), (64, 0), (65, 0), (200, 0), (20, 130)])
+def test_device_neighbors_tiles_of_any_size(leaf, same):
+    """Tiles of 1, 64, 65 and more particles (a leaf is one tile, whatever its
+    size; same particles at one point cannot be split): lists as the FP64
+    restatement's, first search and repeated one."""
+    m, x, _ = host.cluster(3000, "plummer", kroupa=True, f_bin=0.5, seed=47)
+    x[:same] = x[0]
+    rs = 3.0 * R_OUT * np.maximum(np.cbrt(m / m.mean()), 1.0)
+    L = host.build_lists(x, m, rs, theta=0.3, n_leaf_limit=leaf)
+    want = _expected_ngb(L, *O.ngb_walks(L.n_epi, L.n_epj, L.epj_pos, L.epj_rs, L.id_epj, L.epj_pos, L.epj_rs))
+    ctx = sf.Context(0)
+    g = sf.GpuTree(ctx, x, m, rs, theta=0.3, n_leaf_limit=leaf)
+    for _ in range(2):
+        assert all(np.array_equal(a, b) for a, b in zip(g.neighbors()[:3], want))
+    g.close()
+    ctx.close()
+
+
 def test_device_neighbors_one_pass_repeat():
     """A search with as many tiles as the last one writes its candidate lists
     in one pass into regions of the last search's candidate counts, and its
