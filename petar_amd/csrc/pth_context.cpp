@@ -117,7 +117,6 @@ int pth_create(pth_ctx **out, int rank, const pth_params *params)
     c->device = (rank >= 0 ? rank : -rank) % ndev;  // src/force_gpu_cuda.cu:550-553
     if ((e = hipSetDevice(c->device)) != hipSuccess ||
         (e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking)) != hipSuccess ||
-        (e = c->want_sides(2)) != hipSuccess ||  // at once: see resident_enqueue
         (e = hipEventCreateWithFlags(&c->ev_send, hipEventDisableTiming)) != hipSuccess ||
         (e = hipEventCreateWithFlags(&c->ev_upload, hipEventDisableTiming)) != hipSuccess) {
         g_create_err = std::string("pth_create: ") + hipGetErrorName(e);
@@ -219,9 +218,9 @@ void pth_destroy(pth_ctx *c)
     if (c->ev_upload) (void)hipEventDestroy(c->ev_upload);
     if (c->ev_fork) (void)hipEventDestroy(c->ev_fork);
     if (c->ev_join) (void)hipEventDestroy(c->ev_join);
-    for (hipStream_t x : c->sides) {
-        (void)hipStreamSynchronize(x);
-        (void)hipStreamDestroy(x);
+    if (c->side) {
+        (void)hipStreamSynchronize(c->side);
+        (void)hipStreamDestroy(c->side);
     }
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
@@ -670,16 +669,15 @@ int pth_dispatch(pth_ctx *c, int tag, int n_walk, const void *const *epi, const 
     const bool split = c->class_streams && !b.plain && !split_launch(b, 0) && P.seg_count[0] > 0 &&
                        P.seg_count[1] + P.seg_count[2] + P.seg_count[3] > 0;
     if (split) {
-        HIPCHK(c, c->want_sides(1), "hipStreamCreate");
-        const hipStream_t side = c->sides[0];
+        if (!c->side) HIPCHK(c, hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking), "hipStreamCreate");
         if (!c->ev_fork) HIPCHK(c, hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming), "hipEventCreate");
         if (!c->ev_join) HIPCHK(c, hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming), "hipEventCreate");
         HIPCHK(c, launch_stage(b, 0, c->stream), "staging kernel");
         HIPCHK(c, hipEventRecord(c->ev_fork, c->stream), "hipEventRecord");
-        HIPCHK(c, hipStreamWaitEvent(side, c->ev_fork, 0), "hipStreamWaitEvent");
+        HIPCHK(c, hipStreamWaitEvent(c->side, c->ev_fork, 0), "hipStreamWaitEvent");
         HIPCHK(c, launch_force(b, 0, c->stream, 0xEu), "soft-force kernels");
-        HIPCHK(c, launch_force(b, 0, side, 0x1u), "soft-force kernels");
-        HIPCHK(c, hipEventRecord(c->ev_join, side), "hipEventRecord");
+        HIPCHK(c, launch_force(b, 0, c->side, 0x1u), "soft-force kernels");
+        HIPCHK(c, hipEventRecord(c->ev_join, c->side), "hipEventRecord");
         HIPCHK(c, hipStreamWaitEvent(c->stream, c->ev_join, 0), "hipStreamWaitEvent");
         HIPCHK(c, launch_reduce(b, 0, c->stream), "reduction kernel");
     } else {
@@ -991,7 +989,7 @@ static int resident_enqueue(pth_resident *r, hipStream_t st, hipEvent_t fork_ev,
     pth_ctx *c = r->ctx;
     // (segments asked to run on one stream: on st, which needs no events)
     const bool segmented = !r->side.empty() && r->b.n_seg > 1 && (int)r->staged.size() >= r->b.n_seg;
-    if (!segmented || r->n_stream < 2) {
+    if (!segmented || r->side.size() < 2) {
         // one segment: its 1-i items run on a side stream beside the longer
         // classes (the 1-i launch is about one round of waves, whose run-down
         // tail the longer launch then fills)
@@ -1018,29 +1016,20 @@ static int resident_enqueue(pth_resident *r, hipStream_t st, hipEvent_t fork_ev,
         r->ready.clear();
         return PTH_OK;
     }
-    // a pipeline over ns streams: the first side stream stages the segments
-    // one after another; segment k's force and reduce run on st (k mod
-    // (ns - 1) = 0) or another side stream once its staging is done, so the
-    // staging of the segments after k, and the first waves of segment k + 1,
-    // overlap k's force kernels.  HIP gives a process 4 hardware queues, and
-    // streams that share one run in turn: with three side streams of every
-    // evaluation's own and st idle beside them, two of them shared the queue
-    // of a single evaluation (traced at 1,048,576 particles: no two segments
-    // overlapped).  With the context's three streams, made together so that
-    // they get queues of their own: 1,048,576 particles in changeover mode
-    // 12.34 to 11.11 ms, 4,194,304 51.93 to 51.79, a step of 1,048,576 12.58
-    // to 12.47; staging and one force stream (st) alone 12.34, 53.9 and 12.52.
-    const int ns = r->n_stream;
+    // a pipeline: the first side stream stages the segments one after
+    // another; segment k's force and reduce run on side stream
+    // 1 + k mod (n - 1) once its staging is done, so the staging of the
+    // segments after k overlaps k's force kernels
+    const int ns = (int)r->side.size();
     r->ready.clear();
     if (!timed) HIPCHK(c, hipEventRecord(fork_ev, st), "hipEventRecord");
-    for (hipStream_t s : r->side) HIPCHK(c, hipStreamWaitEvent(s, fork_ev, 0), "hipStreamWaitEvent");
+    for (int s = 0; s < ns; s++) HIPCHK(c, hipStreamWaitEvent(r->side[s], fork_ev, 0), "hipStreamWaitEvent");
     for (int k = 0; k < r->b.n_seg; k++) {
         HIPCHK(c, launch_stage(r->b, k, r->side[0]), "stage kernels");
         HIPCHK(c, hipEventRecord(r->staged[k], r->side[0]), "hipEventRecord");
     }
     for (int k = 0; k < r->b.n_seg; k++) {
-        const int f = k % (ns - 1);
-        hipStream_t fs = f == 0 ? st : r->side[f];
+        hipStream_t fs = r->side[1 + k % (ns - 1)];
         HIPCHK(c, hipStreamWaitEvent(fs, r->staged[k], 0), "hipStreamWaitEvent");
         // the last segment's 1-i launch on the staging stream (idle by then)
         // beside its longer classes: nothing else is left to fill its tail
@@ -1064,7 +1053,7 @@ static int resident_enqueue(pth_resident *r, hipStream_t st, hipEvent_t fork_ev,
             r->ready.push_back(ResultsReady{end, r->reduced[k]});
         }
     }
-    for (size_t s = 0; s < r->side.size(); s++) {
+    for (int s = 0; s < ns; s++) {
         HIPCHK(c, hipEventRecord(r->side_done[s], r->side[s]), "hipEventRecord");
         HIPCHK(c, hipStreamWaitEvent(st, r->side_done[s], 0), "hipStreamWaitEvent");
     }
@@ -1115,7 +1104,6 @@ int pth_resident_run(pth_resident *r)
     if (r->co && !r->co_ready)
         return c->fail(PTH_ERR_STATE, "pth_resident_run: changeover mode needs pth_resident_changeover first");
     HIPCHK(c, hipSetDevice(c->device), "hipSetDevice");
-    HIPCHK(c, resident_sides(r), "hipStreamCreate");  // (graph mode may have been set or unset)
     if (c->par.graph) {
         r->ready.clear();
         const int rc = resident_capture(r);
@@ -1309,7 +1297,8 @@ void pth_resident_free(pth_resident *r)
         if (x) (void)hipEventDestroy(x);
     for (hipEvent_t x : r->reduced)
         if (x) (void)hipEventDestroy(x);
-    for (hipStream_t x : r->own) (void)hipStreamDestroy(x);
+    for (hipStream_t x : r->side)
+        if (x) (void)hipStreamDestroy(x);
     if (r->gexec) (void)hipGraphExecDestroy(r->gexec);
     if (r->fork) (void)hipEventDestroy(r->fork);
     if (r->cap) (void)hipStreamDestroy(r->cap);
@@ -1501,25 +1490,6 @@ hipError_t results_to_host(hipStream_t st, ResultRings &rings, const double4 *ac
     return hipSuccess;
 }
 
-// The side streams of r's next run: the context's, or in graph mode, which
-// captures them, streams of r's own, on which nothing else is enqueued.
-hipError_t resident_sides(pth_resident *r)
-{
-    const size_t want = (size_t)std::max(1, r->n_stream - 1);
-    if (!r->ctx->par.graph) {
-        const hipError_t e = r->ctx->want_sides(want);
-        if (e == hipSuccess) r->side.assign(r->ctx->sides.begin(), r->ctx->sides.begin() + (long)want);
-        return e;
-    }
-    while (r->own.size() < want) {
-        hipStream_t s = nullptr;
-        if (const hipError_t e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking)) return e;
-        r->own.push_back(s);
-    }
-    r->side.assign(r->own.begin(), r->own.begin() + (long)want);
-    return hipSuccess;
-}
-
 int resident_setup(pth_resident *r, int n_walk, const int *n_epi, const int *n_epj, const int *n_spj,
                    long long n_ide, long long n_ids, int n_epj_tot, int n_spj_tot, const char *who, Plan *pre,
                    bool pre_ok)
@@ -1561,11 +1531,12 @@ int resident_setup(pth_resident *r, int n_walk, const int *n_epi, const int *n_e
         if (!r->ev[k] && (e = hipEventCreate(&r->ev[k]))) return bail(e, "hipEventCreate");
     {
         // (one side stream also for a single segment: its 1-i class)
+        const int ns = std::max(1, std::min(c->par.streams, (int)P.segs.size()));
         // side streams are only ever added (a later plan may use fewer)
-        r->n_stream = std::max(r->n_stream, std::min(c->par.streams, (int)P.segs.size()));
-        if ((e = resident_sides(r))) return bail(e, "hipStreamCreate");
-        while (r->side_done.size() < r->side.size()) {
+        while ((int)r->side.size() < ns) {
+            r->side.push_back(nullptr);
             r->side_done.push_back(nullptr);
+            if ((e = hipStreamCreateWithFlags(&r->side.back(), hipStreamNonBlocking))) return bail(e, "hipStreamCreate");
             if ((e = hipEventCreateWithFlags(&r->side_done.back(), hipEventDisableTiming)))
                 return bail(e, "hipEventCreate");
         }

@@ -511,21 +511,7 @@ struct pth_ctx {
     // pth_dispatch's kernels write the results straight into the tag's pinned
     // host buffers (PTH_ZERO_COPY=0: device buffers and a copy)
     bool zero_copy = true;
-    // streams beside the context's, for the hooks and for its evaluations
-    // (which its stream orders one after another), made when first wanted
-    std::mutex sides_m;
-    std::vector<hipStream_t> sides;
-    hipError_t want_sides(size_t n)
-    {
-        std::lock_guard<std::mutex> lk(sides_m);
-        sides.reserve(8);  // (streams are at most 8: it never moves)
-        while (sides.size() < n) {
-            hipStream_t s = nullptr;
-            if (const hipError_t e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking)) return e;
-            sides.push_back(s);
-        }
-        return hipSuccess;
-    }
+    hipStream_t side = nullptr;
     hipEvent_t ev_fork = nullptr, ev_join = nullptr;
     hipEvent_t ev_upload = nullptr;  // the last batch's inputs have been read
     ResultRings rings;
@@ -568,9 +554,7 @@ struct pth_resident {
     DevBuf plan_dev;  // work items and reduction items after a re-plan
     int max_ipl = 0, chunk_j = 0;
     int n_seg = 1;                       // walk segments of the plan
-    int n_stream = 1;                    // streams the segments run on: st and side
-    std::vector<hipStream_t> side;       // the context's, or own (graph mode)
-    std::vector<hipStream_t> own;
+    std::vector<hipStream_t> side;       // streams the segments run on
     std::vector<hipEvent_t> side_done;   // one per side stream
     std::vector<hipEvent_t> staged;      // one per segment: its staging is done
     bool pipelined = false;              // the last run used the side streams
@@ -609,8 +593,6 @@ int resident_setup(pth_resident *r, int n_walk, const int *n_epi, const int *n_e
 // Builds the SPJ table and the launch descriptors of a prepared resident
 // whose contents are uploaded (or being uploaded on the context's stream).
 hipError_t resident_finish(pth_resident *r);
-// Sets the side streams of r's next run.
-hipError_t resident_sides(pth_resident *r);
 // Looks up this device's address of the allocation-free entry point's
 // scratch array (once per device; the device must be current).
 void noalloc_setup(int device);
