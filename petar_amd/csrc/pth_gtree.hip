@@ -1898,10 +1898,10 @@ int resident_fill_gtree(pth_resident *r, const pth_gtree *t, const char *who)
     if ((e = r->h_plan.ensure(tables))) return bail(e, "pinned plan");
     copy_tables_to_arena(r->h_plan.as<char>() - A.walks, P, A);
     if ((e = hipMemcpyAsync(d + A.walks, r->h_plan.p, tables, hipMemcpyHostToDevice, st)) ||
-        (!P.items.empty() && (e = hipMemcpyAsync(d + A.items, P.items.data(), sizeof(Item) * P.items.size(),
-                                                 hipMemcpyHostToDevice, st))) ||
-        (!P.ritems.empty() && (e = hipMemcpyAsync(d + A.ritems, P.ritems.data(), sizeof(RItem) * P.ritems.size(),
-                                                  hipMemcpyHostToDevice, st))))
+        (P.item_bytes() &&
+         (e = hipMemcpyAsync(d + A.items, P.items.data(), P.item_bytes(), hipMemcpyHostToDevice, st))) ||
+        (P.ritem_bytes() &&
+         (e = hipMemcpyAsync(d + A.ritems, P.ritems.data(), P.ritem_bytes(), hipMemcpyHostToDevice, st))))
         return bail(e, "resident upload");
     if ((t->n_le && (e = hipMemcpyAsync(d + A.ide, t->id_epj.p, 4 * (size_t)t->n_le, hipMemcpyDeviceToDevice, st))) ||
         (t->n_ls && (e = hipMemcpyAsync(d + A.ids, t->id_spj.p, 4 * (size_t)t->n_ls, hipMemcpyDeviceToDevice, st))))

@@ -453,8 +453,8 @@ inline void copy_tables_to_arena(char *h, const Plan &P, const Arena &A)
 inline void copy_plan_to_arena(char *h, const Plan &P, const Arena &A)
 {
     copy_tables_to_arena(h, P, A);
-    if (!P.items.empty()) std::memcpy(h + A.items, P.items.data(), sizeof(Item) * P.items.size());
-    if (!P.ritems.empty()) std::memcpy(h + A.ritems, P.ritems.data(), sizeof(RItem) * P.ritems.size());
+    if (P.item_bytes()) std::memcpy(h + A.items, P.items.data(), P.item_bytes());
+    if (P.ritem_bytes()) std::memcpy(h + A.ritems, P.ritems.data(), P.ritem_bytes());
 }
 
 }  // namespace pth

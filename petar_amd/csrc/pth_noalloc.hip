@@ -241,8 +241,8 @@ extern "C" int pth_resident_eval_noalloc(pth_ctx *c, int n_walk, const int *n_ep
         (e = up(o_arena + A.ss, P.ss_off.data(), sizeof(long long) * P.ss_off.size())) ||
         (e = up(o_arena + A.wplan, P.wplan.data(), sizeof(WalkPlan) * P.wplan.size())) ||
         (e = up(o_arena + A.splan, P.splan.data(), sizeof(SegPlan) * P.splan.size())) ||
-        (e = up(o_arena + A.items, P.items.data(), sizeof(Item) * P.items.size())) ||
-        (e = up(o_arena + A.ritems, P.ritems.data(), sizeof(RItem) * P.ritems.size())) ||
+        (e = up(o_arena + A.items, P.items.data(), P.item_bytes())) ||
+        (e = up(o_arena + A.ritems, P.ritems.data(), P.ritem_bytes())) ||
         (e = up(o_arena + A.ide, id_epj, sizeof(int) * (size_t)n_ide)) ||
         (e = up(o_arena + A.ids, id_spj, sizeof(int) * (size_t)n_ids)) ||
         (e = up(o_ipos, epi_pos, 24 * (size_t)ni)) || (e = up(o_irs, epi_rs, 8 * (size_t)ni)) ||

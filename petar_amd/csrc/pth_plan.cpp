@@ -270,12 +270,12 @@ bool size_plan(Plan &P, long long cj, int max_ipl, int n_seg, long long min_seg_
 bool make_plan(int n_walk, const int *n_epi, const int *n_epj, const int *n_spj, int exec_mode,
                int chunk_j, int max_ipl, Plan &P, int n_seg, bool mono, long long min_seg_pairs, bool on_device)
 {
-    // the item array keeps its size from the previous plan (every slot is
-    // written below, so growing it is the only initialisation it needs)
+    // the item array keeps its size from the previous plan where this one
+    // writes every slot of it (growing it is then the only initialisation it
+    // needs); a plan without items on the host must not hold the last one's
     std::vector<Item> kept;
     kept.swap(P.items);
     P.reset();
-    P.items.swap(kept);
     P.mono = mono;
     P.walks.resize(n_walk);
     P.es_off.assign(n_walk + 1, 0);
@@ -314,6 +314,7 @@ bool make_plan(int n_walk, const int *n_epi, const int *n_epj, const int *n_spj,
     const long long cj = (chunk_j > 0) ? chunk_j : DEFAULT_CHUNK_J;
     static thread_local Scratch S;
     if (on_device && max_ipl <= 2) return size_plan(P, cj, max_ipl, n_seg, min_seg_pairs, S.wcost);
+    P.items.swap(kept);
     // chunking of walk w: nch chunks, EPJ block / SPJ record bounds
     auto chunks = [&](int w, std::vector<long long> &eb, std::vector<long long> &sb) -> long long {
         const long long nb = (P.es_off[w + 1] - P.es_off[w]) / 8;

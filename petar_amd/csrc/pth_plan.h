@@ -54,6 +54,9 @@ struct Plan {
     std::vector<WalkPlan> wplan;
     std::vector<SegPlan> splan;
     int n_slots = 0, n_ritems = 0;          // items (with empty slots) and reduction items, wherever they are made
+    // bytes of both that the host made and has to upload
+    size_t item_bytes() const { return on_device ? 0 : sizeof(Item) * (size_t)n_slots; }
+    size_t ritem_bytes() const { return on_device ? 0 : sizeof(RItem) * (size_t)n_ritems; }
     int n_part = 0;                         // partial slots of 64 entries
     int n_real_items = 0;
     long long ni_tot = 0, n_e_slots = 0, n_s_rec = 0;

@@ -4,6 +4,7 @@ the entry points fail cleanly where no device exists."""
 import ctypes as C
 import os
 import re
+import subprocess
 
 import numpy as np
 import pytest
@@ -227,3 +228,18 @@ def test_plan_segments_keep_every_walks_items():
                     assert it[0] < 0 or wb <= it[0] < we
             for r in rit[g[10]:g[10] + g[11]]:
                 assert ioff[wb] <= r[0] < ioff[we]
+
+
+def _plan_check(what):
+    """tests/cpp/plan_check, built if it is not there."""
+    d = os.path.join(ROOT, "tests", "cpp")
+    if not os.path.exists(os.path.join(d, "plan_check")):
+        subprocess.run(["make", "plan_check"], cwd=d, check=True, capture_output=True)
+    r = subprocess.run([os.path.join(d, "plan_check"), what], capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout
+
+
+def test_plan_object_reused_holds_no_stale_items():
+    """What a plan makes on the host is what its consumers upload into room
+    sized for it, whatever the object planned before."""
+    _plan_check("reuse")

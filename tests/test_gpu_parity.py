@@ -911,3 +911,29 @@ def test_device_plan_equals_host_plan(max_ipl, segments):
     racc, rpot, rnnb = O.soft_force_walks(**a, eps2=1e-8, rout2=1e-4)
     assert np.median(rel_err(dev[0], racc)[np.abs(racc).sum(1) > 0]) <= MED
     assert np.mean(dev[2] != rnnb) <= 1e-3
+
+
+def test_dispatch_after_a_change_of_plan(c1):
+    """One context's batches, planned by the host, by the device and without
+    items in turn: each batch's results are those of a context that planned
+    no other."""
+    L = c1[0]
+    forms = [dict(max_ipl=4, chunk_j=64), dict(max_ipl=2), dict(max_ipl=3, chunk_j=64), dict(exec_mode=sf.EXEC_PLAIN),
+             dict(max_ipl=1)]
+
+    def replay(kw, fresh):
+        fn = sf.CalcForceWithLinearCutoffMultiWalk(0, 0.0, R_OUT ** 2, 1.0, exec_mode=kw.get("exec_mode", sf.EXEC_FUSED),
+                                                   chunk_j=kw.get("chunk_j", 0))
+        if fresh:
+            fn.close_contexts()
+        c = fn.context()
+        p = c.get_params()
+        p.max_ipl = kw.get("max_ipl", 2)
+        c.set_params(p)
+        return _fdps_replay(L, fn)
+
+    want = [replay(kw, True) for kw in forms]
+    sf.CalcForceWithLinearCutoffMultiWalk.close_contexts()
+    for kw, w in zip(forms, want):
+        assert all(np.array_equal(x, y) for x, y in zip(replay(kw, False), w)), kw
+    sf.CalcForceWithLinearCutoffMultiWalk.close_contexts()

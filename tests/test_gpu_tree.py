@@ -589,3 +589,28 @@ def test_context_close_frees_its_objects_first():
     g.close()
     r.close()
     srv.close()
+
+
+@pytest.mark.parametrize("max_ipl,chunk", [(1, 512), (4, 64)])
+def test_refills_after_a_replan(max_ipl, chunk):
+    """A re-plan leaves items made by the host with the evaluation, which the
+    next refills hand to the tree and back: each refill uploads only what its
+    own plan made on the host."""
+    ctx = sf.Context(0, eps2=0.0, rcut2=R_OUT ** 2, G=1.0)
+    sets = [host.cluster(n, "plummer", f_bin=0.3, seed=n)[:2] for n in (15000, 4000, 9000)]
+    rs = [np.full(len(m), 1.5 * R_OUT) for m, _ in sets]
+    g = sf.GpuTree(ctx, sets[0][1], sets[0][0], rs[0])
+    r = sf.Resident.from_gtree(ctx, g)
+    r.replan(max_ipl, chunk)
+    r.run()
+    for k in (1, 2, 0):
+        g.update(sets[k][1], sets[k][0], rs[k])
+        r.refill(g)
+        r.run()
+        f = sf.Resident.from_gtree(ctx, g)
+        f.run()
+        assert all(np.array_equal(a, b) for a, b in zip(r.results(), f.results()))
+        f.close()
+    r.close()
+    g.close()
+    ctx.close()
