@@ -798,10 +798,28 @@ __global__ __launch_bounds__(256) void k_res_particles(long long n, const double
     epj[k] = j;
 }
 
-// (the SPJ lists name nodes by preorder number)
-__global__ __launch_bounds__(256) void k_res_nodes(long long nn, const int *__restrict__ pre,
-                                                   const double *__restrict__ nmass, const double *__restrict__ ncom,
-                                                   const double *__restrict__ nquad, pth::SpjDev *__restrict__ spj)
+// The tree's SPJ lists name nodes by preorder number; for everyone else the
+// entries become node numbers (level by level) on their way out.  Siblings
+// then lie side by side in the superparticle table: numbered by preorder, with
+// whole subtrees between them, 4,194,304 particles' staging took 4.09 ms for
+// 3.63 and their force 39.7 for 37.8.  A refill copies the lists anyway (53M
+// entries 78 us, by name 114); named where they are put in order, they cost
+// that kernel 50 us (215 to 268) whoever reads them.  Bound by the gathers.
+__global__ __launch_bounds__(256) void k_node_lists(long long n, const int *__restrict__ list,
+                                                    const int *__restrict__ node_at, int *__restrict__ out)
+{
+    const long long k = 4 * ((long long)blockIdx.x * 256 + threadIdx.x);
+    if (k + 4 <= n) {
+        const int4 v = *reinterpret_cast<const int4 *>(list + k);
+        *reinterpret_cast<int4 *>(out + k) = make_int4(node_at[v.x], node_at[v.y], node_at[v.z], node_at[v.w]);
+    } else {
+        for (long long j = k; j < n; j++) out[j] = node_at[list[j]];
+    }
+}
+
+__global__ __launch_bounds__(256) void k_res_nodes(long long nn, const double *__restrict__ nmass,
+                                                   const double *__restrict__ ncom, const double *__restrict__ nquad,
+                                                   pth::SpjDev *__restrict__ spj)
 {
     const long long k = (long long)blockIdx.x * 256 + threadIdx.x;
     if (k >= nn) return;
@@ -818,12 +836,11 @@ __global__ __launch_bounds__(256) void k_res_nodes(long long nn, const int *__re
     r.qxz = (float)q[4];
     r.qyz = (float)q[5];
     r.pad[0] = r.pad[1] = r.pad[2] = 0.f;
-    spj[pre[k]] = r;
+    spj[k] = r;
 }
 
 // monopole superparticles: the node's mass at its centre of mass
-__global__ __launch_bounds__(256) void k_res_nodes_mono(long long nn, const int *__restrict__ pre,
-                                                        const double *__restrict__ nmass,
+__global__ __launch_bounds__(256) void k_res_nodes_mono(long long nn, const double *__restrict__ nmass,
                                                         const double *__restrict__ ncom,
                                                         pth::EpjDev *__restrict__ spj)
 {
@@ -835,7 +852,7 @@ __global__ __launch_bounds__(256) void k_res_nodes_mono(long long nn, const int 
     r.z = ncom[3 * k + 2];
     r.m = (float)nmass[k];
     r.rs = 0.f;
-    spj[pre[k]] = r;
+    spj[k] = r;
 }
 
 struct WalkArgs {
@@ -1854,6 +1871,14 @@ int gtree_run(pth_gtree *t, long long n, const double *pos, const double *mass, 
     return PTH_OK;
 }
 
+// The tree's SPJ lists as node numbers to out (16-byte aligned).
+void node_lists(const pth_gtree *t, int *out, hipStream_t st)
+{
+    if (t->n_ls <= 0) return;
+    hipLaunchKernelGGL(k_node_lists, dim3(blocks((t->n_ls + 3) / 4)), dim3(256), 0, st, t->n_ls, t->id_spj.as<int>(),
+                       t->node_at.as<int>(), out);
+}
+
 // (Re)fills resident r from tree t: plan, buffers, records and lists.
 int resident_fill_gtree(pth_resident *r, const pth_gtree *t, const char *who)
 {
@@ -1903,18 +1928,18 @@ int resident_fill_gtree(pth_resident *r, const pth_gtree *t, const char *who)
         (P.ritem_bytes() &&
          (e = hipMemcpyAsync(d + A.ritems, P.ritems.data(), P.ritem_bytes(), hipMemcpyHostToDevice, st))))
         return bail(e, "resident upload");
-    if ((t->n_le && (e = hipMemcpyAsync(d + A.ide, t->id_epj.p, 4 * (size_t)t->n_le, hipMemcpyDeviceToDevice, st))) ||
-        (t->n_ls && (e = hipMemcpyAsync(d + A.ids, t->id_spj.p, 4 * (size_t)t->n_ls, hipMemcpyDeviceToDevice, st))))
+    if (t->n_le && (e = hipMemcpyAsync(d + A.ide, t->id_epj.p, 4 * (size_t)t->n_le, hipMemcpyDeviceToDevice, st)))
         return bail(e, "resident lists");
+    node_lists(t, reinterpret_cast<int *>(d + A.ids), st);
     hipLaunchKernelGGL(k_res_particles, dim3(blocks(t->n)), dim3(256), 0, st, t->n, t->spos.as<double>(),
                        t->smass.as<double>(), t->srs.as<double>(), reinterpret_cast<EpiDev *>(d + A.epi),
                        r->epj.as<EpjDev>());
     if (P.mono)
         hipLaunchKernelGGL(k_res_nodes_mono, dim3(blocks(t->n_node)), dim3(256), 0, st, t->n_node,
-                           t->pre.as<int>(), t->nmass.as<double>(), t->ncom.as<double>(), r->spj.as<EpjDev>());
+                           t->nmass.as<double>(), t->ncom.as<double>(), r->spj.as<EpjDev>());
     else
-        hipLaunchKernelGGL(k_res_nodes, dim3(blocks(t->n_node)), dim3(256), 0, st, t->n_node, t->pre.as<int>(),
-                           t->nmass.as<double>(), t->ncom.as<double>(), t->nquad.as<double>(), r->spj.as<SpjDev>());
+        hipLaunchKernelGGL(k_res_nodes, dim3(blocks(t->n_node)), dim3(256), 0, st, t->n_node, t->nmass.as<double>(),
+                           t->ncom.as<double>(), t->nquad.as<double>(), r->spj.as<SpjDev>());
     if ((e = hipGetLastError())) return bail(e, "resident records");
     if ((e = resident_finish(r))) return bail(e, "resident SPJ table");
     // the tree's next build waits for its own context's stream: another one's
@@ -1993,12 +2018,15 @@ int pth_gtree_download(const pth_gtree *t, long long *order, long long *node_beg
     HIPCHK(c, d2h(node_com, t->ncom, 24 * nn), "download");
     HIPCHK(c, d2h(node_quad, t->nquad, 48 * nn), "download");
     HIPCHK(c, d2h(id_epj, t->id_epj, 4 * t->n_le), "download");
-    HIPCHK(c, d2h(id_spj, t->id_spj, 4 * t->n_ls), "download");
     if (id_spj && t->n_ls > 0) {
-        // (the lists name nodes by preorder number on the device)
-        std::vector<int> at(nn);
-        HIPCHK(c, d2h(at.data(), t->node_at, 4 * nn), "download");
-        for (long long k = 0; k < t->n_ls; k++) id_spj[k] = at[id_spj[k]];
+        // (by way of the walk's raw lists, which the next walk writes anew:
+        // they held these entries, so they have room for them)
+        const DevBuf &b = t->walk.raw_s;
+        if (b.cap < 4 * (size_t)t->n_ls) return c->fail(PTH_ERR_STATE, "pth_gtree_download: no room for the lists");
+        node_lists(t, b.as<int>(), c->stream);
+        HIPCHK(c, hipGetLastError(), "list kernel");
+        HIPCHK(c, hipStreamSynchronize(c->stream), "download");
+        HIPCHK(c, d2h(id_spj, b, 4 * t->n_ls), "download");
     }
     std::vector<GNode> nodes(nn);
     HIPCHK(c, d2h(nodes.data(), t->nodes, sizeof(GNode) * nn), "download");

@@ -614,3 +614,23 @@ def test_refills_after_a_replan(max_ipl, chunk):
     r.close()
     g.close()
     ctx.close()
+
+
+def test_device_tree_lists_leave_by_node_number():
+    """SPJ lists of every length modulo four, and none at all, leave the
+    device by the host's node numbers, four entries at a time."""
+    ctx = sf.Context(0, eps2=0.0, rcut2=R_OUT ** 2, G=1.0)
+    seen = set()
+    for n in list(range(1200, 1216)) + [30]:
+        m, x, _ = host.cluster(n, "plummer", seed=n)
+        L = host.build_lists(x, m, 1.5 * R_OUT, theta=0.8, n_group_limit=64)
+        g = sf.GpuTree(ctx, x, m, np.full(n, 1.5 * R_OUT), theta=0.8, n_group_limit=64)
+        assert np.array_equal(g.download()["id_spj"], L.id_spj)
+        r, rl = sf.Resident.from_gtree(ctx, g), sf.Resident.from_lists(ctx, L)
+        r.run(), rl.run()
+        assert all(np.array_equal(a, b) for a, b in zip(r.results(), rl.results()))
+        seen.add(len(L.id_spj) % 4 if len(L.id_spj) else -1)
+        for o in (r, rl, g):
+            o.close()
+    ctx.close()
+    assert seen == {-1, 0, 1, 2, 3}
