@@ -896,7 +896,7 @@ template <bool WRITE, bool TILE, int NW>
 __global__ __launch_bounds__(64 * NW) void k_walk(const WalkArgs a)
 {
     __shared__ int stk[WALK_STACK];
-    __shared__ float lim[GT_MAX_LEVEL + 1];  // (L / theta)^2 of each level
+    __shared__ float lim[GT_MAX_LEVEL + 1];  // (L / theta)^2 of each level, NaN where FP32 has too few digits for it
     __shared__ int3 wave_n[NW];              // children, leaves and closed nodes of each wave
     __shared__ int wave_e[NW];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, thread = threadIdx.x;
@@ -904,7 +904,10 @@ __global__ __launch_bounds__(64 * NW) void k_walk(const WalkArgs a)
     const float mg = walk_margin(len, a.meta->rs_max);
     if (thread <= GT_MAX_LEVEL) {
         const double L = len / (double)(1LL << thread);
-        lim[thread] = (float)(L * L * a.inv_theta2);
+        // (near and below FP32's smallest normal number the relative bounds on
+        // squares fail; against NaN the test goes to FP64)
+        const double T = L * L * a.inv_theta2;
+        lim[thread] = T >= 0x1p-100 ? (float)T : NAN;
     }
     const unsigned long long below = lane ? ~0ull >> (64 - lane) : 0ull;
     for (long long g = blockIdx.x; g < a.n_group; g += gridDim.x) {

@@ -634,3 +634,23 @@ def test_device_tree_lists_leave_by_node_number():
             o.close()
     ctx.close()
     assert seen == {-1, 0, 1, 2, 3}
+
+
+@pytest.mark.parametrize("e", [69, 72, 76, 120, 135, 140])
+def test_device_tree_scaled_by_powers_of_two(e):
+    """A cluster scaled by 2^-e has the same tree, lists and neighbours: every
+    FP64 operation scales exactly.  The squares of the opening test (e = 69 to
+    76) and then the coordinates themselves (e = 135, 140) leave the normal
+    FP32 range, where the walks' first tests are made."""
+    m, x, _ = host.cluster(6000, "plummer", f_bin=0.3, seed=23)
+    rs = 1.5 * R_OUT * np.maximum(np.cbrt(m / m.mean()), 1.0)
+    ctx = sf.Context(0)
+    out = []
+    for s in (1.0, 2.0 ** -e):
+        g = sf.GpuTree(ctx, x * s, m, rs * s, theta=0.5)
+        d = g.download()
+        out.append([d[k] for k in ("order", "n_epi", "n_epj", "n_spj", "id_epj", "id_spj")] + list(g.neighbors()[:3]))
+        g.close()
+    ctx.close()
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
