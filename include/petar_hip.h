@@ -118,7 +118,8 @@ typedef struct pth_params {
     int graph;     /* resident evaluations: 1 captures an evaluation's launches
                       (all segments and streams) once as a hipGraph and
                       replays it on later runs; 0 launches them one by one.
-                      Results do not depend on it. */
+                      Results do not depend on it.  Evaluations of several
+                      segments on one stream are launched either way. */
     double min_seg_pairs; /* resident evaluations: fewest pair interactions a
                       pipelined segment gets (0 = 1e9), so a small evaluation
                       runs in fewer segments, down to one on one stream

@@ -1104,7 +1104,12 @@ int pth_resident_run(pth_resident *r)
     if (r->co && !r->co_ready)
         return c->fail(PTH_ERR_STATE, "pth_resident_run: changeover mode needs pth_resident_changeover first");
     HIPCHK(c, hipSetDevice(c->device), "hipSetDevice");
-    if (c->par.graph) {
+    // Segments on one stream are launched in graph mode too: a captured form
+    // of theirs (the stream waiting for its own events) ended in a host
+    // segmentation fault in this call, and as long as its cause is not shown
+    // nothing of the kind is captured.
+    const bool one_stream = r->b.n_seg > 1 && r->side.size() < 2;
+    if (c->par.graph && !one_stream) {
         r->ready.clear();
         const int rc = resident_capture(r);
         if (rc != PTH_OK) return rc;
