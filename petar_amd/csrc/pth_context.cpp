@@ -588,6 +588,15 @@ int pth_dispatch(pth_ctx *c, int tag, int n_walk, const void *const *epi, const 
         if (runs) HIPCHK(c, c->d_ids.ensure(sizeof(int) * (size_t)std::max<long long>(n_ide + n_ids, 1)),
                          "device list allocation");
     }
+    // the SPJ table of the sent superparticles (quadrupole form), for this
+    // batch's eps2; its memory now, so that nothing is left to fail between
+    // the upload and the event that guards the pinned arena
+    const bool make_tab = !c->mono_sent && c->n_spj > 0 && (!c->tab_valid || c->tab_eps2 != (float)c->par.eps2);
+    if (make_tab) {
+        if (sizeof(SpjTab) * (size_t)c->n_spj > c->d_spj_tab.cap)
+            HIPCHK(c, hipStreamSynchronize(c->stream), "hipStreamSynchronize");
+        HIPCHK(c, c->d_spj_tab.ensure(sizeof(SpjTab) * (size_t)c->n_spj), "SPJ table allocation");
+    }
     // the tag's pinned result buffers (nothing of this tag is in flight);
     // with zero_copy the kernels write the results straight into them (host
     // memory the device addresses; the writes are visible to the host once
@@ -636,12 +645,7 @@ int pth_dispatch(pth_ctx *c, int tag, int n_walk, const void *const *epi, const 
     if (c->par.exec_mode == PTH_EXEC_PLAIN) HIPCHK(c, hipStreamSynchronize(c->stream), "upload sync");
     HIPCHK(c, plan_items(P, A, c->d_arena.as<char>(), c->stream), "planning kernel");
     BatchDev b;
-    // the SPJ table of the sent superparticles (quadrupole form), for this
-    // batch's eps2
-    if (!c->mono_sent && c->n_spj > 0 && (!c->tab_valid || c->tab_eps2 != (float)c->par.eps2)) {
-        if (sizeof(SpjTab) * (size_t)c->n_spj > c->d_spj_tab.cap)
-            HIPCHK(c, hipStreamSynchronize(c->stream), "hipStreamSynchronize");
-        HIPCHK(c, c->d_spj_tab.ensure(sizeof(SpjTab) * (size_t)c->n_spj), "SPJ table allocation");
+    if (make_tab) {
         HIPCHK(c, launch_spj_table(c->d_spj.as<SpjDev>(), c->n_spj, (float)c->par.eps2, c->d_spj_tab.as<SpjTab>(),
                                    c->stream), "SPJ table kernel");
         c->tab_valid = true;
