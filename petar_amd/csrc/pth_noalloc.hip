@@ -185,44 +185,57 @@ extern "C" int pth_resident_eval_noalloc(pth_ctx *c, int n_walk, const int *n_ep
     // the plan: one segment on the context's stream (a walk's items and
     // results do not depend on the segmentation)
     Plan &P = c->na_plan;
-    if (!make_plan(n_walk, n_epi, n_epj, n_spj, PTH_EXEC_FUSED, c->par.chunk_j, c->par.max_ipl, P, 1, mono, 0, true))
-        return c->fail(PTH_ERR_CAPACITY, W + ": sizes exceed the int32 index range");
     Arena A{};
-    A.layout(P, n_ide, n_ids, false);
     const bool df = df_enabled(c->par) != 0;
-    const long long nw = (long long)P.walks.size();
+    const long long nw = n_walk;
     const long long ni1 = std::max<long long>(ni, 1), nj1 = std::max(n_epj_tot, 1), ns1 = std::max(n_spj_tot, 1);
-    // inputs and outputs for the whole call
-    Carve cv;
-    const size_t o_arena = cv.take(A.total);
-    const size_t o_epj = cv.take(sizeof(EpjDev) * nj1);
-    const size_t o_spj = cv.take((mono ? sizeof(EpjDev) : sizeof(SpjDev)) * ns1);
-    const size_t o_tab = cv.take(mono ? 0 : sizeof(SpjTab) * ns1);
-    const size_t o_accp = cv.take(sizeof(double4) * ni1);
-    const size_t o_nnb = cv.take(sizeof(int) * ni1);
-    const size_t persist = cv.off;
-    // then, in turn over one region: the caller's FP64 arrays while they are
-    // packed, the work buffers of the evaluation, the unpacked outputs
-    Carve r1{persist};
-    const size_t o_ipos = r1.take(24 * (size_t)ni1), o_irs = r1.take(8 * (size_t)ni1);
-    const size_t o_jpos = r1.take(24 * (size_t)nj1), o_jm = r1.take(8 * (size_t)nj1), o_jrs = r1.take(8 * (size_t)nj1);
-    const size_t o_spos = r1.take(24 * (size_t)ns1), o_sm = r1.take(8 * (size_t)ns1);
-    const size_t o_sq = r1.take(mono ? 0 : 48 * (size_t)ns1);
-    Carve r2{persist};
-    const long long slots = std::max<long long>(P.n_e_slots, 8), recs = std::max<long long>(P.n_s_rec, 1);
-    const long long parts = std::max(P.n_part, 1);
-    const size_t o_centre = r2.take(sizeof(double4) * std::max<long long>(nw, 1));
-    const size_t o_nearb = r2.take(sizeof(int) * std::max<long long>(nw, 1));
-    const size_t o_si = r2.take(sizeof(float4) * ni1);
-    const size_t o_se = r2.take(sizeof(float) * 5 * slots);
-    const size_t o_ss = r2.take(sizeof(float) * PTH_SPJ_STAGED * recs);
-    const size_t o_pa = r2.take(sizeof(double4) * 64 * parts);
-    const size_t o_pn = r2.take(sizeof(int) * 64 * parts);
-    const size_t o_il = r2.take(df ? sizeof(float4) * ni1 : 0);
-    const size_t o_el = r2.take(df ? sizeof(float) * (PTH_DF_EXTRA / 8) * slots : 0);
-    Carve r3{persist};
-    const size_t o_acc = r3.take(24 * (size_t)ni1), o_pot = r3.take(8 * (size_t)ni1), o_nnb64 = r3.take(8 * (size_t)ni1);
-    const size_t need = std::max(r1.off, std::max(r2.off, r3.off));
+    size_t o_arena = 0, o_epj = 0, o_spj = 0, o_tab = 0, o_accp = 0, o_nnb = 0;
+    size_t o_ipos = 0, o_irs = 0, o_jpos = 0, o_jm = 0, o_jrs = 0, o_spos = 0, o_sm = 0, o_sq = 0;
+    size_t o_centre = 0, o_nearb = 0, o_si = 0, o_se = 0, o_ss = 0, o_pa = 0, o_pn = 0, o_il = 0, o_el = 0;
+    size_t o_acc = 0, o_pot = 0, o_nnb64 = 0, need = 0;
+    const auto lay_out = [&](bool on_device) -> bool {
+        if (!make_plan(n_walk, n_epi, n_epj, n_spj, PTH_EXEC_FUSED, c->par.chunk_j, c->par.max_ipl, P, 1, mono, 0,
+                       on_device))
+            return false;
+        A.layout(P, n_ide, n_ids, false);
+        // inputs and outputs for the whole call
+        Carve cv;
+        o_arena = cv.take(A.total);
+        o_epj = cv.take(sizeof(EpjDev) * nj1);
+        o_spj = cv.take((mono ? sizeof(EpjDev) : sizeof(SpjDev)) * ns1);
+        o_tab = cv.take(mono ? 0 : sizeof(SpjTab) * ns1);
+        o_accp = cv.take(sizeof(double4) * ni1);
+        o_nnb = cv.take(sizeof(int) * ni1);
+        const size_t persist = cv.off;
+        // then, in turn over one region: the caller's FP64 arrays while they are
+        // packed, the work buffers of the evaluation, the unpacked outputs
+        Carve r1{persist};
+        o_ipos = r1.take(24 * (size_t)ni1), o_irs = r1.take(8 * (size_t)ni1);
+        o_jpos = r1.take(24 * (size_t)nj1), o_jm = r1.take(8 * (size_t)nj1), o_jrs = r1.take(8 * (size_t)nj1);
+        o_spos = r1.take(24 * (size_t)ns1), o_sm = r1.take(8 * (size_t)ns1);
+        o_sq = r1.take(mono ? 0 : 48 * (size_t)ns1);
+        Carve r2{persist};
+        const long long slots = std::max<long long>(P.n_e_slots, 8), recs = std::max<long long>(P.n_s_rec, 1);
+        const long long parts = std::max(P.n_part, 1);
+        o_centre = r2.take(sizeof(double4) * std::max<long long>(nw, 1));
+        o_nearb = r2.take(sizeof(int) * std::max<long long>(nw, 1));
+        o_si = r2.take(sizeof(float4) * ni1);
+        o_se = r2.take(sizeof(float) * 5 * slots);
+        o_ss = r2.take(sizeof(float) * PTH_SPJ_STAGED * recs);
+        o_pa = r2.take(sizeof(double4) * 64 * parts);
+        o_pn = r2.take(sizeof(int) * 64 * parts);
+        o_il = r2.take(df ? sizeof(float4) * ni1 : 0);
+        o_el = r2.take(df ? sizeof(float) * (PTH_DF_EXTRA / 8) * slots : 0);
+        Carve r3{persist};
+        o_acc = r3.take(24 * (size_t)ni1), o_pot = r3.take(8 * (size_t)ni1), o_nnb64 = r3.take(8 * (size_t)ni1);
+        need = std::max(r1.off, std::max(r2.off, r3.off));
+        return true;
+    };
+    // a plan for the device takes its tables along (32 bytes per walk and
+    // more): an evaluation that only they keep out of the array is planned here
+    bool planned = lay_out(true);
+    if (planned && need > (size_t)PTH_NOALLOC_SCRATCH_BYTES && P.on_device) planned = lay_out(false);
+    if (!planned) return c->fail(PTH_ERR_CAPACITY, W + ": sizes exceed the int32 index range");
     if (need > (size_t)PTH_NOALLOC_SCRATCH_BYTES)
         return c->fail(PTH_ERR_CAPACITY, W + ": the evaluation needs " + std::to_string(need) +
                                              " bytes of scratch, more than its " +

@@ -5,6 +5,8 @@ second on a smaller cluster, so it runs over what the first left in the
 scratch array), with quadrupole and with monopole superparticles; and the
 errors it returns without touching the GPU (an evaluation larger than the
 scratch array, changeover mode, the plain form, an index out of range)."""
+import re
+
 import numpy as np
 import pytest
 
@@ -70,3 +72,35 @@ def test_noalloc_errors():
         with pytest.raises(sf.PthError, match=msg):
             sf.eval_noalloc_lists(c2, L)
         c2.close()
+
+
+def test_noalloc_room_does_not_depend_on_who_plans():
+    """An evaluation that fills the scratch array to within a few kilobytes
+    when the host plans it (max_ipl 4; these walks' tiles are the same at 2)
+    is not refused where the device would plan it, whose tables take more."""
+    rng = np.random.default_rng(11)
+    nw, ni, ne, n_max = 1000, 20, 40, 1900000
+    pos = rng.normal(0, 1, (n_max, 3))
+    mass, rs = np.full(n_max, 1.0 / n_max), np.full(n_max, 1e-3)
+    ide = rng.integers(0, 1000000, nw * ne)
+    n_epi, n_epj, n_spj = np.full(nw, ni), np.full(nw, ne), np.zeros(nw, int)
+
+    def call(ctx, n):
+        return sf.eval_noalloc(ctx, n_epi, n_epj, n_spj, pos[:nw * ni], rs[:nw * ni], ide, [], pos[:n], mass[:n], rs[:n],
+                               [], [], [])
+
+    host_, dev = (sf.Context(0, eps2=1e-4, rcut2=R_OUT ** 2, G=1.0, max_ipl=k) for k in (4, 2))
+    with pytest.raises(sf.PthError, match="bytes of scratch") as e:
+        call(host_, n_max)
+    need, room = (int(x) for x in re.findall(r"(\d+)[- ]bytes? ", str(e.value)))
+    n = n_max - (need - room) // 72  # 72 bytes per EPJ
+    while True:
+        try:
+            want = call(host_, n)
+            break
+        except sf.PthError:
+            n -= 16
+    print(f"[noalloc] {n} EPJ fill the array", flush=True)
+    _same(call(dev, n), want, "planned by the host for want of room")
+    for c in (host_, dev):
+        c.close()
