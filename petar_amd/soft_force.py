@@ -536,7 +536,8 @@ class Resident:
         acc = np.empty((self.ni, 3))
         pot = np.empty(self.ni)
         nnb = np.empty(self.ni, np.int64)
-        pt = np.empty(self.ni if self.co else 0)
+        # (left alone by an evaluation refilled without changeover mode)
+        pt = np.zeros(self.ni if self.co else 0)
         self.ctx.check(lib().pth_resident_results(self._h, _ptr(acc, C.c_double), _ptr(pot, C.c_double),
                                                   _ptr(nnb, C.c_longlong), _ptr(pt, C.c_double) if self.co else None),
                        "pth_resident_results")

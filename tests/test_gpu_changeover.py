@@ -14,7 +14,7 @@ import numpy as np
 import pytest
 
 from oracle import oracle_py as O
-from petar_amd import soft_force as sf
+from petar_amd import host, soft_force as sf
 from tests._common import R_OUT, co_args, co_lists, nnb_check, rel_err, walk_centres
 
 pytestmark = pytest.mark.gpu
@@ -278,3 +278,28 @@ def test_co_group_members_and_artificial_particles():
     r.close()
     ctx.close()
     _check(res, ref, amb, "co group types")
+
+
+def test_results_after_changeover_mode_is_switched_off():
+    """An evaluation made in changeover mode and refilled without it has no
+    total potentials; the array stays zero, not whatever memory held."""
+    m, x, _ = host.cluster(4000, "plummer", seed=2)
+    rs = np.full(4000, 1.5 * R_OUT)
+    ctx = sf.Context(0, eps2=0.0, rcut2=R_OUT ** 2, G=1.0, changeover=1)
+    g = sf.GpuTree(ctx, x, m, rs)
+    r = sf.Resident.from_gtree(ctx, g)
+    p = ctx.get_params()
+    p.changeover = 0
+    ctx.set_params(p)
+    r.refill(g)
+    r.run()
+    junk = [np.full(4000, 7.0) for _ in range(64)]
+    del junk
+    out = r.results()
+    assert len(out) == 4 and np.all(out[3] == 0)
+    ref = sf.Resident.from_gtree(ctx, g)
+    ref.run()
+    assert all(np.array_equal(a, b) for a, b in zip(out[:3], ref.results()))
+    for o in (ref, r, g):
+        o.close()
+    ctx.close()
