@@ -1405,8 +1405,11 @@ __global__ __launch_bounds__(256) void k_results(const double4 *__restrict__ acc
 // search in LDS and is written coalesced.  Bound by the link (1.6 MB of runs
 // per 200-walk batch of the 1,048,576-particle cluster; against copying the
 // runs together and uploading them first, that cluster's hooks 20.2 to 19.3
-// ms).
+// ms).  A list of few runs (at most EXPAND_FEW, 512 bytes for every part to
+// read) is shared out by entries instead: there are too few runs to go round,
+// and one may hold the whole list.
 #define EXPAND_RUNS 1024
+#define EXPAND_FEW 64
 __global__ __launch_bounds__(256) void k_expand_runs(const WalkDev *__restrict__ walks, int n_walk, int n_part,
                                                      const int *__restrict__ rid_e, const int *__restrict__ rpos_e,
                                                      const int *__restrict__ n_re, const int *__restrict__ rid_s,
@@ -1423,7 +1426,10 @@ __global__ __launch_bounds__(256) void k_expand_runs(const WalkDev *__restrict__
     const int *__restrict__ rid = (sp ? rid_s : rid_e) + off;
     const int *__restrict__ rpos = (sp ? rpos_s : rpos_e) + off;
     int *__restrict__ out = (sp ? out_s : out_e) + off;
-    const int r0 = (int)((long long)nr * part / n_part), r1 = (int)((long long)nr * (part + 1) / n_part);
+    const bool few = nr <= EXPAND_FEW;
+    const int r0 = few ? 0 : (int)((long long)nr * part / n_part);
+    const int r1 = few ? nr : (int)((long long)nr * (part + 1) / n_part);
+    const int q0 = few ? (int)((long long)n * part / n_part) : 0, q1 = few ? (int)((long long)n * (part + 1) / n_part) : n;
     const int tid = (int)threadIdx.x;
     for (int c0 = r0; c0 < r1; c0 += EXPAND_RUNS) {
         const int nc = min(EXPAND_RUNS, r1 - c0);
@@ -1433,8 +1439,8 @@ __global__ __launch_bounds__(256) void k_expand_runs(const WalkDev *__restrict__
             l_pos[k] = c0 + k < nr ? rpos[c0 + k] : n;
         }
         __syncthreads();
-        const int p1 = l_pos[nc];
-        for (int k = l_pos[0] + tid; k < p1; k += 256) {
+        const int p1 = min(l_pos[nc], q1);
+        for (int k = max(l_pos[0], q0) + tid; k < p1; k += 256) {
             int lo = 0, hi = nc - 1;
             while (lo < hi) {
                 const int mid = (lo + hi + 1) >> 1;

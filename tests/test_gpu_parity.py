@@ -959,3 +959,49 @@ def test_segments_on_one_stream(c1, graph):
         r.close()
         ctx.close()
     assert all(np.array_equal(x, y) for o in out[1:] for x, y in zip(out[0], o))
+
+
+@pytest.mark.parametrize("nw", [1, 3, 200])
+def test_lists_of_few_and_many_runs(nw, monkeypatch):
+    """Lists of one run, of as many as are shared out by entries and of more
+    (shared out by runs, in one pass over them and in two), also with a run
+    that holds most of the list: the same results as from the lists."""
+    rng = np.random.default_rng(nw)
+    n, ns = 60000, 5000
+    epj, spj = np.zeros(n, sf.EPJ_SOFT), np.zeros(ns, sf.SPJ_SOFT)
+    epj["id"], epj["pos"], epj["mass"] = np.arange(n), rng.normal(0, 1, (n, 3)), rng.uniform(1, 2, n) / n
+    epj["r_search"] = 0.02
+    spj["pos"], spj["mass"] = rng.normal(0, 1, (ns, 3)) + 4.0, 1.0 / ns
+    epi = np.zeros(70, sf.EPI_SOFT)
+    epi["pos"], epi["r_search"] = epj["pos"][:70], 0.02
+
+    def list_of(k, n_tot, longest):
+        # k runs with gaps between them, one of them `longest` entries longer
+        m = rng.integers(1, 4, k)
+        m[rng.integers(k)] += longest
+        first = np.cumsum(np.concatenate([[0], m[:-1] + 2]))
+        assert first[-1] + m[-1] <= n_tot
+        return np.concatenate([np.arange(f, f + q) for f, q in zip(first, m)]).astype(np.int32)
+
+    ks = [1, 2, 7, 8, 63, 64, 65, 66, 511, 1024, 1025, 9000]
+    ide = [list_of(ks[w % len(ks)], n, int(rng.choice([0, 255, 20000]))) for w in range(nw * (12 if nw < 200 else 1))]
+    ids = [list_of(ks[(w + 5) % 9], ns, int(rng.choice([0, 1000]))) for w in range(len(ide))]
+    out = []
+    for form in ("0", "1"):
+        monkeypatch.setenv("PTH_LIST_RUNS", form)
+        sf.CalcForceWithLinearCutoffMultiWalk.close_contexts()
+        f = sf.CalcForceWithLinearCutoffMultiWalk(0, 1e-6, R_OUT ** 2, 1.0)
+        f(0, 0, [], [], [], [], [], [], epj, n, spj, ns, True)
+        got = []
+        for b in range(0, len(ide), nw):
+            e, s = ide[b:b + nw], ids[b:b + nw]
+            force = [np.zeros(70, sf.FORCE_SOFT) for _ in e]
+            ni = np.full(len(e), 70, np.int32)
+            f(0, len(e), [epi] * len(e), ni, e, np.array([len(x) for x in e], np.int32), s,
+              np.array([len(x) for x in s], np.int32), None, 0, None, 0, False)
+            f.retrieve(0, len(e), ni, force)
+            got += force
+        out.append(np.concatenate(got))
+    monkeypatch.delenv("PTH_LIST_RUNS")
+    sf.CalcForceWithLinearCutoffMultiWalk.close_contexts()
+    assert all(np.array_equal(out[0][k], out[1][k]) for k in ("acc", "pot", "n_ngb"))
