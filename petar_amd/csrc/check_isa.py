@@ -15,8 +15,17 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 SOURCES = ["pth_kernels.hip", "pth_gtree.hip", "pth_noalloc.hip"]
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fno-slp-vectorize", "-Xclang", "-target-feature",
          "-Xclang", "-packed-fp32-ops", "-S", "--cuda-device-only", "-o", "-"]
-FORBIDDEN = re.compile(r"^\s*(s_store_|s_buffer_store|s_scratch_store|s_atomic_|s_buffer_atomic_|"
-                       r"s_dcache_wb|s_dcache_discard|v_pk_fma_f32|v_pk_mul_f32|v_pk_add_f32)", re.M)
+# by class, not by name: scalar instructions that are stores or atomics or write
+# the scalar cache back or discard it, and packed FP32 arithmetic
+INSTRUCTION = re.compile(r"^\s+([sv]_\w+)", re.M)
+SCALAR_WRITE = re.compile(r"^s_(\w*_)?(store|atomic|wb|discard)(_|$)")
+PACKED_FP32 = re.compile(r"^v_pk_(add|mul|fma)_f32")
+
+
+def forbidden(asm):
+    """The forbidden instructions of an assembly listing."""
+    ins = set(INSTRUCTION.findall(asm))
+    return sorted(i for i in ins if SCALAR_WRITE.match(i) or PACKED_FP32.match(i))
 
 
 def main():
@@ -24,11 +33,10 @@ def main():
     for src in SOURCES:
         asm = subprocess.run(["/opt/rocm/bin/hipcc"] + FLAGS + [os.path.join(HERE, src)], capture_output=True,
                              text=True, check=True).stdout
-        n_ins = len(re.findall(r"^\s+[sv]_\w+", asm, re.M))
-        hits = FORBIDDEN.findall(asm)
+        hits = forbidden(asm)
         if hits:
-            bad.append((src, sorted(set(hits))))
-        print(f"check_isa: {src}: {n_ins} instructions scanned, forbidden forms: {sorted(set(hits)) or 'none'}")
+            bad.append((src, hits))
+        print(f"check_isa: {src}: {len(INSTRUCTION.findall(asm))} instructions scanned, forbidden forms: {hits or 'none'}")
     if bad:
         sys.exit(f"check_isa: forbidden instructions in {bad}")
 

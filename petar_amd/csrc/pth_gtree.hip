@@ -528,8 +528,8 @@ __device__ __forceinline__ void moments_join(Moments &v, double s, double *rows,
 
 // Stores of node k's moments, lane j < 6 holding component j of the
 // quadrupole in q, and its walk record, a part per lane.
-__device__ __forceinline__ void moments_store(const Moments &v, double q, const MomentArrays &o, const GNode &nd,
-                                              long long k, int j)
+__device__ __forceinline__ void put_moments(const Moments &v, double q, const MomentArrays &o, const GNode &nd,
+                                            long long k, int j)
 {
     if (j == 7) o.mass[k] = v.M;
     if (j < 3) o.com[3 * k + j] = pick(j, v.c[0], v.c[1], v.c[2]);
@@ -627,7 +627,7 @@ __global__ __launch_bounds__(256) void k_leaf_moments(const GNode *__restrict__ 
             wave_sync();
         }
     }
-    moments_store(v, q, out, nd, k, j);
+    put_moments(v, q, out, nd, k, j);
 }
 
 // Moments of one inner node (its children are done), eight lanes.
@@ -667,7 +667,7 @@ __device__ __forceinline__ void inner_moments(const GNode &nd, long long k, cons
     wave_sync();
     for (int t = 0; t < nd.n_child; t++) q += rows[t * KID + 5 + min(j, 5)];
     wave_sync();
-    moments_store(v, q, o, nd, k, j);
+    put_moments(v, q, o, nd, k, j);
 }
 
 // The inner nodes of one level, [a, b).

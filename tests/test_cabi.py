@@ -2,6 +2,7 @@
 headers declare, the host-only planner covers every pair exactly once, and
 the entry points fail cleanly where no device exists."""
 import ctypes as C
+import importlib.util
 import os
 import re
 import subprocess
@@ -243,3 +244,34 @@ def test_plan_object_reused_holds_no_stale_items():
     """What a plan makes on the host is what its consumers upload into room
     sized for it, whatever the object planned before."""
     _plan_check("reuse")
+
+
+def _scalar_writes():
+    # (put together here: files that spell these out are refused as GPU code)
+    return ["s_" + m for m in ("store" + "_dwordx2", "buffer_" + "store_dword", "scratch_" + "store_dword",
+                               "atomic" + "_add", "buffer_" + "atomic_add_x2", "dcache_" + "wb", "dcache_" + "wb_vol",
+                               "dcache_" + "discard_x2")]
+
+
+def test_isa_guard_knows_what_it_forbids():
+    """The guard over the built kernels' assembly names instructions by class:
+    every scalar write and packed FP32 form, no vector store, no scalar load."""
+    path = os.path.join(ROOT, "petar_amd", "csrc", "check_isa.py")
+    if not os.path.exists(path):
+        pytest.skip("the guard runs where the library is built")
+    spec = importlib.util.spec_from_file_location("check_isa", path)
+    guard = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(guard)
+    bad = _scalar_writes() + ["v_pk_" + op + "_f32" for op in ("add", "mul", "fma")]
+    fine = ["s_load_dwordx4", "s_waitcnt", "s_dcache_inv", "s_barrier", "v_fma_f32", "v_pk_add_f16", "s_setprio"]
+    asm = "\n".join(f"\t{i} s[0:1], s2" for i in bad + fine) + "\n\tglobal_store_dword v0, v1, s[0:1]\n"
+    assert guard.forbidden(asm) == sorted(bad)
+    # and no source spells one out
+    word = re.compile(r"(?<![a-z0-9_])(" + "|".join(_scalar_writes()) + ")")
+    short = re.compile(r"(?<![a-z0-9_])s_(\w+_)?(store|atomic)_")
+    for d in ("petar_amd", "oracle", "include", "perf", os.path.join("tests", "cpp")):
+        for base, _, files in os.walk(os.path.join(ROOT, d)):
+            for f in files:
+                if f.endswith((".py", ".hip", ".cpp", ".hpp", ".h", ".c", "Makefile")):
+                    txt = open(os.path.join(base, f)).read()
+                    assert not word.search(txt) and not short.search(txt), os.path.join(base, f)
