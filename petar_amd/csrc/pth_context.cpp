@@ -670,7 +670,7 @@ int pth_dispatch(pth_ctx *c, int tag, int n_walk, const void *const *epi, const 
     // i-per-lane class than the chip has slots: each class launch is one
     // latency-bound round, so the 1-i items run on a second stream beside
     // the longer classes instead of after them
-    const bool split = c->class_streams && !b.plain && !split_launch(b, 0) && P.seg_count[0] > 0 &&
+    const bool split = c->class_streams && !b.plain && !split_launch(b) && P.seg_count[0] > 0 &&
                        P.seg_count[1] + P.seg_count[2] + P.seg_count[3] > 0;
     if (split) {
         if (!c->side) HIPCHK(c, hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking), "hipStreamCreate");
@@ -998,7 +998,7 @@ static int resident_enqueue(pth_resident *r, hipStream_t st, hipEvent_t fork_ev,
         // classes (the 1-i launch is about one round of waves, whose run-down
         // tail the longer launch then fills)
         const SegDev &g0 = r->b.seg[0];
-        const bool split = r->b.n_seg == 1 && c->class_streams && !r->b.plain && !split_launch(r->b, 0) &&
+        const bool split = r->b.n_seg == 1 && c->class_streams && !r->b.plain && !split_launch(r->b) &&
                            !r->side.empty() &&
                            !r->staged.empty() && g0.seg_count[0] > 0 &&
                            g0.seg_count[1] + g0.seg_count[2] + g0.seg_count[3] > 0;
@@ -1039,7 +1039,7 @@ static int resident_enqueue(pth_resident *r, hipStream_t st, hipEvent_t fork_ev,
         // beside its longer classes: nothing else is left to fill its tail
         const SegDev &g = r->b.seg[k];
         const bool split = k == r->b.n_seg - 1 && c->class_streams && !r->b.plain &&
-                           !split_launch(r->b, k) &&
+                           !split_launch(r->b) &&
                            g.seg_count[0] > 0 && g.seg_count[1] + g.seg_count[2] + g.seg_count[3] > 0;
         if (split) {
             HIPCHK(c, launch_force(r->b, k, fs, 0xEu), "force kernel");

@@ -222,9 +222,9 @@ hipError_t launch_plan(const WalkDev *walks, const WalkPlan *wplan, int n_walk, 
 
 // Launches of segment k of a batch (k < b.n_seg).
 hipError_t launch_stage(const BatchDev &b, int k, hipStream_t st);
-// Whether segment k's items run a quarter per wave, classes 1 and 2 together
+// Whether the segments' items run a quarter per wave, classes 1 and 2 together
 // (launch_force then launches them with bit 1 of classes).
-bool split_launch(const BatchDev &b, int k);
+bool split_launch(const BatchDev &b);
 // classes: bit c set launches the items of i-per-lane class c + 1
 hipError_t launch_force(const BatchDev &b, int k, hipStream_t st, unsigned classes = 0xFu);
 hipError_t launch_reduce(const BatchDev &b, int k, hipStream_t st);

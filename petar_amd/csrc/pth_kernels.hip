@@ -1607,21 +1607,35 @@ static unsigned fit_blocks(const void *f)
     return (unsigned)(it->second * cus[dev]);
 }
 
-// Whether segment k's force launch takes an item per workgroup (and both
+// Whether a batch's force launches take an item per workgroup (and both
 // i-per-lane classes at once).  A launch ends with its longest items, and one
 // of a few rounds of waves (8,192 slots) is much of it tail: quarters of items
 // shorten that.  Against that stand the four loads of a tile's i and a
-// barrier.  us per evaluation, a wave against a workgroup per item, by items
-// of a launch: 1,702 (16,384 particles) 259 and 204; 20,000 (262,144) 2,795
-// and 2,540; 37,000 (524,288) 5,700 and 5,030; 29,000 (1,048,576) 10,550 and
-// 10,220; 57,000 (2M) 20,700 and 20,370; 124,000 (4,194,304) 43,050 and
-// 43,830.  The kernel holds 1 and 2 i per lane.
-constexpr int SPLIT_MAX_ITEMS = 65536;
-bool split_launch(const BatchDev &b, int k)
+// barrier, which other segments' launches beside it do not need: they fill the
+// tail.  The changeover kernels wait more than they issue and gain longer.
+// Decided by the largest segment, for all: with the first, half-size one
+// split and the others not, 2,000,000 particles took 22.1 ms, where either
+// form alone takes 21.75 and 22.0.  ms per evaluation, a wave against a
+// workgroup per item, by items of the largest launch:
+//   one segment: 1,641 0.219 and 0.142; 31,000 1.420 and 1.358; 57,000 2.507
+//     and 2.495; 79,000 3.45 and 3.47; 124,000 5.38 and 5.50
+//   eight on three streams: 24,000 7.83 and 7.59; 35,000 11.11 and 11.10;
+//     43,000 13.45 and 13.48; 52,000 15.88 and 16.03; 109,000 33.24 and 33.89
+//   changeover, one: 57,000 2.79 and 2.61; 124,000 5.78 and 5.73; 182,000 8.74
+//     and 8.77; 392,000 16.7 and 17.1
+//   changeover, eight: 35,000 11.86 and 11.38; 72,000 22.03 and 21.49; 147,000
+//     45.4 and 44.6
+// The kernel holds 1 and 2 i per lane.
+constexpr int SPLIT_ITEMS = 65536, SPLIT_ITEMS_SEGMENTS = 40960, SPLIT_ITEMS_CO = 163840;
+bool split_launch(const BatchDev &b)
 {
-    const SegDev &g = b.seg[k];
-    return !b.plain && !b.persistent && !b.j_vgpr && g.seg_count[2] + g.seg_count[3] == 0 &&
-           g.seg_count[0] + g.seg_count[1] <= SPLIT_MAX_ITEMS;
+    if (b.plain || b.persistent || b.j_vgpr) return false;
+    const int limit = b.co ? SPLIT_ITEMS_CO : b.n_seg > 1 ? SPLIT_ITEMS_SEGMENTS : SPLIT_ITEMS;
+    for (int k = 0; k < b.n_seg; k++) {
+        const SegDev &g = b.seg[k];
+        if (g.seg_count[2] + g.seg_count[3] > 0 || g.seg_count[0] + g.seg_count[1] > limit) return false;
+    }
+    return true;
 }
 
 // nblk blocks of one item per wave; persistent (P): as many blocks as the
@@ -1691,7 +1705,7 @@ hipError_t launch_force(const BatchDev &b, int k, hipStream_t st, unsigned class
     a.part_accp = b.part_accp;
     a.part_nnb = b.part_nnb;
     a.part_pott = b.part_pott;
-    if (split_launch(b, k)) {
+    if (split_launch(b)) {
         if (!(classes & 2u)) return hipSuccess;  // both classes go with the 2-i launch
         a.items = b.items + g.seg_begin[1];
         a.n_items = g.seg_count[1];

@@ -11,7 +11,7 @@ import pytest
 
 from oracle import oracle_py as O
 from petar_amd import host, soft_force as sf
-from tests._common import R_OUT, c1_lists, nnb_check, rel_err, walk_centres
+from tests._common import R_OUT, c1_lists, co_lists, nnb_check, rel_err, walk_centres
 
 pytestmark = pytest.mark.gpu
 
@@ -1005,3 +1005,28 @@ def test_lists_of_few_and_many_runs(nw, monkeypatch):
     monkeypatch.delenv("PTH_LIST_RUNS")
     sf.CalcForceWithLinearCutoffMultiWalk.close_contexts()
     assert all(np.array_equal(out[0][k], out[1][k]) for k in ("acc", "pot", "n_ngb"))
+
+
+@pytest.mark.parametrize("co,segments,chunk", [(0, 1, 36), (0, 1, 32), (0, 2, 36), (0, 2, 32), (1, 1, 16), (1, 1, 12),
+                                               (1, 2, 12), (1, 2, 8)])
+def test_split_rule_both_sides(co, segments, chunk):
+    """Evaluations just below and above the item counts up to which launches
+    run an item per workgroup (decided for all segments by the largest): the
+    bits of persistent launches, which run an item per wave."""
+    if co:
+        L, rin, rout = co_lists(20000, seed=4)
+    else:
+        L = c1_lists(20000, seed=4)
+    out, n_items = [], []
+    for persistent in (0, 1):
+        ctx = sf.Context(0, eps2=0.0, rcut2=R_OUT ** 2, G=1.0, segments=segments, streams=3, min_seg_pairs=1,
+                         chunk_j=chunk, changeover=co, persistent=persistent)
+        r = sf.Resident.from_lists(ctx, L, rin, rout) if co else sf.Resident.from_lists(ctx, L)
+        r.run()
+        out.append(r.results())
+        n_items.append(r.stats()["n_items"])
+        r.close()
+        ctx.close()
+    limit = 163840 if co else 65536 if segments == 1 else 40960
+    print(f"[split rule co={co} segments={segments} chunk={chunk}] {n_items[0]} items, limit {limit} per launch", flush=True)
+    assert all(np.array_equal(a, b) for a, b in zip(*out))
