@@ -485,8 +485,10 @@ int pth_dispatch(pth_ctx *c, int tag, int n_walk, const void *const *epi, const 
     const bool encode = c->list_runs != 0;
     const int nj_lim = c->n_epj, ns_lim = c->n_spj;
     if (encode) {
-        // (16 more: the encoder stores whole vectors)
-        const size_t bytes = sizeof(int) * (size_t)(n_ide + n_ids + 16);
+        // (a walk's runs go where its list would; the encoder writes nothing
+        // outside a walk's own entries, which the threads beside it and the
+        // device, reading the runs in place, depend on)
+        const size_t bytes = sizeof(int) * (size_t)std::max<long long>(n_ide + n_ids, 1);
         HIPCHK(c, c->h_rid.ensure(bytes), "pinned list allocation");
         HIPCHK(c, c->h_rpos.ensure(bytes), "pinned list allocation");
     }

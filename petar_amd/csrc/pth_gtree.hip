@@ -13,13 +13,14 @@
 //      level in Morton order (so children follow their parents' order), with
 //      one wait for the host (the counts) in the whole build;
 //   3. moments bottom-up (mass, centre of mass, raw second moment about it,
-//      particle box and box widened by r_search), each node by one thread in
+//      particle box and box widened by r_search), each node by eight lanes in
 //      the host's summation order;
 //   4. i-groups: largest cells with at most n_group_limit particles (or
 //      leaves), in Morton order (decided and counted with the nodes, as are
 //      the neighbour search's tiles of at most 64);
-//   5. walk: one wave per group traverses the tree with a stack in LDS,
-//      popping up to 64 nodes at a time; a node is opened when it contains
+//   5. walk: one wave per group (four of up to WALK_WIDE groups) traverses the
+//      tree with a stack in LDS, popping up to 64 (256) nodes at a time; a node
+//      is opened when it contains
 //      the group, when the group box is closer to its centre of mass than
 //      L/theta, or when the boxes overlap with either side widened by
 //      r_search; opened leaves go to the group's leaf list, closed nodes to
@@ -321,11 +322,9 @@ __global__ __launch_bounds__(64) void k_tree_sizes(const int *__restrict__ off, 
     const int r = threadIdx.x;
     if (r <= ROW_NODES) meta->level_start[r] = off[(size_t)r * nblk];
     if (r == 0) {
-        const int nn = off[(size_t)ROW_NODES * nblk], g0 = off[(size_t)ROW_GROUPS * nblk],
-                  t0 = off[(size_t)ROW_TILES * nblk];
+        const int g0 = off[(size_t)ROW_GROUPS * nblk], t0 = off[(size_t)ROW_TILES * nblk];
         meta->n_group = t0 - g0;
         meta->n_tile = off[(size_t)N_ROWS * nblk] - t0;
-        (void)nn;
     }
 }
 

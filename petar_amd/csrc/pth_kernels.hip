@@ -1457,8 +1457,11 @@ __global__ __launch_bounds__(256) void k_expand_runs(const WalkDev *__restrict__
 // The work items of a plan whose sizes the host made (make_plan with
 // on_device): block b < n_walk writes walk b's items and reduction items,
 // block n_walk + g the empty slots behind the runs of segment g.  A run's
-// items are in walk order (the host's planner puts the most expensive first;
-// their costs differ by at most a factor of two, chunks being of equal size).
+// items are in walk order, where the host's planner puts the most expensive
+// first: the items of walks of several chunks differ by at most a factor of
+// two in cost; those of walks of one chunk may be much cheaper, and of such
+// the order saved nothing (4,194,304 particles' force phase 37.86 ms in walk
+// order, 37.79 in the host's).
 __global__ __launch_bounds__(64) void k_plan(const WalkDev *__restrict__ walks, const WalkPlan *__restrict__ wplan,
                                              int n_walk, const SegPlan *__restrict__ splan,
                                              const long long *__restrict__ es_off,

@@ -10,7 +10,8 @@
 // whatever batch it is part of.  Items are then dealt to the 8 XCDs as 8
 // contiguous runs of equal total cost (neighbouring items share walks,
 // hence staged lists, so each list is fetched into one XCD's L2), most
-// expensive first inside each run, and written in the order the hardware
+// expensive first inside each run (plans left to the device: in walk order),
+// and written in the order the hardware
 // hands workgroups to XCDs (round robin), padding short runs with empty
 // items.  With several segments (contiguous walk ranges of equal cost, the
 // first of half that, pipelined over several streams) the dealing is done
