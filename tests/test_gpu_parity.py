@@ -6,6 +6,8 @@ maximum <= 1e-3 (relative errors of tiny net accelerations); neighbour
 counts exact except for pairs inside the FP32 rounding band of r_search,
 where they may differ by at most the number of such pairs.
 """
+import time
+
 import numpy as np
 import pytest
 
@@ -1030,3 +1032,30 @@ def test_split_rule_both_sides(co, segments, chunk):
     limit = 163840 if co else 65536 if segments == 1 else 40960
     print(f"[split rule co={co} segments={segments} chunk={chunk}] {n_items[0]} items, limit {limit} per launch", flush=True)
     assert all(np.array_equal(a, b) for a, b in zip(*out))
+
+
+def test_transfers_leave_no_spinning_threads():
+    """The threads that copy results and neighbour lists to the caller's arrays
+    sleep soon after: a program that reads results and waits for 100 ms uses
+    no cores meanwhile."""
+    n = 300000
+    m, x, _ = host.cluster(n, "plummer", seed=3)
+    ctx = sf.Context(0, eps2=0.0, rcut2=1e-6)
+    g = sf.GpuTree(ctx, x, m, np.full(n, 1e-3), theta=0.9)
+    r = sf.Resident.from_gtree(ctx, g)
+    r.run()
+    srv = sf.Server(ctx, sf.SERVE_FUSED)
+    k = srv.add_lists(host.build_lists(x[:60000], m[:60000], 1e-3, theta=0.9))
+    srv.wait(srv.submit(k))
+    for what, call in (("results", r.results), ("neighbours", g.neighbors), ("server", lambda: srv.results(k))):
+        time.sleep(0.4)  # (other parallel regions' threads)
+        call()
+        time.sleep(0.01)
+        used = time.process_time()
+        time.sleep(0.1)
+        used = time.process_time() - used
+        print(f"[threads after {what}] {used * 1e3:.1f} ms of processor time in 100 ms", flush=True)
+        assert used < 0.05, what
+    for o in (srv, r, g):
+        o.close()
+    ctx.close()
