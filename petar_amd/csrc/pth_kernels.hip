@@ -985,19 +985,48 @@ __device__ __forceinline__ void store_sums(const ForceArgs &a, const Item &it, i
 // Ends the quarters of an item that one wave takes: the sums up to each cut
 // go to LDS (T, this wave's n_sum IPL rows of 64; in registers they would
 // cost the 2-i kernel a wave per SIMD).  `at` is the next cut among the
-// blocks (records, after records()).
+// blocks (records, after records()).  Scalar registers are short all through
+// the j loops, so the cuts are not held in any: the changeover kernels leave
+// them in LDS (C), the others work them out again from the item (3,000,000
+// particles in changeover mode, pipelined, 33.57 ms with the item read again
+// and 33.15 with the cuts in LDS; 4,194,304 without, force phase 37.6 and 37.85).
 template <int IPL, bool CO> struct Quarters {
     static constexpr int NC = n_sum<CO>;
     const ForceArgs &a;
     int idx, k, at;
     bool first;
     double *T;
+    int *C;
     double (&A)[IPL][4], (&PT)[IPL];
+    __device__ __forceinline__ void start(const Item &it, int near_end)
+    {
+        if constexpr (CO)
+            for (int q = 1; q < 4; q++) {
+                const Cut c = cut_at(it, near_end, q);
+                C[q] = c.in_e ? c.e : ~c.s;
+            }
+        next(it.e_blk_begin, false);
+    }
     // the next cut after position pos (of the blocks or, with rec, records)
     __device__ __forceinline__ void next(int pos, bool rec)
     {
-        // (the item is read again: its words would take scalar registers all
-        // through the j loops, which need every one)
+        if constexpr (CO) {
+            at = INT_MAX;
+#pragma unroll 1
+            for (; k < 4; k++) {
+                const int v = uniform(C[k]);
+                if ((v >= 0) == rec) {
+                    if (!rec) break;  // the cuts left are among the records
+                    continue;
+                }
+                const int c = rec ? ~v : v;
+                if (c > pos) {
+                    at = c;
+                    break;
+                }
+            }
+            return;
+        }
         asm volatile("" : "+s"(idx));
         const Item it = load_item(a.items, idx);
         const int near_end = ((cip)(a.near_blk))[it.walk];
@@ -1005,7 +1034,7 @@ template <int IPL, bool CO> struct Quarters {
         for (; k < 4; k++) {
             const Cut c = cut_at(it, near_end, k);
             if (c.in_e == rec) {
-                if (!rec) break;  // the cuts left are among the records
+                if (!rec) break;
                 continue;
             }
             if ((rec ? c.s : c.e) > pos) {
@@ -1065,7 +1094,7 @@ struct NoQuarters {
 
 // One item by one wave.
 template <int IPL, int NNB_LE, bool VC, bool CO, bool DF>
-__device__ __forceinline__ void run_tile(const ForceArgs &a, int idx, int lane, const Consts &K, double *T)
+__device__ __forceinline__ void run_tile(const ForceArgs &a, int idx, int lane, const Consts &K, double *T, int *C)
 {
     Tile<IPL> t;
     double A[IPL][4], PT[IPL];
@@ -1078,9 +1107,10 @@ __device__ __forceinline__ void run_tile(const ForceArgs &a, int idx, int lane, 
     const Item it = load_item(a.items, idx);
     if (it.walk < 0) return;  // an empty slot
     load_tile<IPL, CO, DF>(a, it, lane, t);
-    const int e_mid = min(max(((cip)(a.near_blk))[it.walk], it.e_blk_begin), it.e_blk_end);
-    Quarters<IPL, CO> end{a, idx, 1, 0, true, T, A, PT};
-    end.next(it.e_blk_begin, false);
+    const int near_end = ((cip)(a.near_blk))[it.walk];
+    const int e_mid = min(max(near_end, it.e_blk_begin), it.e_blk_end);
+    Quarters<IPL, CO> end{a, idx, 1, 0, true, T, C, A, PT};
+    end.start(it, near_end);
     sum_range<IPL, NNB_LE, VC, CO, DF>(end, a, t, it.e_blk_begin, e_mid, it.e_blk_end, it.s_begin, it.s_end, K, A, PT,
                                        nnb);
     end.finish();
@@ -1150,10 +1180,10 @@ __device__ __forceinline__ void run_tile_split(const ForceArgs &a, const Item *i
 
 // Work item idx of this class's launch (empty slots have walk < 0).
 template <int NNB_LE, int IPL, bool VC, bool CO, bool DF>
-__device__ __forceinline__ void force_item(const ForceArgs &a, int idx, double *T)
+__device__ __forceinline__ void force_item(const ForceArgs &a, int idx, double *T, int *C)
 {
     const Consts K{jv<VC>(a.eps2), jv<VC>(a.rout2), jv<VC>(0.5f), jv<VC>(2.5f)};
-    run_tile<IPL, NNB_LE, VC, CO, DF>(a, idx, threadIdx.x & 63, K, T);
+    run_tile<IPL, NNB_LE, VC, CO, DF>(a, idx, threadIdx.x & 63, K, T, C);
 }
 
 // One launch per i-per-lane class: items [0, n_items) of this class, one
@@ -1165,7 +1195,10 @@ template <int NNB_LE, int IPL, bool VC, bool CO, bool DF, bool P>
 __device__ __forceinline__ void force_items(const ForceArgs &a)
 {
     __shared__ double sums[4 * IPL * n_sum<CO> * 64];
-    double *T = sums + (size_t)uniform((int)threadIdx.x >> 6) * (IPL * n_sum<CO> * 64);
+    __shared__ int cuts[4][4];  // (changeover mode)
+    const int wave = uniform((int)threadIdx.x >> 6);
+    double *T = sums + (size_t)wave * (IPL * n_sum<CO> * 64);
+    int *C = cuts[wave];
     if constexpr (P) {
         const int x = (int)blockIdx.x & 7;
         int *cnt = a.counter + x;
@@ -1174,12 +1207,12 @@ __device__ __forceinline__ void force_items(const ForceArgs &a)
             if ((threadIdx.x & 63) == 0) k = atomicAdd(cnt, 1);
             k = uniform(k);
             if (k >= a.n_run) break;
-            force_item<NNB_LE, IPL, VC, CO, DF>(a, ((k >> 2) * 8 + x) * 4 + (k & 3), T);
+            force_item<NNB_LE, IPL, VC, CO, DF>(a, ((k >> 2) * 8 + x) * 4 + (k & 3), T, C);
         }
     } else {
         const int idx = uniform((int)blockIdx.x * 4 + ((int)threadIdx.x >> 6));
         if (idx >= a.n_items) return;
-        force_item<NNB_LE, IPL, VC, CO, DF>(a, idx, T);
+        force_item<NNB_LE, IPL, VC, CO, DF>(a, idx, T, C);
     }
 }
 
