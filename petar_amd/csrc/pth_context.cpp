@@ -1380,6 +1380,22 @@ struct ShortSpin {
     ShortSpin(const ShortSpin &) = delete;
 };
 
+// Threads that copy a chunk of n results, or of `bytes`.
+static int result_threads(long long n) { return (int)std::min<long long>(omp_get_max_threads(), n / 4096); }
+static int copy_threads(size_t bytes)
+{
+    return (int)std::max<size_t>(1, std::min<size_t>(omp_get_max_threads(), bytes >> 17));
+}
+
+// Wakes the threads that the next parallel region of t will use, while the
+// device still works: sleeping ones would cost a transfer 15 to 50 us.
+static void wake_threads(int t)
+{
+    if (t < 2) return;
+#pragma omp parallel num_threads(t)
+    asm volatile("");
+}
+
 void unpack_results(const char *src, long long n, bool co, double *acc, double *pot, long long *nnb, double *pot_tot)
 {
     const double *a = reinterpret_cast<const double *>(src), *p = a + 3 * n, *pt = p + n;
@@ -1393,7 +1409,7 @@ void unpack_results(const char *src, long long n, bool co, double *acc, double *
     };
     // the caller's arrays are often fresh memory: the copy is mostly page
     // faults, which threads take side by side
-    const int t = (int)std::min<long long>(omp_get_max_threads(), n / 4096);
+    const int t = result_threads(n);
     if (t < 2) {
         part(0, n);
         return;
@@ -1455,13 +1471,14 @@ hipError_t copy_to_host(hipStream_t st, ResultRings &rings, const std::vector<Ho
     };
     for (size_t k = 0; k < part.size() && k < RESULT_RING; k++)
         if ((e = start(k))) return e;
+    if (!part.empty()) wake_threads(copy_threads(part[0].bytes));
     for (const HostCopy &c : pieces)
         if (c.dst) map_pages(c.dst, c.bytes);
     for (size_t k = 0; k < part.size(); k++) {
         if ((e = hipEventSynchronize(ring.ev[k % RESULT_RING]))) return e;
         const char *src = ring.buf[k % RESULT_RING].as<char>();
         const size_t n = part[k].bytes;
-        const int t = (int)std::max<size_t>(1, std::min<size_t>(omp_get_max_threads(), n >> 17));
+        const int t = copy_threads(n);
 #pragma omp parallel for num_threads(t) schedule(static, 1) if (t > 1)
         for (int q = 0; q < t; q++)
             std::memcpy((char *)part[k].dst + n * q / t, src + n * q / t, n * (q + 1) / t - n * q / t);
@@ -1505,6 +1522,7 @@ hipError_t results_to_host(hipStream_t st, ResultRings &rings, const double4 *ac
     for (long long k = 0; k < nb; k++)
         if ((e = pack(k))) return e;
     // (while the evaluation is still running)
+    wake_threads(result_threads(count(0)));
     map_pages(acc, 24 * (size_t)n);
     map_pages(pot, 8 * (size_t)n);
     map_pages(nnb, 8 * (size_t)n);
