@@ -855,8 +855,8 @@ __device__ __forceinline__ Item load_item(const Item *items, int idx)
 // the quarters in turn and four waves that take one each give the same bits,
 // and a launch is free to do either.  A wave that takes all four pays for
 // them: force phase of 4,194,304 particles at chunk 1024 37.3 to 37.6 ms,
-// changeover 30.1 to 30.75 (3,000,000); of 8,388,608 at chunk 2048 with 3 i per
-// lane nothing in one segment, 0.5 of 89 ms pipelined.
+// changeover 30.3 to 30.65 (3,000,000); of 8,388,608 with 3 i per lane nothing
+// in one segment, 0.8 of 89.3 ms pipelined, changeover 1.4 of 95.3.
 struct Cut {
     bool in_e;  // among the EPJ blocks (at most their end), or the SPJ records
     int e, s;   // blocks before e and records before s come before the cut
